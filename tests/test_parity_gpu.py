@@ -109,6 +109,31 @@ def test_dequantize_bit_exact(gpu, oracle, t, N, K):
 
 
 @pytest.mark.parametrize("t", ALL_TYPES)
+@pytest.mark.parametrize("N,K", [(3, 768), (5, 1280), (129, 4352), (1023, 2048), (1025, 2048), (8200, 4096)])
+def test_dequantize_bit_exact_around_its_chunks(gpu, oracle, t, N, K):
+    """Last chunks of 256 and 1024 quads that are partly filled; both lane widths; an output of more than 128 MB (written
+    around the caches)."""
+    W = np.tile(synth.weights(t, 15 + t, min(N, 129), K), (-(-N // 129), 1))[:N]
+    got = nn.dequantize(dev(gpu, W), t).cpu().numpy()
+    want = np.tile(oracle.c_dequantize(t, W[:129], K), (-(-N // 129), 1))[:N]
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("t", ALL_TYPES)
+@pytest.mark.parametrize("K,count", [(256, 1), (256, 517), (768, 1), (768, 31), (1280, 40), (4096, 700), (4352, 300)])
+def test_gather_row_lengths_around_its_chunks(gpu, oracle, t, K, count):
+    """Several rows to a workgroup (under 256 quads), one row in one or several chunks, and an index out of range among them."""
+    vocab = 50
+    table = synth.weights(t, 115 + t, vocab, K)
+    idx = synth.randint(116, t, count, 0, vocab - 1).astype(np.int32).reshape(count, 1)
+    out = nn.quantized_gather(dev(gpu, table), dev(gpu, idx), Quantization(ggml_type=t)).cpu().numpy()
+    assert np.array_equal(out.view(np.uint32), oracle.c_embedding_lookup(t, table, K, idx).view(np.uint32))
+    idx[-1] = vocab
+    with pytest.raises(IndexError):
+        nn.quantized_gather(dev(gpu, table), dev(gpu, idx), Quantization(ggml_type=t))
+
+
+@pytest.mark.parametrize("t", ALL_TYPES)
 def test_dequantize_bit_exact_on_extreme_scales(gpu, oracle, t):
     """Random bytes everywhere, including the fp16 scale fields (subnormals, large values)."""
     K, N = 1024, 64
