@@ -92,6 +92,12 @@ class NotImplementedByBackend(HipqError):
 
 _lib = None
 _initialised = False
+fast = None  # the native host path (csrc/binding.cpp), bound to the loaded library by init()
+
+# Entry points the native host path calls, in the order in which csrc/binding.cpp takes them.
+_BOUND = ("gq_qdense_check", "gq_qdense_f32", "gq_qdense_bf16", "gq_qdense_block_f32", "gq_qdense_block_bf16", "gq_qdense_gated_f32",
+          "gq_qdense_gated_bf16", "gq_qdense_f32_batch", "gq_qdense_norm_f32_batch", "gq_qdense_norm_bf16_batch", "gq_dequantize",
+          "gq_embedding_lookup", "gq_row_bytes", "gq_bytes_per_block", "gq_values_per_block")
 
 
 def lib() -> ctypes.CDLL:
@@ -121,7 +127,10 @@ def check(status: int) -> None:
 
 def init(device: int = 0) -> None:
     """gq_init once per process; raises if there is no gfx950 device."""
-    global _initialised
+    global _initialised, fast
     if not _initialised:
         check(lib().gq_init(device))
+        from . import _binding
+        _binding.bind(*(ctypes.cast(getattr(lib(), name), ctypes.c_void_p).value for name in _BOUND))
+        fast = _binding
         _initialised = True

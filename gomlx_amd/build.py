@@ -18,6 +18,8 @@ OBJ = os.path.join(HERE, "csrc", "build")
 LIB = os.path.join(HERE, "libgomlx_hipq.so")
 YARDSTICK_LIB = os.path.join(HERE, "libgq_yardstick.so")  # read-only kernels for the benchmark; not part of the product library
 
+BINDING = os.path.join(HERE, "_binding.so")  # native host path of nn.py (csrc/binding.cpp)
+
 HOST = os.path.join(HERE, "host")
 HOST_TEST = os.path.join(HOST, "build", "hipq_backend_test")
 WORKSPACE_TEST = os.path.join(HOST, "build", "workspace_test")
@@ -102,8 +104,27 @@ def build(verbose: bool = True) -> str:
         raise RuntimeError(f"yardstick build failed:\n{r.stdout}\n{r.stderr}")
     if verbose:
         print(f"built {YARDSTICK_LIB}")
+    build_binding(verbose)
     build_host_test(verbose)
     return LIB
+
+
+def build_binding(verbose: bool = True) -> str:
+    """The CPython module behind nn.py (host code: g++ against torch's headers)."""
+    import sysconfig
+
+    import torch
+    T = os.path.dirname(torch.__file__)
+    inc = [os.path.join(T, "include"), os.path.join(T, "include", "torch", "csrc", "api", "include"), "/opt/rocm/include", sysconfig.get_paths()["include"]]
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-DUSE_ROCM", "-D__HIP_PLATFORM_AMD__=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *(x for i in inc for x in ("-isystem", i)),
+           os.path.join(CSRC, "binding.cpp"), "-o", BINDING, "-L" + os.path.join(T, "lib"), "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"binding build failed:\n{r.stdout}\n{r.stderr}")
+    if verbose:
+        print(f"built {BINDING}")
+    return BINDING
 
 
 def build_host_test(verbose: bool = True) -> str:

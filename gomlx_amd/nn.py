@@ -9,6 +9,10 @@ device tensors.  Names, argument meaning and error behaviour follow
 
 torch only supplies device memory and the current stream; all arithmetic runs in
 libgomlx_hipq.so.  There is no CPU path: tensors must live on the GPU.
+
+The operators of a decode loop first try the same steps in native code (``_lib.fast``,
+csrc/binding.cpp; bound when the library is initialised, so from a process's second call on);
+it returns None for whatever it does not take, and the Python steps below then run or raise.
 """
 from __future__ import annotations
 
@@ -82,6 +86,8 @@ def _weights_2d(weights: torch.Tensor) -> None:
 
 def dequantize(weights: torch.Tensor, ggml_type: int) -> torch.Tensor:
     """ggml.Dequantize: [N, bytesPerRow] uint8 -> [N, K] float32, bit-exact."""
+    if _lib.fast is not None and (out := _lib.fast.dequantize(weights, ggml_type)) is not None:
+        return out
     _require_cuda("weights", weights)
     _weights_2d(weights)
     _lib.init(weights.device.index or 0)
@@ -132,6 +138,8 @@ def gated_feed_forward(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor
     """The front of a gated feed-forward block (ml/zoo/transformer/transformer.go:1276-1287):
     ``activation(dense(xn, w_gate)) * dense(xn, w_up)`` with ``xn = rms_norm(x)`` when ``norm`` is given.
     x: [batch..., K] float32 or bfloat16 (gain, biases and the result stay float32); both weights [N, bytesPerRow] uint8 of one GGML type."""
+    if _lib.fast is not None and (y := _lib.fast.gated(x, w_gate, w_up, quant, activation, bias_gate, bias_up, norm)) is not None:
+        return y
     if quant is None or quant.scheme != QuantizationScheme.GGML:
         raise _lib.NotImplementedByBackend(_lib.ERR_NOT_IMPLEMENTED, "only the GGML scheme is on this path")
     for name, t in (("x", x), ("w_gate", w_gate), ("w_up", w_up)):
@@ -178,6 +186,10 @@ def quantized_dense(x: torch.Tensor, weights: torch.Tensor, quant: Quantization,
     ([batch..., N] float32) is added to the result (gain and residual are float32 also for bfloat16 x): Model.normalize followed by a
     projection and Add(residual, ...) after it, ml/zoo/transformer/transformer.go:1099-1101, 1045, 1055.
     """
+    if _lib.fast is not None and len(optional_activation) <= 1:
+        y = _lib.fast.dense(x, weights, quant, bias, optional_activation[0] if optional_activation else None, norm, residual)
+        if y is not None:
+            return y
     if len(optional_activation) > 1:
         raise ValueError(f"quantized_dense can only take one optional activation, got {optional_activation}")
     act = optional_activation[0] if optional_activation else Activation.NONE
@@ -230,6 +242,8 @@ def quantized_dense(x: torch.Tensor, weights: torch.Tensor, quant: Quantization,
 def quantized_gather(table: torch.Tensor, indices: torch.Tensor, quant: Quantization) -> torch.Tensor:
     """nn.QuantizedGather: indices [batch..., 1] (int32) -> [batch..., K] float32 rows of the
     dequantised table.  An out-of-range index raises IndexError."""
+    if _lib.fast is not None and (out := _lib.fast.gather(table, indices, quant)) is not None:
+        return out
     if quant.scheme != QuantizationScheme.GGML:
         raise ValueError("quantized_gather: only the GGML scheme is supported")  # quantized_gather.go:31-33
     _require_cuda("table", table)
@@ -263,6 +277,8 @@ def quantized_dense_batch(problems, norm: RMSNorm | None = None) -> list:
     activations (with ``norm``: all float32 or all bfloat16); returns the list of outputs.  Results equal those of separate calls; problems
     of one GGML type and one batch size of up to 8 rows share a single kernel launch.
     """
+    if _lib.fast is not None and (outs := _lib.fast.batch(problems, norm)) is not None:
+        return outs
     import ctypes
     L = _lib.lib()
     descs = (_lib.DenseDesc * len(problems))()

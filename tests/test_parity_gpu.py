@@ -1666,6 +1666,39 @@ def test_gather_out_of_range_index_raises(gpu):
             nn.quantized_gather(dev(gpu, table), dev(gpu, np.array([[3], [bad]], np.int32)), Quantization(ggml_type=Q8_0))
 
 
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("shape", [(1, 1024), (2, 3, 1024), (0, 1024)])
+def test_native_host_path_equals_the_python_steps(gpu, monkeypatch, shape, bf16):
+    """The same operators through csrc/binding.cpp and through the Python steps of nn.py: the same bits, shapes and types."""
+    from gomlx_amd import _lib
+    t, K, N = Q4_K, 1024, 192
+    q = Quantization(ggml_type=t)
+    w = [dev(gpu, synth.weights(t, 700 + i, N, K)) for i in range(2)]
+    g = gpu.Generator(device="cuda").manual_seed(3)
+    x = gpu.randn(shape, device="cuda", generator=g)
+    x = x.to(gpu.bfloat16) if bf16 else x
+    bias, gain = gpu.randn(N, device="cuda", generator=g), gpu.rand(K, device="cuda", generator=g)
+    res = gpu.randn(shape[:-1] + (N,), device="cuda", generator=g)
+    norm = nn.RMSNorm(gain=gain, epsilon=1e-5, scale_offset=1.0)
+    idx = gpu.tensor([[3], [0], [191]], dtype=gpu.int32, device="cuda")
+
+    def calls():
+        out = [nn.quantized_dense(x, w[0], q), nn.quantized_dense(x, w[0], q, bias, nn.Activation.GELU),
+               nn.quantized_dense(x, w[1], q, None, nn.Activation.SILU, norm=norm, residual=res),
+               nn.gated_feed_forward(x, w[0], w[1], q, nn.Activation.SWISH, bias, None, nn.RMSNorm()), nn.dequantize(w[0], t),
+               nn.quantized_gather(w[0], idx, q)]
+        out += nn.quantized_dense_batch([(x, w[0], q, bias, None), (x, w[1], q, None, nn.Activation.RELU)], norm)
+        return out if bf16 else out + nn.quantized_dense_batch([(x, w[0], q, bias, None), (x, w[1], q, None, None)])
+
+    _lib.init(0)
+    native = calls()
+    monkeypatch.setattr(_lib, "fast", None)
+    python = calls()
+    assert len(native) == len(python)
+    for a, b in zip(native, python):
+        assert a.dtype == b.dtype and a.shape == b.shape and a.device == b.device and gpu.equal(a, b)
+
+
 # ------------------------------------------------------------------------------ recorded replays and timing hooks
 
 def test_recorded_chain_replays_match_eager(gpu, oracle):
