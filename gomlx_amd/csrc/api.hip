@@ -258,6 +258,40 @@ int64_t gated_split_k_to(int type, int64_t K, int64_t N) {
     }
 }
 
+// Whether 3 to 16 rows of up to 4096 values take the one-launch kernel of mmv.hip.  It costs about 5 us of activation conversion per
+// workgroup and then streams W once; the GEMV it replaces costs a pass per row over small matrices, per four rows (two with a
+// normalisation, a residual or a gated pair: `extras`) over those of 24 MB and more, the split-K kernels three launches.
+// Measured (us per call on rotating weights; rows 2 3 4 6 8 12 16; the routes before | this one):
+//   Q8_0   4096x1024   3.5  4.2  4.3  6.0  6.4  8.7 11.1 |  7.8  7.8  7.9  8.9  8.8 10.8 10.9    4096x14336  13.3 15.4 15.4 28.9 28.6 29.2 29.4 | 17.1 17.0 17.2 17.9 17.9 21.6 21.4
+//          4096x4096   7.5 10.0 12.2 14.1 14.1 14.4 14.5 |  9.8  9.7  9.9 10.6 10.7 13.2 13.2    gated pair  23.8 40.7 40.7 48.2 49.3 50.0 50.6 | 25.3 25.5 25.6 26.5 26.7 31.7 31.8
+//   Q4_0   4096x4096   5.6  7.3  8.9 12.2 12.4 12.7 12.9 |  8.1  8.0  8.1  8.7  8.7 11.8 11.9    4096x14336   9.6 14.0 14.0 22.8 23.3 23.8 23.9 | 14.0 14.0 14.3 15.3 15.5 20.3 20.4
+//   Q4_K   4096x4096   6.7  8.8 10.9 12.0 12.3 12.4 12.6 |  8.0  7.9  8.0  9.6  9.6 13.1 12.9    4096x14336  11.1 14.8 14.8 18.3 18.6 19.0 19.3 | 12.4 12.3 12.5 13.8 13.9 20.4 20.4
+//          gated pair  8.6 11.1 13.6 19.8 14.8 15.5 15.6 | 10.1 10.1 10.1 11.4 11.5 15.6 15.5    gated pair  18.9 26.3 26.6 27.1 27.2 27.8 28.5 | 17.7 17.7 18.0 19.4 19.5 26.3 26.3
+//   Q6_K   4096x4096   8.0 10.6 13.2 17.0 17.3 17.5 17.7 |  9.8  9.5  9.6 10.6 10.6 14.1 14.1    4096x14336  14.6 24.5 24.1 31.5 32.1 32.8 32.8 | 17.3 17.2 17.4 18.2 18.1 24.1 24.5
+//   IQ4_NL 4096x4096   6.8  9.0 11.0 13.1 13.3 13.6 13.8 |  8.5  8.5  8.5  9.3  9.4 12.6 12.6    4096x14336  12.3 16.0 16.1 25.6 26.3 26.9 27.1 | 16.1 16.0 16.1 17.0 17.3 22.3 22.5
+// Below 9 MB a pass per row comes out of the caches: there the product of rows and bytes decides (Q8_0 4096x1024, 4.5 MB: even at 16 rows;
+// a gated pair of them: 10.8 | 10.7 at 8; Q4_K: 14.5 | 14.5 at 12).
+bool takes_mmv(int type, int64_t M, int64_t K, int64_t N, const void *x, const void *gain, int matrices, bool extras) {
+    if (M < 3 || !mmv_one_launch(K) || !mmv_supported(type, M, K, N, x, gain)) return false;
+    const int64_t bytes = weight_bytes_of(type, K, N) * matrices, MB = (int64_t)1 << 20;
+    if (bytes < 9 * MB) return M * bytes >= 64 * MB;
+    if (type == GQ_Q4_0 && M == 3 && bytes < kLargeWeightBytes) return false;
+    if (!extras && M <= 4 && bytes >= kLargeWeightBytes && (type == GQ_Q8_0 || (type == GQ_Q4_0 && bytes < 64 * MB))) return false;  // one GEMV pass of four rows
+    if (type == GQ_Q4_K && M > 8 && matrices == 1) return false;  // the split-K kernels, whose Q4_K conversion is as cheap and shared by 32 rows
+    return true;
+}
+// What the split-K kernels were chosen for: rows of more than 4096 values, up to sixteen of them (eight for Q4_K), take mmv.hip's two
+// launches instead of the three of mmq.hip (8 and 16 rows on 14336 -> 4096: Q8_0 29.7 30.0 | 20.6 24.7 us, Q4_0 24.2 24.6 | 18.7 23.3,
+// Q6_K 32.8 33.3 | 21.6 27.2, IQ4_NL 27.5 27.7 | 20.6 25.6, Q4_K 17.8 18.1 | 17.8 23.6).  Their scratch memory is the smaller one.
+int split_k(int type, const void *x, bool x_is_bf16, int64_t M, int64_t K, int count, const MmqSetItem *items, const MmqExtra *ex, hipStream_t s) {
+    const void *gain = ex && ex->norm ? ex->norm->gain : nullptr;
+    bool mmv = type != GQ_Q4_K || M <= 8;
+    for (int i = 0; i < count; i++) mmv = mmv && mmv_supported(type, M, K, items[i].N, x, gain);
+    if (mmv) return launch_mmv(type, x, x_is_bf16, M, K, count, items, ex, s);
+    if (count > 1) return launch_mmq_set(type, x, x_is_bf16, M, K, count, items, ex ? ex->norm : nullptr, s);
+    return launch_mmq(type, x, x_is_bf16, M, K, items[0].W, items[0].N, items[0].bias, items[0].act, items[0].y, s, ex);
+}
+
 // large batches: W dequantised once into the stream's workspace, then a plain 16-bit GEMM
 int two_pass(int type, bool x_is_bf16, const void *x, int64_t M, int64_t K, const void *W, int64_t N, const float *bias, int act,
              float *y, hipStream_t s) {
@@ -437,12 +471,14 @@ int gq_qdense_f32(int type, const float *dX, int64_t M, int64_t K, const void *d
     // MFMA kernels cost 19 .. 26 us (Q8_0 / Q4_0, K = 4096, N = 4096 .. 14336) for up to 32 rows and
     // 5 .. 18 us per further 32; the two passes 33 .. 62 us for anything up to 128 rows.  Measured
     // crossovers: split_k_from() / split_k_to().
+    const MmqSetItem one{(const uint8_t *)dW, N, dBias, act, dY};
+    if (takes_mmv(type, M, K, N, dX, nullptr, 1, false)) return launch_mmv(type, dX, false, M, K, 1, &one, nullptr, (hipStream_t)stream);
     const bool tp = gemm_two_pass_supported(type, false, M, K, N, dX);
     const bool ks = M <= kGemvMaxRows && gemv_ks_supported(type, K, N, dX);
     const bool sk = M >= split_k_from(type, weight_bytes_of(type, K, N)) && mmq_supported(type, M, K, N, dX, dBias, dY) &&
                     (M <= split_k_to(type, K, N) || !tp);
     if (ks && !sk) return launch_gemv_ks(type, dX, false, M, K, (const uint8_t *)dW, N, dBias, act, dY, (hipStream_t)stream);
-    if (sk) return launch_mmq(type, dX, false, M, K, (const uint8_t *)dW, N, dBias, act, dY, (hipStream_t)stream);
+    if (sk) return split_k(type, dX, false, M, K, 1, &one, nullptr, (hipStream_t)stream);
     // Shapes without a K-sliced plan (K not a multiple of 256: rare in models): a pass over W per row for up to 16
     // rows.  The 16-bit operands of the GEMMs below lean on averaging over many outputs and terms; on these few-row
     // problems seeded sweeps measured up to 0.9e-3 (1.25e-3 over a single block) through them, too close to the bound.
@@ -470,6 +506,7 @@ int gq_qdense_f32_static(int type, const float *dX, int64_t M, int64_t K, const 
 }
 
 namespace {
+bool set_takes_mmv(int count, const gq_dense_desc *descs, const float *gain, MmqSetItem *set);
 bool takes_shared_pass(int count, const gq_dense_desc *descs, const float *gain, MmqSetItem *set);  // (defined with the dispatch thresholds below)
 // From 6 rows the shared split-K pass is ahead of the merged GEMV launch: a decoder layer's q / k / v, 4096 -> 4096 + 2 x 1024,
 // with the rest of the layer: 79.2 against 80.0 us at 5 rows, 81.6 against 79.9 at 6, 84.7 against 80.3 at 8.
@@ -487,8 +524,10 @@ int gq_qdense_f32_batch(int count, const gq_dense_desc *descs, void *stream) {
     CallScope scope;
     {   // projections of one input beyond the GEMV's best rows: one split-K pass for all of them
         MmqSetItem set[4];
+        if (set_takes_mmv(count, descs, nullptr, set))
+            return launch_mmv(descs[0].type, descs[0].dX, false, descs[0].M, descs[0].K, count, set, nullptr, (hipStream_t)stream);
         if (descs[0].M >= kSharedPassFromRows && takes_shared_pass(count, descs, nullptr, set))
-            return launch_mmq_set(descs[0].type, descs[0].dX, false, descs[0].M, descs[0].K, count, set, nullptr, (hipStream_t)stream);
+            return split_k(descs[0].type, descs[0].dX, false, descs[0].M, descs[0].K, count, set, nullptr, (hipStream_t)stream);
     }
     // merge runs of batch-1 problems of one type that the streaming GEMV handles; the rest go one by one
     int i = 0;
@@ -504,7 +543,10 @@ int gq_qdense_f32_batch(int count, const gq_dense_desc *descs, void *stream) {
         const int64_t rows = descs[i].M;
         const bool rows_ok = rows == 1 || (use_ks && rows >= 1 && rows <= batch_rows_max());
         // (several rows per problem: only over matrices below the size from which one pass serves several rows)
-        auto size_ok = [&](const gq_dense_desc &d) { return rows == 1 || weight_bytes_of(d.type, d.K, d.N) < kLargeWeightBytes; };
+        // (and none that a call of its own would hand to the one-launch kernel: a submission returns what its calls return one by one)
+        auto size_ok = [&](const gq_dense_desc &d) {
+            return rows == 1 || (weight_bytes_of(d.type, d.K, d.N) < kLargeWeightBytes && !takes_mmv(d.type, d.M, d.K, d.N, d.dX, nullptr, 1, false));
+        };
         while (j < count && j - i < 8 && rows_ok && descs[j].type == descs[i].type && descs[j].M == rows && descs[j].N > 0 && fits(descs[j]) &&
                size_ok(descs[j])) {
             const gq_dense_desc &d = descs[j];
@@ -534,12 +576,14 @@ int gq_qdense_bf16(int type, const uint16_t *dX, int64_t M, int64_t K, const voi
     // Same crossovers as for fp32 activations: bf16 widens exactly to fp32 for the GEMV passes and to
     // the fp16 activation image of the split-K kernels (which have no bf16 rounding of W: tighter than
     // the bf16 MFMA paths).
+    const MmqSetItem one{(const uint8_t *)dW, N, dBias, act, dY};
+    if (takes_mmv(type, M, K, N, dX, nullptr, 1, false)) return launch_mmv(type, dX, true, M, K, 1, &one, nullptr, (hipStream_t)stream);
     const bool tp = gemm_two_pass_supported(type, true, M, K, N, dX);
     const bool ks = M <= kGemvMaxRows && gemv_ks_supported(type, K, N, dX);
     const bool sk = M >= split_k_from(type, weight_bytes_of(type, K, N)) && mmq_supported(type, M, K, N, dX, dBias, dY) &&
                     (M <= split_k_to(type, K, N) || !tp);
     if (ks && !sk) return launch_gemv_ks(type, dX, true, M, K, (const uint8_t *)dW, N, dBias, act, dY, (hipStream_t)stream);
-    if (sk) return launch_mmq(type, dX, true, M, K, (const uint8_t *)dW, N, dBias, act, dY, (hipStream_t)stream);
+    if (sk) return split_k(type, dX, true, M, K, 1, &one, nullptr, (hipStream_t)stream);
     if (tp) return two_pass(type, true, dX, M, K, dW, N, dBias, act, dY, (hipStream_t)stream);
     return launch_gemm(type, true, dX, M, K, (const uint8_t *)dW, N, dBias, act, dY, (hipStream_t)stream);
 }
@@ -629,6 +673,12 @@ bool same_input_set(int count, const gq_dense_desc *descs, MmqSetItem *set) {
     }
     return true;
 }
+bool set_takes_mmv(int count, const gq_dense_desc *descs, const float *gain, MmqSetItem *set) {
+    if (!same_input_set(count, descs, set)) return false;
+    int64_t ntot = 0;
+    for (int i = 0; i < count; i++) ntot += descs[i].N;
+    return takes_mmv(descs[0].type, descs[0].M, descs[0].K, ntot, descs[0].dX, gain, 1, true);
+}
 bool takes_shared_pass(int count, const gq_dense_desc *descs, const float *gain, MmqSetItem *set) {
     if ((gain && !aligned_to(gain, 16)) || !same_input_set(count, descs, set)) return false;
     const int type = descs[0].type;
@@ -653,6 +703,9 @@ int gq_qdense_block_f32(int type, const float *dX, int64_t M, int64_t K, const g
     CallScope scope;
     RmsNorm rn{nullptr, 0.f, 0.f};
     if (norm) rn = RmsNorm{norm->dGain, norm->eps, norm->gain_offset};
+    const MmqSetItem one{(const uint8_t *)dW, N, dBias, act, dY};
+    const MmqExtra ex{nullptr, nullptr, dResidual, norm ? &rn : nullptr};
+    if (takes_mmv(type, M, K, N, dX, rn.gain, 1, true)) return launch_mmv(type, dX, false, M, K, 1, &one, &ex, (hipStream_t)stream);
     if (fold_into_gemv(type, M, K, N, dX, rn.gain, dBias, dY, false))
         return launch_gemv_ks_ext(type, dX, false, M, K, norm ? &rn : nullptr, (const uint8_t *)dW, dBias, nullptr, nullptr, dResidual, N, act, dY,
                                   (hipStream_t)stream);
@@ -663,10 +716,8 @@ int gq_qdense_block_f32(int type, const float *dX, int64_t M, int64_t K, const g
                                           dY, ws, (hipStream_t)stream);
     }
     // split-K range: the normalisation rides on the activation pre-pass and the reduction, the residual on the reduction
-    if (block_takes_split_k(type, M, K, N, dX, dBias, dY, false) && (!dResidual || aligned_to(dResidual, 16)) && (!rn.gain || aligned_to(rn.gain, 16))) {
-        const MmqExtra ex{nullptr, nullptr, dResidual, norm ? &rn : nullptr};
-        return launch_mmq(type, dX, false, M, K, (const uint8_t *)dW, N, dBias, act, dY, (hipStream_t)stream, &ex);
-    }
+    if (block_takes_split_k(type, M, K, N, dX, dBias, dY, false) && (!dResidual || aligned_to(dResidual, 16)) && (!rn.gain || aligned_to(rn.gain, 16)))
+        return split_k(type, dX, false, M, K, 1, &one, &ex, (hipStream_t)stream);
     // composed: normalised activations into the stream's second workspace, the dense call, then the residual.  When y
     // overlaps the residual (a residual stream updated in place) the dense result goes to the workspace first: written
     // straight to y it would destroy the residual before the addition reads it.
@@ -687,8 +738,8 @@ int gq_qdense_block_f32(int type, const float *dX, int64_t M, int64_t K, const g
         }
     }
     if (dResidual && dense_takes_split_k(type, M, K, N, x, dBias, dY) && aligned_to(dResidual, 16)) {  // the residual rides on the reduction
-        const MmqExtra ex{nullptr, nullptr, dResidual, nullptr};
-        return launch_mmq(type, x, false, M, K, (const uint8_t *)dW, N, dBias, act, dY, (hipStream_t)stream, &ex);
+        const MmqExtra plain{nullptr, nullptr, dResidual, nullptr};
+        return split_k(type, x, false, M, K, 1, &one, &plain, (hipStream_t)stream);
     }
     float *dense_out = in_place ? tmp : dY;
     if (int rc = gq_qdense_f32(type, x, M, K, dW, N, dBias, act, dense_out, stream)) return rc;
@@ -729,23 +780,21 @@ int gq_qdense_norm_f32_batch(int count, const gq_dense_desc *descs, const gq_rms
     // over all their rows, one reduction - where the matrices taken together are in that kernel's range (three calls
     // would convert the activations three times and pay nine launches).
     MmqSetItem set[4];
+    const RmsNorm rn{norm->dGain, norm->eps, norm->gain_offset};
+    const MmqExtra ex{nullptr, nullptr, nullptr, &rn};
+    if (set_takes_mmv(count, descs, norm->dGain, set))
+        return launch_mmv(descs[0].type, descs[0].dX, false, rows, descs[0].K, count, set, &ex, (hipStream_t)stream);
     const bool shared_pass = takes_shared_pass(count, descs, norm->dGain, set);
     XsBatchItem items[8];
-    if (merges_into_gemv(count, descs, norm, shared_pass, items)) {
-        const RmsNorm rn{norm->dGain, norm->eps, norm->gain_offset};
+    if (merges_into_gemv(count, descs, norm, shared_pass, items))
         return launch_gemv_ks_batch_norm(descs[0].type, count, items, &rn, (hipStream_t)stream, (int)rows);
-    }
-    if (shared_pass) {
-        const RmsNorm rn{norm->dGain, norm->eps, norm->gain_offset};
-        return launch_mmq_set(descs[0].type, descs[0].dX, false, rows, descs[0].K, count, set, &rn, (hipStream_t)stream);
-    }
+    if (shared_pass) return split_k(descs[0].type, descs[0].dX, false, rows, descs[0].K, count, set, &ex, (hipStream_t)stream);
     // Past the split-K range the same projections share the two passes: one activation conversion, one image of all the
     // matrices, one GEMM (a decoder layer's q / k / v at 128 rows: two launches instead of six).
     if (same_input_set(count, descs, set) && rows > kGemvMaxRows && (!norm->dGain || aligned_to(norm->dGain, 16)) &&
         gemm_two_pass_set_supported(descs[0].type, count, set, rows, descs[0].K, descs[0].dX)) {
         void *ws = nullptr;
         if (int rc = stream_workspace((hipStream_t)stream, gemm_two_pass_set_workspace(count, set, rows, descs[0].K), &ws)) return rc;
-        const RmsNorm rn{norm->dGain, norm->eps, norm->gain_offset};
         return launch_gemm_two_pass_set(descs[0].type, descs[0].dX, rows, descs[0].K, &rn, count, set, ws, (hipStream_t)stream);
     }
     for (int i = 0; i < count; i++) {
@@ -766,6 +815,9 @@ int gq_qdense_gated_f32(int type, const float *dX, int64_t M, int64_t K, const g
     CallScope scope;
     RmsNorm rn{nullptr, 0.f, 0.f};
     if (norm) rn = RmsNorm{norm->dGain, norm->eps, norm->gain_offset};
+    const MmqSetItem one{(const uint8_t *)dWgate, N, dBiasGate, act, dY};
+    const MmqExtra ex{(const uint8_t *)dWup, dBiasUp, nullptr, norm ? &rn : nullptr};
+    if (takes_mmv(type, M, K, N, dX, rn.gain, 2, true)) return launch_mmv(type, dX, false, M, K, 1, &one, &ex, (hipStream_t)stream);
     if (fold_into_gemv(type, M, K, N, dX, rn.gain, dBiasGate, dY, true))
         return launch_gemv_ks_ext(type, dX, false, M, K, norm ? &rn : nullptr, (const uint8_t *)dWgate, dBiasGate, (const uint8_t *)dWup, dBiasUp,
                                   nullptr, N, act, dY, (hipStream_t)stream);
@@ -775,11 +827,9 @@ int gq_qdense_gated_f32(int type, const float *dX, int64_t M, int64_t K, const g
         return launch_gemm_two_pass_block(type, dX, M, K, norm ? &rn : nullptr, (const uint8_t *)dWgate, dBiasGate, (const uint8_t *)dWup, dBiasUp,
                                           nullptr, N, act, dY, ws, (hipStream_t)stream);
     }
-    if (block_takes_split_k(type, M, K, N, dX, dBiasGate, dY, true) && (!dBiasUp || aligned_to(dBiasUp, 16)) && (!rn.gain || aligned_to(rn.gain, 16))) {
-        // both matrices against one activation image (which carries the gain); the reduction normalises and forms act(gate) * up
-        const MmqExtra ex{(const uint8_t *)dWup, dBiasUp, nullptr, norm ? &rn : nullptr};
-        return launch_mmq(type, dX, false, M, K, (const uint8_t *)dWgate, N, dBiasGate, act, dY, (hipStream_t)stream, &ex);
-    }
+    // (split-K: both matrices against one activation image, which carries the gain; the reduction normalises and forms act(gate) * up)
+    if (block_takes_split_k(type, M, K, N, dX, dBiasGate, dY, true) && (!dBiasUp || aligned_to(dBiasUp, 16)) && (!rn.gain || aligned_to(rn.gain, 16)))
+        return split_k(type, dX, false, M, K, 1, &one, &ex, (hipStream_t)stream);
     // composed: [normalised activations,] act(gate) into the stream's second workspace, up into y, y *= act(gate)
     const size_t xn_bytes = norm ? ((size_t)M * (size_t)K * sizeof(float) + 255) / 256 * 256 : 0;
     void *ws = nullptr;
@@ -792,8 +842,8 @@ int gq_qdense_gated_f32(int type, const float *dX, int64_t M, int64_t K, const g
     }
     if (dense_takes_split_k(type, M, K, N, x, dBiasGate, dY) && (!dBiasUp || aligned_to(dBiasUp, 16))) {
         // both matrices against one activation image; the reduction forms act(gate) * up
-        const MmqExtra ex{(const uint8_t *)dWup, dBiasUp, nullptr, nullptr};
-        return launch_mmq(type, x, false, M, K, (const uint8_t *)dWgate, N, dBiasGate, act, dY, (hipStream_t)stream, &ex);
+        const MmqExtra plain{(const uint8_t *)dWup, dBiasUp, nullptr, nullptr};
+        return split_k(type, x, false, M, K, 1, &one, &plain, (hipStream_t)stream);
     }
     float *gate = reinterpret_cast<float *>(static_cast<uint8_t *>(ws) + xn_bytes);
     if (int rc = gq_qdense_f32(type, x, M, K, dWgate, N, dBiasGate, act, gate, stream)) return rc;
@@ -824,19 +874,19 @@ int gq_qdense_block_bf16(int type, const uint16_t *dX, int64_t M, int64_t K, con
     if (M == 0 || N == 0) return GQ_OK;
     if (int rc = use_device()) return rc;
     CallScope scope;
+    const RmsNorm rn = norm ? RmsNorm{norm->dGain, norm->eps, norm->gain_offset} : RmsNorm{nullptr, 0.f, 0.f};
+    const MmqSetItem one{(const uint8_t *)dW, N, dBias, act, dY};
+    const MmqExtra ex{nullptr, nullptr, dResidual, norm ? &rn : nullptr};
+    if (takes_mmv(type, M, K, N, dX, rn.gain, 1, true)) return launch_mmv(type, dX, true, M, K, 1, &one, &ex, (hipStream_t)stream);
     if (fold_into_gemv(type, M, K, N, reinterpret_cast<const float *>(dX), norm ? norm->dGain : nullptr, dBias, dY, false)) {
-        const RmsNorm rn = norm ? RmsNorm{norm->dGain, norm->eps, norm->gain_offset} : RmsNorm{nullptr, 0.f, 0.f};
         return launch_gemv_ks_ext(type, dX, true, M, K, norm ? &rn : nullptr, (const uint8_t *)dW, dBias, nullptr, nullptr, dResidual, N, act, dY,
                                   (hipStream_t)stream);
     }
     {   // the split-K kernels' pre-pass reads bf16 as well (where the fp32 call would take them too)
         const float *xa = reinterpret_cast<const float *>(dX), *gain = norm ? norm->dGain : nullptr;  // (only their alignment is looked at)
         if (!block_takes_two_pass(type, M, K, N, xa, gain, dBias, dY, false) && block_takes_split_k(type, M, K, N, xa, dBias, dY, false) &&
-            (!dResidual || aligned_to(dResidual, 16)) && (!gain || aligned_to(gain, 16))) {
-            const RmsNorm rn = norm ? RmsNorm{norm->dGain, norm->eps, norm->gain_offset} : RmsNorm{nullptr, 0.f, 0.f};
-            const MmqExtra ex{nullptr, nullptr, dResidual, norm ? &rn : nullptr};
-            return launch_mmq(type, dX, true, M, K, (const uint8_t *)dW, N, dBias, act, dY, (hipStream_t)stream, &ex);
-        }
+            (!dResidual || aligned_to(dResidual, 16)) && (!gain || aligned_to(gain, 16)))
+            return split_k(type, dX, true, M, K, 1, &one, &ex, (hipStream_t)stream);
     }
     void *ws = nullptr;
     if (int rc = stream_workspace((hipStream_t)stream, widened_bytes(M, K), &ws, kWsWidenSlot)) return rc;
@@ -854,19 +904,19 @@ int gq_qdense_gated_bf16(int type, const uint16_t *dX, int64_t M, int64_t K, con
     if (M == 0 || N == 0) return GQ_OK;
     if (int rc = use_device()) return rc;
     CallScope scope;
+    const RmsNorm rn = norm ? RmsNorm{norm->dGain, norm->eps, norm->gain_offset} : RmsNorm{nullptr, 0.f, 0.f};
+    const MmqSetItem one{(const uint8_t *)dWgate, N, dBiasGate, act, dY};
+    const MmqExtra ex{(const uint8_t *)dWup, dBiasUp, nullptr, norm ? &rn : nullptr};
+    if (takes_mmv(type, M, K, N, dX, rn.gain, 2, true)) return launch_mmv(type, dX, true, M, K, 1, &one, &ex, (hipStream_t)stream);
     if (fold_into_gemv(type, M, K, N, reinterpret_cast<const float *>(dX), norm ? norm->dGain : nullptr, dBiasGate, dY, true)) {
-        const RmsNorm rn = norm ? RmsNorm{norm->dGain, norm->eps, norm->gain_offset} : RmsNorm{nullptr, 0.f, 0.f};
         return launch_gemv_ks_ext(type, dX, true, M, K, norm ? &rn : nullptr, (const uint8_t *)dWgate, dBiasGate, (const uint8_t *)dWup, dBiasUp, nullptr,
                                   N, act, dY, (hipStream_t)stream);
     }
     {
         const float *xa = reinterpret_cast<const float *>(dX), *gain = norm ? norm->dGain : nullptr;  // (only their alignment is looked at)
         if (!block_takes_two_pass(type, M, K, N, xa, gain, dBiasGate, dY, true) && block_takes_split_k(type, M, K, N, xa, dBiasGate, dY, true) &&
-            (!dBiasUp || aligned_to(dBiasUp, 16)) && (!gain || aligned_to(gain, 16))) {
-            const RmsNorm rn = norm ? RmsNorm{norm->dGain, norm->eps, norm->gain_offset} : RmsNorm{nullptr, 0.f, 0.f};
-            const MmqExtra ex{(const uint8_t *)dWup, dBiasUp, nullptr, norm ? &rn : nullptr};
-            return launch_mmq(type, dX, true, M, K, (const uint8_t *)dWgate, N, dBiasGate, act, dY, (hipStream_t)stream, &ex);
-        }
+            (!dBiasUp || aligned_to(dBiasUp, 16)) && (!gain || aligned_to(gain, 16)))
+            return split_k(type, dX, true, M, K, 1, &one, &ex, (hipStream_t)stream);
     }
     void *ws = nullptr;
     if (int rc = stream_workspace((hipStream_t)stream, widened_bytes(M, K), &ws, kWsWidenSlot)) return rc;
@@ -888,16 +938,15 @@ int gq_qdense_norm_bf16_batch(int count, const gq_dense_desc *descs, const gq_rm
     CallScope scope;
     if (norm && count <= 8) {  // the list as one launch of the decode GEMV, on the bf16 data as it is
         MmqSetItem set[4];
+        const RmsNorm rn{norm->dGain, norm->eps, norm->gain_offset};
+        const MmqExtra ex{nullptr, nullptr, nullptr, &rn};
+        if (set_takes_mmv(count, descs, norm->dGain, set))
+            return launch_mmv(descs[0].type, descs[0].dX, true, descs[0].M, descs[0].K, count, set, &ex, (hipStream_t)stream);
         const bool shared_pass = takes_shared_pass(count, descs, norm->dGain, set);
         XsBatchItem items[8];
-        if (merges_into_gemv(count, descs, norm, shared_pass, items)) {
-            const RmsNorm rn{norm->dGain, norm->eps, norm->gain_offset};
+        if (merges_into_gemv(count, descs, norm, shared_pass, items))
             return launch_gemv_ks_batch_norm(descs[0].type, count, items, &rn, (hipStream_t)stream, (int)descs[0].M, true);
-        }
-        if (shared_pass) {
-            const RmsNorm rn{norm->dGain, norm->eps, norm->gain_offset};
-            return launch_mmq_set(descs[0].type, descs[0].dX, true, descs[0].M, descs[0].K, count, set, &rn, (hipStream_t)stream);
-        }
+        if (shared_pass) return split_k(descs[0].type, descs[0].dX, true, descs[0].M, descs[0].K, count, set, &ex, (hipStream_t)stream);
     }
     // every distinct activation matrix (q / k / v share theirs) is widened once
     gq_dense_desc wide[64];

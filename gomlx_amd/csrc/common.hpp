@@ -95,6 +95,15 @@ struct MmqSetItem { const uint8_t *W; int64_t N; const float *bias; int act; flo
 bool mmq_set_supported(int type, int count, const MmqSetItem *items, int64_t M, int64_t K, const void *x);
 int launch_mmq_set(int type, const void *x, bool x_is_bf16, int64_t M, int64_t K, int count, const MmqSetItem *items, const RmsNorm *norm,
                    hipStream_t s);
+// 2 to 16 activation rows in one launch on the matrix cores (mmv.hip); more than 4096 values of K take a second launch, workspace
+// and what mmq_supported asks of N, bias, residual and y.
+bool mmv_supported(int type, int64_t M, int64_t K, int64_t N, const void *x, const void *gain);
+bool mmv_one_launch(int64_t K);
+int launch_mmv(int type, const void *x, bool x_is_bf16, int64_t M, int64_t K, int count, const MmqSetItem *items, const MmqExtra *ex, hipStream_t s);
+// The reduction behind it: sums partial[slices][M][all columns] (partial2: the second matrix of a gated pair) and, with a normalisation,
+// sums of squares xss[slices][M] -> the finished outputs of `count` matrices.
+int launch_split_k_finish(const float *partial, const float *partial2, const float *xss, int nslices, int64_t M, int64_t K, int count,
+                          const MmqSetItem *items, const MmqExtra *ex, hipStream_t s);
 // The K-sliced GEMV with the normalisation folded in and, when W2 is given, the gated product
 // act(x.W + bias) * (x.W2 + bias2); fp32 or bf16 activations, at most 16 rows (the entry points use it below 8 rows, where a pass per row still wins).
 bool gemv_ks_ext_supported(int type, int64_t M, int64_t K, int64_t N, const void *x, const void *gain);

@@ -20,6 +20,7 @@
 // row r = 8 * block + (l >> 3), so every 128-byte row is still read as one full line.
 #include "blocks.hpp"
 #include "common.hpp"
+#include "lds_dma.hpp"
 
 #include <algorithm>
 #include <type_traits>
@@ -33,7 +34,6 @@ namespace {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef int i32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int DK = 64;
 constexpr int ROWB = 128;  // bytes per LDS row
@@ -261,27 +261,6 @@ int launch_x_to_f16(const float *x, int64_t M, int64_t K, const RmsNorm *norm, u
 }
 
 // ---- pass 2: 16-bit GEMM with global -> LDS DMA --------------------------------------------------
-// One 16-byte-per-lane buffer load whose data goes to LDS at lds_addr + 16 * lane.  The compiler
-// does not see that the instruction writes LDS or that it is counted by vmcnt: the kernel orders
-// these loads against its LDS reads with explicit waits and barriers.  (The s_nop is the wait
-// state the hardware wants between a write of M0 and an LDS DMA; the assembler does not add it
-// inside inline assembly.)
-__device__ __forceinline__ void dma16(uint32_t lds_addr, i32x4 rsrc, uint32_t voff, uint32_t soff) {
-    lds_addr = __builtin_amdgcn_readfirstlane(lds_addr);  // both are uniform by construction
-    soff = __builtin_amdgcn_readfirstlane(soff);
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds_addr), "v"(voff), "s"(rsrc), "s"(soff) : "memory");
-}
-
-__device__ __forceinline__ i32x4 make_rsrc(const void *base, uint64_t bytes) {
-    const uint64_t b = reinterpret_cast<uint64_t>(base);
-    i32x4 r;
-    r.x = __builtin_amdgcn_readfirstlane((int)(uint32_t)b);
-    r.y = __builtin_amdgcn_readfirstlane((int)(uint32_t)(b >> 32));  // stride 0: raw buffer, byte offsets
-    r.z = __builtin_amdgcn_readfirstlane((int)(uint32_t)(bytes > 0xFFFFFFFFull ? 0xFFFFFFFFull : bytes));
-    r.w = 0x00020000;  // 32-bit data format, no swizzle
-    return r;
-}
-
 // X [M, K] and Wh [N, K] 16-bit, K % 64 == 0, both 16-byte aligned.  The workgroup tile is
 // (128 TM) x (64 TN): 4 x 2 wavefronts of (32 TM) x (32 TN) each.  TM = TN = 2 is the tile for
 // large problems; the smaller ones keep the chip full when M x N yields too few big tiles.

@@ -2124,6 +2124,29 @@ int run_q4k_set(const void *x, bool x_is_bf16, int64_t M, int64_t K, int count, 
 }
 }  // namespace
 
+int launch_split_k_finish(const float *partial, const float *partial2, const float *xss, int nslices, int64_t M, int64_t K, int count,
+                          const MmqSetItem *items, const MmqExtra *ex, hipStream_t s) {
+    const RmsNorm *norm = ex ? ex->norm : nullptr;
+    const float eps = norm ? norm->eps : 0.f, inv_k = 1.0f / (float)K;
+    if (!norm) xss = nullptr;
+    int64_t N = 0;
+    MmqSetOut out = {};
+    for (int i = 0; i < count; i++) {
+        out.bias[i] = items[i].bias; out.y[i] = items[i].y; out.N[i] = (int)items[i].N; out.n0[i] = (int)N; out.act[i] = items[i].act;
+        N += items[i].N;
+    }
+    out.count = count;
+    out.ntot = (int)N;
+    const int64_t MN = M * N;
+    const int threads = MN / 4 / 256 >= 2 * device_cu_count() ? 256 : 64;
+    const dim3 grid((unsigned)((MN / 4 + threads - 1) / threads));
+    if (count == 1)
+        return launch(mmq_reduce_kernel, grid, dim3(threads), 0, s, partial, partial2, nslices, MN, (int)N, items[0].bias, ex ? ex->bias2 : nullptr, items[0].act,
+                      ex ? ex->residual : nullptr, items[0].y, (const float *)nullptr, xss, eps, inv_k, (uint32_t *)nullptr, 0);
+    return launch(mmq_reduce_set_kernel, grid, dim3(threads), 0, s, partial, nslices, (int)M, out, (const float *)nullptr, xss, eps, inv_k,
+                  (uint32_t *)nullptr, 0);
+}
+
 int launch_mmq(int type, const void *x, bool x_is_bf16, int64_t M, int64_t K, const uint8_t *W, int64_t N, const float *bias,
                int act, float *y, hipStream_t s, const MmqExtra *ex) {
     // (four row tiles per workgroup measured a little faster than two)

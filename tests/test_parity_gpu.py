@@ -392,6 +392,64 @@ def test_output_head_of_a_128k_vocabulary(gpu, oracle, t):
 
 
 @pytest.mark.parametrize("t", ALL_TYPES)
+@pytest.mark.parametrize("M,K,kind", [(3, 768, "plain"), (4, 4096, "block"), (5, 256, "plain"), (8, 4096, "gated"), (8, 2048, "set"), (9, 1280, "gated"),
+                                      (16, 4096, "bf16"), (6, 4352, "block"), (16, 8192, "gated")])
+def test_few_rows_in_one_launch(gpu, oracle, t, M, K, kind):
+    """3 to 16 rows on the matrix cores with the activations in registers: a last half slice (K % 512 == 256), fewer than eight slices,
+    two groups of slices (K > 4096), partly filled row tiles, rows of very different magnitude, and a row that is not finite.
+
+    Bound: the activations keep 20 bits (hi + lo, both truncated), sums are fp32 over at most a few hundred blocks and the minima of
+    Q4_K cancel a term about four times the result: 4 * (2^-20 + 2^-22) is 4.8e-6 of the row's 2-norm; twice that for a product."""
+    if t == Q6_K and K % 512:
+        K += 256
+    if t == Q4_K and M > 8 and (K > 4096 or kind != "gated"):
+        M = 8   # (beyond, Q4_K stays with the split-K kernels)
+    if t == Q4_0:
+        M = max(M, 4)
+    row_bytes = ggml.row_bytes(t, K)
+    N = (9 << 20) // row_bytes + 1
+    N += -N % 4 if K > 4096 else (N + 1) % 2 * 2 + (N % 16 == 0)   # ragged row tiles, except where the reduction asks for N % 4 == 0
+    nmat = {"gated": 2, "set": 3}.get(kind, 1)
+    sizes = [N] + [max(4, N // 5) // 4 * 4 + (1 if K <= 4096 else 0)] * 2 if kind == "set" else [N] * nmat
+    rng = np.random.default_rng(7 * M + K)
+    Ws = [np.tile(synth.weights(t, 71 + i, 131, K), (-(-n // 131), 1))[:n] for i, n in enumerate(sizes)]
+    x = rng.standard_normal((M, K)).astype(np.float32) * (10.0 ** rng.integers(-12, 12, (M, 1))).astype(np.float32)
+    x[2, K - 3] = np.inf if M % 2 else np.nan
+    if kind == "bf16":
+        x = bf16_round(x)
+    gain = (1 + 0.1 * rng.standard_normal(K)).astype(np.float32)
+    bias = rng.standard_normal(N).astype(np.float32)
+    res = rng.standard_normal((M, N)).astype(np.float32)
+    torch, q = gpu, Quantization(ggml_type=t)
+    norm = nn.RMSNorm(gain=dev(torch, gain), epsilon=0.0) if kind in ("block", "gated", "set") else None
+    xd, Wd = dev(torch, x), [dev(torch, w) for w in Ws]
+    if kind == "bf16":
+        xd = xd.to(torch.bfloat16)
+    if kind == "gated":
+        got = [nn.gated_feed_forward(xd, Wd[0], Wd[1], q, Activation.SILU, norm=norm)]
+    elif kind == "set":
+        got = nn.quantized_dense_batch([(xd, w, q, None, None) for w in Wd], norm=norm)
+    elif kind == "block":
+        got = [nn.quantized_dense(xd, Wd[0], q, dev(torch, bias), norm=norm, residual=dev(torch, res))]
+    else:
+        got = [nn.quantized_dense(xd, Wd[0], q)]
+    got = [g.cpu().numpy().astype(np.float64) for g in got]
+    keep = [m for m in range(M) if m != 2]
+    h = x[keep].astype(np.float64)
+    if norm is not None:
+        h = h / np.sqrt((h * h).mean(-1, keepdims=True)) * gain
+    want = [np.tile(h @ oracle.c_dequantize(t, w[:131], K).astype(np.float64).T, (1, -(-len(w) // 131)))[:, :len(w)] for w in Ws]
+    if kind == "gated":
+        want = [want[0] / (1 + np.exp(-want[0])) * want[1]]
+    elif kind == "block":
+        want = [want[0] + bias + res[keep]]
+    for g, w in zip(got, want):
+        assert not np.isfinite(g[2]).any()
+        err = np.linalg.norm(g[keep] - w, axis=1) / np.linalg.norm(w, axis=1)
+        assert err.max() <= (1e-5 if kind == "gated" else 4.8e-6), err
+
+
+@pytest.mark.parametrize("t", ALL_TYPES)
 def test_gemv_long_k_is_chunked(gpu, oracle, t):
     """K above the 16384 values one LDS pass holds."""
     K, N = 16384 + 4096, 19
