@@ -68,13 +68,11 @@ __device__ __forceinline__ float iq4nl_value(uint32_t nib) {
 __device__ __forceinline__ void q4k_scale_min(uint32_t a, uint32_t b, uint32_t c, int j, uint32_t &sc, uint32_t &mn) {
     const int sh = (j & 3) * 8;
     const uint32_t aj = a >> sh, bj = b >> sh, cj = c >> sh;
-    if (j < 4) {
-        sc = aj & 63u;
-        mn = bj & 63u;
-    } else {
-        sc = (cj & 0x0Fu) | (((aj >> 6) & 3u) << 4);
-        mn = ((cj >> 4) & 0x0Fu) | (((bj >> 6) & 3u) << 4);
-    }
+    // (selects of values, not of branches: lanes of one wavefront hold different j)
+    const bool low = j < 4;
+    const uint32_t mask = low ? 63u : 15u, top = low ? 0u : 0x30u;
+    sc = ((low ? aj : cj) & mask) | ((aj >> 2) & top);
+    mn = ((low ? bj : cj >> 4) & mask) | ((bj >> 2) & top);
 }
 
 // Exact dequantisation of 16 consecutive values of one weight row:

@@ -73,49 +73,146 @@ template <> struct Op16<false> {
 __host__ __device__ inline int64_t padded_k(int64_t K) { return (K + 63) / 64 * 64; }
 
 // ---- pass 1: GGML blocks -> 16-bit [N, K] -------------------------------------------------------
-// One thread per run of 16 weights (32 output bytes).  half = 0: image row = weight row.  half = 1 / 2:
-// the matrix is the first / second of a gated pair, whose images interleave in chunks of 32 rows
-// (image rows 64 c .. 64 c + 31 = rows 32 c .. of the first matrix, the next 32 = the same rows of
-// the second), so that a wavefront's 64-column tile holds both projections of 32 outputs.
-// The image's rows hold runs_per_row runs, of which the first `runs` come from W and the rest (padding
-// of K to the GEMM's step of 64) are zero.
-template <int T, bool BF16>
-__device__ __forceinline__ void dequant16bit_body(const uint8_t *__restrict__ W, uint16_t *__restrict__ out, uint32_t runs_per_row,
-                                                  uint32_t total_runs, int64_t row_bytes, int half, uint32_t runs, uint32_t block) {
-    // The 16-byte halves of the runs meet in LDS so that consecutive lanes store consecutive 16 bytes
-    // (whole cache lines per store instruction; a lane storing its own 32 bytes in two instructions
-    // half-fills twice as many).  An image holds at most 2^27 runs: 32-bit index arithmetic.
-    __shared__ uint4 halves[512];
-    const uint32_t tid = threadIdx.x, g0 = block * 256u, g = g0 + tid;
-    if (g < total_runs) {
-        const uint32_t row = g / runs_per_row, run = g % runs_per_row;
-        float w[16];
-        if (run < runs) {
-            dequant16<T>(W + (int64_t)row * row_bytes, run, w);
-        } else {
-#pragma unroll
-            for (int i = 0; i < 16; i++) w[i] = 0.f;
-        }
-        halves[2 * tid] = make_uint4(Op16<BF16>::pack(w[0], w[1]), Op16<BF16>::pack(w[2], w[3]), Op16<BF16>::pack(w[4], w[5]),
-                                     Op16<BF16>::pack(w[6], w[7]));
-        halves[2 * tid + 1] = make_uint4(Op16<BF16>::pack(w[8], w[9]), Op16<BF16>::pack(w[10], w[11]), Op16<BF16>::pack(w[12], w[13]),
-                                         Op16<BF16>::pack(w[14], w[15]));
+// The bytes that eight consecutive values (octet `o` of a run of blocks at `row`) come from and their exact fp32 values: the
+// arithmetic of dequant16<T>, eight values at a time (a product of a scale and a code is exact, so that a fused multiply-add
+// rounds where the separate subtraction does).
+struct __attribute__((packed, aligned(2))) u64_a2 { uint32_t v[2]; };
+__device__ __forceinline__ void bytes_as_float(uint32_t u, float *v) { v[0] = ubyte0(u); v[1] = ubyte1(u); v[2] = ubyte2(u); v[3] = ubyte3(u); }
+__device__ __forceinline__ void sbytes_as_float(uint32_t u, float *v) { v[0] = sbyte0(u); v[1] = sbyte1(u); v[2] = sbyte2(u); v[3] = sbyte3(u); }
+
+template <int T> struct Octet;
+template <> struct Octet<kQ8_0> {
+    uint32_t d;
+    u64_a2 c;
+    __device__ __forceinline__ void load(const uint8_t *row, uint32_t o) {
+        const uint8_t *b = row + (o >> 2) * 34u;
+        d = load_u16(b);
+        c = *reinterpret_cast<const u64_a2 *>(b + 2 + 8 * (o & 3));
     }
-    __syncthreads();
+    __device__ __forceinline__ void value(uint32_t, float *v) const {
+        const float s = half_bits_to_float(d);
+        sbytes_as_float(c.v[0], v);
+        sbytes_as_float(c.v[1], v + 4);
 #pragma unroll
-    for (int p = 0; p < 2; p++) {
-        const uint32_t c = tid + 256u * p, gg = g0 + (c >> 1);
-        if (gg >= total_runs) continue;
-        const uint32_t row = gg / runs_per_row, run = gg % runs_per_row;
-        const int64_t out_row = half == 0 ? (int64_t)row : (int64_t)(row >> 5) * 64 + (half - 1) * 32 + (row & 31);
-        *reinterpret_cast<uint4 *>(out + (out_row * runs_per_row + run) * 16 + (c & 1u) * 8u) = halves[c];
+        for (int j = 0; j < 8; j++) v[j] *= s;
+    }
+};
+template <int T> struct OctetNibble {  // Q4_0, IQ4_NL: octets 0, 1 in the low nibbles, 2, 3 in the high ones
+    uint32_t d;
+    u64_a2 c;
+    __device__ __forceinline__ void load(const uint8_t *row, uint32_t o) {
+        const uint8_t *b = row + (o >> 2) * 18u;
+        d = load_u16(b);
+        c = *reinterpret_cast<const u64_a2 *>(b + 2 + 8 * (o & 1));
+    }
+    __device__ __forceinline__ void value(uint32_t o, float *v) const {
+        const float s = half_bits_to_float(d);
+#pragma unroll
+        for (int w = 0; w < 2; w++) {
+            const uint32_t n = (c.v[w] >> (2 * (o & 2))) & 0x0F0F0F0Fu;
+            if constexpr (T == kQ4_0) {
+                bytes_as_float(n, v + 4 * w);
+#pragma unroll
+                for (int j = 0; j < 4; j++) v[4 * w + j] = (v[4 * w + j] - 8.0f) * s;
+            } else {  // four code-book entries (int8) at a time by byte permutes: see iq4nl_value
+                const uint32_t low3 = n & 0x07070707u;
+                const uint32_t lo = __builtin_amdgcn_perm(0xF6EADDCFu, 0xBFAD9881u, low3), hi = __builtin_amdgcn_perm(0x71594535u, 0x26190D01u, low3);
+                sbytes_as_float(__builtin_amdgcn_perm(hi, lo, 0x03020100u | ((n & 0x08080808u) >> 1)), v + 4 * w);
+#pragma unroll
+                for (int j = 0; j < 4; j++) v[4 * w + j] *= s;
+            }
+        }
+    }
+};
+template <> struct Octet<kQ4_0> : OctetNibble<kQ4_0> {};
+template <> struct Octet<kIQ4_NL> : OctetNibble<kIQ4_NL> {};
+template <> struct Octet<kQ4_K> {
+    uint4 hd;
+    uint2 c;
+    __device__ __forceinline__ void load(const uint8_t *row, uint32_t o) {
+        const uint8_t *sb = row + (o >> 5) * 144u;
+        hd = *reinterpret_cast<const uint4 *>(sb);
+        c = *reinterpret_cast<const uint2 *>(sb + 16 + 32 * ((o >> 3) & 3) + 8 * (o & 3));
+    }
+    __device__ __forceinline__ void value(uint32_t o, float *v) const {
+        uint32_t sc, mn;
+        q4k_scale_min(hd.y, hd.z, hd.w, (int)((o >> 2) & 7), sc, mn);
+        const float ds = half_bits_to_float(hd.x & 0xFFFFu) * (float)sc, dm = half_bits_to_float(hd.x >> 16) * (float)mn;
+        const uint32_t sh = o & 4;
+        bytes_as_float((c.x >> sh) & 0x0F0F0F0Fu, v);
+        bytes_as_float((c.y >> sh) & 0x0F0F0F0Fu, v + 4);
+#pragma unroll
+        for (int j = 0; j < 8; j++) v[j] = fmaf(ds, v[j], -dm);
+    }
+};
+template <> struct Octet<kQ6_K> {  // (block layout: see dequant16<kQ6_K>)
+    uint32_t d;
+    u64_a2 ql, qh;
+    int sc;
+    __device__ __forceinline__ void load(const uint8_t *row, uint32_t o) {
+        const uint8_t *sb = row + (o >> 5) * 210u;
+        const uint32_t h = (o >> 4) & 1, qd = (o >> 2) & 3;
+        ql = *reinterpret_cast<const u64_a2 *>(sb + 64 * h + 32 * (qd & 1) + 8 * (o & 3));
+        qh = *reinterpret_cast<const u64_a2 *>(sb + 128 + 32 * h + 8 * (o & 3));
+        sc = (int)(int8_t)sb[192 + ((o & 31) >> 1)];
+        d = load_u16(sb + 208);
+    }
+    __device__ __forceinline__ void value(uint32_t o, float *v) const {
+        const uint32_t qd = (o >> 2) & 3, nsh = (qd >> 1) * 4, hsh = 2 * qd;
+        const float s = half_bits_to_float(d) * (float)sc;
+#pragma unroll
+        for (int w = 0; w < 2; w++)
+            bytes_as_float(((ql.v[w] >> nsh) & 0x0F0F0F0Fu) | (((qh.v[w] >> hsh) & 0x03030303u) << 4), v + 4 * w);
+#pragma unroll
+        for (int j = 0; j < 8; j++) v[j] = s * (v[j] - 32.0f);
+    }
+};
+
+// half = 0: image row = weight row.  half = 1 / 2: the matrix is the first / second of a gated pair, whose images interleave
+// in chunks of 32 rows (image rows 64 c .. 64 c + 31 = rows 32 c .. of the first matrix, the next 32 = the same rows of
+// the second), so that a wavefront's 64-column tile holds both projections of 32 outputs.
+// The image's rows hold octs_per_row octets, of which the first `octs` come from W and the rest (padding of K to the GEMM's
+// step of 64) are zero.
+// A workgroup writes 256 kPrepOctets consecutive octets, a lane one of them (16 bytes) per store: whole lines, and all of a lane's
+// loads are issued before its first value is formed.  Bound by the writes (with the activations of 512 rows beside them): the two
+// 14336 x 4096 matrices of a Q4_K pair take 53 us (5.6 TB/s), a Q8_0 4096 x 4096 8.6; sixteen values per thread with an integer division per half,
+// exchanged through LDS, took 82 and 9.9.
+constexpr uint32_t kPrepOctets = 4;
+template <int T, bool BF16>
+__device__ __forceinline__ void dequant16bit_body(const uint8_t *__restrict__ W, uint16_t *__restrict__ out, uint32_t octs_per_row,
+                                                  uint32_t total_octs, int64_t row_bytes, int half, uint32_t octs, uint32_t block) {
+    // (an image holds at most 2^28 octets: 32-bit index arithmetic)
+    const uint32_t g0 = block * (256u * kPrepOctets), row0 = g0 / octs_per_row, rem0 = g0 - row0 * octs_per_row;  // uniform
+    // rows from row0 on: (l + 1/2) / octs_per_row is at least 1 / (2 octs_per_row) from a whole number, l is below 2^20 + 2^10 and the
+    // float quotient's relative error 2^-22, so that truncation finds the row
+    const float inv = 1.0f / (float)octs_per_row;
+    Octet<T> b[kPrepOctets];
+    uint32_t row[kPrepOctets], col[kPrepOctets];
+#pragma unroll
+    for (uint32_t u = 0; u < kPrepOctets; u++) {
+        const uint32_t l = min(rem0 + threadIdx.x + 256u * u, total_octs - 1u - g0 + rem0);
+        const uint32_t r = (uint32_t)(((float)l + 0.5f) * inv);
+        row[u] = row0 + r;
+        col[u] = l - r * octs_per_row;
+        b[u].load(W + (int64_t)row[u] * row_bytes, min(col[u], octs - 1u));
+    }
+#pragma unroll
+    for (uint32_t u = 0; u < kPrepOctets; u++) {
+        if (g0 + threadIdx.x + 256u * u >= total_octs) continue;
+        float w[8];
+        b[u].value(col[u], w);
+        uint4 v = make_uint4(Op16<BF16>::pack(w[0], w[1]), Op16<BF16>::pack(w[2], w[3]), Op16<BF16>::pack(w[4], w[5]), Op16<BF16>::pack(w[6], w[7]));
+        if (col[u] >= octs) v = make_uint4(0u, 0u, 0u, 0u);
+        const int64_t out_row = half == 0 ? (int64_t)row[u] : (int64_t)(row[u] >> 5) * 64 + (half - 1) * 32 + (row[u] & 31);
+        *reinterpret_cast<uint4 *>(out + (out_row * octs_per_row + col[u]) * 8) = v;
     }
 }
+uint32_t prep_blocks(int64_t total_octs) { return (uint32_t)((total_octs + 256 * kPrepOctets - 1) / (256 * kPrepOctets)); }
 
 template <int T, bool BF16>
-__global__ __launch_bounds__(256) void dequant16bit_kernel(const uint8_t *__restrict__ W, uint16_t *__restrict__ out, uint32_t runs_per_row,
-                                                          uint32_t total_runs, int64_t row_bytes, int half, uint32_t runs) {
-    dequant16bit_body<T, BF16>(W, out, runs_per_row, total_runs, row_bytes, half, runs, blockIdx.x);
+__global__ __launch_bounds__(256) void dequant16bit_kernel(const uint8_t *__restrict__ W, uint16_t *__restrict__ out, uint32_t octs_per_row,
+                                                          uint32_t total_octs, int64_t row_bytes, int half, uint32_t octs) {
+    dequant16bit_body<T, BF16>(W, out, octs_per_row, total_octs, row_bytes, half, octs, blockIdx.x);
 }
 
 // fp32 activations -> fp16 [M, K], one workgroup per row: the row is scaled by a power of two
@@ -552,11 +649,11 @@ __global__ __launch_bounds__(256) void gemm_slices_reduce_kernel(const float *__
 
 template <int T, bool BF16>
 int launch_dequant16bit(const uint8_t *W, int64_t N, int64_t K, uint16_t *out, hipStream_t s, int half) {
-    const int64_t runs = K / 16, runs_per_row = padded_k(K) / 16, total = N * runs_per_row;
+    const int64_t octs = K / 8, octs_per_row = padded_k(K) / 8, total = N * octs_per_row;
     const int64_t row_bytes = (K / Geom<T>::vpb) * Geom<T>::bpb;
-    if (total > ((int64_t)1 << 27)) return fail(GQ_ERR_INVALID, "gemm: a 16-bit image of %lld x %lld values is too large", (long long)N, (long long)K);
-    return launch(dequant16bit_kernel<T, BF16>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, W, out, (uint32_t)runs_per_row, (uint32_t)total,
-                  row_bytes, half, (uint32_t)runs);
+    if (total > ((int64_t)1 << 28)) return fail(GQ_ERR_INVALID, "gemm: a 16-bit image of %lld x %lld values is too large", (long long)N, (long long)K);
+    return launch(dequant16bit_kernel<T, BF16>, dim3(prep_blocks(total)), dim3(256), 0, s, W, out, (uint32_t)octs_per_row, (uint32_t)total, row_bytes, half,
+                  (uint32_t)octs);
 }
 
 template <bool BF16>
@@ -572,7 +669,7 @@ int launch_dequant16bit_type(int type, const uint8_t *W, int64_t N, int64_t K, u
 }
 
 // Both pre-passes of the fp32-activation route in ONE launch (they do not depend on each other): the first M workgroups
-// convert an activation row each (x_row_to_f16_body), the others 256 runs of weights each (dequant16bit_body), of W and -
+// convert an activation row each (x_row_to_f16_body), the others 1024 octets of weights each (dequant16bit_body), of W and -
 // for a gated pair, whose images interleave - of W2.  Rows of up to 16384 values (longer ones keep their own two-read kernel).
 // The matrices of one pre-pass: matrix i is W[i] with rows[i] rows, written from image row row0[i] on with the interleaving
 // `half[i]` of dequant16bit_body (a gated pair: both matrices at row 0 with halves 1 and 2; a set: halves 0, one after the other).
@@ -585,7 +682,7 @@ struct PrepMatrices {
 template <int T, int IT, bool NORM>
 __global__ __launch_bounds__(256) void prep_f32_kernel(const float *__restrict__ X, const float *__restrict__ gain, float gain_offset, float eps, int K,
                                                        uint16_t *__restrict__ xh, float *__restrict__ rowscale, uint32_t xblocks, PrepMatrices pm,
-                                                       uint16_t *__restrict__ wh, uint32_t runs_per_row, int64_t row_bytes, uint32_t runs) {
+                                                       uint16_t *__restrict__ wh, uint32_t octs_per_row, int64_t row_bytes, uint32_t octs) {
     const uint32_t b = blockIdx.x;
     if (b < xblocks) {
         x_row_to_f16_body<IT, NORM>(X, gain, gain_offset, eps, K, xh, rowscale, b);
@@ -597,20 +694,20 @@ __global__ __launch_bounds__(256) void prep_f32_kernel(const float *__restrict__
     for (int q = 1; q < 4; q++)
         if (q < pm.count && wb >= pm.blocks_end[q - 1]) i = q;
     const uint32_t first = i ? pm.blocks_end[i - 1] : 0u;
-    dequant16bit_body<T, false>(pm.W[i], wh + (size_t)pm.row0[i] * runs_per_row * 16, runs_per_row, pm.rows[i] * runs_per_row, row_bytes, pm.half[i], runs,
+    dequant16bit_body<T, false>(pm.W[i], wh + (size_t)pm.row0[i] * octs_per_row * 8, octs_per_row, pm.rows[i] * octs_per_row, row_bytes, pm.half[i], octs,
                                 wb - first);
 }
 
 template <int T>
 int launch_prep_f32_t(const float *x, int64_t M, int64_t K, const RmsNorm *norm, uint16_t *xh, float *rowscale, PrepMatrices pm, uint16_t *wh,
                       hipStream_t s) {
-    const int64_t runs = K / 16, runs_per_row = padded_k(K) / 16;
+    const int64_t octs = K / 8, octs_per_row = padded_k(K) / 8;
     const int64_t row_bytes = (K / Geom<T>::vpb) * Geom<T>::bpb;
     int64_t wblocks = 0;
     for (int i = 0; i < pm.count; i++) {
-        const int64_t total = (int64_t)pm.rows[i] * runs_per_row;
-        if (total > ((int64_t)1 << 27)) return fail(GQ_ERR_INVALID, "gemm: a 16-bit image of %u x %lld values is too large", pm.rows[i], (long long)K);
-        wblocks += (total + 255) / 256;
+        const int64_t total = (int64_t)pm.rows[i] * octs_per_row;
+        if (total > ((int64_t)1 << 28)) return fail(GQ_ERR_INVALID, "gemm: a 16-bit image of %u x %lld values is too large", pm.rows[i], (long long)K);
+        wblocks += prep_blocks(total);
         if (wblocks > INT32_MAX) return fail(GQ_ERR_INVALID, "gemm: too many workgroups in the pre-pass");
         pm.blocks_end[i] = (uint32_t)wblocks;
     }
@@ -620,7 +717,7 @@ int launch_prep_f32_t(const float *x, int64_t M, int64_t K, const RmsNorm *norm,
     const float off = norm ? norm->gain_offset : 0.f, eps = norm ? norm->eps : 0.f;
     const dim3 grid((unsigned)blocks), block(256);
     auto go = [&](auto kernel) {
-        return launch(kernel, grid, block, 0, s, x, gain, off, eps, (int)K, xh, rowscale, (uint32_t)M, pm, wh, (uint32_t)runs_per_row, row_bytes, (uint32_t)runs);
+        return launch(kernel, grid, block, 0, s, x, gain, off, eps, (int)K, xh, rowscale, (uint32_t)M, pm, wh, (uint32_t)octs_per_row, row_bytes, (uint32_t)octs);
     };
     if (padded_k(K) <= 4096) return norm ? go(prep_f32_kernel<T, 2, true>) : go(prep_f32_kernel<T, 2, false>);
     if (padded_k(K) <= 8192) return norm ? go(prep_f32_kernel<T, 4, true>) : go(prep_f32_kernel<T, 4, false>);

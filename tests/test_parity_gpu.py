@@ -450,6 +450,26 @@ def test_few_rows_in_one_launch(gpu, oracle, t, M, K, kind):
 
 
 @pytest.mark.parametrize("t", ALL_TYPES)
+@pytest.mark.parametrize("K,N", [(96, 131), (32, 2051), (2080, 67), (768, 1), (4352, 515)])
+@pytest.mark.parametrize("bf16", [False, True])
+def test_weight_image_of_the_two_pass_gemm_is_exact(gpu, oracle, t, K, N, bf16):
+    """Unit vectors through the two-pass GEMM return the columns of its 16-bit weight image: the exact values, rounded once.  Rows shorter
+    than a workgroup's 1024 octets and longer, last workgroups that are partly filled, K padded to the GEMM's step of 64 (N % 4 != 0 keeps
+    the split-K kernels away)."""
+    K = -(-K // ggml.values_per_block(t)) * ggml.values_per_block(t)
+    if bf16:
+        K = -(-K // 64) * 64   # (other K go to the fused kernel)
+    W = np.tile(synth.weights(t, 77 + t, min(N, 67), K), (-(-N // 67), 1))[:N]
+    w = np.tile(oracle.c_dequantize(t, W[:67], K), (-(-N // 67), 1))[:N]
+    cols = np.linspace(0, K - 1, 40).astype(int)
+    x = np.zeros((40, K), np.float32)
+    x[np.arange(40), cols] = 1.0
+    want = (bf16_round(w) if bf16 else w.astype(np.float16).astype(np.float32))[:, cols].T
+    got = run_dense(gpu, t, x, W, bf16=bf16)
+    assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("t", ALL_TYPES)
 def test_gemv_long_k_is_chunked(gpu, oracle, t):
     """K above the 16384 values one LDS pass holds."""
     K, N = 16384 + 4096, 19
