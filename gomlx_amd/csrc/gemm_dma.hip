@@ -11,8 +11,8 @@
 // both operands from global memory straight into LDS (buffer loads with the LDS modifier: no
 // registers, no vector-ALU instructions) two K steps ahead through a ring of three LDS stages.
 //
-// Tile: 256 x 128 per workgroup, 8 wavefronts x (64 x 64 = 2 x 2 v_mfma_f32_32x32x16), or 128 x 128
-// and 128 x 64 when the problem has too few large tiles to fill the chip; K in steps of 64.  LDS
+// Tile: 256 x 128 per workgroup, 8 wavefronts x (64 x 64 = 2 x 2 v_mfma_f32_32x32x16), 256 x 256 where
+// that fills the chip's rounds, 128 x 128 and 128 x 64 when the problem has too few large tiles for it (plan_gemm); K in steps of 64.  LDS
 // rows are 128 bytes, unpadded (the DMA writes 1 KB = 8 rows per wavefront instruction, lane l ->
 // bytes 16 l ..), and 16-byte chunk c of row r is kept in slot
 // c ^ ((r >> 1) & 7): 16 consecutive lanes of a fragment read then cover all 64 banks once.  The
@@ -359,7 +359,7 @@ int launch_x_to_f16(const float *x, int64_t M, int64_t K, const RmsNorm *norm, u
 
 // ---- pass 2: 16-bit GEMM with global -> LDS DMA --------------------------------------------------
 // X [M, K] and Wh [N, K] 16-bit, K % 64 == 0, both 16-byte aligned.  The workgroup tile is
-// (128 TM) x (64 TN): 4 x 2 wavefronts of (32 TM) x (32 TN) each.  TM = TN = 2 is the tile for
+// (128 TM) x (64 TN): 4 x 2 wavefronts of (32 TM) x (32 TN) each.  TM = 2 with TN = 2 or 4 are the tiles for
 // large problems; the smaller ones keep the chip full when M x N yields too few big tiles.
 template <int TM, int TN> struct DmaTile {
     static constexpr int DM = 128 * TM, DN = 64 * TN;
@@ -369,7 +369,7 @@ template <int TM, int TN> struct DmaTile {
     // because they leave room for one workgroup per CU instead of two.  (Also measured: the 256 x 128
     // tile on four wavefronts of 128 x 64, which reads a quarter less from LDS per MFMA but leaves a
     // SIMD a single wavefront: 112 .. 120 us against 81 .. 89 us at 2048 rows.)
-    static constexpr int NS = 3;
+    static constexpr int NS = kStageBytes * 3 <= 160 * 1024 ? 3 : 2;  // (256 x 256: two stages of 64 KB)
     static constexpr int kLdsBytes = NS * kStageBytes;
 };
 
@@ -509,39 +509,46 @@ __global__ __launch_bounds__(512) void gemm_dma_kernel(const uint16_t *X, const 
     // instructions per element: C3 through the two passes took 83.3 us against 75.9, fp32 prefill 98.3 against 87.3.)
     const int m0 = bm + wm + 4 * (lane >> 5);
     if constexpr (GATED) {
-        static_assert(TN == 2, "a gated tile pairs two 32-column blocks");
+        static_assert(TN % 2 == 0, "a gated tile pairs 32-column blocks");
         // (the image of a gated pair may have more rows than 2 n_out: the bound is on the output columns)
-        const int n = ((bn + wn) >> 1) + (lane & 31);
-        if (n >= n_out) return;
-        const float bg = bias ? bias[n] : 0.f, bu = bias2 ? bias2[n] : 0.f;
-        const int64_t at0 = (int64_t)m0 * n_out + n;
+        const int n0 = ((bn + wn) >> 1) + (lane & 31);
         auto store_all = [&](auto bounded, auto scaled, auto with_residual, auto activate) __attribute__((always_inline)) {
 #pragma unroll
-            for (int i = 0; i < TM; i++) {
-                const int rows_left = decltype(bounded)::value ? M - (bm + wm + i * 32) : 32;  // (see the plain form below)
-                if (rows_left <= 0) continue;
-                auto store16 = [&](auto checked) __attribute__((always_inline)) {
+            for (int jp = 0; jp < TN / 2; jp++) {
+                const int n = n0 + jp * 32;
+                if (n >= n_out) continue;
+                const float bg = bias ? bias[n] : 0.f, bu = bias2 ? bias2[n] : 0.f;
+                const int64_t at0 = (int64_t)m0 * n_out + n;
 #pragma unroll
-                    for (int r = 0; r < 16; r++) {
-                        const int dm = i * 32 + 8 * (r >> 2) + (r & 3);
-                        if constexpr (decltype(checked)::value) { if (m0 + dm >= M) continue; }
-                        float rs = 1.f;
-                        if (is_on(scaled)) rs = rowscale[m0 + dm];
-                        float v = activate(fmaf(acc[i][0][r], rs, bg)) * fmaf(acc[i][1][r], rs, bu);
-                        if (is_on(with_residual)) v += residual[at0 + (int64_t)dm * n_out];
-                        Y[at0 + (int64_t)dm * n_out] = v;
-                    }
-                };
-                if (rows_left >= 32) store16(std::false_type());
-                else store16(std::true_type());
+                for (int i = 0; i < TM; i++) {
+                    const int rows_left = decltype(bounded)::value ? M - (bm + wm + i * 32) : 32;  // (see the plain form below)
+                    if (rows_left <= 0) continue;
+                    auto store16 = [&](auto checked) __attribute__((always_inline)) {
+#pragma unroll
+                        for (int r = 0; r < 16; r++) {
+                            const int dm = i * 32 + 8 * (r >> 2) + (r & 3);
+                            if constexpr (decltype(checked)::value) { if (m0 + dm >= M) continue; }
+                            float rs = 1.f;
+                            if (is_on(scaled)) rs = rowscale[m0 + dm];
+                            float v = activate(fmaf(acc[i][2 * jp][r], rs, bg)) * fmaf(acc[i][2 * jp + 1][r], rs, bu);
+                            if (is_on(with_residual)) v += residual[at0 + (int64_t)dm * n_out];
+                            Y[at0 + (int64_t)dm * n_out] = v;
+                        }
+                    };
+                    if (rows_left >= 32) store16(std::false_type());
+                    else store16(std::true_type());
+                }
             }
         };
         // (SiLU, the activation of the feed-forward blocks this form exists for, gets the compile-time switches; the
         // others take row scales and residual as run-time tests, uniform over the wavefront: a quarter of the code)
         auto by_edge = [&](auto bounded) __attribute__((always_inline)) {
             auto silu = [](float v) { return v / (1.0f + __expf(-v)); };
-            if (act != kActSilu) store_all(bounded, rowscale != nullptr, residual != nullptr, [act](float v) { return apply_act(act, v); });
-            else if (rowscale && residual) store_all(bounded, std::true_type(), std::true_type(), silu);
+            // (the 256 x 256 tile is launched for SiLU only: 128 copies of the general activation are more than the compiler unrolls)
+            if constexpr (TN == 2) {
+                if (act != kActSilu) return store_all(bounded, rowscale != nullptr, residual != nullptr, [act](float v) { return apply_act(act, v); });
+            }
+            if (rowscale && residual) store_all(bounded, std::true_type(), std::true_type(), silu);
             else if (rowscale) store_all(bounded, std::true_type(), std::false_type(), silu);
             else if (residual) store_all(bounded, std::false_type(), std::true_type(), silu);
             else store_all(bounded, std::false_type(), std::false_type(), silu);
@@ -561,6 +568,7 @@ __global__ __launch_bounds__(512) void gemm_dma_kernel(const uint16_t *X, const 
             float *Y = Yall;               // (shadow the kernel's arguments: a segment brings its own output, row length and bias)
             const float *bias = bias_all;
             int N = Nall;
+            if constexpr (TN > 2 && !SEGS) asm volatile("" : "+s"(N)::"memory");  // (row offsets and the residual's loads of one column block at a time: of all four they spill)
             if constexpr (SEGS) {
                 int sg = 0;
 #pragma unroll
@@ -601,8 +609,10 @@ __global__ __launch_bounds__(512) void gemm_dma_kernel(const uint16_t *X, const 
     // residual are run-time tests, uniform over the wavefront: a quarter of the code)
     auto by_edge = [&](auto bounded) __attribute__((always_inline)) {
         auto none = [](float v) { return v; };
-        if (act != kActNone) store_all(bounded, rowscale != nullptr, residual != nullptr, [act](float v) { return apply_act(act, v); });
-        else if (rowscale && residual) store_all(bounded, std::true_type(), std::true_type(), none);
+        if constexpr (TN <= 2) {  // (the 256 x 256 tile is launched without an activation only, see above)
+            if (act != kActNone) return store_all(bounded, rowscale != nullptr, residual != nullptr, [act](float v) { return apply_act(act, v); });
+        }
+        if (rowscale && residual) store_all(bounded, std::true_type(), std::true_type(), none);
         else if (rowscale) store_all(bounded, std::true_type(), std::false_type(), none);
         else if (residual) store_all(bounded, std::false_type(), std::true_type(), none);
         else store_all(bounded, std::false_type(), std::false_type(), none);
@@ -772,50 +782,54 @@ int launch_gemm16_tile(const uint16_t *x, int64_t M, int64_t K, const uint16_t *
                   bias2, (int)n_out, residual, rowscale, segs ? *segs : GemmSegs{});
 }
 
-// GOMLX_HIPQ_GEMM_TILE=0|1|2 forces the 256x128 / 128x128 / 128x64 tile (tuning runs only).
+// GOMLX_HIPQ_GEMM_TILE=0|1|2|3 forces the 256x128 / 128x128 / 128x64 / 256x256 tile, GOMLX_HIPQ_GEMM_K_SLICES=n the number of K
+// slices where K may be split (tuning runs only).
 int tile_env() {
     static const int v = [] { const char *e = std::getenv("GOMLX_HIPQ_GEMM_TILE"); return e ? std::atoi(e) : -1; }();
     return v;
 }
-
-// Which tile: 0 = 256 x 128, 1 = 128 x 128 (one workgroup per CU each), 2 = 128 x 64 (two per CU).  The workgroups run in
-// rounds of one per CU; a round of 128 x 128 tiles takes about 0.61 of a round of 256 x 128 tiles, and a last round that is
-// only partly filled still costs a good half of a full one (the chip clocks higher and the memory system is less
-// crowded, but every workgroup walks all of K).  Estimated that way, the choice matches the faster tile in 22 of 24
-// measured cases (K = 4096 and 14336, N = 4096 and 14336, 640 .. 1536 rows) - e.g. 1280 rows on 4096 x 4096 are 160
-// large tiles in one round (57 us) or 320 small ones in two (70 us), where a rule by tile count alone took the small ones.
-int pick_tile(int64_t M, int64_t N) {
-    const int64_t cus = device_cu_count();
-    auto tiles = [&](int64_t dm, int64_t dn) { return ((M + dm - 1) / dm) * ((N + dn - 1) / dn); };
-    if (tiles(128, 64) <= cus) return 2;  // small problems: as long as the smallest tiles run in one round they win (512 rows on 4096 x 4096: 35 against 38 us; 640 rows: 48 against 39)
-    if (M <= 128) return 1;                       // (no half-empty 256-row tiles)
-    auto rounds = [&](int64_t wgs, double empty_round) {
-        const int64_t full = wgs / cus;
-        const double frac = (double)(wgs % cus) / (double)cus;
-        return (double)full + (frac > 0.0 ? empty_round + (1.0 - empty_round) * frac : 0.0);
-    };
-    const double t0 = rounds(tiles(256, 128), 0.6), t1 = 0.61 * rounds(tiles(128, 128), 0.5);
-    return t0 <= t1 ? 0 : 1;
-}
-
-// Few rows on a matrix with few columns leave most of the chip without a workgroup, each of the few walking all of K
-// (128 rows on 14336 -> 4096: 64 tiles of 128 x 64 on 256 CUs).  Then K is split into slices, as many as fill the chip
-// with at least 16 steps (1024 values) each, eight at most; the slices' sums go to `partial` ([slices][M][N] fp32) and a
-// small kernel adds them up and finishes them.  GOMLX_HIPQ_GEMM_K_SLICES=n forces n where it applies (1: never split).
 int k_slices_env() {
     static const int v = [] { const char *e = std::getenv("GOMLX_HIPQ_GEMM_K_SLICES"); return e ? std::atoi(e) : 0; }();
     return v;
 }
-int gemm_k_slices(int64_t M, int64_t K, int64_t N) {
-    if (N % 4 != 0) return 1;
-    const int64_t steps = K / DK, tiles = ((M + 127) / 128) * ((N + 63) / 64);
-    int64_t ns = std::min<int64_t>(std::min<int64_t>(device_cu_count() / tiles, steps / 16), 8);
-    if (k_slices_env() > 0) ns = std::min<int64_t>(std::min<int64_t>(k_slices_env(), steps), 8);
-    while (ns > 1 && (ns - 1) * ((steps + ns - 1) / ns) >= steps) ns--;  // no empty slice
-    return ns < 2 ? 1 : (int)ns;
+
+// Which tile - 0 = 256 x 128, 1 = 128 x 128, 2 = 128 x 64, 3 = 256 x 256 - and how many slices of K (whole steps each; their sums go to
+// `partial`, [slices][M][N] fp32, and a small kernel adds them up and finishes them): the smallest estimated time decides.  Workgroups
+// run in rounds of one per CU; a round costs its steps plus 6.5 (filling the ring, the epilogue) times the tile's time per step, and a
+// last round that is partly filled nearly as much as a full one; slices cost a launch and their sums' way through memory.  The constants
+// are fitted to 63 problems (K x N 4096x4096, 14336x4096, 4096x6144, 4096x14336, 2048x1536 and gated pairs, 64 .. 2048 rows) timed with
+// every tile and 1 2 3 4 6 8 slices: the choice is the fastest or within 3 % of it in 57 of them, within 7 % in the others.  E.g. (us,
+// weight image included, the former rule | this one; Q8_0):  4096x14336 at 768, 1024, 2048 rows 139 155 281 | 125 145 261 (256 x 256: a
+// wavefront's 64 x 128 share reads a quarter less from LDS per matrix instruction than 64 x 64, which that tile's time per step is
+// bound by), its gated pair at 512 and 1024 209 338 | 191 304, 4096x6144 at 2048 136 | 122; 14336x4096 at 256 and 512 rows 97 114 | 79 105
+// (slices where one round of small tiles filled the chip before).
+struct GemmPlan { int tile, slices; };
+GemmPlan plan_gemm(int64_t M, int64_t K, int64_t N, bool gated = false) {
+    constexpr int kTiles = 4, dm[kTiles] = {256, 128, 128, 256}, dn[kTiles] = {128, 128, 64, 256};
+    constexpr double step_us[kTiles] = {0.88, 0.61, 0.343, 1.476};
+    const int64_t cus = device_cu_count(), steps = (K + DK - 1) / DK;
+    GemmPlan best{1, 1};
+    double best_us = 1e30;
+    for (int t = 0; t < kTiles; t++) {
+        if (gated && t == 2) continue;
+        if (tile_env() >= 0 && tile_env() < kTiles && t != tile_env() && !(gated && tile_env() == 2)) continue;
+        const int64_t tiles = ((M + dm[t] - 1) / dm[t]) * ((N + dn[t] - 1) / dn[t]);
+        const int max_slices = gated || N % 4 != 0 ? 1 : (int)std::min<int64_t>(8, steps / 8);
+        for (int ns = 1; ns == 1 || ns <= max_slices; ns++) {
+            const int64_t per = (steps + ns - 1) / ns;
+            if (ns > 1 && (ns - 1) * per >= steps) continue;  // no empty slice
+            if (k_slices_env() > 0 && ns != std::max(1, std::min(k_slices_env(), max_slices))) continue;
+            const int64_t wgs = tiles * ns, full = wgs / cus;
+            const double frac = (double)(wgs % cus) / (double)cus;
+            double us = ((double)full + (frac > 0 ? 0.89 + 0.11 * frac : 0)) * ((double)per + 6.5) * step_us[t];
+            if (ns > 1) us += 2.05 + (double)(2 * ns + 1) * (double)M * (double)N * 4.0 / 3.6e6;
+            if (us < best_us) { best_us = us; best = {t, ns}; }
+        }
+    }
+    return best;
 }
 size_t gemm_partial_bytes(int64_t M, int64_t K, int64_t N) {
-    const int ns = gemm_k_slices(M, K, N);
+    const int ns = plan_gemm(M, K, N).slices;
     return ns > 1 ? (size_t)ns * (size_t)M * (size_t)N * sizeof(float) : 0;
 }
 template <class... P> bool aligned16(P... p) { return (((reinterpret_cast<uintptr_t>(p)) | ...) & 15) == 0; }  // (the reduction's float4 accesses)
@@ -826,21 +840,29 @@ int launch_slices_reduce(const float *partial, int slices, int64_t M, int64_t N,
                   residual, y, segs ? *segs : GemmSegs{}, segs ? 1 : 0);
 }
 
+// one launch of the chosen tile
+template <bool BF16, bool SEGS>
+int launch_gemm16_choice(int tile, const uint16_t *x, int64_t M, int64_t K, const uint16_t *Wh, int64_t N, const float *bias, int act, float *y,
+                         const float *residual, const float *rowscale, hipStream_t s, const GemmSegs *segs, int slices) {
+    switch (tile) {
+    case 3: return launch_gemm16_tile<BF16, 2, 4, false, SEGS>(x, M, K, Wh, N, bias, act, y, nullptr, N, residual, rowscale, s, segs, slices);
+    case 0: return launch_gemm16_tile<BF16, 2, 2, false, SEGS>(x, M, K, Wh, N, bias, act, y, nullptr, N, residual, rowscale, s, segs, slices);
+    case 1: return launch_gemm16_tile<BF16, 1, 2, false, SEGS>(x, M, K, Wh, N, bias, act, y, nullptr, N, residual, rowscale, s, segs, slices);
+    default: return launch_gemm16_tile<BF16, 1, 1, false, SEGS>(x, M, K, Wh, N, bias, act, y, nullptr, N, residual, rowscale, s, segs, slices);
+    }
+}
+
 // partial: room for gemm_partial_bytes(M, K, N), or null (then K is never split)
 template <bool BF16>
 int launch_gemm16(const uint16_t *x, int64_t M, int64_t K, const uint16_t *Wh, int64_t N, const float *bias, int act, float *y, hipStream_t s,
                   const float *residual = nullptr, const float *rowscale = nullptr, float *partial = nullptr) {
-    if (const int ns = partial && aligned16(bias, residual, y) ? gemm_k_slices(M, K, N) : 1; ns > 1) {
-        if (int rc = launch_gemm16_tile<BF16, 1, 1>(x, M, K, Wh, N, nullptr, kActNone, partial, nullptr, N, nullptr, nullptr, s, nullptr, ns)) return rc;
-        return launch_slices_reduce(partial, ns, M, N, rowscale, bias, act, residual, y, nullptr, s);
+    GemmPlan p = plan_gemm(M, K, N);
+    if (p.slices > 1 && partial && aligned16(bias, residual, y)) {
+        if (int rc = launch_gemm16_choice<BF16, false>(p.tile, x, M, K, Wh, N, nullptr, kActNone, partial, nullptr, nullptr, s, nullptr, p.slices)) return rc;
+        return launch_slices_reduce(partial, p.slices, M, N, rowscale, bias, act, residual, y, nullptr, s);
     }
-    int choice = pick_tile(M, N);
-    if (tile_env() >= 0 && tile_env() <= 2) choice = tile_env();
-    switch (choice) {
-    case 0: return launch_gemm16_tile<BF16, 2, 2>(x, M, K, Wh, N, bias, act, y, nullptr, N, residual, rowscale, s);
-    case 1: return launch_gemm16_tile<BF16, 1, 2>(x, M, K, Wh, N, bias, act, y, nullptr, N, residual, rowscale, s);
-    default: return launch_gemm16_tile<BF16, 1, 1>(x, M, K, Wh, N, bias, act, y, nullptr, N, residual, rowscale, s);
-    }
+    if (p.tile == 3 && act != kActNone) p.tile = 0;
+    return launch_gemm16_choice<BF16, false>(p.tile, x, M, K, Wh, N, bias, act, y, residual, rowscale, s, nullptr, 1);
 }
 
 // Several matrices' images one after the other, one GEMM, each segment's columns to its own output (fp16 operands).
@@ -849,17 +871,13 @@ int launch_gemm16_set(const uint16_t *x, int64_t M, int64_t K, const uint16_t *W
     const int64_t N = segs.n0[segs.count];
     bool aligned = true;
     for (int i = 0; i < segs.count; i++) aligned = aligned && aligned16(segs.bias[i], segs.y[i]);
-    if (const int ns = partial && aligned ? gemm_k_slices(M, K, N) : 1; ns > 1) {
-        if (int rc = launch_gemm16_tile<false, 1, 1>(x, M, K, Wh, N, nullptr, kActNone, partial, nullptr, N, nullptr, nullptr, s, nullptr, ns)) return rc;
-        return launch_slices_reduce(partial, ns, M, N, rowscale, nullptr, act, nullptr, nullptr, &segs, s);
+    GemmPlan p = plan_gemm(M, K, N);
+    if (p.slices > 1 && partial && aligned) {
+        if (int rc = launch_gemm16_choice<false, false>(p.tile, x, M, K, Wh, N, nullptr, kActNone, partial, nullptr, nullptr, s, nullptr, p.slices)) return rc;
+        return launch_slices_reduce(partial, p.slices, M, N, rowscale, nullptr, act, nullptr, nullptr, &segs, s);
     }
-    int choice = pick_tile(M, N);
-    if (tile_env() >= 0 && tile_env() <= 2) choice = tile_env();
-    switch (choice) {
-    case 0: return launch_gemm16_tile<false, 2, 2, false, true>(x, M, K, Wh, N, nullptr, act, nullptr, nullptr, N, nullptr, rowscale, s, &segs);
-    case 1: return launch_gemm16_tile<false, 1, 2, false, true>(x, M, K, Wh, N, nullptr, act, nullptr, nullptr, N, nullptr, rowscale, s, &segs);
-    default: return launch_gemm16_tile<false, 1, 1, false, true>(x, M, K, Wh, N, nullptr, act, nullptr, nullptr, N, nullptr, rowscale, s, &segs);
-    }
+    if (p.tile == 3 && act != kActNone) p.tile = 0;
+    return launch_gemm16_choice<false, true>(p.tile, x, M, K, Wh, N, nullptr, act, nullptr, nullptr, rowscale, s, &segs, 1);
 }
 
 // Gated pair (fp16 operands): the interleaved image has 64 rows per 32 outputs.
@@ -867,8 +885,9 @@ int64_t gated_image_rows(int64_t N) { return (N + 31) / 32 * 64; }
 int launch_gemm16_gated(const uint16_t *x, int64_t M, int64_t K, const uint16_t *Wh, int64_t N, const float *bias, const float *bias2, int act,
                         float *y, const float *residual, const float *rowscale, hipStream_t s) {
     const int64_t rows = gated_image_rows(N);
-    const bool big = pick_tile(M, rows) == 0;  // (the gated kernel exists for the two 128-column tiles)
-    if (big && tile_env() != 1) return launch_gemm16_tile<false, 2, 2, true>(x, M, K, Wh, rows, bias, act, y, bias2, N, residual, rowscale, s);
+    const int tile = plan_gemm(M, K, rows, true).tile;  // (the gated kernel exists for the tiles of 128 columns and more)
+    if (tile == 3 && act == kActSilu) return launch_gemm16_tile<false, 2, 4, true>(x, M, K, Wh, rows, bias, act, y, bias2, N, residual, rowscale, s);
+    if (tile == 3 || tile == 0) return launch_gemm16_tile<false, 2, 2, true>(x, M, K, Wh, rows, bias, act, y, bias2, N, residual, rowscale, s);
     return launch_gemm16_tile<false, 1, 2, true>(x, M, K, Wh, rows, bias, act, y, bias2, N, residual, rowscale, s);
 }
 

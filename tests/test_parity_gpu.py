@@ -469,6 +469,46 @@ def test_weight_image_of_the_two_pass_gemm_is_exact(gpu, oracle, t, K, N, bf16):
     assert np.array_equal(got, want)
 
 
+@pytest.mark.parametrize("M,K,N,kind", [(1000, 512, 14340, "plain"), (1000, 512, 14340, "bf16"), (1023, 512, 14339, "block"), (770, 256, 14336, "gated"),
+                                        (1000, 512, 7201, "gated"), (900, 512, 14336, "set"), (500, 8192, 2052, "block"), (300, 4096, 516, "set"),
+                                        (1000, 512, 14340, "gelu")])
+def test_large_tiles_and_slices_of_the_two_pass_gemm(gpu, oracle, M, K, N, kind):
+    """The 256 x 256 tile (edges in both directions, segments, the gated pairing, residual, an activation that keeps it away) and tiles whose K
+    is split.  Bound: both operands are rounded to 11 bits, 2^-11 each at most, 2^-11 / sqrt(3) in the mean, so 2^-11 * sqrt(2 / 3) of the
+    2-norm (4.0e-4); once more that for a product; bfloat16 operands of 8 bits eight times it."""
+    torch, t = gpu, Q8_0
+    q = Quantization(ggml_type=t)
+    gen = np.random.default_rng(M + N)
+    sizes = {"gated": [N, N], "set": [N // 2 // 32 * 32, N // 4 // 32 * 32, 64]}.get(kind, [N])
+    Ws = [np.tile(synth.weights(t, 91 + i, 131, K), (-(-n // 131), 1))[:n] for i, n in enumerate(sizes)]
+    ref = [torch.from_numpy(np.tile(oracle.c_dequantize(t, w[:131], K), (-(-len(w) // 131), 1))[:len(w)]).cuda().double() for w in Ws]
+    x = dev(torch, gen.standard_normal((M, K)).astype(np.float32))
+    if kind == "bf16":
+        x = x.to(torch.bfloat16)
+    Wd = [dev(torch, w) for w in Ws]
+    gain, bias = (dev(torch, gen.standard_normal(n).astype(np.float32)) for n in (K, N))
+    res = dev(torch, gen.standard_normal((M, N)).astype(np.float32))
+    norm = nn.RMSNorm(gain=gain, epsilon=1e-6) if kind in ("block", "gated", "set") else None
+    h = x.double()
+    if norm is not None:
+        h = h / torch.sqrt((h * h).mean(-1, keepdim=True) + 1e-6) * gain.double()
+    want = [h @ w.T for w in ref]
+    if kind == "gated":
+        got, want = [nn.gated_feed_forward(x, Wd[0], Wd[1], q, Activation.SILU, norm=norm)], [torch.nn.functional.silu(want[0]) * want[1]]
+    elif kind == "set":
+        got = nn.quantized_dense_batch([(x, w, q, None, None) for w in Wd], norm=norm)
+    elif kind == "block":
+        got, want = [nn.quantized_dense(x, Wd[0], q, bias, norm=norm, residual=res)], [want[0] + bias.double() + res.double()]
+    elif kind == "gelu":
+        got, want = [nn.quantized_dense(x, Wd[0], q, bias, Activation.GELU)], [torch.nn.functional.gelu(want[0] + bias.double())]
+    else:
+        got = [nn.quantized_dense(x, Wd[0], q)]
+    bound = 4.0e-4 * {"gated": 2, "bf16": 8}.get(kind, 1)
+    for g, w in zip(got, want):
+        err = ((g.double() - w).norm() / w.norm()).item()
+        assert err <= bound, err
+
+
 @pytest.mark.parametrize("t", ALL_TYPES)
 def test_gemv_long_k_is_chunked(gpu, oracle, t):
     """K above the 16384 values one LDS pass holds."""
