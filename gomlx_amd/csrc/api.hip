@@ -121,6 +121,10 @@ int stream_workspace(hipStream_t s, size_t bytes, void **out, int slot, uint32_t
     return GQ_OK;
 }
 
+namespace {
+bool serves_static_scratch() { return t_scope && t_scope->static_ptr; }  // (inside gq_qdense_f32_static)
+}  // namespace
+
 ProfileState &profile_state() {
     thread_local ProfileState ps;
     return ps;
@@ -199,22 +203,24 @@ int64_t split_k_from(int type, int64_t weight_bytes) {
     }
 }
 int64_t weight_bytes_of(int type, int64_t K, int64_t N) { return (int64_t)gq_row_bytes(type, K) * N; }
-// Last batch size of the split-K kernels before the two-pass GEMM takes over.  The split-K route streams W once per 32
-// batch rows; the two passes pay the 16-bit image (written once and read once, in proportion to N K) and a GEMM that splits
-// K itself while its tiles are fewer than the CUs.
-// Measured (python -m gomlx_amd.tune.crossover with GOMLX_HIPQ_SPLIT_K_TO=100000 and =16: us per call in a replayed graph of 20
-// calls on rotating weights, fp32 activations; rows 32 64 96 128 160 192; split-K | two passes at the same rows):
-//   Q8_0   4096x4096  16 22 27 29 35 36 | 27 28 29 30 31 31    4096x14336  32 37  43  49  69  76 | 56 56 55 58 69 69    14336x4096  32 38 44 49  70  77 | 63 70 72 73 81 82
-//   Q4_0   4096x4096  15 20 25 26 32 33 | 25 26 26 27 29 29    4096x14336  27 33  40  45  61  67 | 57 55 55 56 67 69    14336x4096  28 34 40 45  62  69 | 62 63 69 68 79 79
-//   Q4_K   4096x4096  15 17 21 29 36 38 | 26 26 27 29 30 30    4096x14336  25 28  34  38  53  57 | 61 59 60 60 73 72    14336x4096  21 30 36 41  55  59 | 69 73 72 71 85 85
-//          (at 256 320 384 rows: 4096x14336 74 96 108 | 74 94 95; 14336x4096 77 99 112 | 87 108 109.  Q4_K walks up to four tiles of 32 batch rows per
-//          launch; with one launch per 32 rows, as the other formats' kernels still work, it took 14 23 32 39 46 52, 27 44 61 79 96 113 and 22 36 49 63 77 92)
-//   Q6_K   4096x4096  19 22 30 32 39 40 | 26 28 29 30 31 32    4096x14336  36 56  76  89 109 130 | 61 57 58 59 70 71    14336x4096  36 56 77 90 111 132 | 68 68 74 74 82 83
-//   IQ4_NL 4096x4096  16 21 28 29 37 37 | 27 28 29 30 31 32    4096x14336  30 36  43  48  66  72 | 63 62 62 64 76 77    14336x4096  31 37 43 48  67  74 | 70 75 78 78 87 88
-//          (Q8_0, Q4_0 and IQ4_NL walk up to four tiles of 32 batch rows per launch on the large matrices, like Q4_K; one pass per 32 rows took
-//          33 52 71 84 100 118 / 33 52 72 85 104 121, 27 42 56 66 80 94 / 28 43 57 68 83 97 and 30 48 65 78 95 112 / 31 49 66 80 97 114; at 256
-//          rows the tiles take 79 - 90 against 70 - 90)
-// (Before the GEMM split K on narrow problems the two passes took 33 us on 4096x4096 and 92 .. 102 us on 14336x4096 at these rows.)
+// Last batch size of the split-K kernels before the two-pass GEMM takes over.  The split-K route streams W once per up to four tiles of
+// 32 batch rows (Q6_K: per tile); the two passes pay the 16-bit image (written once and read once, in proportion to N K) and a GEMM that
+// splits K itself where its tiles leave CUs idle.
+// Measured (GOMLX_HIPQ_SPLIT_K_TO=100000 and =16; us per call on rotating weights, fp32 activations; rows 32 64 96 128 160 192 256;
+// split-K | two passes at the same rows):
+//   Q8_0   4096x4096  16 22 27 29 35 36 44 | 24 24 24 25 29 29 30
+//          4096x14336 31 36 43 49 69 76 88 | 51 54 53 54 64 65 65    14336x4096 31 37 44 50 70 77 90 | 53 55 56 58 68 74 76
+//   Q4_0   4096x4096  14 19 24 26 32 33 39 | 23 24 24 25 28 28 29
+//          4096x14336 25 32 39 44 61 67 79 | 47 48 49 50 59 60 60    14336x4096 26 33 39 44 62 69 82 | 51 51 53 55 66 71 73
+//   Q4_K   4096x4096  14 17 20 28 36 38 44 | 25 24 25 25 29 29 30
+//          4096x14336 21 27 32 37 52 57 68 | 48 49 50 51 61 61 61    14336x4096 21 28 33 38 54 59 71 | 50 52 54 56 66 72 74
+//   Q6_K   4096x4096  18 21 29 32 39 41 50 | 25 25 25 27 30 30 31
+//          4096x14336 34 55 76 89 109 130 163 | 53 54 55 56 66 66 66    14336x4096 35 55 77 90 111 132 167 | 54 56 57 59 70 75 77
+//   IQ4_NL 4096x4096  15 21 27 29 37 37 45 | 23 24 24 25 28 29 30
+//          4096x14336 28 34 41 46 65 72 84 | 47 48 49 50 60 61 61    14336x4096 29 35 41 47 67 73 86 | 51 52 54 56 66 71 74
+//          (Q4_K at 320 rows: 4096x14336 88 | 85, 14336x4096 92 | 92)
+// The hand-over lies up to 64 rows beyond the point where the two passes are level: the split-K kernels contract exact weights, the two passes
+// weights rounded to 16 bits (a relative error of 5.6e-4 for Q4_K where the split-K kernels have 2.6e-4), and these few per cent do not buy that.
 // GOMLX_HIPQ_SPLIT_K_TO=rows overrides the table (tuning runs only).
 int64_t split_k_to_env() {
     static const int64_t v = [] { const char *e = std::getenv("GOMLX_HIPQ_SPLIT_K_TO"); return e ? (int64_t)std::atoll(e) : (int64_t)-1; }();
@@ -224,7 +230,7 @@ int64_t split_k_to(int type, int64_t K, int64_t N) {
     if (split_k_to_env() >= 0) return split_k_to_env();
     const bool large = weight_bytes_of(type, K, N) >= kLargeWeightBytes, long_k = K > N;
     switch (type) {
-    case GQ_Q8_0: return !large ? 128 : long_k ? 192 : 128;  // (4096x6144, 27 MB: 34 46 | 34 39 at 128 and 160 rows)
+    case GQ_Q8_0: return !large ? 128 : long_k ? 192 : 128;
     case GQ_Q4_0: return !large ? 128 : 192;
     case GQ_Q4_K: return !large ? 128 : long_k ? 320 : 256;
     case GQ_Q6_K: return !large ? 96 : 64;
@@ -234,14 +240,19 @@ int64_t split_k_to(int type, int64_t K, int64_t N) {
 }
 
 // The same point for a gated pair act(x.Wgate) * (x.Wup): both matrices are contracted against one activation image by the
-// split-K kernels, or dequantised into one interleaved image for ONE GEMM by the two passes.  Measured (same tool, mode
-// `gated`, SiLU; rows 32 64 96 128 160 192 256; split-K | two passes):
-//   Q8_0   4096x4096  24 35 39 45 52 58 73 | 46 45 46 46 47 46 46    4096x14336  50 60  72  86 122 136 161 | 112 117 123 129 142 145 151
-//   Q4_0   4096x4096  20 27 34 41 47 52 66 | 45 44 44 45 45 45 45    4096x14336  42 53  65  75 107 119 141 | 107 114 121 118 138 133 141
-//   Q4_K   4096x4096  17 22 27 32 44 48 60 | 46 45 45 45 46 46 45    4096x14336  37 46  55  65  92 101 121 | 118 125 131 128 147 142 151
-//          (one launch per 32 rows: 17 28 37 45 53 61 78 and 37 65 93 120 149 178 233; at 320 384 448 rows the large pair takes 173 198 243 | 203 205 209)
-//   Q6_K   4096x4096  28 33 43 51 59 67 85 | 46 46 46 46 47 46 46    4096x14336  57 89 129 161 200 231 302 | 112 117 124 127 138 137 146
-//   IQ4_NL 4096x4096  22 29 39 47 54 61 77 | 49 48 48 47 48 48 48    4096x14336  48 58  70  81 117 130 151 | 120 125 131 128 147 144 150
+// split-K kernels, or dequantised into one interleaved image for ONE GEMM by the two passes.  Measured (the same way, SiLU behind a
+// normalisation; rows 32 64 96 128 160 192 256; split-K | two passes):
+//   Q8_0   4096x4096  23 28 33 37 51 54 66 | 45 46 46 47 48 49 49
+//          4096x14336 53 63 76 88 126 139 165 | 115 118 123 129 144 145 152
+//   Q4_0   4096x4096  20 25 30 34 45 49 61 | 45 45 46 46 46 46 46
+//          4096x14336 43 54 67 78 110 122 144 | 106 111 113 120 135 131 137
+//   Q4_K   4096x4096  17 22 27 31 42 46 56 | 46 46 47 48 49 48 47
+//          4096x14336 31 45 55 64 93 103 125 | 108 112 115 122 137 133 139
+//   Q6_K   4096x4096  29 34 44 53 63 70 88 | 46 46 47 48 48 48 48
+//          4096x14336 58 92 132 166 204 235 308 | 117 120 126 131 144 146 153
+//   IQ4_NL 4096x4096  21 26 31 35 48 52 62 | 46 45 46 46 48 47 47
+//          4096x14336 48 59 72 82 120 133 155 | 108 111 114 120 130 132 131
+//          (Q4_K at 320 and 384 rows: 165 187 | 171 166; where the line lies and why: as above)
 // (The pair composed of two dense calls and a multiplication is never ahead of the one GEMM: 127 - 159 against 118 - 143 us
 // for Q4_K 4096 -> 2 x 14336 at 64 - 256 rows.)
 int64_t gated_split_k_to(int type, int64_t K, int64_t N) {
@@ -296,8 +307,10 @@ int split_k(int type, const void *x, bool x_is_bf16, int64_t M, int64_t K, int c
 int two_pass(int type, bool x_is_bf16, const void *x, int64_t M, int64_t K, const void *W, int64_t N, const float *bias, int act,
              float *y, hipStream_t s) {
     void *ws = nullptr;
-    if (int rc = stream_workspace(s, gemm_two_pass_workspace(x_is_bf16, M, K, N), &ws)) return rc;
-    return launch_gemm_two_pass(type, x_is_bf16, x, M, K, static_cast<const uint8_t *>(W), N, bias, act, y, ws, s);
+    // (K in one piece where the static scratch array holds the images but not the sums of its slices)
+    const bool split_k = !serves_static_scratch() || gemm_two_pass_workspace(x_is_bf16, M, K, N) <= kStaticScratchBytes - kWsSyncBytes;
+    if (int rc = stream_workspace(s, gemm_two_pass_workspace(x_is_bf16, M, K, N, split_k), &ws)) return rc;
+    return launch_gemm_two_pass(type, x_is_bf16, x, M, K, static_cast<const uint8_t *>(W), N, bias, act, y, ws, s, split_k);
 }
 
 }  // namespace

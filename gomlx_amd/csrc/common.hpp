@@ -105,7 +105,7 @@ int launch_mmv(int type, const void *x, bool x_is_bf16, int64_t M, int64_t K, in
 int launch_split_k_finish(const float *partial, const float *partial2, const float *xss, int nslices, int64_t M, int64_t K, int count,
                           const MmqSetItem *items, const MmqExtra *ex, hipStream_t s);
 // The K-sliced GEMV with the normalisation folded in and, when W2 is given, the gated product
-// act(x.W + bias) * (x.W2 + bias2); fp32 or bf16 activations, at most 16 rows (the entry points use it below 8 rows, where a pass per row still wins).
+// act(x.W + bias) * (x.W2 + bias2); fp32 or bf16 activations, at most 16 rows (the entry points use it for one and two rows, and where mmv.hip and the split-K kernels do not apply or are not ahead).
 bool gemv_ks_ext_supported(int type, int64_t M, int64_t K, int64_t N, const void *x, const void *gain);
 int launch_gemv_ks_ext(int type, const void *x, bool x_is_bf16, int64_t M, int64_t K, const RmsNorm *norm, const uint8_t *W, const float *bias,
                        const uint8_t *W2, const float *bias2, const float *residual, int64_t N, int act, float *y, hipStream_t s);
@@ -122,9 +122,10 @@ int launch_gemv_ks_batch_norm(int type, int count, const XsBatchItem *items, con
 // Large batches: dequantise W once into a 16-bit image (in `workspace`, gemm_two_pass_workspace()
 // bytes), then a plain 16-bit MFMA GEMM.
 bool gemm_two_pass_supported(int type, bool x_is_bf16, int64_t M, int64_t K, int64_t N, const void *x);
-size_t gemm_two_pass_workspace(bool x_is_bf16, int64_t M, int64_t K, int64_t N);
+// (split_k = false: K stays in one piece, and the workspace without room for the sums of its slices)
+size_t gemm_two_pass_workspace(bool x_is_bf16, int64_t M, int64_t K, int64_t N, bool split_k = true);
 int launch_gemm_two_pass(int type, bool x_is_bf16, const void *x, int64_t M, int64_t K, const uint8_t *W, int64_t N, const float *bias,
-                         int act, float *y, void *workspace, hipStream_t s);
+                         int act, float *y, void *workspace, hipStream_t s, bool split_k = true);
 // The two passes with the neighbours of a projection folded in (fp32 activations; same conditions as
 // gemm_two_pass_supported): RMS normalisation in the activation pass, residual in the GEMM epilogue;
 // with W2 one GEMM over the interleaved image of both matrices forms the gated product in registers.

@@ -804,7 +804,7 @@ int k_slices_env() {
 // bound by), its gated pair at 512 and 1024 209 338 | 191 304, 4096x6144 at 2048 136 | 122; 14336x4096 at 256 and 512 rows 97 114 | 79 105
 // (slices where one round of small tiles filled the chip before).
 struct GemmPlan { int tile, slices; };
-GemmPlan plan_gemm(int64_t M, int64_t K, int64_t N, bool gated = false) {
+GemmPlan plan_gemm(int64_t M, int64_t K, int64_t N, bool gated = false, bool may_split = true) {
     constexpr int kTiles = 4, dm[kTiles] = {256, 128, 128, 256}, dn[kTiles] = {128, 128, 64, 256};
     constexpr double step_us[kTiles] = {0.88, 0.61, 0.343, 1.476};
     const int64_t cus = device_cu_count(), steps = (K + DK - 1) / DK;
@@ -814,7 +814,7 @@ GemmPlan plan_gemm(int64_t M, int64_t K, int64_t N, bool gated = false) {
         if (gated && t == 2) continue;
         if (tile_env() >= 0 && tile_env() < kTiles && t != tile_env() && !(gated && tile_env() == 2)) continue;
         const int64_t tiles = ((M + dm[t] - 1) / dm[t]) * ((N + dn[t] - 1) / dn[t]);
-        const int max_slices = gated || N % 4 != 0 ? 1 : (int)std::min<int64_t>(8, steps / 8);
+        const int max_slices = gated || !may_split || N % 4 != 0 ? 1 : (int)std::min<int64_t>(8, steps / 8);
         for (int ns = 1; ns == 1 || ns <= max_slices; ns++) {
             const int64_t per = (steps + ns - 1) / ns;
             if (ns > 1 && (ns - 1) * per >= steps) continue;  // no empty slice
@@ -856,8 +856,9 @@ int launch_gemm16_choice(int tile, const uint16_t *x, int64_t M, int64_t K, cons
 template <bool BF16>
 int launch_gemm16(const uint16_t *x, int64_t M, int64_t K, const uint16_t *Wh, int64_t N, const float *bias, int act, float *y, hipStream_t s,
                   const float *residual = nullptr, const float *rowscale = nullptr, float *partial = nullptr) {
-    GemmPlan p = plan_gemm(M, K, N);
-    if (p.slices > 1 && partial && aligned16(bias, residual, y)) {
+    const bool may_split = partial && aligned16(bias, residual, y);
+    GemmPlan p = plan_gemm(M, K, N, false, may_split);
+    if (p.slices > 1) {
         if (int rc = launch_gemm16_choice<BF16, false>(p.tile, x, M, K, Wh, N, nullptr, kActNone, partial, nullptr, nullptr, s, nullptr, p.slices)) return rc;
         return launch_slices_reduce(partial, p.slices, M, N, rowscale, bias, act, residual, y, nullptr, s);
     }
@@ -871,8 +872,8 @@ int launch_gemm16_set(const uint16_t *x, int64_t M, int64_t K, const uint16_t *W
     const int64_t N = segs.n0[segs.count];
     bool aligned = true;
     for (int i = 0; i < segs.count; i++) aligned = aligned && aligned16(segs.bias[i], segs.y[i]);
-    GemmPlan p = plan_gemm(M, K, N);
-    if (p.slices > 1 && partial && aligned) {
+    GemmPlan p = plan_gemm(M, K, N, false, partial && aligned);
+    if (p.slices > 1) {
         if (int rc = launch_gemm16_choice<false, false>(p.tile, x, M, K, Wh, N, nullptr, kActNone, partial, nullptr, nullptr, s, nullptr, p.slices)) return rc;
         return launch_slices_reduce(partial, p.slices, M, N, rowscale, nullptr, act, nullptr, nullptr, &segs, s);
     }
@@ -926,16 +927,16 @@ size_t two_pass_front_bytes(bool x_is_bf16, int64_t M, int64_t Kp, int64_t rows)
     return align256((size_t)rows * Kp * 2) + (x_is_bf16 ? 0 : align256((size_t)M * Kp * 2) + align256((size_t)M * sizeof(float)));
 }
 }  // namespace
-size_t gemm_two_pass_workspace(bool x_is_bf16, int64_t M, int64_t K, int64_t N) {
+size_t gemm_two_pass_workspace(bool x_is_bf16, int64_t M, int64_t K, int64_t N, bool split_k) {
     K = padded_k(K);
-    return two_pass_front_bytes(x_is_bf16, M, K, N) + gemm_partial_bytes(M, K, N);
+    return two_pass_front_bytes(x_is_bf16, M, K, N) + (split_k ? gemm_partial_bytes(M, K, N) : 0);
 }
 
 int launch_gemm_two_pass(int type, bool x_is_bf16, const void *x, int64_t M, int64_t K, const uint8_t *W, int64_t N, const float *bias,
-                         int act, float *y, void *workspace, hipStream_t s) {
+                         int act, float *y, void *workspace, hipStream_t s, bool split_k) {
     uint16_t *wh = static_cast<uint16_t *>(workspace);
     const int64_t Kp = padded_k(K);
-    float *partial = reinterpret_cast<float *>(static_cast<uint8_t *>(workspace) + two_pass_front_bytes(x_is_bf16, M, Kp, N));
+    float *partial = split_k ? reinterpret_cast<float *>(static_cast<uint8_t *>(workspace) + two_pass_front_bytes(x_is_bf16, M, Kp, N)) : nullptr;
     if (x_is_bf16) {
         if (int rc = launch_dequant16bit_type<true>(type, W, N, K, wh, s)) return rc;
         return launch_gemm16<true>(static_cast<const uint16_t *>(x), M, K, wh, N, bias, act, y, s, nullptr, nullptr, partial);

@@ -105,3 +105,14 @@ def test_static_scratch_entry_rejects_what_does_not_fit(gpu):
     assert b"static buffer" in L.gq_last_error()
     gpu.cuda.synchronize()
     assert float(y.min()) == 7.0 and float(y.max()) == 7.0  # nothing was launched
+
+
+@pytest.mark.parametrize("t,M,K,N", [(ggml.Q4_0, 80, 4096, 4096), (ggml.Q8_0, 300, 2048, 2048)])
+def test_static_scratch_entry_serves_a_gemm_without_room_for_its_slices(gpu, oracle, t, M, K, N):
+    """A split-K batch of more than 64 rows, and a two-pass GEMM whose K slices' sums have no room beside the weight image: K in one piece."""
+    L = _lib.lib()
+    W, x = synth.weights(t, 9500 + t, N, K), synth.activations(9501 + t, M, K)
+    xd, Wd, y = _dev(gpu, x), _dev(gpu, W), gpu.full((M, N), float("nan"), device="cuda")
+    _lib.check(L.gq_qdense_f32_static(t, xd.data_ptr(), M, K, Wd.data_ptr(), N, None, 0, y.data_ptr(), gpu.cuda.current_stream().cuda_stream))
+    want = oracle.c_qdense(t, x, W)
+    assert float(np.max(np.abs(y.cpu().numpy().astype(np.float64) - want))) / float(np.max(np.abs(want))) < 1e-3
