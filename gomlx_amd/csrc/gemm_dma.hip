@@ -370,6 +370,11 @@ template <int TM, int TN> struct DmaTile {
     // tile on four wavefronts of 128 x 64, which reads a quarter less from LDS per MFMA but leaves a
     // SIMD a single wavefront: 112 .. 120 us against 81 .. 89 us at 2048 rows.)
     static constexpr int NS = kStageBytes * 3 <= 160 * 1024 ? 3 : 2;  // (256 x 256: two stages of 64 KB)
+    // A step's DMAs go out behind the fragment reads of its first groups, not all in front of them: issued at once they hold the
+    // wavefront's first LDS reads back (Q8_0 4096 x 4096 at 2048 rows 84.8 -> 82.9 us, 4096 -> 14336 at 512 rows 92.7 -> 90.1).  The
+    // 256 x 256 tile has one step for them to land and sends them in the first two groups; its matrix instructions run at raised
+    // priority over the other wavefront's reads (4096 -> 14336 at 2048 rows 262 -> 253; the smaller tiles lose 1 % by it).
+    static constexpr int kDmaGroups = NS == 3 ? 3 : 2;
     static constexpr int kLdsBytes = NS * kStageBytes;
 };
 
@@ -422,15 +427,17 @@ __global__ __launch_bounds__(512) void gemm_dma_kernel(const uint16_t *X, const 
     const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>(lds);
     const uint32_t xdst = __builtin_amdgcn_readfirstlane(lds0 + (uint32_t)(G::XI * wave) * 1024u);
     const uint32_t wdst = __builtin_amdgcn_readfirstlane(lds0 + (uint32_t)(G::DM * ROWB) + (uint32_t)(G::WI * wave) * 1024u);
-    auto issue = [&](int kt, int stage) __attribute__((always_inline)) {  // steps past the end re-read the last one (the data is never used)
+    // part `part` of `parts` of a step's DMAs (steps past the end re-read the last one: the data is never used)
+    auto issue = [&](int kt, int stage, int part, int parts) __attribute__((always_inline)) {
         const uint32_t soff = (uint32_t)(k0 + min(kt, nk - 1)) * (uint32_t)(DK * 2);
         const uint32_t sb = (uint32_t)stage * (uint32_t)G::kStageBytes;
 #pragma unroll
-        for (int j = 0; j < G::XI; j++) dma16(xdst + sb + (uint32_t)j * 1024u, xrsrc, xvoff[j], soff);
-#pragma unroll
-        for (int j = 0; j < G::WI; j++) dma16(wdst + sb + (uint32_t)j * 1024u, wrsrc, wvoff[j], soff);
+        for (int d = 0; d < G::XI + G::WI; d++) {
+            if (d * parts / (G::XI + G::WI) != part) continue;
+            if (d < G::XI) dma16(xdst + sb + (uint32_t)d * 1024u, xrsrc, xvoff[d < G::XI ? d : 0], soff);
+            else dma16(wdst + sb + (uint32_t)(d - G::XI) * 1024u, wrsrc, wvoff[d >= G::XI ? d - G::XI : 0], soff);
+        }
     };
-
     // ---- fragment addresses: row (w? + 32 t + lane % 32), chunk 2 kk + lane / 32, swizzled
     uint32_t aoff[4], boff[4];
     {
@@ -473,18 +480,20 @@ __global__ __launch_bounds__(512) void gemm_dma_kernel(const uint16_t *X, const 
     };
 
 #pragma unroll
-    for (int p = 0; p < G::NS - 1; p++) issue(p, p);
+    for (int p = 0; p < G::NS - 1; p++) issue(p, p, 0, 1);
     publish();
     // Step kt computes out of stage kt % NS while the DMAs of step kt + NS - 1 fill the stage that
     // every wavefront finished reading before the barrier that ended step kt - 1.  The MFMA groups
     // are skewed by one against the barriers (group 3 of a step issues after the barrier, behind
     // the first fragment reads of the next step).
     auto step = [&](int kt, int stage, bool first) __attribute__((always_inline)) {
-        issue(kt + G::NS - 1, (stage + G::NS - 1) % G::NS);
 #pragma unroll
         for (int kk = 0; kk < 4; kk++) {
             frags(stage, kk);
+            if (kk < G::kDmaGroups) issue(kt + G::NS - 1, (stage + G::NS - 1) % G::NS, kk, G::kDmaGroups);
+            if constexpr (G::NS == 2) __builtin_amdgcn_s_setprio(1);
             if (kk > 0 || !first) mfma_group((kk + 1) & 1);
+            if constexpr (G::NS == 2) __builtin_amdgcn_s_setprio(0);
             __builtin_amdgcn_sched_barrier(0);
         }
         publish();
