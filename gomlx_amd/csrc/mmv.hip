@@ -563,7 +563,8 @@ __global__ __launch_bounds__(512) void mmv_kernel(const void *__restrict__ X, co
                 am[m] = max3_abs(v[m][7], v[m][7], am[m]);
             }
             float my_sc, my_iv;
-            pow2_scale(rows_reduce<R>(am, lane, [](float a, float b) { return max3_abs(a, b, b); }), my_sc, my_iv);
+            const float top = rows_reduce<R>(am, lane, [](float a, float b) { return max3_abs(a, b, b); });
+            pow2_scale(top, my_sc, my_iv);
             if (row_writer<R>(lane)) invs[mine_row] = my_iv;
             uint32_t hi[R][4], lo[R][4];
 #pragma unroll
@@ -595,6 +596,17 @@ __global__ __launch_bounds__(512) void mmv_kernel(const void *__restrict__ X, co
                     sp.y = (_Float16)(sum - (float)sp.x);
                     if ((lane & 7) < 2) sums[m * 16 + 8 * (lane & 1) + (lane >> 3)] = as_u(sp);
                 }
+            }
+            // An infinite activation leaves lo = inf - inf: it becomes 0, and hi alone carries the infinity through the products as the
+            // reference's own sums do (NaN stays in hi; rows without an infinity never come here).
+            if (__builtin_amdgcn_ballot_w64(top == __builtin_inff()) != 0) {
+#pragma unroll
+                for (int m = 0; m < R; m++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        const uint32_t l = lo[m][e];
+                        lo[m][e] = ((l & 0x7C00u) == 0x7C00u ? 0u : l & 0xFFFFu) | ((l & 0x7C000000u) == 0x7C000000u ? 0u : l & 0xFFFF0000u);
+                    }
             }
             wave_fence();
             inv[s][0] = invs[2 * kg];

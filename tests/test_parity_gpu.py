@@ -449,6 +449,27 @@ def test_few_rows_in_one_launch(gpu, oracle, t, M, K, kind):
         assert err.max() <= (1e-5 if kind == "gated" else 4.8e-6), err
 
 
+@pytest.mark.parametrize("t", [Q4_0, Q8_0, Q6_K, IQ4_NL])
+@pytest.mark.parametrize("M,K,N,bf16", [(6, 4096, 4096, False), (16, 4096, 4096, True), (8, 8192, 2048, False), (12, 2560, 8192, False)])
+def test_infinite_activations_of_a_few_rows(gpu, oracle, t, M, K, N, bf16):
+    """Rows with +inf, with -inf and with both: every output is the infinity or the NaN that its weights' signs and zeros make of it
+    (inf * 0 and inf - inf), exactly as in 64 bits; the other rows stay finite.  (Q4_K's sub-block minima are a second sum,
+    so that an infinity meets its opposite there on every route.)"""
+    rng = np.random.default_rng(M + K)
+    W = np.tile(synth.weights(t, 77, 256, K), (N // 256, 1))
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    x[1, K - 3], x[3, 5], x[4, 17], x[4, K - 300] = np.inf, -np.inf, np.inf, -np.inf
+    if bf16:
+        x = bf16_round(x)
+    got = run_dense(gpu, t, x, W, bf16=bf16)
+    with np.errstate(invalid="ignore"):
+        want = np.tile(x.astype(np.float64) @ oracle.c_dequantize(t, W[:256], K).astype(np.float64).T, (1, N // 256))
+    for m in (1, 3, 4):
+        assert not np.isfinite(want[m]).any()
+        np.testing.assert_array_equal(got[m], want[m])
+    assert np.isfinite(np.delete(got, (1, 3, 4), axis=0)).all()
+
+
 @pytest.mark.parametrize("t", ALL_TYPES)
 @pytest.mark.parametrize("K,N", [(96, 131), (32, 2051), (2080, 67), (768, 1), (4352, 515)])
 @pytest.mark.parametrize("bf16", [False, True])
