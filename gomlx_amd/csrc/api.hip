@@ -269,6 +269,13 @@ int64_t gated_split_k_to(int type, int64_t K, int64_t N) {
     }
 }
 
+// Whether y [M, N] lies over any part of x [M, K].  The split-K kernels and the two passes have read x before the launch that writes y; a kernel
+// whose workgroups read x while others write y must not have such a call.
+bool y_over_x(const void *x, bool x_is_bf16, const float *y, int64_t M, int64_t K, int64_t N) {
+    const uintptr_t xa = reinterpret_cast<uintptr_t>(x), ya = reinterpret_cast<uintptr_t>(y);
+    return ya < xa + (uintptr_t)(M * K) * (x_is_bf16 ? 2 : 4) && xa < ya + (uintptr_t)(M * N) * sizeof(float);
+}
+
 // Whether 3 to 16 rows of up to 4096 values take the one-launch kernel of mmv.hip.  It costs about 5 us of activation conversion per
 // workgroup and then streams W once; the GEMV it replaces costs a pass per row over small matrices, per four rows (two with a
 // normalisation, a residual or a gated pair: `extras`) over those of 24 MB and more, the split-K kernels three launches.
@@ -297,7 +304,8 @@ bool takes_mmv(int type, int64_t M, int64_t K, int64_t N, const void *x, const v
 int split_k(int type, const void *x, bool x_is_bf16, int64_t M, int64_t K, int count, const MmqSetItem *items, const MmqExtra *ex, hipStream_t s) {
     const void *gain = ex && ex->norm ? ex->norm->gain : nullptr;
     bool mmv = type != GQ_Q4_K || M <= 8;
-    for (int i = 0; i < count; i++) mmv = mmv && mmv_supported(type, M, K, items[i].N, x, gain);
+    for (int i = 0; i < count; i++)
+        mmv = mmv && mmv_supported(type, M, K, items[i].N, x, gain) && !(mmv_one_launch(K) && y_over_x(x, x_is_bf16, items[i].y, M, K, items[i].N));
     if (mmv) return launch_mmv(type, x, x_is_bf16, M, K, count, items, ex, s);
     if (count > 1) return launch_mmq_set(type, x, x_is_bf16, M, K, count, items, ex ? ex->norm : nullptr, s);
     return launch_mmq(type, x, x_is_bf16, M, K, items[0].W, items[0].N, items[0].bias, items[0].act, items[0].y, s, ex);
@@ -485,7 +493,8 @@ int gq_qdense_f32(int type, const float *dX, int64_t M, int64_t K, const void *d
     // 5 .. 18 us per further 32; the two passes 33 .. 62 us for anything up to 128 rows.  Measured
     // crossovers: split_k_from() / split_k_to().
     const MmqSetItem one{(const uint8_t *)dW, N, dBias, act, dY};
-    if (takes_mmv(type, M, K, N, dX, nullptr, 1, false)) return launch_mmv(type, dX, false, M, K, 1, &one, nullptr, (hipStream_t)stream);
+    if (takes_mmv(type, M, K, N, dX, nullptr, 1, false) && !y_over_x(dX, false, dY, M, K, N))
+        return launch_mmv(type, dX, false, M, K, 1, &one, nullptr, (hipStream_t)stream);
     const bool tp = gemm_two_pass_supported(type, false, M, K, N, dX);
     const bool ks = M <= kGemvMaxRows && gemv_ks_supported(type, K, N, dX);
     const bool sk = M >= split_k_from(type, weight_bytes_of(type, K, N)) && mmq_supported(type, M, K, N, dX, dBias, dY) &&
@@ -590,7 +599,8 @@ int gq_qdense_bf16(int type, const uint16_t *dX, int64_t M, int64_t K, const voi
     // the fp16 activation image of the split-K kernels (which have no bf16 rounding of W: tighter than
     // the bf16 MFMA paths).
     const MmqSetItem one{(const uint8_t *)dW, N, dBias, act, dY};
-    if (takes_mmv(type, M, K, N, dX, nullptr, 1, false)) return launch_mmv(type, dX, true, M, K, 1, &one, nullptr, (hipStream_t)stream);
+    if (takes_mmv(type, M, K, N, dX, nullptr, 1, false) && !y_over_x(dX, true, dY, M, K, N))
+        return launch_mmv(type, dX, true, M, K, 1, &one, nullptr, (hipStream_t)stream);
     const bool tp = gemm_two_pass_supported(type, true, M, K, N, dX);
     const bool ks = M <= kGemvMaxRows && gemv_ks_supported(type, K, N, dX);
     const bool sk = M >= split_k_from(type, weight_bytes_of(type, K, N)) && mmq_supported(type, M, K, N, dX, dBias, dY) &&
@@ -718,7 +728,8 @@ int gq_qdense_block_f32(int type, const float *dX, int64_t M, int64_t K, const g
     if (norm) rn = RmsNorm{norm->dGain, norm->eps, norm->gain_offset};
     const MmqSetItem one{(const uint8_t *)dW, N, dBias, act, dY};
     const MmqExtra ex{nullptr, nullptr, dResidual, norm ? &rn : nullptr};
-    if (takes_mmv(type, M, K, N, dX, rn.gain, 1, true)) return launch_mmv(type, dX, false, M, K, 1, &one, &ex, (hipStream_t)stream);
+    if (takes_mmv(type, M, K, N, dX, rn.gain, 1, true) && !y_over_x(dX, false, dY, M, K, N))
+        return launch_mmv(type, dX, false, M, K, 1, &one, &ex, (hipStream_t)stream);
     if (fold_into_gemv(type, M, K, N, dX, rn.gain, dBias, dY, false))
         return launch_gemv_ks_ext(type, dX, false, M, K, norm ? &rn : nullptr, (const uint8_t *)dW, dBias, nullptr, nullptr, dResidual, N, act, dY,
                                   (hipStream_t)stream);
@@ -830,7 +841,8 @@ int gq_qdense_gated_f32(int type, const float *dX, int64_t M, int64_t K, const g
     if (norm) rn = RmsNorm{norm->dGain, norm->eps, norm->gain_offset};
     const MmqSetItem one{(const uint8_t *)dWgate, N, dBiasGate, act, dY};
     const MmqExtra ex{(const uint8_t *)dWup, dBiasUp, nullptr, norm ? &rn : nullptr};
-    if (takes_mmv(type, M, K, N, dX, rn.gain, 2, true)) return launch_mmv(type, dX, false, M, K, 1, &one, &ex, (hipStream_t)stream);
+    if (takes_mmv(type, M, K, N, dX, rn.gain, 2, true) && !y_over_x(dX, false, dY, M, K, N))
+        return launch_mmv(type, dX, false, M, K, 1, &one, &ex, (hipStream_t)stream);
     if (fold_into_gemv(type, M, K, N, dX, rn.gain, dBiasGate, dY, true))
         return launch_gemv_ks_ext(type, dX, false, M, K, norm ? &rn : nullptr, (const uint8_t *)dWgate, dBiasGate, (const uint8_t *)dWup, dBiasUp,
                                   nullptr, N, act, dY, (hipStream_t)stream);
@@ -890,7 +902,8 @@ int gq_qdense_block_bf16(int type, const uint16_t *dX, int64_t M, int64_t K, con
     const RmsNorm rn = norm ? RmsNorm{norm->dGain, norm->eps, norm->gain_offset} : RmsNorm{nullptr, 0.f, 0.f};
     const MmqSetItem one{(const uint8_t *)dW, N, dBias, act, dY};
     const MmqExtra ex{nullptr, nullptr, dResidual, norm ? &rn : nullptr};
-    if (takes_mmv(type, M, K, N, dX, rn.gain, 1, true)) return launch_mmv(type, dX, true, M, K, 1, &one, &ex, (hipStream_t)stream);
+    if (takes_mmv(type, M, K, N, dX, rn.gain, 1, true) && !y_over_x(dX, true, dY, M, K, N))
+        return launch_mmv(type, dX, true, M, K, 1, &one, &ex, (hipStream_t)stream);
     if (fold_into_gemv(type, M, K, N, reinterpret_cast<const float *>(dX), norm ? norm->dGain : nullptr, dBias, dY, false)) {
         return launch_gemv_ks_ext(type, dX, true, M, K, norm ? &rn : nullptr, (const uint8_t *)dW, dBias, nullptr, nullptr, dResidual, N, act, dY,
                                   (hipStream_t)stream);
@@ -920,7 +933,8 @@ int gq_qdense_gated_bf16(int type, const uint16_t *dX, int64_t M, int64_t K, con
     const RmsNorm rn = norm ? RmsNorm{norm->dGain, norm->eps, norm->gain_offset} : RmsNorm{nullptr, 0.f, 0.f};
     const MmqSetItem one{(const uint8_t *)dWgate, N, dBiasGate, act, dY};
     const MmqExtra ex{(const uint8_t *)dWup, dBiasUp, nullptr, norm ? &rn : nullptr};
-    if (takes_mmv(type, M, K, N, dX, rn.gain, 2, true)) return launch_mmv(type, dX, true, M, K, 1, &one, &ex, (hipStream_t)stream);
+    if (takes_mmv(type, M, K, N, dX, rn.gain, 2, true) && !y_over_x(dX, true, dY, M, K, N))
+        return launch_mmv(type, dX, true, M, K, 1, &one, &ex, (hipStream_t)stream);
     if (fold_into_gemv(type, M, K, N, reinterpret_cast<const float *>(dX), norm ? norm->dGain : nullptr, dBiasGate, dY, true)) {
         return launch_gemv_ks_ext(type, dX, true, M, K, norm ? &rn : nullptr, (const uint8_t *)dWgate, dBiasGate, (const uint8_t *)dWup, dBiasUp, nullptr,
                                   N, act, dY, (hipStream_t)stream);

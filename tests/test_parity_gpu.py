@@ -1209,6 +1209,45 @@ def test_residual_in_place_on_the_composed_path(gpu, oracle):
         assert err < TOL_F32, (ggml.name(t), M, K, N, use_norm, err)
 
 
+@pytest.mark.parametrize("t", ALL_TYPES)
+@pytest.mark.parametrize("call", ["dense", "block", "gated"])
+def test_output_over_its_own_input(gpu, oracle, t, call):
+    """8 rows of 4096 values, y written over x itself (a block: x, residual and y one buffer) and over half of it: the routes that take such
+    calls have read x before they write y, so that the result is the oracle's (bounds of a contraction, twice that for a product)."""
+    import ctypes
+    from gomlx_amd import _lib
+    torch = gpu
+    L, M, K, sp = _lib.lib(), 8, 4096, torch.cuda.current_stream().cuda_stream
+    Ws = [np.tile(synth.weights(t, 90 + i, 256, K), (K // 256, 1)) for i in range(2)]
+    x = synth.activations(92, M, K)
+    W0, W1 = (dev(torch, w) for w in Ws)
+    norm = ctypes.byref(_lib.RmsNormDesc(None, 1e-5, 0.0))
+    want = np.tile(oracle.c_qdense(t, x, Ws[0][:256]), (1, K // 256))
+    if call != "dense":
+        xn = oracle.c_rmsnorm(x, np.ones(K, np.float32), 1e-5, 0.0)
+        g, u = (np.tile(oracle.c_qdense(t, xn, w[:256]), (1, K // 256)).astype(np.float64) for w in Ws)
+        want = g + x if call == "block" else g / (1 + np.exp(-g)) * u
+    for shift in (0, M * K // 2):
+        buf = torch.zeros(2 * M * K, device="cuda")
+        buf[:M * K] = dev(torch, x).flatten()
+        xp, yp = buf.data_ptr(), buf.data_ptr() + 4 * shift
+        _lib.check(L.gq_profile_begin())
+        if call == "dense":
+            rc = L.gq_qdense_f32(t, xp, M, K, W0.data_ptr(), K, None, 0, yp, sp)
+        elif call == "block":
+            res = buf if shift == 0 else buf[:M * K].clone()
+            rc = L.gq_qdense_block_f32(t, xp, M, K, norm, W0.data_ptr(), K, None, 0, res.data_ptr(), yp, sp)
+        else:
+            rc = L.gq_qdense_gated_f32(t, xp, M, K, norm, W0.data_ptr(), None, W1.data_ptr(), None, K, 3, yp, sp)
+        _lib.check(rc)
+        launches, us = ctypes.c_int(0), ctypes.c_double(0.0)
+        _lib.check(L.gq_profile_end(ctypes.byref(launches), ctypes.byref(us)))
+        assert launches.value > 1  # (one launch would read x and write y at once, and be right only by luck)
+        got = buf[shift:shift + M * K].view(M, K).cpu().numpy()
+        scale = np.abs(want - x).max() if call == "block" else np.abs(g).max() * np.abs(u).max() if call == "gated" else np.abs(want).max()
+        assert np.abs(got - want).max() < (2 if call == "gated" else 1) * TOL_F32 * scale, (call, shift)
+
+
 def test_two_host_threads_share_the_null_stream(gpu, oracle):
     """Split-K calls (three kernels that share the stream's workspace) issued concurrently from two host threads on the
     null stream: every result matches the oracle, i.e. the launch sequences were not interleaved."""
