@@ -315,7 +315,8 @@ int split_k(int type, const void *x, bool x_is_bf16, int64_t M, int64_t K, int c
 int two_pass(int type, bool x_is_bf16, const void *x, int64_t M, int64_t K, const void *W, int64_t N, const float *bias, int act,
              float *y, hipStream_t s) {
     void *ws = nullptr;
-    // (K in one piece where the static scratch array holds the images but not the sums of its slices)
+    // (K in one piece where the static scratch array holds the images but not the sums of its slices: another order of the same fp32 sums, as
+    // the header says.  Held to the slices that fit, gq_qdense_f32 would return the same bits, at 28.7 us for 21.5 on 4096 -> 1024 at 520 rows.)
     const bool split_k = !serves_static_scratch() || gemm_two_pass_workspace(x_is_bf16, M, K, N) <= kStaticScratchBytes - kWsSyncBytes;
     if (int rc = stream_workspace(s, gemm_two_pass_workspace(x_is_bf16, M, K, N, split_k), &ws)) return rc;
     return launch_gemm_two_pass(type, x_is_bf16, x, M, K, static_cast<const uint8_t *>(W), N, bias, act, y, ws, s, split_k);

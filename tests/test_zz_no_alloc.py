@@ -1,6 +1,6 @@
 """The entry point that allocates nothing (gq_qdense_f32_static) against gq_qdense_f32, through the C ABI.
 
-Same kernels, so the results must be bit-identical; the scratch memory is the library's fixed device
+Same kernels, so the results must be bit-identical (but where the slices of a two-pass GEMM have no room: see the last test); the scratch memory is the library's fixed device
 array, which keeps the previous call's contents: two calls in a row, the second smaller, both checked.
 Collected last on purpose (a failure here must not hide the tests before it)."""
 import numpy as np
@@ -116,3 +116,22 @@ def test_static_scratch_entry_serves_a_gemm_without_room_for_its_slices(gpu, ora
     _lib.check(L.gq_qdense_f32_static(t, xd.data_ptr(), M, K, Wd.data_ptr(), N, None, 0, y.data_ptr(), gpu.cuda.current_stream().cuda_stream))
     want = oracle.c_qdense(t, x, W)
     assert float(np.max(np.abs(y.cpu().numpy().astype(np.float64) - want))) / float(np.max(np.abs(want))) < 1e-3
+
+
+@pytest.mark.parametrize("t,M,K,N,fits", [(ggml.Q8_0, 300, 2048, 2048, True), (ggml.Q6_K, 130, 2048, 3072, True), (ggml.IQ4_NL, 520, 1056, 4096, True),
+                                          (ggml.Q4_0, 512, 4096, 1024, False), (ggml.Q8_0, 700, 4096, 1024, False)])
+def test_static_scratch_entry_against_the_allocating_one_around_the_limit(gpu, oracle, t, M, K, N, fits):
+    """Two-pass GEMMs of a few megabytes of image.  With room for the K slices' sums: the same bits.  Without: the same products summed in one piece;
+    either side's fp32 sums of K terms are within 2^-24 sqrt(K) of the products' 2-norm in the mean, four times that allowed."""
+    if fits:
+        return _both(gpu, oracle, t, M, K, N, 9600 + t, act=3)
+    L = _lib.lib()
+    W, x = synth.weights(t, 9600 + t, N, K), synth.normal(9601 + t, 0, M * K).reshape(M, K).astype(np.float32)
+    xd, Wd, stream = _dev(gpu, x), _dev(gpu, W), gpu.cuda.current_stream().cuda_stream
+    y = [gpu.full((M, N), float("nan"), device="cuda") for _ in range(2)]
+    for entry, out in zip((L.gq_qdense_f32, L.gq_qdense_f32_static), y):
+        _lib.check(entry(t, xd.data_ptr(), M, K, Wd.data_ptr(), N, None, 0, out.data_ptr(), stream))
+    a, b = (v.cpu().numpy().astype(np.float64) for v in y)
+    w = oracle.c_dequantize(t, W, K).astype(np.float64)
+    size = np.linalg.norm(x.astype(np.float64)) * np.linalg.norm(w) / K ** 0.5   # 2-norm over the outputs of sums of independent products
+    assert np.linalg.norm(a - b) <= 4 * 2.0 ** -24 * K ** 0.5 * size
