@@ -7,6 +7,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import warnings
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libgomlx_hipq.so")
@@ -92,7 +93,8 @@ class NotImplementedByBackend(HipqError):
 
 _lib = None
 _initialised = False
-fast = None  # the native host path (csrc/binding.cpp), bound to the loaded library by init()
+fast = None  # the native host path (csrc/binding.cpp), bound to the loaded library by bind_fast()
+_fast_tried = False
 
 # Entry points the native host path calls, in the order in which csrc/binding.cpp takes them.
 _BOUND = ("gq_qdense_check", "gq_qdense_f32", "gq_qdense_bf16", "gq_qdense_block_f32", "gq_qdense_block_bf16", "gq_qdense_gated_f32",
@@ -127,10 +129,27 @@ def check(status: int) -> None:
 
 def init(device: int = 0) -> None:
     """gq_init once per process; raises if there is no gfx950 device."""
-    global _initialised, fast
+    global _initialised
     if not _initialised:
         check(lib().gq_init(device))
-        from . import _binding
-        _binding.bind(*(ctypes.cast(getattr(lib(), name), ctypes.c_void_p).value for name in _BOUND))
-        fast = _binding
         _initialised = True
+
+
+def bind_fast() -> None:
+    """Binds the native host path, once per process, for callers that work on torch tensors (the module links torch's libraries and
+    needs them loaded).  Where it does not load - another build of torch - or the library in use lacks an entry point - an older
+    build under comparison - ``fast`` stays None, and the Python steps of nn.py do the same work."""
+    global fast, _fast_tried
+    if _fast_tried:
+        return
+    _fast_tried = True
+    L = lib()
+    if not all(hasattr(L, name) for name in _BOUND):
+        return
+    try:
+        from . import _binding
+    except ImportError as e:
+        warnings.warn(f"gomlx_amd: calls take the slower host path in Python ({e})")
+        return
+    _binding.bind(*(ctypes.cast(getattr(L, name), ctypes.c_void_p).value for name in _BOUND))
+    fast = _binding

@@ -11,8 +11,8 @@ torch only supplies device memory and the current stream; all arithmetic runs in
 libgomlx_hipq.so.  There is no CPU path: tensors must live on the GPU.
 
 The operators of a decode loop first try the same steps in native code (``_lib.fast``,
-csrc/binding.cpp; bound when the library is initialised, so from a process's second call on);
-it returns None for whatever it does not take, and the Python steps below then run or raise.
+csrc/binding.cpp; bound by the first of these calls, so used from a process's second one on); it
+returns None for whatever it does not take, and the Python steps below then run or raise.
 """
 from __future__ import annotations
 
@@ -68,6 +68,11 @@ class Quantization:
     block_size: int = 0
 
 
+def _init(device: int) -> None:
+    _lib.init(device)
+    _lib.bind_fast()
+
+
 def _stream_ptr(t: torch.Tensor) -> int:
     return torch.cuda.current_stream(t.device).cuda_stream
 
@@ -90,7 +95,7 @@ def dequantize(weights: torch.Tensor, ggml_type: int) -> torch.Tensor:
         return out
     _require_cuda("weights", weights)
     _weights_2d(weights)
-    _lib.init(weights.device.index or 0)
+    _init(weights.device.index or 0)
     N, rb = weights.shape
     bpb = ggml.bytes_per_block(ggml_type)
     if rb % bpb:
@@ -125,7 +130,7 @@ def rms_norm(x: torch.Tensor, norm: RMSNorm) -> torch.Tensor:
         raise _lib.NotImplementedByBackend(_lib.ERR_NOT_IMPLEMENTED, f"rms_norm: dtype {x.dtype} is not implemented")
     K = x.shape[-1]
     d = norm._desc(K)
-    _lib.init(x.device.index or 0)
+    _init(x.device.index or 0)
     y = torch.empty_like(x)
     _lib.check(_lib.lib().gq_rmsnorm_f32(x.data_ptr(), x.numel() // K if K else 0, K, d.dGain, d.eps, d.gain_offset, y.data_ptr(),
                                          _stream_ptr(x)))
@@ -166,7 +171,7 @@ def gated_feed_forward(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor
             blen = b.shape[0]
         _lib.check(L.gq_qdense_check(quant.ggml_type, xd, M, K_in, N, rb, blen, activation.to_backend(), ctypes.byref(K)))
     d = None if norm is None else norm._desc(K.value)
-    _lib.init(x.device.index or 0)
+    _init(x.device.index or 0)
     y = torch.empty(x.shape[:-1] + (N,), dtype=torch.float32, device=x.device)
     fn = L.gq_qdense_gated_f32 if xd == _lib.F32 else L.gq_qdense_gated_bf16
     _lib.check(fn(quant.ggml_type, x.data_ptr(), M, K.value, None if d is None else ctypes.byref(d),
@@ -220,7 +225,7 @@ def quantized_dense(x: torch.Tensor, weights: torch.Tensor, quant: Quantization,
     import ctypes
     K = ctypes.c_int64(0)
     _lib.check(L.gq_qdense_check(quant.ggml_type, xd, M, K_in, N, rb, blen, act.to_backend(), ctypes.byref(K)))
-    _lib.init(x.device.index or 0)
+    _init(x.device.index or 0)
     y = torch.empty(x.shape[:-1] + (N,), dtype=torch.float32, device=x.device)
     if norm is not None or residual is not None:
         d = None if norm is None else norm._desc(K.value)
@@ -252,7 +257,7 @@ def quantized_gather(table: torch.Tensor, indices: torch.Tensor, quant: Quantiza
     if indices.dim() < 1 or indices.shape[-1] != 1:
         raise ValueError("indices must have last dimension 1")
     idx = indices.to(torch.int32).contiguous()
-    _lib.init(table.device.index or 0)
+    _init(table.device.index or 0)
     vocab, rb = table.shape
     bpb = ggml.bytes_per_block(quant.ggml_type)
     if rb % bpb:
@@ -309,7 +314,7 @@ def quantized_dense_batch(problems, norm: RMSNorm | None = None) -> list:
         d.type, d.act, d.dX, d.M, d.K = quant.ggml_type, act.to_backend(), x.data_ptr(), M, K.value
         d.dW, d.N, d.dBias, d.dY = weights.data_ptr(), N, (None if bias is None else bias.data_ptr()), y.data_ptr()
     if problems:
-        _lib.init(problems[0][0].device.index or 0)
+        _init(problems[0][0].device.index or 0)
         if norm is None:
             _lib.check(L.gq_qdense_f32_batch(len(problems), descs, _stream_ptr(problems[0][0])))
         else:

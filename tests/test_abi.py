@@ -4,6 +4,7 @@ like the reference's graph-build checks.  No kernel is launched here."""
 import ctypes
 import os
 import re
+import sys
 
 import pytest
 
@@ -210,6 +211,33 @@ def test_python_wrapper_maps_statuses_to_exceptions():
     assert e.value.status == _lib.ERR_INVALID and not isinstance(e.value, _lib.NotImplementedByBackend)
     with pytest.raises(_lib.NotImplementedByBackend):
         _lib.check(_lib.lib().gq_qdense_f32(99, 16, 1, 32, 16, 1, None, 0, 16, None))
+
+
+def test_initialisation_needs_neither_torch_nor_the_native_host_path():
+    """gq_init through ctypes in a process that never loads torch (a stub stands in for the device), and a second library
+    that lacks an entry point the native host path calls: both stay usable."""
+    import subprocess
+    code = """
+import sys
+from gomlx_amd import _lib
+L = _lib.lib()
+L.gq_init = lambda device: _lib.OK
+_lib.init(0)
+assert _lib._initialised and _lib.fast is None and "torch" not in sys.modules
+
+class Older:  # what hasattr sees of a library without one of the entry points
+    def __getattr__(self, name):
+        if name == "gq_qdense_norm_bf16_batch":
+            raise AttributeError(name)
+        return getattr(L, name)
+
+_lib._lib = Older()
+_lib.init(0)
+_lib.bind_fast()
+assert _lib.fast is None and "torch" not in sys.modules
+"""
+    r = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
 
 
 def test_activation_mapping_quirks():
