@@ -135,8 +135,8 @@ def init(device: int = 0) -> None:
         _initialised = True
 
 
-def bind_fast() -> None:
-    """Binds the native host path, once per process, for callers that work on torch tensors (the module links torch's libraries and
+def bind_fast(activation: type) -> None:
+    """Binds the native host path (``activation``: the enumeration nn.Activation), once per process, for callers that work on torch tensors (the module links torch's libraries and
     needs them loaded).  Where it does not load - another build of torch - or the library in use lacks an entry point - an older
     build under comparison - ``fast`` stays None, and the Python steps of nn.py do the same work."""
     global fast, _fast_tried
@@ -151,5 +151,5 @@ def bind_fast() -> None:
     except ImportError as e:
         warnings.warn(f"gomlx_amd: calls take the slower host path in Python ({e})")
         return
-    _binding.bind(*(ctypes.cast(getattr(L, name), ctypes.c_void_p).value for name in _BOUND))
+    _binding.bind(activation, *(ctypes.cast(getattr(L, name), ctypes.c_void_p).value for name in _BOUND))
     fast = _binding

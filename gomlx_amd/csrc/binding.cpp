@@ -12,6 +12,7 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <climits>
 #include <initializer_list>
 
 #include "../../include/gomlx_hipq.h"
@@ -37,6 +38,7 @@ struct Entry {
 } g;
 constexpr int kEntries = 15;
 bool g_bound = false;
+PyTypeObject *g_activation = nullptr;  // nn.Activation
 PyObject *s_scheme, *s_ggml_type, *s_gain, *s_epsilon, *s_scale_offset;
 
 // activation.Type.ToBackend by the numeric value of nn.Activation
@@ -48,7 +50,7 @@ bool to_long(PyObject *o, long &v) {
     if (!PyLong_Check(o)) return false;  // (IntEnum members are ints)
     v = PyLong_AsLong(o);
     if (v == -1 && PyErr_Occurred()) { PyErr_Clear(); return false; }
-    return true;
+    return v >= INT_MIN && v <= INT_MAX;
 }
 bool attr_long(PyObject *o, PyObject *name, long &v) {
     PyObject *a = PyObject_GetAttr(o, name);
@@ -72,10 +74,10 @@ bool ggml_type_of(PyObject *quant, int &type) {
     type = (int)t;
     return true;
 }
+// A member of nn.Activation itself: a bare number or a member of another enumeration says nothing about which function is meant.
 bool backend_act(PyObject *act, int &v) {
-    long a = 0;
-    if (act != Py_None && !to_long(act, a)) return false;
-    if (a < 0 || a >= 13) return false;
+    long a;
+    if (Py_TYPE(act) != g_activation || !to_long(act, a) || a < 0 || a >= 13) return false;
     v = kBackendAct[a];
     return true;
 }
@@ -158,7 +160,7 @@ template <class F> PyObject *guarded(F f) {
     }
 }
 
-// dense(x, weights, quant, bias, activation | None, norm, residual)
+// dense(x, weights, quant, bias, activation, norm, residual)
 PyObject *dense(PyObject *, PyObject *const *a, Py_ssize_t n) {
     return guarded([&]() -> PyObject * {
         int type, act;
@@ -195,7 +197,7 @@ PyObject *gated(PyObject *, PyObject *const *a, Py_ssize_t n) {
         int type, act;
         Operands o;
         Norm norm;
-        if (n != 8 || !ggml_type_of(a[3], type) || a[4] == Py_None || !backend_act(a[4], act)) return none();
+        if (n != 8 || !ggml_type_of(a[3], type) || !backend_act(a[4], act)) return none();
         const at::Tensor *up = gpu_tensor(a[2]);
         if (!o.read(a[0], a[1], type, act, -1) || !up || up->scalar_type() != at::kByte || up->sizes() != o.w->sizes()) return none();
         const float *bg, *bu;
@@ -212,7 +214,7 @@ PyObject *gated(PyObject *, PyObject *const *a, Py_ssize_t n) {
     });
 }
 
-// batch(problems, norm): up to eight (x, weights, quant, bias, activation) tuples
+// batch(problems, norm): up to eight (x, weights, quant, bias, activation | None) tuples
 PyObject *batch(PyObject *, PyObject *const *a, Py_ssize_t n) {
     return guarded([&]() -> PyObject * {
         if (n != 2 || !(PyList_Check(a[0]) || PyTuple_Check(a[0]))) return none();
@@ -224,9 +226,9 @@ PyObject *batch(PyObject *, PyObject *const *a, Py_ssize_t n) {
         bool bf16 = false;
         for (Py_ssize_t i = 0; i < count; i++) {
             PyObject *p = PySequence_Fast_GET_ITEM(a[0], i);
-            int type, act;
-            if (!PyTuple_Check(p) || PyTuple_GET_SIZE(p) != 5 || !ggml_type_of(PyTuple_GET_ITEM(p, 2), type) || !backend_act(PyTuple_GET_ITEM(p, 4), act))
-                return none();
+            int type, act = GQ_ACT_NONE;
+            if (!PyTuple_Check(p) || PyTuple_GET_SIZE(p) != 5 || !ggml_type_of(PyTuple_GET_ITEM(p, 2), type)) return none();
+            if (PyTuple_GET_ITEM(p, 4) != Py_None && !backend_act(PyTuple_GET_ITEM(p, 4), act)) return none();
             const float *bias;
             if (!o.read(PyTuple_GET_ITEM(p, 0), PyTuple_GET_ITEM(p, 1), type, act, -1) || vector_of(PyTuple_GET_ITEM(p, 3), o.N, bias) < 0) return none();
             if (i == 0) bf16 = o.bf16;
@@ -303,12 +305,12 @@ PyObject *gather(PyObject *, PyObject *const *a, Py_ssize_t n) {
     });
 }
 
-// bind(address, ...): the entry points in the order of Entry
+// bind(Activation, address, ...): the enumeration of nn.py, the entry points in the order of Entry
 PyObject *bind(PyObject *, PyObject *const *a, Py_ssize_t n) {
-    if (n != kEntries) { PyErr_Format(PyExc_TypeError, "bind takes %d addresses", kEntries); return nullptr; }
+    if (n != kEntries + 1 || !PyType_Check(a[0])) { PyErr_Format(PyExc_TypeError, "bind takes a type and %d addresses", kEntries); return nullptr; }
     void *p[kEntries];
     for (int i = 0; i < kEntries; i++) {
-        p[i] = PyLong_AsVoidPtr(a[i]);
+        p[i] = PyLong_AsVoidPtr(a[i + 1]);
         if (!p[i]) {
             if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "null address");
             return nullptr;
@@ -316,6 +318,9 @@ PyObject *bind(PyObject *, PyObject *const *a, Py_ssize_t n) {
     }
     static_assert(sizeof(Entry) == sizeof p, "one pointer per entry point");
     std::memcpy(static_cast<void *>(&g), p, sizeof p);
+    Py_INCREF(a[0]);
+    Py_XDECREF(reinterpret_cast<PyObject *>(g_activation));
+    g_activation = reinterpret_cast<PyTypeObject *>(a[0]);
     g_bound = true;
     return none();
 }

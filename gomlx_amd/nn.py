@@ -70,7 +70,7 @@ class Quantization:
 
 def _init(device: int) -> None:
     _lib.init(device)
-    _lib.bind_fast()
+    _lib.bind_fast(Activation)
 
 
 def _stream_ptr(t: torch.Tensor) -> int:
@@ -192,7 +192,7 @@ def quantized_dense(x: torch.Tensor, weights: torch.Tensor, quant: Quantization,
     projection and Add(residual, ...) after it, ml/zoo/transformer/transformer.go:1099-1101, 1045, 1055.
     """
     if _lib.fast is not None and len(optional_activation) <= 1:
-        y = _lib.fast.dense(x, weights, quant, bias, optional_activation[0] if optional_activation else None, norm, residual)
+        y = _lib.fast.dense(x, weights, quant, bias, optional_activation[0] if optional_activation else Activation.NONE, norm, residual)
         if y is not None:
             return y
     if len(optional_activation) > 1:

@@ -233,7 +233,7 @@ class Older:  # what hasattr sees of a library without one of the entry points
 
 _lib._lib = Older()
 _lib.init(0)
-_lib.bind_fast()
+_lib.bind_fast(int)
 assert _lib.fast is None and "torch" not in sys.modules
 """
     r = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True)

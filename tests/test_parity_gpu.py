@@ -1877,6 +1877,29 @@ def test_native_host_path_equals_the_python_steps(gpu, monkeypatch, shape, bf16)
         assert a.dtype == b.dtype and a.shape == b.shape and a.device == b.device and gpu.equal(a, b)
 
 
+def test_an_activation_is_a_member_of_its_enumeration(gpu):
+    """Bare numbers, None where the argument is given, and members of other enumerations (the C ABI's Relu is 2, nn's Sigmoid too)
+    are refused, with the native host path bound as without it."""
+    import enum
+
+    class Abi(enum.IntEnum):
+        RELU = 2
+
+    K, N = 256, 32
+    w = dev(gpu, synth.weights(Q8_0, 710, N, K))
+    q, x = Quantization(ggml_type=Q8_0), gpu.ones(1, K, device="cuda")
+    nn.quantized_dense(x, w, q, None, Activation.RELU)  # (binds the native path)
+    for bad in (0, 1, 2, Abi.RELU, True):
+        for call in (lambda: nn.quantized_dense(x, w, q, None, bad), lambda: nn.gated_feed_forward(x, w, w, q, bad),
+                     lambda: nn.quantized_dense_batch([(x, w, q, None, bad)]), lambda: nn.quantized_dense_batch([(x, w, q, None, None)] * 2 + [(x, w, q, None, bad)])):
+            with pytest.raises(AttributeError):
+                call()
+    for call in (lambda: nn.quantized_dense(x, w, q, None, None), lambda: nn.gated_feed_forward(x, w, w, q, None)):
+        with pytest.raises(AttributeError):
+            call()
+    assert gpu.equal(nn.quantized_dense_batch([(x, w, q, None, None)])[0], nn.quantized_dense(x, w, q))
+
+
 # ------------------------------------------------------------------------------ recorded replays and timing hooks
 
 def test_recorded_chain_replays_match_eager(gpu, oracle):
