@@ -4,6 +4,7 @@
 #include "blocks.hpp"
 #include "common.hpp"
 
+#include <algorithm>
 #include <climits>
 
 namespace gq {
@@ -111,13 +112,14 @@ template <> struct Quad<kQ6_K> {  // (block layout: see dequant16<kQ6_K>)
 template <int T, int U, bool NT>
 __global__ __launch_bounds__(256) void dequant_rows_kernel(const uint8_t *__restrict__ W, float *__restrict__ out, int64_t rows,
                                                            int64_t quads_per_row, uint32_t rows_per_wg, uint32_t chunks, int64_t row_bytes, const int32_t *__restrict__ indices,
-                                                           int64_t vocab, int32_t *__restrict__ err_flag) {
+                                                           int64_t vocab, int32_t *__restrict__ err_flag, uint32_t first_wg) {
     int64_t r = 0, src = 0;
-    uint32_t chunk = blockIdx.x, lane = threadIdx.x;
+    const uint32_t wg = first_wg + blockIdx.x;
+    uint32_t chunk = wg, lane = threadIdx.x;
     bool bad = false;
     if (indices) {  // gather: row r of the output is row indices[r] of the table
-        const uint32_t group = blockIdx.x / chunks;
-        chunk = blockIdx.x - group * chunks;
+        const uint32_t group = wg / chunks;
+        chunk = wg - group * chunks;
         r = group;
         if (rows_per_wg > 1) {  // (rows of fewer than 256 quads: several of them to a workgroup; U is 1 then)
             const uint32_t sub = lane / (uint32_t)quads_per_row;
@@ -163,9 +165,14 @@ int launch_rows(const uint8_t *W, float *out, int64_t N, int64_t K, const int32_
     const int64_t chunks = wide ? (quads + 1023) / 1024 : (quads + 255) / 256, per_wg = quads >= 256 || !indices ? 1 : 256 / quads;
     const int64_t groups = (rows + per_wg - 1) / per_wg;
     if (chunks > INT_MAX / groups) return fail(GQ_ERR_NOT_IMPLEMENTED, "dequantize: %lld x %lld values in one call", (long long)N, (long long)K);
+    // (a launch takes fewer than 2^32 threads: a gather of more than 2^24 rows of 1024 values, 64 GB of them, needs several)
+    constexpr int64_t kMaxWgs = ((int64_t)1 << 24) - 1;
     auto go = [&](auto kernel) {
-        return launch(kernel, dim3((unsigned)(groups * chunks)), dim3(256), 0, s, W, out, rows, quads, (uint32_t)per_wg, (uint32_t)chunks, row_bytes,
-                      indices, vocab, err_flag);
+        for (int64_t first = 0; first < groups * chunks; first += kMaxWgs)
+            if (int rc = launch(kernel, dim3((unsigned)std::min(groups * chunks - first, kMaxWgs)), dim3(256), 0, s, W, out, rows, quads, (uint32_t)per_wg,
+                                (uint32_t)chunks, row_bytes, indices, vocab, err_flag, (uint32_t)first))
+                return rc;
+        return (int)GQ_OK;
     };
     if (!wide) return go(dequant_rows_kernel<T, 1, false>);
     return rows * quads * 16 >= kStreamBytes ? go(dequant_rows_kernel<T, 4, true>) : go(dequant_rows_kernel<T, 4, false>);

@@ -1837,6 +1837,25 @@ def test_gather_random_rows_bit_exact(gpu, oracle, t):
     assert np.array_equal(out.view(np.uint32), want.view(np.uint32))
 
 
+def test_gather_of_more_rows_than_one_launch_holds(gpu):
+    """2^24 + 3 rows of 544 values (36.5 GB), a workgroup per row: more threads than a launch takes.  Rows around the seam and at both
+    ends against the dequantised table, bit for bit, an index out of range behind the seam reported."""
+    import ctypes
+    from gomlx_amd import _lib
+    K, vocab, count = 544, 64, (1 << 24) + 3
+    table = dev(gpu, synth.weights(Q8_0, 125, vocab, K))
+    rows = nn.dequantize(table, Q8_0)
+    idx = (gpu.arange(count, dtype=gpu.int64, device="cuda") * 7 % vocab).to(gpu.int32)
+    idx[-1] = vocab
+    out = gpu.empty((count, K), dtype=gpu.float32, device="cuda")
+    flag = gpu.zeros(1, dtype=gpu.int32, device="cuda")
+    _lib.check(_lib.lib().gq_embedding_lookup(Q8_0, table.data_ptr(), vocab, K, idx.data_ptr(), count, out.data_ptr(), flag.data_ptr(),
+                                              gpu.cuda.current_stream().cuda_stream))
+    for lo, hi in ((0, 1000), ((1 << 23) - 500, (1 << 23) + 500), (count - 1000, count - 1)):
+        assert gpu.equal(out[lo:hi], rows[idx[lo:hi].long()])
+    assert int(flag.item()) == 1 and bool(gpu.isnan(out[-1]).all())
+
+
 def test_gather_out_of_range_index_raises(gpu):
     table = synth.weights(Q8_0, 120, 10, 64)
     for bad in (10, -1):
