@@ -747,9 +747,16 @@ int launch_mmv_rows(const void *x, const MmvArgs &a, const Plan &p, hipStream_t 
                                    L::bytes(kMaxWaves)) == hipSuccess;
     }();
     if (!lds_ok) return fail(GQ_ERR_HIP, "mmv: cannot reserve %d bytes of LDS", L::bytes(kMaxWaves));
-    // one workgroup per CU (two of up to four wavefronts), the slices' groups sharing them; the tiles are dealt out round-robin
-    const int per_cu = p.waves <= 4 && SETS == 1 ? 2 : 1;
-    const int gx = std::max(1, std::min(a.ntiles, device_cu_count() * per_cu / p.groups));
+    // Eight wavefronts per CU, two per SIMD, as registers and LDS hold them: one workgroup of five to eight, two of three or four, four of
+    // two, eight of one; the slices' groups share them, the tiles are dealt out round-robin.  (With one workgroup per CU, short rows left
+    // three quarters of the chip's loads unissued from nine rows on: Q4_0 1024 -> 32768 at 12 rows 32.2 us for 18.8, Q8_0
+    // 256 -> 32768 46.8 for 15.3 at 16.)  Two sets of rows convert for half a microsecond longer where a SIMD has both wavefronts
+    // converting: a second workgroup of three or four wavefronts pays from three tiles per CU on (Q8_0 2048 -> 8192 at 12 rows, two tiles:
+    // 13.1 us with it, 12.4 without; -> 16384, four tiles: 17.4 and 18.2).
+    const int cus = device_cu_count();
+    int per_cu = kMaxWaves / p.waves;
+    if (SETS == 2 && per_cu == 2 && a.ntiles < 3 * cus) per_cu = 1;
+    const int gx = std::max(1, std::min(a.ntiles, cus * per_cu / p.groups));
     return launch(mmv_kernel<T, BF, SETS, R>, dim3((unsigned)gx, (unsigned)p.groups), dim3((unsigned)p.waves * 64), (size_t)L::bytes(p.waves), s, x, a);
 }
 
