@@ -276,6 +276,67 @@ bool y_over_x(const void *x, bool x_is_bf16, const float *y, int64_t M, int64_t 
     return ya < xa + (uintptr_t)(M * K) * (x_is_bf16 ? 2 : 4) && xa < ya + (uintptr_t)(M * N) * sizeof(float);
 }
 
+// Rows x MB up to which the GEMV stays ahead of mmv.hip over 9 to 24 MB (0: nowhere).  Three things decide besides the product.  From 2^24
+// values on the GEMV's workgroups have three row-steps and more, below one or two, and a row's conversion costs more than its share of
+// the weights; rows of 2049 to 3584 values leave some of a CU's wavefront slots empty in it; and extras cost it registers.  Measured (us on rotating
+// weights, rows 3 4 5; GEMV | mmv.hip):
+//   Q8_0  1536x6144   6.1  7.1  8.1 |  8.0  8.2  9.1   2048x6144  7.2  8.4  9.5 |  8.7  8.7  9.5   2048x8192   8.8 10.4 12.0 |  9.5  9.6 10.4
+//         3072x3072   6.9  8.5  9.6 |  8.0  8.2  9.0   4096x3072  8.8  9.5 11.2 |  8.6  8.6  9.5   4096x4096  10.0 12.1 14.5 |  9.4  9.6 10.3
+//         three 4096x1024 of one input 7.1 7.7 8.8 | 8.2 8.2 9.2;  gated 4096x1536 8.9 9.5 14.2 | 10.0 10.0 11.0;  behind a norm 1536x6144 7.8 12.9 13.0 | 8.7 8.7 9.8
+//   Q6_K  2048x6144   8.3 10.1 11.7 |  9.2  9.3 10.3   4096x3072  8.9 10.4 12.7 |  9.1  9.2 10.3   1024x16384 10.4 12.6 15.0 |  9.7  9.8 10.6
+//   Q4_0  1536x12288  6.5  7.8  8.8 |  8.6  8.5 10.1   4096x6144  7.9  9.3 10.9 | 10.0 10.1 10.8   4096x4096 (2^24 values) 7.6 9.2 11.0 | 8.2 8.3 9.0
+//         gated 1536x6144 7.5 8.5 10.2 | 9.9 9.9 11.0
+//   Q4_K  1536x12288  7.6  9.2 10.7 |  8.8  8.7 10.2   4096x6144  9.1 10.9 12.9 |  9.5  9.6 11.1   4096x4096   9.2 11.2 13.3 |  8.2  8.2  9.8
+//   IQ4_NL gated 1536x6144 10.1 11.8 14.6 | 11.1 11.1 12.1
+// (K from 1024: narrower matrices of 9 MB have 12000 rows and more; Q8_0 768x12544 at 3 rows takes 8.5 us where the GEMV took 7.0.)
+int64_t gemv_reach(int type, int64_t K, int64_t values, int matrices, bool extras, bool set) {
+    if (K < 1024) return 0;
+    const bool shallow = values <= (int64_t)1 << 24, is_short = K <= 2048, gaps = !is_short && K <= 3584;
+    if (matrices == 2) {
+        if (gaps || type == GQ_Q6_K) return 0;
+        if (type == GQ_Q8_0) return 58;
+        if (is_short && shallow) return 0;
+        return type != GQ_Q4_0 ? 32 : is_short ? 55 : 37;
+    }
+    if (extras) return !is_short ? 0 : type == GQ_Q8_0 ? 40 : type == GQ_Q4_K && !shallow ? 32 : 0;
+    switch (type) {
+    case GQ_Q8_0: return is_short || set ? 58 : 36;
+    case GQ_Q6_K: return K < 1536 ? 0 : is_short || set ? 38 : 28;
+    case GQ_Q4_0: return shallow ? 0 : gaps ? 52 : 58;
+    case GQ_Q4_K: return shallow || gaps ? 0 : 40;
+    default: return 0;
+    }
+}
+
+// Whether the split-K kernels are ahead of mmv.hip where both take a call (a matrix - of a pair: each - of 6 MB and more).  mmv.hip contracts
+// 9 to 16 rows as two sets of 8, the split-K kernels up to 32 at one price: Q4_K and the other 4-bit formats, whose weights take least of
+// the time, feel that from 9 rows on.  And where the slices of K do not come out in groups of eight, mmv.hip leaves wavefront slots
+// empty.  Measured (us, split-K | mmv.hip):
+//   Q4_K    K <= 4096, 12 rows: 4096x14336 19.0 | 20.5, gated pairs of it 27.8 | 26.3, of 3072x6144 17.3 | 18.8, of 1024x16384 16.1 | 17.2
+//           8 and 12 rows: 14336x4096 17.8 18.1 | 17.6 22.7, 8192x8192 22.5 22.9 | 17.2 23.5; 8 rows: 4608x4096 12.6 | 13.2, behind a norm 10240x4096 16.6 | 18.2
+//           (at 4 rows 16.2 | 15.1) and 6144x8192 17.6 | 18.4, gated pairs of 4608x4096 16.0 | 17.1, of 6144x8192 26.5 | 24.3
+//   Q4_0    12 rows: 4096x14336 24.2 | 20.3, 1024x32768 16.5 | 18.8; 8 and 12 rows: 6144x4096 14.9 15.5 | 13.5 17.1, 14336x4096 24.2 24.7 | 18.7 22.5,
+//           gated pairs at 12 rows: 8192x4096 24.9 | 24.5, 9216x4096 28.7 | 31.4
+//   IQ4_NL  8 and 12 rows: 8192x4096 17.0 17.7 | 15.4 18.7; 12 rows: 12288x4096 26.5 | 24.3, 2048x16384 behind a norm 17.9 | 18.9
+//   Q8_0    8 and 12 rows: 8192x1024 13.4 13.6 | 11.7 14.8, 9216x1024 14.2 14.4 | 11.6 13.6; 12 rows: 256x32768 13.5 | 14.2
+// Their scratch memory is the larger one.
+bool split_k_ahead(int type, int64_t M, int64_t K, int64_t one, int matrices) {
+    const int64_t MB = (int64_t)1 << 20, slices = (K + 511) / 512, slots = (slices + 7) / 8 * 8;
+    const bool gaps = K > 2048 && slices * 20 < slots * 17;
+    if (M < 5 || one < kTinyWeightBytes) return false;
+    if (mmv_one_launch(K)) {
+        if (type == GQ_Q4_K) return M > 8 && (matrices == 1 || gaps || K <= 1024);
+        return M > 8 && matrices == 1 && one >= 8 * MB && type != GQ_Q6_K && K <= (type == GQ_Q8_0 ? 512 : one >= 16 * MB ? 2048 : 1024);
+    }
+    switch (type) {
+    case GQ_Q4_K: return M > 8 || (gaps && one >= 10 * MB && one < (matrices == 1 ? 28 : 13) * MB);
+    case GQ_Q4_0:
+    case GQ_IQ4_NL: return M > 8 && one >= 9 * MB && one < 26 * MB && (matrices == 1 || gaps);
+    case GQ_Q8_0: return M > 8 && one < 9 * MB;
+    default: return false;
+    }
+}
+
 // Whether 3 to 16 rows of up to 4096 values take the one-launch kernel of mmv.hip.  It costs about 5 us of activation conversion per
 // workgroup and then streams W once; the GEMV it replaces costs a pass per row over small matrices, per four rows (two with a
 // normalisation, a residual or a gated pair: `extras`) over those of 24 MB and more, the split-K kernels three launches.
@@ -287,23 +348,26 @@ bool y_over_x(const void *x, bool x_is_bf16, const float *y, int64_t M, int64_t 
 //          gated pair  8.6 11.1 13.6 19.8 14.8 15.5 15.6 | 10.1 10.1 10.1 11.4 11.5 15.6 15.5    gated pair  18.9 26.3 26.6 27.1 27.2 27.8 28.5 | 17.7 17.7 18.0 19.4 19.5 26.3 26.3
 //   Q6_K   4096x4096   8.0 10.6 13.2 17.0 17.3 17.5 17.7 |  9.8  9.5  9.6 10.6 10.6 14.1 14.1    4096x14336  14.6 24.5 24.1 31.5 32.1 32.8 32.8 | 17.3 17.2 17.4 18.2 18.1 24.1 24.5
 //   IQ4_NL 4096x4096   6.8  9.0 11.0 13.1 13.3 13.6 13.8 |  8.5  8.5  8.5  9.3  9.4 12.6 12.6    4096x14336  12.3 16.0 16.1 25.6 26.3 26.9 27.1 | 16.1 16.0 16.1 17.0 17.3 22.3 22.5
-// Below 9 MB a pass per row comes out of the caches: there the product of rows and bytes decides (Q8_0 4096x1024, 4.5 MB: even at 16 rows;
-// a gated pair of them: 10.8 | 10.7 at 8; Q4_K: 14.5 | 14.5 at 12).
-bool takes_mmv(int type, int64_t M, int64_t K, int64_t N, const void *x, const void *gain, int matrices, bool extras) {
+// The GEMV's passes over matrices of less than 24 MB come out of the caches and cost rows x bytes, so that the product of both decides:
+// below 9 MB mmv.hip takes over at 64 MB (Q8_0 4096x1024, 4.5 MB: even at 16 rows; a gated pair of them: 10.8 | 10.7 at 8; Q4_K: 14.5 | 14.5 at
+// 12), above at gemv_reach().
+// set: N counts the columns of several matrices that share x, which a call of its own would not take together
+bool takes_mmv(int type, int64_t M, int64_t K, int64_t N, const void *x, const void *gain, int matrices, bool extras, bool set = false) {
     if (M < 3 || !mmv_one_launch(K) || !mmv_supported(type, M, K, N, x, gain)) return false;
-    const int64_t bytes = weight_bytes_of(type, K, N) * matrices, MB = (int64_t)1 << 20;
+    const int64_t one = weight_bytes_of(type, K, N), bytes = one * matrices, MB = (int64_t)1 << 20;
+    if ((!set || type == GQ_Q4_K) && N % 4 == 0 && split_k_ahead(type, M, K, one, matrices)) return false;  // (what the split-K kernels take)
     if (bytes < 9 * MB) return M * bytes >= 64 * MB;
-    if (type == GQ_Q4_0 && M == 3 && bytes < kLargeWeightBytes) return false;
-    if (!extras && M <= 4 && bytes >= kLargeWeightBytes && (type == GQ_Q8_0 || (type == GQ_Q4_0 && bytes < 64 * MB))) return false;  // one GEMV pass of four rows
-    if (type == GQ_Q4_K && M > 8 && matrices == 1) return false;  // the split-K kernels, whose Q4_K conversion is as cheap and shared by 32 rows
+    if (bytes < kLargeWeightBytes) return !(type == GQ_Q4_0 && M == 3) && M * bytes >= gemv_reach(type, K, K * N * matrices, matrices, extras, set) * MB;
+    if (!extras && !set && M <= 4 && (type == GQ_Q8_0 || (type == GQ_Q4_0 && bytes < 64 * MB))) return false;  // one GEMV pass of four rows
     return true;
 }
-// What the split-K kernels were chosen for: rows of more than 4096 values, up to sixteen of them (eight for Q4_K), take mmv.hip's two
-// launches instead of the three of mmq.hip (8 and 16 rows on 14336 -> 4096: Q8_0 29.7 30.0 | 20.6 24.7 us, Q4_0 24.2 24.6 | 18.7 23.3,
-// Q6_K 32.8 33.3 | 21.6 27.2, IQ4_NL 27.5 27.7 | 20.6 25.6, Q4_K 17.8 18.1 | 17.8 23.6).  Their scratch memory is the smaller one.
+// What the split-K kernels were chosen for: up to 16 rows take mmv.hip (rows of more than 4096 values its two launches instead of the three
+// of mmq.hip) where split_k_ahead() says so.
 int split_k(int type, const void *x, bool x_is_bf16, int64_t M, int64_t K, int count, const MmqSetItem *items, const MmqExtra *ex, hipStream_t s) {
     const void *gain = ex && ex->norm ? ex->norm->gain : nullptr;
-    bool mmv = type != GQ_Q4_K || M <= 8;
+    int64_t ntot = 0;
+    for (int i = 0; i < count; i++) ntot += items[i].N;
+    bool mmv = !split_k_ahead(type, M, K, weight_bytes_of(type, K, ntot), ex && ex->W2 ? 2 : 1);
     for (int i = 0; i < count; i++)
         mmv = mmv && mmv_supported(type, M, K, items[i].N, x, gain) && !(mmv_one_launch(K) && y_over_x(x, x_is_bf16, items[i].y, M, K, items[i].N));
     if (mmv) return launch_mmv(type, x, x_is_bf16, M, K, count, items, ex, s);
@@ -529,7 +593,7 @@ int gq_qdense_f32_static(int type, const float *dX, int64_t M, int64_t K, const 
 }
 
 namespace {
-bool set_takes_mmv(int count, const gq_dense_desc *descs, const float *gain, MmqSetItem *set);
+bool set_takes_mmv(int count, const gq_dense_desc *descs, const float *gain, bool normed, MmqSetItem *set);
 bool takes_shared_pass(int count, const gq_dense_desc *descs, const float *gain, MmqSetItem *set);  // (defined with the dispatch thresholds below)
 // From 6 rows the shared split-K pass is ahead of the merged GEMV launch: a decoder layer's q / k / v, 4096 -> 4096 + 2 x 1024,
 // with the rest of the layer: 79.2 against 80.0 us at 5 rows, 81.6 against 79.9 at 6, 84.7 against 80.3 at 8.
@@ -547,7 +611,7 @@ int gq_qdense_f32_batch(int count, const gq_dense_desc *descs, void *stream) {
     CallScope scope;
     {   // projections of one input beyond the GEMV's best rows: one split-K pass for all of them
         MmqSetItem set[4];
-        if (set_takes_mmv(count, descs, nullptr, set))
+        if (set_takes_mmv(count, descs, nullptr, false, set))
             return launch_mmv(descs[0].type, descs[0].dX, false, descs[0].M, descs[0].K, count, set, nullptr, (hipStream_t)stream);
         if (descs[0].M >= kSharedPassFromRows && takes_shared_pass(count, descs, nullptr, set))
             return split_k(descs[0].type, descs[0].dX, false, descs[0].M, descs[0].K, count, set, nullptr, (hipStream_t)stream);
@@ -697,11 +761,11 @@ bool same_input_set(int count, const gq_dense_desc *descs, MmqSetItem *set) {
     }
     return true;
 }
-bool set_takes_mmv(int count, const gq_dense_desc *descs, const float *gain, MmqSetItem *set) {
+bool set_takes_mmv(int count, const gq_dense_desc *descs, const float *gain, bool normed, MmqSetItem *set) {
     if (!same_input_set(count, descs, set)) return false;
     int64_t ntot = 0;
     for (int i = 0; i < count; i++) ntot += descs[i].N;
-    return takes_mmv(descs[0].type, descs[0].M, descs[0].K, ntot, descs[0].dX, gain, 1, true);
+    return takes_mmv(descs[0].type, descs[0].M, descs[0].K, ntot, descs[0].dX, gain, 1, normed, true);
 }
 bool takes_shared_pass(int count, const gq_dense_desc *descs, const float *gain, MmqSetItem *set) {
     if ((gain && !aligned_to(gain, 16)) || !same_input_set(count, descs, set)) return false;
@@ -807,7 +871,7 @@ int gq_qdense_norm_f32_batch(int count, const gq_dense_desc *descs, const gq_rms
     MmqSetItem set[4];
     const RmsNorm rn{norm->dGain, norm->eps, norm->gain_offset};
     const MmqExtra ex{nullptr, nullptr, nullptr, &rn};
-    if (set_takes_mmv(count, descs, norm->dGain, set))
+    if (set_takes_mmv(count, descs, norm->dGain, true, set))
         return launch_mmv(descs[0].type, descs[0].dX, false, rows, descs[0].K, count, set, &ex, (hipStream_t)stream);
     const bool shared_pass = takes_shared_pass(count, descs, norm->dGain, set);
     XsBatchItem items[8];
@@ -968,7 +1032,7 @@ int gq_qdense_norm_bf16_batch(int count, const gq_dense_desc *descs, const gq_rm
         MmqSetItem set[4];
         const RmsNorm rn{norm->dGain, norm->eps, norm->gain_offset};
         const MmqExtra ex{nullptr, nullptr, nullptr, &rn};
-        if (set_takes_mmv(count, descs, norm->dGain, set))
+        if (set_takes_mmv(count, descs, norm->dGain, true, set))
             return launch_mmv(descs[0].type, descs[0].dX, true, descs[0].M, descs[0].K, count, set, &ex, (hipStream_t)stream);
         const bool shared_pass = takes_shared_pass(count, descs, norm->dGain, set);
         XsBatchItem items[8];

@@ -449,6 +449,36 @@ def test_few_rows_in_one_launch(gpu, oracle, t, M, K, kind):
         assert err.max() <= (1e-5 if kind == "gated" else 4.8e-6), err
 
 
+@pytest.mark.parametrize("t,M,K,N,kind,route", [
+    (Q8_0, 3, 2048, 6144, "plain", "gemv"), (Q8_0, 5, 2048, 8192, "plain", "mmv"), (Q8_0, 3, 4096, 4096, "plain", "mmv"),
+    (Q4_0, 4, 4096, 6144, "plain", "gemv"), (Q4_0, 5, 4096, 6144, "plain", "mmv"), (Q4_0, 4, 1536, 6144, "gated", "gemv"),
+    (Q4_K, 3, 1536, 12288, "plain", "gemv"), (Q4_K, 4, 1536, 12288, "plain", "mmv"), (Q4_K, 3, 4096, 4096, "plain", "mmv"),
+    (Q6_K, 3, 2048, 6144, "plain", "gemv"), (Q6_K, 4, 2048, 6144, "plain", "mmv"), (IQ4_NL, 3, 1536, 6144, "gated", "gemv"),
+    (Q4_0, 8, 6144, 4096, "plain", 2), (Q4_0, 9, 6144, 4096, "plain", 3), (IQ4_NL, 12, 12288, 4096, "plain", 2), (IQ4_NL, 12, 1024, 32768, "plain", 3),
+    (Q4_K, 8, 8192, 4096, "plain", 2), (Q4_K, 8, 9216, 4096, "plain", 3), (Q4_K, 12, 3072, 8192, "gated", 3), (Q4_K, 12, 4096, 8192, "gated", "mmv"),
+    (Q8_0, 12, 8192, 1024, "plain", 3), (Q8_0, 12, 9216, 1024, "plain", 2), (Q4_0, 12, 1024, 8192, "plain", "gemv"), (Q4_0, 12, 2048, 8192, "plain", "mmv")])
+def test_routes_of_a_few_rows(gpu, t, M, K, N, kind, route):
+    """Both sides of the lines between the GEMV, the few-row kernel and the split-K kernels (gomlx_amd/csrc/api.hip).  The split-K kernels
+    make three launches, the few-row kernel two where K > 4096 and one else; the GEMV's passes of one row give each row the bits of a
+    call of its own, the few-row kernel others."""
+    import ctypes
+    from gomlx_amd import _lib
+    W = [dev(gpu, np.tile(synth.weights(t, 80 + i, 512, K), (N // 512, 1))) for i in range(2)]
+    x = gpu.randn(M, K, device="cuda", generator=gpu.Generator(device="cuda").manual_seed(1))
+    q, L = Quantization(ggml_type=t), _lib.lib()
+
+    def call(x):
+        return nn.quantized_dense(x, W[0], q) if kind == "plain" else nn.gated_feed_forward(x, W[0], W[1], q, Activation.SILU)
+
+    launches, us = ctypes.c_int(0), ctypes.c_double(0.0)
+    _lib.check(L.gq_profile_begin())
+    y = call(x)
+    _lib.check(L.gq_profile_end(ctypes.byref(launches), ctypes.byref(us)))
+    assert launches.value == (route if isinstance(route, int) else 1)
+    if launches.value == 1:
+        assert gpu.equal(y, gpu.cat([call(x[m:m + 1]) for m in range(M)])) == (route == "gemv")
+
+
 @pytest.mark.parametrize("t", [Q4_0, Q8_0, Q6_K, IQ4_NL])
 @pytest.mark.parametrize("M,K,N,bf16", [(6, 4096, 4096, False), (16, 4096, 4096, True), (8, 8192, 2048, False), (12, 2560, 8192, False)])
 def test_infinite_activations_of_a_few_rows(gpu, oracle, t, M, K, N, bf16):
