@@ -616,9 +616,36 @@ int gq_qdense_f32_batch(int count, const gq_dense_desc *descs, void *stream) {
         if (descs[0].M >= kSharedPassFromRows && takes_shared_pass(count, descs, nullptr, set))
             return split_k(descs[0].type, descs[0].dX, false, descs[0].M, descs[0].K, count, set, nullptr, (hipStream_t)stream);
     }
+    // problems that calls of their own would hand to the few-row kernel: up to four of one type, batch size and K in one launch, each with
+    // its own input and share of the workgroups, and the bits of a call of its own (two Q4_K 4096x4096 at 3 and 5 rows 9.8 and 11.6 us; one launch each took 16.0 18.7,
+    // the merged GEMV launch 10.0 14.5)
+    uint64_t done = 0;
+    auto few = [&](const gq_dense_desc &d) { return d.N > 0 && takes_mmv(d.type, d.M, d.K, d.N, d.dX, nullptr, 1, false); };
+    for (int i = 0; i < count && i < 64; i++) {
+        if ((done >> i & 1) || !few(descs[i])) continue;
+        MmqSetItem items[4];
+        const void *xs[4];
+        uint64_t mine = 0;
+        int n = 0;
+        for (int j = i; j < count && j < 64 && n < 4; j++) {
+            const gq_dense_desc &d = descs[j];
+            if ((done >> j & 1) || d.type != descs[i].type || d.M != descs[i].M || d.K != descs[i].K || !few(d)) continue;
+            items[n] = MmqSetItem{(const uint8_t *)d.dW, d.N, d.dBias, d.act, d.dY};
+            xs[n++] = d.dX;
+            mine |= (uint64_t)1 << j;
+        }
+        if (n < 2) continue;
+        if (int rc = launch_mmv(descs[i].type, nullptr, false, descs[i].M, descs[i].K, n, items, nullptr, (hipStream_t)stream, xs)) return rc;
+        done |= mine;
+    }
     // merge runs of batch-1 problems of one type that the streaming GEMV handles; the rest go one by one
+    auto is_done = [&](int k) { return k < 64 && (done >> k & 1); };
     int i = 0;
     while (i < count) {
+        if (is_done(i)) {
+            i++;
+            continue;
+        }
         int j = i;
         XsBatchItem items[8];
         // the kernel family of the run is that of its first problem: K-sliced where that applies, else
@@ -630,11 +657,11 @@ int gq_qdense_f32_batch(int count, const gq_dense_desc *descs, void *stream) {
         const int64_t rows = descs[i].M;
         const bool rows_ok = rows == 1 || (use_ks && rows >= 1 && rows <= batch_rows_max());
         // (several rows per problem: only over matrices below the size from which one pass serves several rows)
-        // (and none that a call of its own would hand to the one-launch kernel: a submission returns what its calls return one by one)
+        // (and none for the few-row kernel: one that is alone in the list takes it in a call of its own)
         auto size_ok = [&](const gq_dense_desc &d) {
-            return rows == 1 || (weight_bytes_of(d.type, d.K, d.N) < kLargeWeightBytes && !takes_mmv(d.type, d.M, d.K, d.N, d.dX, nullptr, 1, false));
+            return rows == 1 || (weight_bytes_of(d.type, d.K, d.N) < kLargeWeightBytes && !few(d));
         };
-        while (j < count && j - i < 8 && rows_ok && descs[j].type == descs[i].type && descs[j].M == rows && descs[j].N > 0 && fits(descs[j]) &&
+        while (j < count && !is_done(j) && j - i < 8 && rows_ok && descs[j].type == descs[i].type && descs[j].M == rows && descs[j].N > 0 && fits(descs[j]) &&
                size_ok(descs[j])) {
             const gq_dense_desc &d = descs[j];
             items[j - i] = XsBatchItem{d.dX, (const uint8_t *)d.dW, d.dBias, d.dY, d.K, d.N, d.act};

@@ -99,7 +99,9 @@ int launch_mmq_set(int type, const void *x, bool x_is_bf16, int64_t M, int64_t K
 // and what mmq_supported asks of N, bias, residual and y.
 bool mmv_supported(int type, int64_t M, int64_t K, int64_t N, const void *x, const void *gain);
 bool mmv_one_launch(int64_t K);
-int launch_mmv(int type, const void *x, bool x_is_bf16, int64_t M, int64_t K, int count, const MmqSetItem *items, const MmqExtra *ex, hipStream_t s);
+// xs: every matrix with activations of its own (two to four of them, K in one launch, no extras).
+int launch_mmv(int type, const void *x, bool x_is_bf16, int64_t M, int64_t K, int count, const MmqSetItem *items, const MmqExtra *ex, hipStream_t s,
+               const void *const *xs = nullptr);
 // The reduction behind it: sums partial[slices][M][all columns] (partial2: the second matrix of a gated pair) and, with a normalisation,
 // sums of squares xss[slices][M] -> the finished outputs of `count` matrices.
 int launch_split_k_finish(const float *partial, const float *partial2, const float *xss, int nslices, int64_t M, int64_t K, int count,

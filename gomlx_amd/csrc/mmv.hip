@@ -83,6 +83,8 @@ struct MmvArgs {
     float *y[kMaxProblems];
     int N[kMaxProblems], act[kMaxProblems], tile0[kMaxProblems], n0[kMaxProblems];
     int count, ntiles, M, K, nslices, ntot;
+    const void *X[kMaxProblems];  // apart: every matrix has its own activations and wgs[j] workgroups from wg0[j] on
+    int wg0[kMaxProblems], wgs[kMaxProblems], apart;
     const uint8_t *W2;       // gated pair: the second matrix, its bias
     const float *bias2;
     const float *residual;
@@ -436,7 +438,7 @@ __device__ __forceinline__ void wave_fence() {  // LDS operations of one wavefro
 
 // SETS sets of R activation rows (R = 4: half the columns of a set stay empty, and half the conversion undone)
 template <int T, bool BF, int SETS, int R>
-__global__ __launch_bounds__(512) void mmv_kernel(const void *__restrict__ X, const MmvArgs A) {
+__global__ __launch_bounds__(512) void mmv_kernel(const void *__restrict__ Xall, const MmvArgs A) {
     typedef MV<T> F;
     typedef MVG<T> G;
     typedef MVLds<T, SETS> L;
@@ -446,9 +448,27 @@ __global__ __launch_bounds__(512) void mmv_kernel(const void *__restrict__ X, co
     const int i16 = lane & 15, kg = lane >> 4;
     const int waves = (int)(blockDim.x >> 6);
     const int slice0 = (int)blockIdx.y * waves, live = min(waves, A.nslices - slice0), slice = slice0 + wave;
-    const int gx = (int)gridDim.x, bx = (int)blockIdx.x;
+    // this workgroup's tiles: bx, bx + gx, .. below end
+    int gx = (int)gridDim.x, bx = (int)blockIdx.x, end = A.ntiles;
+    const void *X = Xall;
+    if (A.apart) {
+        int wg0 = 0, first = 0;
+        X = A.X[0];
+        gx = A.wgs[0];
+        end = A.tile0[1];
+#pragma unroll
+        for (int j = 1; j < kMaxProblems; j++) {
+            const bool in = j < A.count && (int)blockIdx.x >= A.wg0[j];
+            X = in ? A.X[j] : X;
+            gx = in ? A.wgs[j] : gx;
+            wg0 = in ? A.wg0[j] : wg0;
+            first = in ? A.tile0[j] : first;
+            end = in ? (j + 1 < kMaxProblems && j + 1 < A.count ? A.tile0[(j + 1) % kMaxProblems] : A.ntiles) : end;
+        }
+        bx = first + bx - wg0;
+    }
     const int dual = A.W2 ? 1 : 0;
-    const int nmt = ((A.ntiles - bx + gx - 1) / gx) << dual;  // matrix tiles of this workgroup (a gated pair's alternate)
+    const int nmt = ((end - bx + gx - 1) / gx) << dual;  // matrix tiles of this workgroup (a gated pair's alternate)
     const int64_t row_bytes = (int64_t)(A.K / 256) * F::kBytes;
 
     uint8_t *const mine = lds + wave * L::kWave;
@@ -756,8 +776,19 @@ int launch_mmv_rows(const void *x, const MmvArgs &a, const Plan &p, hipStream_t 
     const int cus = device_cu_count();
     int per_cu = kMaxWaves / p.waves;
     if (SETS == 2 && per_cu == 2 && a.ntiles < 3 * cus) per_cu = 1;
-    const int gx = std::max(1, std::min(a.ntiles, cus * per_cu / p.groups));
-    return launch(mmv_kernel<T, BF, SETS, R>, dim3((unsigned)gx, (unsigned)p.groups), dim3((unsigned)p.waves * 64), (size_t)L::bytes(p.waves), s, x, a);
+    int gx = std::max(1, std::min(a.ntiles, cus * per_cu / p.groups));
+    MmvArgs b = a;
+    if (a.apart) {  // every matrix its share of the workgroups, in proportion to its tiles
+        const int total = gx;
+        gx = 0;
+        for (int j = 0; j < a.count; j++) {
+            const int tiles = (j + 1 < a.count ? a.tile0[j + 1] : a.ntiles) - a.tile0[j];
+            b.wg0[j] = gx;
+            b.wgs[j] = std::max(1, (int)((int64_t)total * tiles / a.ntiles));
+            gx += b.wgs[j];
+        }
+    }
+    return launch(mmv_kernel<T, BF, SETS, R>, dim3((unsigned)gx, (unsigned)p.groups), dim3((unsigned)p.waves * 64), (size_t)L::bytes(p.waves), s, x, b);
 }
 
 template <int T>
@@ -779,11 +810,16 @@ bool mmv_supported(int type, int64_t M, int64_t K, int64_t N, const void *x, con
 }
 
 // The same activations against `count` matrices (one with W2, bias2: a gated pair; a residual goes with one matrix only).  K of
-// more than eight slices needs workspace, N % 4 == 0 and 16-byte aligned bias, residual and y for the reduction.
-int launch_mmv(int type, const void *x, bool x_is_bf16, int64_t M, int64_t K, int count, const MmqSetItem *items, const MmqExtra *ex, hipStream_t s) {
+// more than eight slices needs workspace, N % 4 == 0 and 16-byte aligned bias, residual and y for the reduction.  xs: activations of
+// their own for every matrix (two or more of up to eight slices, no extras).
+int launch_mmv(int type, const void *x, bool x_is_bf16, int64_t M, int64_t K, int count, const MmqSetItem *items, const MmqExtra *ex, hipStream_t s,
+               const void *const *xs) {
     if (count < 1 || count > kMaxProblems) return fail(GQ_ERR_NOT_IMPLEMENTED, "mmv: a set of %d matrices is not implemented", count);
     const Plan p = plan_of(K);
+    if (xs && (count < 2 || ex || p.groups > 1)) return fail(GQ_ERR_NOT_IMPLEMENTED, "mmv: activations per matrix in this form are not implemented");
     MmvArgs a = {};
+    a.apart = xs ? 1 : 0;
+    for (int i = 0; xs && i < count; i++) a.X[i] = xs[i];
     int64_t tiles = 0, ntot = 0;
     for (int i = 0; i < count; i++) {
         a.W[i] = items[i].W; a.bias[i] = items[i].bias; a.y[i] = items[i].y; a.N[i] = (int)items[i].N; a.act[i] = items[i].act;

@@ -1854,6 +1854,33 @@ def test_batched_submission_equals_separate_calls(gpu, oracle):
         assert rel_err(y.cpu().numpy(), want) < TOL_F32
 
 
+@pytest.mark.parametrize("t", ALL_TYPES)
+@pytest.mark.parametrize("M,K,counts", [(6, 4096, (1, 3)), (8, 1536, (2, 1)), (16, 4096, (1, 1, 2, 1)), (5, 512, (3, 2))])
+def test_batched_problems_with_inputs_of_their_own_in_the_few_row_kernel(gpu, t, M, K, counts):
+    """Problems of one K that the few-row kernel takes, each with its own input, between two small ones that it does not: the bits of
+    separate calls, in one launch.  Widths of `counts` times 9 to 12 MB, off every tile: shares of the workgroups from
+    a sixth up, ragged last tiles."""
+    import ctypes
+    from gomlx_amd import _lib
+    if t == Q4_K:
+        M = min(M, 8)
+    q, g, L = Quantization(ggml_type=t), gpu.Generator(device="cuda").manual_seed(7), _lib.lib()
+    rb = ggml.row_bytes(t, K)
+    probs = []
+    for i, n in enumerate((0,) + counts + (0,)):
+        N = (12 << 20) * n // rb + 5 + 2 * i if n else 24
+        w = dev(gpu, np.tile(synth.weights(t, 730 + i, 131, K), (-(-N // 131), 1))[:N])
+        probs.append((gpu.randn(M, K, device="cuda", generator=g), w, q, gpu.randn(N, device="cuda", generator=g), Activation.SILU if i % 2 else None))
+    single = [nn.quantized_dense(p[0], p[1], q, p[3], p[4] or Activation.NONE) for p in probs]
+    launches, us = ctypes.c_int(0), ctypes.c_double(0.0)
+    _lib.check(L.gq_profile_begin())
+    outs = nn.quantized_dense_batch(probs)
+    _lib.check(L.gq_profile_end(ctypes.byref(launches), ctypes.byref(us)))
+    for a, b in zip(single, outs):
+        assert gpu.equal(a, b)
+    assert launches.value == 1 + 2
+
+
 # ------------------------------------------------------------------------------ gather
 
 @pytest.mark.parametrize("t", ALL_TYPES)
