@@ -132,9 +132,13 @@ int gq_qdense_bf16(int type, const uint16_t *dX, int64_t M, int64_t K, const voi
 /* ---- Several FusedQuantizedDense nodes of one compiled graph that do not depend on each other
  * (e.g. the q/k/v or gate/up projections of a decoder layer) submitted together: the work an
  * Executable.Execute (core/graph/graph.go:669) is free to overlap.  Equivalent to calling
- * gq_qdense_f32 once per descriptor, in any order; outputs must not alias any input.  Batch-1
- * problems of one GGML type are merged into a single launch; two to four Q4_K projections of the
- * same activation buffer with 6 rows or more share one split-K pass (activations converted once). ---- */
+ * gq_qdense_f32 once per descriptor, in any order; outputs must not alias any input.  Problems of one
+ * GGML type and one batch size of up to 8 rows over matrices of less than 24 MB are merged into a single
+ * launch; up to four problems of one type, batch size of 3 to 16 rows and K that calls of their own hand to
+ * the few-row kernel share one of its launches; two to four projections of the same activation buffer do so
+ * where their weights together are worth it, and in Q4_K share one split-K pass beyond (activations converted
+ * once).  The kernel that serves a list may be another than the one that serves its members alone: results
+ * then agree to the rounding of the activations, not bit for bit (batches of 1 and 2 rows: bit for bit). ---- */
 typedef struct {
     int type;            /* gq_type */
     int act;             /* gq_act */
@@ -177,8 +181,9 @@ int gq_qdense_block_f32(int type, const float *dX, int64_t M, int64_t K, const g
 /* gq_qdense_f32_batch with one RMS normalisation applied to the activations of every problem:
  * the q/k/v projections behind a layer's input norm (transformer.go:1099-1130) in one launch
  * when all are problems of one type, one K and one batch size of at most 8 rows.  Two to four
- * Q4_K projections of the SAME activation buffer (equal dX, M, K) with more rows than that share
- * one split-K pass (activations converted once, one main launch, one reduction; uses the
+ * projections of the SAME activation buffer (equal dX, M, K; 3 to 16 rows of up to 4096 values, any one type) share a
+ * launch of the few-row kernel where their weights together are worth it; in Q4_K, from 6 rows, they share one split-K
+ * pass beyond (activations converted once, one main launch, one reduction; uses the
  * per-stream workspace); past the split-K kernels' range such projections of any one type, with
  * widths that are multiples of 32 and one activation function, share the two-pass GEMM (one activation
  * conversion, one 16-bit image of all the matrices, one GEMM that writes each matrix's columns to its

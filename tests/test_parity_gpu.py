@@ -1855,6 +1855,26 @@ def test_batched_submission_equals_separate_calls(gpu, oracle):
 
 
 @pytest.mark.parametrize("t", ALL_TYPES)
+@pytest.mark.parametrize("M", [2, 3, 4, 6, 8, 12, 16, 40])
+def test_projections_of_one_input_against_separate_calls(gpu, t, M):
+    """q / k / v shapes of one input as one submission and as three calls, with and without a norm: the same bits at 2 rows, to the
+    rounding of the activations from 3.  The GEMV's 16-bit fixed point keeps a value to 2^-16 of the largest of its 512, at most five
+    times their root mean square: 5 * 2^-16 / sqrt(3) is 4.4e-5 of a sum's 2-norm, twice that for Q4_K, whose minima cancel part of the
+    result.  One fp16 (Q4_K in the split-K kernels from 9 rows, every format beyond 16) rounds to 2^-11 / sqrt(3), 2.8e-4, against
+    another rounding of that size at most; Q4_K twice."""
+    K, g, q = 4096, gpu.Generator(device="cuda").manual_seed(M), Quantization(ggml_type=t)
+    W = [dev(gpu, np.tile(synth.weights(t, 740 + i, 256, K), (n, 1))) for i, n in enumerate((16, 4, 4))]
+    x, norm = gpu.randn(M, K, device="cuda", generator=g), nn.RMSNorm(gain=gpu.rand(K, device="cuda", generator=g) + 0.5)
+    fp16 = M > 16 or (t == Q4_K and M > 8)
+    bound = 0.0 if M == 2 else (2 if t == Q4_K else 1) * (5.7e-4 if fp16 else 4.4e-5)
+    for n in (None, norm):
+        outs = nn.quantized_dense_batch([(x, w, q, None, None) for w in W], n)
+        for w, y in zip(W, outs):
+            one = nn.quantized_dense(x, w, q, norm=n).double()
+            assert float(((y.double() - one).norm(dim=1) / one.norm(dim=1)).max()) <= bound
+
+
+@pytest.mark.parametrize("t", ALL_TYPES)
 @pytest.mark.parametrize("M,K,counts", [(6, 4096, (1, 3)), (8, 1536, (2, 1)), (16, 4096, (1, 1, 2, 1)), (5, 512, (3, 2))])
 def test_batched_problems_with_inputs_of_their_own_in_the_few_row_kernel(gpu, t, M, K, counts):
     """Problems of one K that the few-row kernel takes, each with its own input, between two small ones that it does not: the bits of
