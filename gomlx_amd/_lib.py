@@ -99,7 +99,7 @@ _fast_tried = False
 # Entry points the native host path calls, in the order in which csrc/binding.cpp takes them.
 _BOUND = ("gq_qdense_check", "gq_qdense_f32", "gq_qdense_bf16", "gq_qdense_block_f32", "gq_qdense_block_bf16", "gq_qdense_gated_f32",
           "gq_qdense_gated_bf16", "gq_qdense_f32_batch", "gq_qdense_norm_f32_batch", "gq_qdense_norm_bf16_batch", "gq_dequantize",
-          "gq_embedding_lookup", "gq_row_bytes", "gq_bytes_per_block", "gq_values_per_block")
+          "gq_embedding_lookup", "gq_bytes_per_block", "gq_values_per_block")
 
 
 def lib() -> ctypes.CDLL:

@@ -32,11 +32,10 @@ struct Entry {
     decltype(&gq_qdense_norm_bf16_batch) norm_batch_bf16;
     decltype(&gq_dequantize) dequantize;
     decltype(&gq_embedding_lookup) lookup;
-    decltype(&gq_row_bytes) row_bytes;
     decltype(&gq_bytes_per_block) bytes_per_block;
     decltype(&gq_values_per_block) values_per_block;
 } g;
-constexpr int kEntries = 15;
+constexpr int kEntries = 14;
 bool g_bound = false;
 PyTypeObject *g_activation = nullptr;  // nn.Activation
 PyObject *s_scheme, *s_ggml_type, *s_gain, *s_epsilon, *s_scale_offset;

@@ -1973,6 +1973,48 @@ def test_native_host_path_equals_the_python_steps(gpu, monkeypatch, shape, bf16)
         assert a.dtype == b.dtype and a.shape == b.shape and a.device == b.device and gpu.equal(a, b)
 
 
+@pytest.mark.parametrize("bf16", [False, True])
+def test_native_host_path_is_the_one_that_serves(gpu, bf16):
+    """csrc/binding.cpp itself: it returns a result for every form of the five operators that nn.py hands it - so that a path that
+    declines everything does not pass for the Python steps - with the Python steps' bits, and None for what it does not take."""
+    from gomlx_amd import _lib
+    t, K, N = Q8_0, 512, 96
+    q, g = Quantization(ggml_type=t), gpu.Generator(device="cuda").manual_seed(5)
+    w = [dev(gpu, synth.weights(t, 720 + i, N, K)) for i in range(2)]
+    x = gpu.randn(3, K, device="cuda", generator=g)
+    x = x.to(gpu.bfloat16) if bf16 else x
+    bias, gain, res = (gpu.randn(*s, device="cuda", generator=g) for s in ((N,), (K,), (3, N)))
+    norm, none = nn.RMSNorm(gain=gain, epsilon=1e-5), Activation.NONE
+    nn.quantized_dense(x, w[0], q)  # (binds the native path)
+    fast, idx = _lib.fast, gpu.tensor([[3], [95]], dtype=gpu.int32, device="cuda")
+    assert fast is not None
+    calls = [(fast.dense, (x, w[0], q, bias, a, None, None), lambda a=a: nn.quantized_dense(x, w[0], q, bias, a)) for a in Activation]
+    calls += [(fast.gated, (x, w[0], w[1], q, a, None, bias, norm), lambda a=a: nn.gated_feed_forward(x, w[0], w[1], q, a, None, bias, norm)) for a in Activation]
+    calls += [(fast.dense, (x, w[0], q, None, none, norm, res), lambda: nn.quantized_dense(x, w[0], q, norm=norm, residual=res)),
+              (fast.batch, ([(x, w[0], q, bias, None), (x, w[1], q, None, Activation.TANH)], norm),
+               lambda: nn.quantized_dense_batch([(x, w[0], q, bias, None), (x, w[1], q, None, Activation.TANH)], norm)),
+              (fast.dequantize, (w[0], t), lambda: nn.dequantize(w[0], t)), (fast.gather, (w[0], idx, q), lambda: nn.quantized_gather(w[0], idx, q))]
+    if not bf16:
+        calls.append((fast.batch, (((x, w[0], q, None, None),), None), lambda: nn.quantized_dense_batch(((x, w[0], q, None, None),))))
+    got = [f(*args) for f, args, _ in calls]
+    try:
+        _lib.fast = None
+        want = [f() for _, _, f in calls]
+    finally:
+        _lib.fast = fast
+    for a, b in zip(got, want):
+        assert a is not None
+        for u, v in zip(a, b) if isinstance(b, list) else ((a, b),):
+            assert u.dtype == v.dtype and u.shape == v.shape and u.device == v.device and gpu.equal(u, v)
+    for f, args in [(fast.dense, (x.t().contiguous().t(), w[0], q, None, none, None, None)), (fast.dense, (x, w[0], q, bias.double(), none, None, None)),
+                    (fast.dense, (x, w[0], q, bias[:-1], none, None, None)), (fast.dense, (x, w[0], None, None, none, None, None)),
+                    (fast.dense, (x, w[0], q, None, none, nn.RMSNorm(gain=gain[:-1]), None)), (fast.dense, (x, w[0], q, None, none, None, res[:2])),
+                    (fast.dense, (x.cpu(), w[0], q, None, none, None, None)), (fast.dense, (x, w[0], Quantization(ggml_type=3), None, none, None, None)),
+                    (fast.dense, (x[:, :-32].contiguous(), w[0], q, None, none, None, None)), (fast.gated, (x, w[0], w[1][:-1], q, none, None, None, None)),
+                    (fast.batch, ([], None)), (fast.dequantize, (w[0], 2 ** 32 + t)), (fast.gather, (w[0], idx + 95, q)), (fast.gather, (w[0], idx.long(), q))]:
+        assert f(*args) is None
+
+
 def test_an_activation_is_a_member_of_its_enumeration(gpu):
     """Bare numbers, None where the argument is given, and members of other enumerations (the C ABI's Relu is 2, nn's Sigmoid too)
     are refused, with the native host path bound as without it."""
