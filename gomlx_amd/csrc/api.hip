@@ -186,6 +186,10 @@ int check_dense_args(const char *fn, int type, const void *x, int64_t M, int64_t
 //          4096x1024 (3 MB)    5.1  6.1  6.2  7.2  7.3  8.4  8.5 | 16.4   14336x4096         28.6 37.1 37.3 46.9 48.0 57.6 58.8 | 34.0
 //   IQ4_NL 4096x4096          11.8 12.9 15.0 16.9 18.9 20.9 22.8 | 13.7   4096x14336         17.0 24.0 26.7 31.1 29.4 37.7 40.4 | 26.3
 //          4096x1024           4.8  5.7  5.7  6.6  6.7  7.6  7.7 | 12.8   14336x4096         20.9 28.6 31.1 37.7 35.9 45.0 47.8 | 27.2
+// These are the three launches of mmq.hip.  Rows of up to 4096 values meet this line only where takes_mmv() has declined them; longer ones take,
+// from it to 16 rows, mmv.hip's two launches (split_k_ahead()), which the line was not moved for.  They are ahead of the GEMV below it on the
+// larger matrices - rows 4 and 5 on the GEMV | 6 on the two launches: 14336x4096 Q8_0 19.9 31.2 | 20.3, Q4_0 18.3 25.4 | 18.5, Q6_K 25.8 21.3 | 21.3 (at 5 already
+// the two launches), IQ4_NL 19.7 28.6 | 20.5; 8192x8192 18.6 30.4 | 20.9, 16.6 23.6 | 18.2, 28.5 21.0 | 20.9, 18.6 28.3 | 20.3.
 // The split-K route is three dependent launches with a floor of about 12 us: matrices of a few megabytes (the k / v
 // projections of a grouped-query layer) stay on GEMV passes for every batch the GEMV takes.
 // (The Q6_K kernel pays 16 scale groups per super-block: twice the time of the others per byte.)
@@ -726,7 +730,10 @@ namespace {
 //   Q4_K   4096x4096  9 12 15 18 20 23 26 | 13   4096x14336 13 22 22 31 31 40 40 | 19      10 12 15 17 20 22 24 | 21   21 36 35 50 50 65 65 | 33
 //   Q6_K   4096x4096 11 14 17 20 23 26 30 | 19   4096x14336 16 28 28 39 39 51 51 | 33      12 20 20 28 28 35 35 | 31   29 47 47 64 64 83 83 | 59
 //   IQ4_NL 4096x4096 10 13 16 19 22 25 28 | 14   4096x14336 14 25 25 35 35 46 46 | 28      12 15 18 21 24 27 31 | 19   24 42 41 59 59 77 77 | 46
-// (14336x4096 behaves like 4096x14336.)  Matrices of a few megabytes stay on the GEMV for every batch it takes.
+// (14336x4096 behaves like 4096x14336.)  Matrices of a few megabytes stay on the GEMV for every batch it takes.  As above, the line is that of the
+// three launches: rows of up to 4096 values come here only where takes_mmv() has declined them, and the two launches that longer ones now take are
+// ahead below it (behind a norm, rows 4 on the GEMV | 5 on the two launches: 14336x4096 Q8_0 29.1 | 21.0, Q4_0 23.2 | 19.0, Q6_K 30.8 | 22.5, IQ4_NL 27.2 | 21.4;
+// gated 46.4 | 30.4, 35.6 | 26.7, 46.8 | 32.8, 43.2 | 31.2).
 int64_t block_split_k_from(int type, int64_t weight_bytes, bool gated) {
     if (weight_bytes < kTinyWeightBytes) return kGemvMaxRows + 1;
     if (weight_bytes >= kLargeWeightBytes) return type == GQ_Q4_K ? 3 : 5;

@@ -95,7 +95,7 @@ struct MmqSetItem { const uint8_t *W; int64_t N; const float *bias; int act; flo
 bool mmq_set_supported(int type, int count, const MmqSetItem *items, int64_t M, int64_t K, const void *x);
 int launch_mmq_set(int type, const void *x, bool x_is_bf16, int64_t M, int64_t K, int count, const MmqSetItem *items, const RmsNorm *norm,
                    hipStream_t s);
-// 2 to 16 activation rows in one launch on the matrix cores (mmv.hip); more than 4096 values of K take a second launch, workspace
+// 3 to 16 activation rows in one launch on the matrix cores (mmv.hip); more than 4096 values of K take a second launch, workspace
 // and what mmq_supported asks of N, bias, residual and y.
 bool mmv_supported(int type, int64_t M, int64_t K, int64_t N, const void *x, const void *gain);
 bool mmv_one_launch(int64_t K);

@@ -371,7 +371,7 @@ template <int TM, int TN> struct DmaTile {
     // SIMD a single wavefront: 112 .. 120 us against 81 .. 89 us at 2048 rows.)
     static constexpr int NS = kStageBytes * 3 <= 160 * 1024 ? 3 : 2;  // (256 x 256: two stages of 64 KB)
     // A step's DMAs go out behind the fragment reads of its first groups, not all in front of them: issued at once they hold the
-    // wavefront's first LDS reads back (Q8_0 4096 x 4096 at 2048 rows 84.8 -> 82.9 us, 4096 -> 14336 at 512 rows 92.7 -> 90.1).  The
+    // wavefront's first LDS reads back (weight images included: Q8_0 4096 x 4096 at 2048 bf16 rows 70.9 -> 66.4 us, 4096 -> 14336 at 512 92.7 -> 90.1).  The
     // 256 x 256 tile has one step for them to land and sends them in the first two groups; its matrix instructions run at raised
     // priority over the other wavefront's reads (4096 -> 14336 at 2048 rows 262 -> 253; the smaller tiles lose 1 % by it).
     static constexpr int kDmaGroups = NS == 3 ? 3 : 2;

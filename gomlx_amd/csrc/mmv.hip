@@ -1,4 +1,4 @@
-// Quantised Dense for 2 to 16 activation rows in one launch on the matrix cores (Q4_K, Q8_0, Q4_0, IQ4_NL, Q6_K; K % 256 == 0).
+// Quantised Dense for 3 to 16 activation rows in one launch on the matrix cores (Q4_K, Q8_0, Q4_0, IQ4_NL, Q6_K; K % 256 == 0).
 //
 // At these batch sizes the weights' bytes bound the work, but the vector ALUs contract at most four rows per reading of W
 // (gemv_ks_body.hpp), and the split-K kernels (mmq.hip) need three dependent launches and 32-row tiles.  Here the activations
@@ -7,8 +7,8 @@
 // wavefront waits for another before the sums of up to sixteen tiles meet in LDS, where the workgroup adds the slices and
 // applies normalisation, bias, activation, gate and residual.
 //
-// Activations: x * 2^e (a power of two per row and slice) as the sum of two fp16 numbers, hi = fp16(x), lo = fp16(x - hi): 22
-// significant bits, more than the 16-bit fixed point of the GEMV.  With up to 8 rows hi and lo share one 16-column operand
+// Activations: x * 2^e (a power of two per row and slice) as the sum of two fp16 numbers, hi = fp16(x), lo = fp16(x - hi), both
+// truncated: 20 significant bits, more than the 16-bit fixed point of the GEMV.  With up to 8 rows hi and lo share one 16-column operand
 // (columns 4 g + {0, 1}: hi of rows 2 g, 2 g + 1; + {2, 3}: their lo, so that a lane holds both halves of its sums); up to 16
 // rows are two such sets against the same converted weights.
 //
@@ -804,7 +804,7 @@ bool mmv_one_launch(int64_t K) { return plan_of(K).groups == 1; }
 
 bool mmv_supported(int type, int64_t M, int64_t K, int64_t N, const void *x, const void *gain) {
     if (type != kQ4_K && type != kQ8_0 && type != kQ4_0 && type != kIQ4_NL && type != kQ6_K) return false;
-    if (M < 2 || M > 16 || N < 1 || N > (int64_t)INT32_MAX / 64 || K < 256 || K > (1 << 20)) return false;
+    if (M < 3 || M > 16 || N < 1 || N > (int64_t)INT32_MAX / 64 || K < 256 || K > (1 << 20)) return false;
     if (K % (type == kQ6_K ? 512 : 256) != 0) return false;  // (Q6_K: rows of whole dwords)
     return ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(gain)) & 15) == 0;
 }

@@ -97,9 +97,10 @@ int gq_dequantize(int type, const void *dW, int64_t N, int64_t K, float *dOut, v
 /* ---- compute.Function.FusedQuantizedDense (core/graph/fused_ops.go:231-232), run time:
  * y = act(x . dequant(W)^T + bias), the contract of nn.QuantizedDense
  * (ml/nn/quantized_dense.go:31-57) and ggml.DenseDecomposed (ml/ggml/dense.go:23-62).
- * dBias may be NULL.  fp32 activations, fp32 accumulation.  The first few rows (4 to 6, depending
- * on format and matrix size; 16 for matrices of a few megabytes) run as bandwidth-bound GEMV
- * passes; larger batches contract on the matrix cores with the activations (and, from 65 to 385
+ * dBias may be NULL.  fp32 activations, fp32 accumulation.  One and two rows (more on matrices that the caches
+ * hold, up to 16 on those of a few megabytes) run as bandwidth-bound GEMV passes on 16-bit fixed-point activations; up to 16
+ * rows (most of Q4_K: 8) on the matrix cores with the activations as the sum of two fp16 numbers, 20 bits together;
+ * larger batches contract on the matrix cores with the activations (and, from 65 to 385
  * rows on, depending on format and shape, the dequantised weights) rounded to fp16 operands (each batch row scaled by a power of two first, so the magnitude of x does not
  * matter).  Batches of 5 rows and more may use a
  * per-stream workspace that is created on the first such call on the stream: make
@@ -169,8 +170,8 @@ typedef struct {
  * (Model.normalize followed by a projection, transformer.go:1099-1101; Add(residual, ...) after
  * the output and down projections, :1045, :1055, :1291-1292).  norm and dResidual may each be
  * NULL (both NULL is plain gq_qdense_f32); dY may be dResidual itself (a residual stream updated
- * in place).  Small batches (a few rows; up to 16 where the split-K kernels do not apply) run in
- * the decode GEMV itself when K is a multiple of 256 and x and gain are 16-byte aligned; large batches (those a plain call hands to the two-pass GEMM) fold the
+ * in place).  Small batches (up to 16 rows of at most 4096 values, fewer or none of longer ones) run in one launch of
+ * the decode GEMV or of the few-row kernel when K is a multiple of 256 and x and gain are 16-byte aligned; large batches (those a plain call hands to the two-pass GEMM) fold the
  * normalisation into the activation pass and the residual into the GEMM epilogue; the batches in
  * between (split-K kernels) apply the gain where their activation image is written and the
  * division and the residual in their reduction; what is left is composed of an RMSNorm kernel,
@@ -192,9 +193,9 @@ int gq_qdense_norm_f32_batch(int count, const gq_dense_desc *descs, const gq_rms
                              void *stream);
 /* The gated feed-forward front (transformer.go:1279-1287, after the pre_feedforward_norm of
  * :1276 when norm != NULL): y = act(xn . Wgate^T + bgate) * (xn . Wup^T + bup), xn = RMSNorm(x)
- * or x.  Both matrices are [N, gq_row_bytes(type, K)] of one type.  A few rows run as one launch
- * of the decode GEMV (conditions as for gq_qdense_block_f32); from 256 rows the two matrices are
- * dequantised into one interleaved 16-bit image and a single GEMM forms the product in
+ * or x.  Both matrices are [N, gq_row_bytes(type, K)] of one type.  Up to 16 rows run as one launch of the
+ * decode GEMV or of the few-row kernel (rows of at most 4096 values; conditions as for gq_qdense_block_f32); from 65 to 385 rows on, by
+ * format and shape, the two matrices are dequantised into one interleaved 16-bit image and a single GEMM forms the product in
  * registers; in between, the split-K kernels contract both matrices against one activation
  * image in one launch (the normalisation in their pre-pass and reduction, the product in the
  * reduction) up to their batch limit, and dense calls are composed beyond it.  All but the
