@@ -316,27 +316,40 @@ int64_t gemv_reach(int type, int64_t K, int64_t values, int matrices, bool extra
 // 9 to 16 rows as two sets of 8, the split-K kernels up to 32 at one price: Q4_K and the other 4-bit formats, whose weights take least of
 // the time, feel that from 9 rows on.  And where the slices of K do not come out in groups of eight, mmv.hip leaves wavefront slots
 // empty.  Measured (us, split-K | mmv.hip):
-//   Q4_K    K <= 4096, 12 rows: 4096x14336 19.0 | 20.5, gated pairs of it 27.8 | 26.3, of 3072x6144 17.3 | 18.8, of 1024x16384 16.1 | 17.2
-//           8 and 12 rows: 14336x4096 17.8 18.1 | 17.6 22.7, 8192x8192 22.5 22.9 | 17.2 23.5; 8 rows: 4608x4096 12.6 | 13.2, behind a norm 10240x4096 16.6 | 18.2
-//           (at 4 rows 16.2 | 15.1) and 6144x8192 17.6 | 18.4, gated pairs of 4608x4096 16.0 | 17.1, of 6144x8192 26.5 | 24.3
-//   Q4_0    12 rows: 4096x14336 24.2 | 20.3, 1024x32768 16.5 | 18.8; 8 and 12 rows: 6144x4096 14.9 15.5 | 13.5 17.1, 14336x4096 24.2 24.7 | 18.7 22.5,
-//           gated pairs at 12 rows: 8192x4096 24.9 | 24.5, 9216x4096 28.7 | 31.4
+//   Q4_K    K <= 4096, 12 rows: 4096x14336 19.0 | 20.5, gated pairs of it 27.8 | 26.3, of 3072x6144 17.3 | 18.8, of 3072x11008 27.3 | 21.9, of 1024x16384 16.1 | 17.2
+//           8 and 12 rows: 14336x4096 17.8 18.1 | 17.6 22.7, 8192x8192 22.5 22.9 | 17.2 23.5; 8 rows: 4608x4096 12.6 | 13.2, 5120x20480 behind a norm 25.9 | 27.2, 6144x8192 17.6 |
+//           18.4, 6144x11008 24.6 | 19.7, 10240x4096 16.6 | 18.2 (at 4 rows 16.2 | 15.1), 10240x2560 16.6 | 14.7, gated pairs of 4608x4096 16.0 | 17.1, of 6144x8192 26.5 | 24.3,
+//           of 4608x20480 35.1 | 40.6
+//   Q4_0    12 rows: 4096x14336 24.2 | 20.3, 1024x32768 16.5 | 18.8; 8 and 12 rows: 6144x4096 14.9 15.5 | 13.5 17.1, 14336x4096 24.2 24.7 | 18.7 22.5; mmv.hip over split-K at 12 rows:
+//           5120x3072 (8 MB) 1.17, 5120x8192 1.10, 6144x8192 .96, 9216x1536 1.09, 9216x2048 .98, 9216x3072 1.13; gated pairs: 5120x8192 1.13, 8192x4096 .98, 9216x4096 1.08, 9984x2560 .89
 //   IQ4_NL  8 and 12 rows: 8192x4096 17.0 17.7 | 15.4 18.7; 12 rows: 12288x4096 26.5 | 24.3, 2048x16384 behind a norm 17.9 | 18.9
-//   Q8_0    8 and 12 rows: 8192x1024 13.4 13.6 | 11.7 14.8, 9216x1024 14.2 14.4 | 11.6 13.6; 12 rows: 256x32768 13.5 | 14.2
+//   Q8_0    8 and 12 rows: 8192x1024 13.4 13.6 | 11.7 14.8, 9216x1024 14.2 14.4 | 11.6 13.6; 12 rows: 256x32768 13.5 | 14.2, 5120x3072 14.4 | 16.5 (two rounds of tiles, the
+//           second half empty), 5120x4096 19.3 | 16.8.  Q6_K 5120x3072 16.7 | 18.1
+// (Widths move both kernels by whole rounds of tiles, so that single shapes lie up to 15 % on the other side of these lines.)
 // Their scratch memory is the larger one.
 bool split_k_ahead(int type, int64_t M, int64_t K, int64_t one, int matrices) {
     const int64_t MB = (int64_t)1 << 20, slices = (K + 511) / 512, slots = (slices + 7) / 8 * 8;
     const bool gaps = K > 2048 && slices * 20 < slots * 17;
+    auto within = [&](int64_t lo, int64_t hi) { return one >= lo * MB && one < hi * MB; };
     if (M < 5 || one < kTinyWeightBytes) return false;
     if (mmv_one_launch(K)) {
-        if (type == GQ_Q4_K) return M > 8 && (matrices == 1 || gaps || K <= 1024);
-        return M > 8 && matrices == 1 && one >= 8 * MB && type != GQ_Q6_K && K <= (type == GQ_Q8_0 ? 512 : one >= 16 * MB ? 2048 : 1024);
+        if (M <= 8) return false;
+        if (type == GQ_Q4_K) return matrices == 1 || K <= 1024 || (gaps && one < 14 * MB);
+        return matrices == 1 && one >= 8 * MB && type != GQ_Q6_K && K <= (type == GQ_Q8_0 ? 512 : one >= 16 * MB ? 2048 : 1024);
     }
     switch (type) {
-    case GQ_Q4_K: return M > 8 || (gaps && one >= 10 * MB && one < (matrices == 1 ? 28 : 13) * MB);
+    case GQ_Q4_K:
+        if (M > 8) return true;
+        if (!gaps || (matrices == 2 && K > 6144)) return false;
+        if (matrices == 2) return within(7, 13) || (K <= 5120 && one >= 48 * MB);
+        return K <= 5120 ? one >= 10 * MB : K <= 6144 ? within(10, 28) : within(18, 24);
     case GQ_Q4_0:
-    case GQ_IQ4_NL: return M > 8 && one >= 9 * MB && one < 26 * MB && (matrices == 1 || gaps);
-    case GQ_Q8_0: return M > 8 && one < 9 * MB;
+    case GQ_IQ4_NL:
+        if (M <= 8 || (matrices == 2 && !gaps)) return false;
+        if (!gaps) return within(9, 26);
+        return K <= 6144 ? within(7, K <= 5120 ? 31 : 24) : within(7, 9) || within(15, matrices == 1 ? 26 : 24);
+    case GQ_Q8_0: return M > 8 && (one < 9 * MB || (matrices == 1 && K <= 5120 && within(13, 17)));
+    case GQ_Q6_K: return M > 8 && matrices == 1 && K <= 5120 && within(10, 13);
     default: return false;
     }
 }
