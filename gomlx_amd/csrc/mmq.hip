@@ -26,6 +26,7 @@
 // lane's sixteen results belong to ONE weight row, the one whose header it has already loaded.
 #include "blocks.hpp"
 #include "common.hpp"
+#include "lds_dma.hpp"
 
 #include <algorithm>
 #include <cstdlib>
@@ -296,13 +297,38 @@ __device__ __forceinline__ void q4k_contract_sb(const RawSB &cur, const uint8_t 
 // halves (steps 2 H and 2 H + 1 of the super-block's four), so that the images can be staged half a super-block at a time:
 // `img` holds tile t's half at 8192 t - 16 slots of (32 columns x 16 bytes) in the order of stage_x, whose slot index
 // modulo 16 is the position inside the half.
+//
+// Everything a matrix instruction needs is prepared one group of RM of them ahead: the operands of a step (`w`, two sets: they
+// stay in registers from one half to the next) a quarter per group of the step before it, the activations of a group during the
+// group before it, one LDS read and a few vector-ALU instructions behind each matrix instruction (sched_group_barrier).  Left to
+// itself the compiler puts a group's reads behind its matrix instructions and then waits for all of them in front of the
+// next group's first.
+struct Q4KScales { h2 s0, s1, k0, k1; };
+__device__ __forceinline__ Q4KScales q4k_step_scales(const uint4 &hd, int st) {
+    const uint32_t sc = st < 2 ? (hd.y & 0x3F3F3F3Fu) : ((hd.w & 0x0F0F0F0Fu) | ((hd.y >> 2) & 0x30303030u));  // scales 0..3 / 4..7 as bytes
+    const uint32_t scw = sc >> (16 * (st & 1));
+    const float s0f = (float)(scw & 0xFFu), s1f = (float)((scw >> 8) & 0xFFu);
+    return Q4KScales{as_h2(pack_h2(s0f, s0f)), as_h2(pack_h2(s1f * 0.0625f, s1f * 0.0625f)),  // high-nibble pairs arrive as 1024 + 16 n
+                     as_h2(pack_h2(-1024.f * s0f, -1024.f * s0f)), as_h2(pack_h2(-64.f * s1f, -64.f * s1f))};
+}
+// dword i of a step's four code dwords: operands 2 i, 2 i + 1 of its low nibbles (w[0 .. 7]) and of its high ones (w[8 .. 15])
+__device__ __forceinline__ void q4k_step_quarter(const Q4KScales &k, uint32_t u, int i, uint32_t magic, uint32_t (&w)[16]) {
+    const uint32_t v = u >> 8;
+    w[2 * i] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(magic_pair(u, 0x000F000Fu, magic), k.s0, k.k0));
+    w[2 * i + 1] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(magic_pair(v, 0x000F000Fu, magic), k.s0, k.k0));
+    w[8 + 2 * i] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(magic_pair(u, 0x00F000F0u, magic), k.s1, k.k1));
+    w[8 + 2 * i + 1] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(magic_pair(v, 0x00F000F0u, magic), k.s1, k.k1));
+}
+__device__ __forceinline__ uint32_t q4k_dword(const RawSB &r, int st, int i) { return i == 0 ? r.c[st].x : i == 1 ? r.c[st].y : i == 2 ? r.c[st].z : r.c[st].w; }
+__device__ __forceinline__ void q4k_step(const RawSB &cur, int st, uint32_t magic, uint32_t (&w)[16]) {
+    const Q4KScales k = q4k_step_scales(cur.hd, st);
+#pragma unroll
+    for (int i = 0; i < 4; i++) q4k_step_quarter(k, q4k_dword(cur, st, i), i, magic, w);
+}
+
+// w[0]: the operands of step 2 H on entry (q4k_step for H = 0), of step 2 H + 2 on return
 template <int RM, int H>
-__device__ __forceinline__ void q4k_tiles_half(const RawSB &cur, const uint8_t *img, int kg, int col, uint32_t magic, f16v (&p1)[RM]) {
-    const uint32_t a = cur.hd.y, c = cur.hd.w;
-    const uint32_t sc = H == 0 ? (a & 0x3F3F3F3Fu) : ((c & 0x0F0F0F0Fu) | ((a >> 2) & 0x30303030u));  // scales 0..3 / 4..7 as bytes
-    // Eight groups (step s2, fragment q) of RM MFMAs each; the activations of group g + 1 are requested from LDS before the
-    // MFMAs of group g are issued and nothing moves across the group boundaries, so that two groups' fragments are all the
-    // registers the reads take (left to itself the compiler hoists sixteen reads and more, and four tiles spill).
+__device__ __forceinline__ void q4k_tiles_half(const RawSB &cur, const uint8_t *img, int kg, int col, uint32_t magic, uint32_t (&w)[2][16], f16v (&p1)[RM]) {
     h8 xf[2][RM];
     auto request = [&](int g) __attribute__((always_inline)) {
         const int slot = (2 * (g >> 2) + kg) * 4 + (g & 3);  // fragment 4 st + q sits in slot 32 sb + 8 st + 4 kg + q of the image: this is that modulo 16
@@ -310,39 +336,35 @@ __device__ __forceinline__ void q4k_tiles_half(const RawSB &cur, const uint8_t *
         for (int t = 0; t < RM; t++) xf[g & 1][t] = *reinterpret_cast<const h8 *>(img + t * 8192 + (slot * kMT + (col ^ slot)) * 16);
     };
     request(0);
-    uint32_t wl[8], wh[8];
+    __builtin_amdgcn_sched_barrier(0);
+    Q4KScales k;
 #pragma unroll
     for (int g = 0; g < 8; g++) {
-        const int s2 = g >> 2, q = g & 3;
-        if (q == 0) {
-            const int st = 2 * H + s2;
-            const uint32_t scw = sc >> (16 * s2);
-            const float s0f = (float)(scw & 0xFFu), s1f = (float)((scw >> 8) & 0xFFu);
-            const h2 s0 = as_h2(pack_h2(s0f, s0f));
-            const h2 s1 = as_h2(pack_h2(s1f * 0.0625f, s1f * 0.0625f));  // high-nibble pairs arrive as 1024 + 16 n
-            const h2 k0h = as_h2(pack_h2(-1024.f * s0f, -1024.f * s0f));
-            const h2 k1h = as_h2(pack_h2(-64.f * s1f, -64.f * s1f));
-            const uint32_t dw[4] = {cur.c[st].x, cur.c[st].y, cur.c[st].z, cur.c[st].w};
-#pragma unroll
-            for (int w = 0; w < 4; w++) {
-                const uint32_t u = dw[w], v = dw[w] >> 8;
-                wl[2 * w] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(magic_pair(u, 0x000F000Fu, magic), s0, k0h));
-                wl[2 * w + 1] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(magic_pair(v, 0x000F000Fu, magic), s0, k0h));
-                wh[2 * w] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(magic_pair(u, 0x00F000F0u, magic), s1, k1h));
-                wh[2 * w + 1] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(magic_pair(v, 0x00F000F0u, magic), s1, k1h));
-            }
-        }
+        const int s2 = g >> 2, q = g & 3, next = 2 * H + s2 + 1;
         if (g + 1 < 8) request(g + 1);
-        const uint32_t *src = (q < 2 ? wl : wh) + 4 * (q & 1);
+        if (next < 4) {
+            if (q == 0) k = q4k_step_scales(cur.hd, next);
+            q4k_step_quarter(k, q4k_dword(cur, next, q), q, magic, w[(s2 + 1) & 1]);
+        }
+        const uint32_t *src = w[s2 & 1] + 8 * (q >> 1) + 4 * (q & 1);
         const h8 wfrag = __builtin_bit_cast(h8, make_uint4(src[0], src[1], src[2], src[3]));
+        f16v zero16;
 #pragma unroll
-        for (int t = 0; t < RM; t++) p1[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xf[g & 1][t], wfrag, p1[t], 0, 0, 0);
+        for (int r = 0; r < 16; r++) zero16[r] = 0.f;
+#pragma unroll
+        for (int t = 0; t < RM; t++) p1[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xf[g & 1][t], wfrag, H == 0 && g == 0 ? zero16 : p1[t], 0, 0, 0);
+#pragma unroll
+        for (int t = 0; t < RM; t++) {
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            if (q == 0) __builtin_amdgcn_sched_group_barrier(0x002, 9, 0);
+            else __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
+        }
         __builtin_amdgcn_sched_barrier(0);
     }
 }
 
-// The end of a super-block: the minima against the tiles' sub-block sums (tile t's at sums + 1024 t), then d and dmin in fp32;
-// p1 starts the next super-block at zero.  Only k-group 0 carries operands of the minima's MFMA (the sums are read by
+// The end of a super-block: the minima against the tiles' sub-block sums (tile t's at sums + 1024 t), then d and dmin in fp32.  Only k-group 0 carries operands of the minima's MFMA (the sums are read by
 // every lane and cleared by a mask in k-group 1: no branch around an LDS read).
 template <int RM>
 __device__ __forceinline__ void q4k_tiles_finish(const RawSB &cur, const uint8_t *sums, int kg, int col, uint32_t magic, f16v (&p1)[RM], f16v (&acc)[RM]) {
@@ -372,8 +394,6 @@ __device__ __forceinline__ void q4k_tiles_finish(const RawSB &cur, const uint8_t
         for (int r = 0; r < 16; r++) acc[t][r] = fmaf(d, p1[t][r], acc[t][r]);
 #pragma unroll
         for (int r = 0; r < 16; r++) acc[t][r] = fmaf(-dmin, p2[r], acc[t][r]);
-#pragma unroll
-        for (int r = 0; r < 16; r++) p1[t][r] = 0.f;
     }
 }
 
@@ -566,51 +586,51 @@ __global__ __launch_bounds__(64 * Q4KTiles::kWaves) void mmq_q4k_tiles_kernel(co
     const uint8_t *__restrict__ W = blockIdx.z ? W2 : set.W[prob];
     float *__restrict__ partial = blockIdx.z ? partial2 : partial0;
     const int N = set.N[prob], xblk = (int)blockIdx.x - set.wg0[prob];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int kg = lane >> 5, col = lane & 31;
     const int slice = blockIdx.y, nslices = gridDim.y;
     const int nsb = ((K >> 8) - slice + nslices - 1) / nslices;  // slice s holds super-blocks s, s + nslices, ... of every row (at least one)
     const int row0 = xblk * G::kRows + wave * 32;
     const int n = row0 + col;  // this lane's weight row
 
-    const uint8_t *wtile = W + (int64_t)min(row0, N - 1) * row_bytes + slice * 144;
+    // The copies into LDS are dma16's: behind the compiler's own form of them it waits for every LDS read in flight in front of each use of one.
+    const int rowc = min(row0, N - 1);
+    const i32x4 wrsrc = make_rsrc(W + (int64_t)rowc * row_bytes + slice * 144, (uint64_t)(N - rowc) * (uint64_t)row_bytes - (uint64_t)slice * 144);
     uint32_t csrc[kParkLoads];
 #pragma unroll
     for (int l = 0; l < kParkLoads; l++) {
         const int c = min(lane + 64 * l, 32 * 9 - 1);
-        csrc[l] = (uint32_t)(min(row0 + c / 9, N - 1) - min(row0, N - 1)) * (uint32_t)row_bytes + (uint32_t)((c % 9) * 16);
+        csrc[l] = (uint32_t)(min(row0 + c / 9, N - 1) - rowc) * (uint32_t)row_bytes + (uint32_t)((c % 9) * 16);
     }
+    const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>(lds);
     uint8_t *const park0 = lds + L::kRingBytes + L::kSumBytes + wave * (L::kParks * kParkBytes);
+    const uint32_t park_at = lds0 + (uint32_t)(L::kRingBytes + L::kSumBytes + wave * (L::kParks * kParkBytes));
     // super-block j of this wavefront's row tile -> park j % kParks: exactly kParkLoads load instructions
     auto fetch = [&](int sb) __attribute__((always_inline)) {
-        const uint8_t *base = wtile + sb * nslices * 144;
-        uint8_t *park = park0 + (sb % L::kParks) * kParkBytes;
+        const uint32_t soff = (uint32_t)(sb * nslices) * 144u, park = park_at + (uint32_t)((sb % L::kParks) * kParkBytes);
 #pragma unroll
         for (int l = 0; l < kParkLoads; l++)
             if (64 * l + 64 <= 32 * 9 || lane < 32 * 9 - 64 * l)  // (the last instruction carries 32 chunks)
-                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(base + csrc[l]),
-                                                 (__attribute__((address_space(3))) void *)(park + l * 1024), 16, 0, 0);
+                dma16(park + l * 1024u, wrsrc, csrc[l], soff);
     };
     // tile t's image of this slice: fragments of super-block j at 16384 j (its second half 8192 further), sums at kXFBytes + 512 j
     const uint8_t *img0 = ximg + ((size_t)(m0 / kMT) * nslices + slice) * kLdsBytes;
     const size_t tile_stride = (size_t)nslices * kLdsBytes;
-    // half `h` of super-block `sb` of every tile -> ring stage h; with the second half come the super-block's sub-block sums, which
-    // are read at its end and not again (one buffer, at a fixed address: the compiler's own wait insertion can tell it from the ring)
+    i32x4 irsrc[NT];
+#pragma unroll
+    for (int t = 0; t < NT; t++) irsrc[t] = make_rsrc(img0 + t * tile_stride, kLdsBytes);
+    const i32x4 srsrc = make_rsrc(img0 + (wave % NT) * tile_stride, kLdsBytes);
+    // half `h` of super-block `sb` of every tile -> ring stage h (a wavefront copies one kilobyte of each); with the second half come the super-block's
+    // sub-block sums, which are read at its end and not again (one buffer, at a fixed address)
     auto stage = [&](int sb, int h) __attribute__((always_inline)) {
-        uint8_t *dst = lds + h * L::kStageBytes;
-        for (int i = wave; i < NT * 8; i += G::kWaves) {
-            const int t = i >> 3, ck = i & 7;
-            __builtin_amdgcn_global_load_lds(
-                (const __attribute__((address_space(1))) void *)(img0 + t * tile_stride + sb * 16384 + h * G::kHalfBytes + ck * 1024 + lane * 16),
-                (__attribute__((address_space(3))) void *)(dst + t * G::kHalfBytes + ck * 1024), 16, 0, 0);
-        }
+        const uint32_t soff = (uint32_t)(sb * 16384 + h * G::kHalfBytes + wave * 1024);
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+            dma16(lds0 + (uint32_t)(h * L::kStageBytes + t * G::kHalfBytes + wave * 1024), irsrc[t], (uint32_t)lane * 16u, soff);
         // (every wavefront copies the 512 bytes of one tile's sums, with all 64 lanes - the upper half lands behind them, unused -
-        // and several wavefronts may copy the same tile's: no branch around a load into LDS, behind which the compiler would wait
-        // for every load in flight in front of the next LDS read)
+        // and several wavefronts may copy the same tile's)
         if (h == 1)
-            __builtin_amdgcn_global_load_lds(
-                (const __attribute__((address_space(1))) void *)(img0 + (wave % NT) * tile_stride + kXFBytes + sb * 512 + (lane & 31) * 16),
-                (__attribute__((address_space(3))) void *)(lds + L::kRingBytes + (wave % NT) * 1024), 16, 0, 0);
+            dma16(lds0 + (uint32_t)(L::kRingBytes + (wave % NT) * 1024), srsrc, (uint32_t)(lane & 31) * 16u, (uint32_t)(kXFBytes + sb * 512));
     };
     // (no fence: the loads that must have landed are waited for by count, and LDS reads have been consumed before a wavefront arrives)
     auto meet = [&](bool all) __attribute__((always_inline)) {
@@ -627,7 +647,7 @@ __global__ __launch_bounds__(64 * Q4KTiles::kWaves) void mmq_q4k_tiles_kernel(co
 #pragma unroll
     for (int t = 0; t < NT; t++)
 #pragma unroll
-        for (int r = 0; r < 16; r++) acc[t][r] = p1[t][r] = 0.f;
+        for (int r = 0; r < 16; r++) acc[t][r] = 0.f;
     uint32_t magic;
     asm volatile("v_mov_b32 %0, 0x64006400" : "=v"(magic));
 
@@ -656,11 +676,13 @@ __global__ __launch_bounds__(64 * Q4KTiles::kWaves) void mmq_q4k_tiles_kernel(co
         __builtin_amdgcn_wave_barrier();
         const bool more = sb + L::kParks < nsb;
         if (more) fetch(sb + L::kParks);
-        q4k_tiles_half<NT, 0>(cur, lds, kg, col, magic, p1);
+        uint32_t w[2][16];
+        q4k_step(cur, 0, magic, w[0]);
+        q4k_tiles_half<NT, 0>(cur, lds, kg, col, magic, w, p1);
         // second half: the image requested above must be there (the request of a weight tile, issued after it, may still be out)
         meet(!more);
         if (sb + 1 < nsb) stage(sb + 1, 0);
-        q4k_tiles_half<NT, 1>(cur, lds + L::kStageBytes, kg, col, magic, p1);
+        q4k_tiles_half<NT, 1>(cur, lds + L::kStageBytes, kg, col, magic, w, p1);
         q4k_tiles_finish<NT>(cur, lds + L::kRingBytes, kg, col, magic, p1, acc);
     }
 
@@ -2016,22 +2038,27 @@ int run_q4k_set(const void *x, bool x_is_bf16, int64_t M, int64_t K, int count, 
     }
     set.count = out.count = count;
     set.ntot = out.ntot = (int)N;
-    // Super-blocks per K-slice (at most 7: the image shares LDS with the parked tiles): the count that needs the fewest
-    // rounds of workgroups over the chip times the length of a round (+3: what a workgroup costs beyond its
-    // super-blocks); ties go to the longer slice (fewer partial sums).
-    int slice_sb = Tile::kMaxSliceSB;
+    // Super-blocks per K-slice: the count that needs the fewest rounds of workgroups over the chip times the length of a round; ties go to
+    // the longer slice (fewer partial sums).  mmq_q4k_kernel: at most 7 (the image shares LDS with the parked tiles), a workgroup costs 3
+    // super-blocks beyond its own.  mmq_q4k_tiles_kernel: at most the 8 of an image (it holds two halves of one at a time); with four tiles of
+    // 32 rows a workgroup costs 2 of its 3.9 us steps beyond them, and each slice's sums a store and a load at about 4.5 TB/s together (the gated pair of
+    // 4096 x 14336 at 128 rows: 4 slices of 4 in two rounds 69.6 us, 2 of 8 in one round 56.8).
+    const int max_slice_sb = together ? kSliceSB : Tile::kMaxSliceSB;
+    int slice_sb = max_slice_sb;
     {
         const int64_t cus = device_cu_count(), z = W2 ? 2 : 1;
+        const int64_t sums = together ? (int64_t)std::min<int64_t>(M, 128) * N * z * 8 / 4500 : 0;  // ns per slice
+        const int64_t sb_ns = 1100 + 700 * std::min(mtiles, 4);
         int64_t best_cost = INT64_MAX;
-        for (int ssb = Tile::kMaxSliceSB; ssb >= 2; ssb--) {
-            const int64_t wgs = rowwgs * ((sbs + ssb - 1) / ssb) * z;
-            const int64_t cost = ((wgs + cus - 1) / cus) * (ssb + 3);
+        for (int ssb = max_slice_sb; ssb >= 2; ssb--) {
+            const int64_t ns = (sbs + ssb - 1) / ssb, rounds = (rowwgs * ns * z + cus - 1) / cus;
+            const int64_t cost = together ? rounds * (ssb * sb_ns + 8000) + ns * sums : rounds * (ssb + 3);
             if (cost < best_cost) { best_cost = cost; slice_sb = ssb; }
         }
     }
     if (const char *e = std::getenv("GOMLX_HIPQ_Q4K_SLICE_SB")) {  // (tuning runs only)
         const int v = std::atoi(e);
-        if (v >= 1 && v <= Tile::kMaxSliceSB) slice_sb = v;
+        if (v >= 1 && v <= max_slice_sb) slice_sb = v;
     }
     const int nslices = (int)((sbs + slice_sb - 1) / slice_sb);
     const int64_t row_bytes = (K / 256) * 144;
