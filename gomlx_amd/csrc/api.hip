@@ -398,8 +398,8 @@ int two_pass(int type, bool x_is_bf16, const void *x, int64_t M, int64_t K, cons
     void *ws = nullptr;
     // (K in one piece where the static scratch array holds the images but not the sums of its slices: another order of the same fp32 sums, as
     // the header says.  Held to the slices that fit, gq_qdense_f32 would return the same bits, at 28.7 us for 21.5 on 4096 -> 1024 at 520 rows.)
-    const bool split_k = !serves_static_scratch() || gemm_two_pass_workspace(x_is_bf16, M, K, N) <= kStaticScratchBytes - kWsSyncBytes;
-    if (int rc = stream_workspace(s, gemm_two_pass_workspace(x_is_bf16, M, K, N, split_k), &ws)) return rc;
+    const bool split_k = !serves_static_scratch() || gemm_two_pass_workspace(type, x_is_bf16, M, K, N) <= kStaticScratchBytes - kWsSyncBytes;
+    if (int rc = stream_workspace(s, gemm_two_pass_workspace(type, x_is_bf16, M, K, N, split_k), &ws)) return rc;
     return launch_gemm_two_pass(type, x_is_bf16, x, M, K, static_cast<const uint8_t *>(W), N, bias, act, y, ws, s, split_k);
 }
 
@@ -847,7 +847,7 @@ int gq_qdense_block_f32(int type, const float *dX, int64_t M, int64_t K, const g
                                   (hipStream_t)stream);
     if (block_takes_two_pass(type, M, K, N, dX, rn.gain, dBias, dY, false)) {
         void *ws = nullptr;
-        if (int rc = stream_workspace((hipStream_t)stream, gemm_two_pass_block_workspace(M, K, N, false), &ws)) return rc;
+        if (int rc = stream_workspace((hipStream_t)stream, gemm_two_pass_block_workspace(type, M, K, N, false), &ws)) return rc;
         return launch_gemm_two_pass_block(type, dX, M, K, norm ? &rn : nullptr, (const uint8_t *)dW, dBias, nullptr, nullptr, dResidual, N, act,
                                           dY, ws, (hipStream_t)stream);
     }
@@ -930,7 +930,7 @@ int gq_qdense_norm_f32_batch(int count, const gq_dense_desc *descs, const gq_rms
     if (same_input_set(count, descs, set) && rows > kGemvMaxRows && (!norm->dGain || aligned_to(norm->dGain, 16)) &&
         gemm_two_pass_set_supported(descs[0].type, count, set, rows, descs[0].K, descs[0].dX)) {
         void *ws = nullptr;
-        if (int rc = stream_workspace((hipStream_t)stream, gemm_two_pass_set_workspace(count, set, rows, descs[0].K), &ws)) return rc;
+        if (int rc = stream_workspace((hipStream_t)stream, gemm_two_pass_set_workspace(descs[0].type, count, set, rows, descs[0].K), &ws)) return rc;
         return launch_gemm_two_pass_set(descs[0].type, descs[0].dX, rows, descs[0].K, &rn, count, set, ws, (hipStream_t)stream);
     }
     for (int i = 0; i < count; i++) {
@@ -960,7 +960,7 @@ int gq_qdense_gated_f32(int type, const float *dX, int64_t M, int64_t K, const g
                                   nullptr, N, act, dY, (hipStream_t)stream);
     if (block_takes_two_pass(type, M, K, N, dX, rn.gain, dBiasGate, dY, true)) {
         void *ws = nullptr;
-        if (int rc = stream_workspace((hipStream_t)stream, gemm_two_pass_block_workspace(M, K, N, true), &ws)) return rc;
+        if (int rc = stream_workspace((hipStream_t)stream, gemm_two_pass_block_workspace(type, M, K, N, true), &ws)) return rc;
         return launch_gemm_two_pass_block(type, dX, M, K, norm ? &rn : nullptr, (const uint8_t *)dWgate, dBiasGate, (const uint8_t *)dWup, dBiasUp,
                                           nullptr, N, act, dY, ws, (hipStream_t)stream);
     }

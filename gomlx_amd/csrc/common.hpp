@@ -125,13 +125,13 @@ int launch_gemv_ks_batch_norm(int type, int count, const XsBatchItem *items, con
 // bytes), then a plain 16-bit MFMA GEMM.
 bool gemm_two_pass_supported(int type, bool x_is_bf16, int64_t M, int64_t K, int64_t N, const void *x);
 // (split_k = false: K stays in one piece, and the workspace without room for the sums of its slices)
-size_t gemm_two_pass_workspace(bool x_is_bf16, int64_t M, int64_t K, int64_t N, bool split_k = true);
+size_t gemm_two_pass_workspace(int type, bool x_is_bf16, int64_t M, int64_t K, int64_t N, bool split_k = true);
 int launch_gemm_two_pass(int type, bool x_is_bf16, const void *x, int64_t M, int64_t K, const uint8_t *W, int64_t N, const float *bias,
                          int act, float *y, void *workspace, hipStream_t s, bool split_k = true);
 // The two passes with the neighbours of a projection folded in (fp32 activations; same conditions as
 // gemm_two_pass_supported): RMS normalisation in the activation pass, residual in the GEMM epilogue;
 // with W2 one GEMM over the interleaved image of both matrices forms the gated product in registers.
-size_t gemm_two_pass_block_workspace(int64_t M, int64_t K, int64_t N, bool gated);
+size_t gemm_two_pass_block_workspace(int type, int64_t M, int64_t K, int64_t N, bool gated);
 bool gemm_two_pass_block_supported(int type, int64_t M, int64_t K, int64_t N, const void *x, bool gated);
 int launch_gemm_two_pass_block(int type, const float *x, int64_t M, int64_t K, const RmsNorm *norm, const uint8_t *W, const float *bias,
                                const uint8_t *W2, const float *bias2, const float *residual, int64_t N, int act, float *y, void *workspace,
@@ -139,9 +139,13 @@ int launch_gemm_two_pass_block(int type, const float *x, int64_t M, int64_t K, c
 // Two to four matrices against the same fp32 activations through the two passes: one activation conversion, one image, one
 // GEMM that writes each matrix's columns to its own output (every N a multiple of 32, one activation for all).
 bool gemm_two_pass_set_supported(int type, int count, const MmqSetItem *items, int64_t M, int64_t K, const void *x);
-size_t gemm_two_pass_set_workspace(int count, const MmqSetItem *items, int64_t M, int64_t K);
+size_t gemm_two_pass_set_workspace(int type, int count, const MmqSetItem *items, int64_t M, int64_t K);
 int launch_gemm_two_pass_set(int type, const float *x, int64_t M, int64_t K, const RmsNorm *norm, int count, const MmqSetItem *items, void *workspace,
                              hipStream_t s);
+// One GEMM on the blocks themselves, weights converted in registers (gemm_wreg.hip): the main launch behind gemm_dma.hip's entry points.
+bool gemm_wreg_supported(int type, int64_t M, int64_t K, int64_t cols);
+int launch_gemm_wreg(int type, bool bf16, const uint16_t *x16, int64_t M, int64_t K, int count, const MmqSetItem *items, const uint8_t *W2,
+                     const float *bias2, int act, const float *residual, const float *rowscale, float *partial, int tm, int slices, hipStream_t s);
 int launch_gemm(int type, bool x_is_bf16, const void *x, int64_t M, int64_t K, const uint8_t *W, int64_t N,
                 const float *bias, int act, float *y, hipStream_t s);
 

@@ -26,6 +26,7 @@
 #include <type_traits>
 
 #include <cstdlib>
+#include <cstring>
 
 namespace gq {
 
@@ -812,13 +813,12 @@ int k_slices_env() {
 // wavefront's 64 x 128 share reads a quarter less from LDS per matrix instruction than 64 x 64, which that tile's time per step is
 // bound by), its gated pair at 512 and 1024 209 338 | 191 304, 4096x6144 at 2048 136 | 122; 14336x4096 at 256 and 512 rows 97 114 | 79 105
 // (slices where one round of small tiles filled the chip before).
-struct GemmPlan { int tile, slices; };
+struct GemmPlan { int tile, slices; double us; };
 GemmPlan plan_gemm(int64_t M, int64_t K, int64_t N, bool gated = false, bool may_split = true) {
     constexpr int kTiles = 4, dm[kTiles] = {256, 128, 128, 256}, dn[kTiles] = {128, 128, 64, 256};
     constexpr double step_us[kTiles] = {0.88, 0.61, 0.343, 1.476};
     const int64_t cus = device_cu_count(), steps = (K + DK - 1) / DK;
-    GemmPlan best{1, 1};
-    double best_us = 1e30;
+    GemmPlan best{1, 1, 1e30};
     for (int t = 0; t < kTiles; t++) {
         if (gated && t == 2) continue;
         if (tile_env() >= 0 && tile_env() < kTiles && t != tile_env() && !(gated && tile_env() == 2)) continue;
@@ -832,7 +832,7 @@ GemmPlan plan_gemm(int64_t M, int64_t K, int64_t N, bool gated = false, bool may
             const double frac = (double)(wgs % cus) / (double)cus;
             double us = ((double)full + (frac > 0 ? 0.89 + 0.11 * frac : 0)) * ((double)per + 6.5) * step_us[t];
             if (ns > 1) us += 2.05 + (double)(2 * ns + 1) * (double)M * (double)N * 4.0 / 3.6e6;
-            if (us < best_us) { best_us = us; best = {t, ns}; }
+            if (us < best.us) best = {t, ns, us};
         }
     }
     return best;
@@ -936,9 +936,104 @@ size_t two_pass_front_bytes(bool x_is_bf16, int64_t M, int64_t Kp, int64_t rows)
     return align256((size_t)rows * Kp * 2) + (x_is_bf16 ? 0 : align256((size_t)M * Kp * 2) + align256((size_t)M * sizeof(float)));
 }
 }  // namespace
-size_t gemm_two_pass_workspace(bool x_is_bf16, int64_t M, int64_t K, int64_t N, bool split_k) {
-    K = padded_k(K);
-    return two_pass_front_bytes(x_is_bf16, M, K, N) + (split_k ? gemm_partial_bytes(M, K, N) : 0);
+// ---- the one-GEMM form (gemm_wreg.hip)
+namespace {
+// Whether a call takes gemm_wreg.hip's kernel - one launch that converts weights in registers - in place of the image and the GEMM over it,
+// with how many rows of activations per workgroup (32 tm) and slices of K.  Both ways are estimated: rounds of workgroups of one per CU,
+// each its steps of 64 values of K and a fixed part (first bytes from memory, epilogue); slices cost a launch and their sums' way through
+// memory; the image 2 bytes per value written and the blocks read.  The constants are fitted to 540 problems (K x N 4096x4096, 4096x6144,
+// 4096x14336 and its pair, 14336x4096, 2048x2048, 8192x2048, 3072x8192, 5120x5120, 2048x16384, pairs of 2048x8192 and 1024x4096; 80 .. 2048 rows; Q4_K, Q8_0,
+// Q4_0, IQ4_NL) timed both ways with every tile and 1 2 3 4 6 8 slices.  The step and the fixed part are longer than the plain GEMM's, which
+// an image of few values does not pay for: from 2^25 values on, and where the estimate is 8 % ahead, the choice is the faster one in 130 of 133 problems
+// (the others 3 to 5 % behind).  E.g. (us, two passes | this): gated pair of 4096x14336 in Q4_K at 384, 512, 768 and 2048 rows 163 165 251 481 | 95 119 188 451;
+// 14336x4096 at 256, 384 and 512 rows 78 97 101 | 52 67 83; Q8_0: the pair 172 174 259 492 | 110 134 222 516 (not taken), 14336x4096 82 100 103 | 62 75 93; at
+// 4096x4096 and 512 rows, Q4_K 36 | 38 (not taken).
+// GOMLX_HIPQ_GEMM_WREG=0 keeps every call on the two passes, =tm or =tm,slices (tm 4, 6 or 8) forces this way wherever it applies (tuning runs
+// and tests; read at every call).
+constexpr int64_t kWregValues = (int64_t)1 << 25;
+struct WregPlan { bool take; int tm, slices; };
+struct WregEnv { int tm, slices; };  // (tm: -1 not set, 0 never)
+WregEnv wreg_env() {
+    const char *e = std::getenv("GOMLX_HIPQ_GEMM_WREG");
+    if (!e) return WregEnv{-1, 0};
+    const char *comma = std::strchr(e, ',');
+    return WregEnv{std::atoi(e), comma ? std::atoi(comma + 1) : 0};
+}
+// tiles: workgroups along the weight rows; cols: columns of the sums; values: of all matrices
+WregPlan plan_wreg(int type, bool bf16, int64_t M, int64_t K, int64_t tiles, int64_t cols, int64_t values, bool gated, bool may_split) {
+    WregPlan best{false, 8, 1};
+    const WregEnv env = wreg_env();
+    if (env.tm == 0 || !gemm_wreg_supported(type, M, K, cols) || (env.tm < 0 && values < kWregValues)) return best;
+    constexpr int kTm[3] = {8, 6, 4};
+    constexpr double kStep[4][3] = {{1.39, 1.11, 0.90}, {1.82, 1.46, 1.24}, {1.55, 1.25, 1.03}, {1.81, 1.44, 1.22}}, kFixed[3] = {14.2, 11.9, 10.8};
+    const int row = type == kQ4_K ? 0 : type == kQ8_0 ? 1 : type == kQ4_0 ? 2 : 3;
+    const int64_t cus = device_cu_count(), units = K / 256;
+    double best_us = 1e30;
+    for (int t = 0; t < 3; t++) {
+        if (env.tm > 0 && env.tm != kTm[t]) continue;
+        for (int ns = 1; ns <= (gated || !may_split || cols % 4 != 0 ? 1 : 8); ns++) {
+            const int64_t per = (units + ns - 1) / ns;
+            if ((ns - 1) * per >= units || (env.slices > 0 && ns > 1 && ns != env.slices)) continue;
+            const int64_t wgs = tiles * ((M + 32 * kTm[t] - 1) / (32 * kTm[t])) * ns, full = wgs / cus;
+            const double frac = (double)(wgs % cus) / (double)cus;
+            double us = ((double)full + (frac > 0 ? 0.77 + 0.23 * frac : 0)) * ((double)(4 * per) * kStep[row][t] + kFixed[t]);
+            if (ns > 1) us += 3.4 + (double)(2 * ns + 1) * (double)M * (double)cols * 4.0 / 15.4e6;
+            if (us < best_us || (ns > 1 && ns == env.slices)) { best_us = us; best.tm = kTm[t]; best.slices = ns; }
+        }
+    }
+    const double image = 4.5 + (double)values * (2.0 + (double)gq_bytes_per_block(type) / (double)gq_values_per_block(type)) / 7.4e6;
+    const int64_t image_rows = gated ? gated_image_rows(cols) : cols;
+    best.take = env.tm > 0 || best_us * 1.08 < plan_gemm(M, K, image_rows, gated, may_split).us + image - (bf16 ? 0.0 : 4.0);
+    return best;
+}
+WregPlan plan_wreg_one(int type, bool bf16, int64_t M, int64_t K, int64_t N, bool gated, bool may_split) {
+    return plan_wreg(type, bf16, M, K, gated ? (N + 127) / 128 : (N + 255) / 256, N, N * K * (gated ? 2 : 1), gated, may_split);
+}
+WregPlan plan_wreg_set(int type, int64_t M, int64_t K, int count, const MmqSetItem *items, bool may_split) {
+    int64_t tiles = 0, cols = 0;
+    for (int i = 0; i < count; i++) {
+        tiles += (items[i].N + 255) / 256;
+        cols += items[i].N;
+    }
+    return plan_wreg(type, false, M, K, tiles, cols, cols * K, false, may_split);
+}
+// [fp32 activations: fp16 rows, row scales (whole tiles of rows)][sums of the slices]
+size_t wreg_front_bytes(bool bf16, int64_t M, int64_t K) {
+    return bf16 ? 0 : align256((size_t)M * K * 2) + align256((size_t)((M + 255) / 256 * 256) * sizeof(float));
+}
+// (whatever the alignment of the outputs lets the plan be at the launch)
+size_t wreg_bytes(const WregPlan &split, bool bf16, int64_t M, int64_t K, int64_t cols) {
+    return wreg_front_bytes(bf16, M, K) + (split.take && split.slices > 1 ? (size_t)split.slices * M * cols * sizeof(float) : 0);
+}
+int run_wreg(int type, bool bf16, const void *x, int64_t M, int64_t K, const RmsNorm *norm, int count, const MmqSetItem *items, const uint8_t *W2,
+             const float *bias2, const float *residual, int act, void *workspace, const WregPlan &p, hipStream_t s) {
+    const uint16_t *x16 = static_cast<const uint16_t *>(x);
+    float *rowscale = nullptr;
+    if (!bf16) {
+        uint16_t *xh = static_cast<uint16_t *>(workspace);
+        rowscale = reinterpret_cast<float *>(xh + align256((size_t)M * K * 2) / 2);
+        if (int rc = launch_x_to_f16(static_cast<const float *>(x), M, K, norm, xh, rowscale, s)) return rc;
+        x16 = xh;
+    }
+    float *partial = reinterpret_cast<float *>(static_cast<uint8_t *>(workspace) + wreg_front_bytes(bf16, M, K));
+    if (int rc = launch_gemm_wreg(type, bf16, x16, M, K, count, items, W2, bias2, act, residual, rowscale, partial, p.tm, p.slices, s)) return rc;
+    if (p.slices == 1) return GQ_OK;
+    if (count == 1)
+        return launch_slices_reduce(partial, p.slices, M, items[0].N, rowscale, items[0].bias, act, residual, items[0].y, nullptr, s);
+    GemmSegs segs{};
+    segs.count = count;
+    for (int i = 0; i < count; i++) {
+        segs.y[i] = items[i].y; segs.bias[i] = items[i].bias;
+        segs.n0[i + 1] = segs.n0[i] + (int)items[i].N;
+    }
+    return launch_slices_reduce(partial, p.slices, M, segs.n0[count], rowscale, nullptr, act, nullptr, nullptr, &segs, s);
+}
+}  // namespace
+// (The image's bytes also where gemm_wreg.hip needs none: an output that is not aligned for slices may take the other way at the launch.)
+size_t gemm_two_pass_workspace(int type, bool x_is_bf16, int64_t M, int64_t K, int64_t N, bool split_k) {
+    const int64_t Kp = padded_k(K);
+    return std::max(two_pass_front_bytes(x_is_bf16, M, Kp, N) + (split_k ? gemm_partial_bytes(M, Kp, N) : 0),
+                    wreg_bytes(plan_wreg_one(type, x_is_bf16, M, K, N, false, split_k), x_is_bf16, M, K, N));
 }
 
 int launch_gemm_two_pass(int type, bool x_is_bf16, const void *x, int64_t M, int64_t K, const uint8_t *W, int64_t N, const float *bias,
@@ -946,6 +1041,10 @@ int launch_gemm_two_pass(int type, bool x_is_bf16, const void *x, int64_t M, int
     uint16_t *wh = static_cast<uint16_t *>(workspace);
     const int64_t Kp = padded_k(K);
     float *partial = split_k ? reinterpret_cast<float *>(static_cast<uint8_t *>(workspace) + two_pass_front_bytes(x_is_bf16, M, Kp, N)) : nullptr;
+    if (const WregPlan wp = plan_wreg_one(type, x_is_bf16, M, K, N, false, split_k && aligned16(bias, y)); wp.take) {
+        const MmqSetItem one{W, N, bias, act, y};
+        return run_wreg(type, x_is_bf16, x, M, K, nullptr, 1, &one, nullptr, nullptr, nullptr, act, workspace, wp, s);
+    }
     if (x_is_bf16) {
         if (int rc = launch_dequant16bit_type<true>(type, W, N, K, wh, s)) return rc;
         return launch_gemm16<true>(static_cast<const uint16_t *>(x), M, K, wh, N, bias, act, y, s, nullptr, nullptr, partial);
@@ -960,10 +1059,10 @@ int launch_gemm_two_pass(int type, bool x_is_bf16, const void *x, int64_t M, int
 // is folded into the activation pass, the residual into the GEMM's epilogue; a gated pair
 // act(xn.W + bias) * (xn.W2 + bias2) is ONE GEMM over the interleaved image of both matrices, the
 // product formed in registers, so neither projection is ever written out.
-size_t gemm_two_pass_block_workspace(int64_t M, int64_t K, int64_t N, bool gated) {
-    const int64_t rows = gated ? gated_image_rows(N) : N;
-    K = padded_k(K);
-    return two_pass_front_bytes(false, M, K, rows) + (gated ? 0 : gemm_partial_bytes(M, K, N));
+size_t gemm_two_pass_block_workspace(int type, int64_t M, int64_t K, int64_t N, bool gated) {
+    const int64_t rows = gated ? gated_image_rows(N) : N, Kp = padded_k(K);
+    return std::max(two_pass_front_bytes(false, M, Kp, rows) + (gated ? 0 : gemm_partial_bytes(M, Kp, N)),
+                    wreg_bytes(plan_wreg_one(type, false, M, K, N, gated, !gated), false, M, K, N));
 }
 
 bool gemm_two_pass_block_supported(int type, int64_t M, int64_t K, int64_t N, const void *x, bool gated) {
@@ -980,6 +1079,10 @@ int launch_gemm_two_pass_block(int type, const float *x, int64_t M, int64_t K, c
     uint16_t *xh = wh + align256((size_t)rows * Kp * 2) / 2;
     float *rowscale = reinterpret_cast<float *>(xh + align256((size_t)M * Kp * 2) / 2);
     float *partial = reinterpret_cast<float *>(static_cast<uint8_t *>(workspace) + two_pass_front_bytes(false, M, Kp, rows));
+    if (const WregPlan wp = plan_wreg_one(type, false, M, K, N, W2 != nullptr, !W2 && aligned16(bias, residual, y)); wp.take) {
+        const MmqSetItem one{W, N, bias, act, y};
+        return run_wreg(type, false, x, M, K, norm, 1, &one, W2, bias2, residual, act, workspace, wp, s);
+    }
     if (int rc = launch_prep_f32(type, x, M, K, norm, xh, rowscale, prep_one_or_pair(W, W2, N), wh, s)) return rc;
     if (!W2) return launch_gemm16<false>(xh, M, Kp, wh, N, bias, act, y, s, residual, rowscale, partial);
     return launch_gemm16_gated(xh, M, Kp, wh, N, bias, bias2, act, y, residual, rowscale, s);
@@ -999,10 +1102,12 @@ bool gemm_two_pass_set_supported(int type, int count, const MmqSetItem *items, i
     return gemm_two_pass_supported(type, false, M, K, ntot, x);
 }
 
-size_t gemm_two_pass_set_workspace(int count, const MmqSetItem *items, int64_t M, int64_t K) {
+size_t gemm_two_pass_set_workspace(int type, int count, const MmqSetItem *items, int64_t M, int64_t K) {
     int64_t ntot = 0;
     for (int i = 0; i < count; i++) ntot += items[i].N;
-    return gemm_two_pass_block_workspace(M, K, ntot, false);
+    const int64_t Kp = padded_k(K);
+    return std::max(two_pass_front_bytes(false, M, Kp, ntot) + gemm_partial_bytes(M, Kp, ntot),
+                    wreg_bytes(plan_wreg_set(type, M, K, count, items, true), false, M, K, ntot));
 }
 
 int launch_gemm_two_pass_set(int type, const float *x, int64_t M, int64_t K, const RmsNorm *norm, int count, const MmqSetItem *items, void *workspace,
@@ -1017,6 +1122,10 @@ int launch_gemm_two_pass_set(int type, const float *x, int64_t M, int64_t K, con
         ntot += items[i].N;
     }
     segs.n0[count] = (int)ntot;
+    bool aligned = true;
+    for (int i = 0; i < count; i++) aligned = aligned && aligned16(items[i].bias, items[i].y);
+    if (const WregPlan wp = plan_wreg_set(type, M, K, count, items, aligned); wp.take)
+        return run_wreg(type, false, x, M, K, norm, count, items, nullptr, nullptr, nullptr, items[0].act, workspace, wp, s);
     uint16_t *wh = static_cast<uint16_t *>(workspace);
     const int64_t Kp = padded_k(K);
     uint16_t *xh = wh + align256((size_t)ntot * Kp * 2) / 2;

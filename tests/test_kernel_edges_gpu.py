@@ -37,3 +37,62 @@ def test_q4_k_several_tiles_over_every_slice_length(gpu, monkeypatch, M, slice_s
     up = oracle.c_qdense(ggml.Q4_K, x, W2, None, oracle.ACT_NONE)
     got = nn.gated_feed_forward(xd, wd, dev(gpu, W2), q, Activation.RELU).cpu().numpy()
     assert np.max(np.abs(got - np.maximum(want, 0) * up)) < 2 * TOL_F32 * np.max(np.abs(want)) * np.max(np.abs(up))
+
+
+GEMM_TYPES = [ggml.Q4_K, ggml.Q8_0, ggml.Q4_0, ggml.IQ4_NL]
+
+
+@pytest.mark.parametrize("t", GEMM_TYPES)
+@pytest.mark.parametrize("tm,slices,M,K,N", [
+    (4, 1, 17, 256, 257),      # a single unit of K, one partly filled tile, N odd: element-wise stores
+    (4, 3, 129, 768, 260),     # one row into the second tile, a slice per unit, four columns into the second workgroup
+    (6, 1, 193, 1280, 36),     # one row over, N inside the first wavefront's tiles
+    (8, 2, 255, 1280, 516),    # one row short, uneven slices
+    (8, 1, 288, 512, 320),     # a whole tile and a whole 32-row part of the second
+])
+def test_gemm_with_weights_converted_in_registers(gpu, monkeypatch, t, tm, slices, M, K, N):
+    """Every epilogue of gemm_wreg.hip (plain, bias and activation, residual behind a norm, gated pair, q / k / v of one input) at the edges of
+    its tiles, fp32 and bfloat16 activations."""
+    torch = gpu
+    monkeypatch.setenv("GOMLX_HIPQ_GEMM_WREG", f"{tm},{slices}")
+    W, W2, x = synth.weights(t, 3, N, K), synth.weights(t, 4, N, K), synth.activations(5 + M, M, K)
+    rng = np.random.default_rng(M)
+    bias, res = rng.standard_normal(N).astype(np.float32), rng.standard_normal((M, N)).astype(np.float32)
+    q, wd, w2d, xd = Quantization(ggml_type=t), dev(torch, W), dev(torch, W2), dev(torch, x)
+    gate, up = (oracle.c_qdense(t, x, w, None, oracle.ACT_NONE) for w in (W, W2))
+    peak = float(np.max(np.abs(gate))) * float(np.max(np.abs(up)))
+    assert rel(nn.quantized_dense(xd, wd, q).cpu().numpy(), gate) < TOL_F32
+    got = nn.quantized_dense(xd, wd, q, dev(torch, bias), Activation.RELU).cpu().numpy()
+    assert np.max(np.abs(got - np.maximum(gate + bias, 0))) < TOL_F32 * np.max(np.abs(gate))
+    for act, f in ((Activation.SILU, lambda v: v / (1 + np.exp(-v))), (Activation.RELU, lambda v: np.maximum(v, 0))):
+        got = nn.gated_feed_forward(xd, wd, w2d, q, act).cpu().numpy()
+        assert np.max(np.abs(got - f(gate.astype(np.float64)) * up)) < 2 * TOL_F32 * peak
+    norm = nn.RMSNorm(gain=dev(torch, np.ones(K, np.float32)), epsilon=1e-5)
+    scale = np.sqrt(np.mean(x.astype(np.float64) ** 2, axis=1, keepdims=True) + 1e-5)
+    got = nn.quantized_dense(xd, wd, q, norm=norm, residual=dev(torch, res)).cpu().numpy()
+    assert np.max(np.abs(got - res - gate / scale)) < TOL_F32 * np.max(np.abs(gate / scale)) + 1e-6 * np.max(np.abs(res))
+    if N % 32 == 0:
+        outs = nn.quantized_dense_batch([(xd, w, q, None, None) for w in (wd, w2d, wd)], norm=norm)
+        for o, w in zip(outs, (gate, up, gate)):
+            assert rel(o.cpu().numpy(), w / scale) < TOL_F32
+    xb = xd.to(torch.bfloat16)
+    want = oracle.c_qdense(t, xb.float().cpu().numpy(), W, bias, oracle.ACT_NONE)
+    assert rel(nn.quantized_dense(xb, wd, q, dev(torch, bias)).cpu().numpy(), want) < TOL_BF16
+
+
+def test_gemm_with_weights_converted_in_registers_keeps_infinities(gpu, monkeypatch):
+    """A block of infinite scale in one weight row: that output column is infinite or NaN as the reference's, every other one untouched."""
+    torch = gpu
+    K, N, M = 512, 63, 40  # (an N that the split-K kernels do not take)
+    for t in (ggml.Q8_0, ggml.Q4_0, ggml.IQ4_NL):
+        W = synth.weights(t, 3, N, K)
+        W[5, 0:2] = np.frombuffer(np.float16(np.inf).tobytes(), np.uint8)
+        bpb = ggml.bytes_per_block(t)
+        W[5, 2:bpb] = 0x7F if t == ggml.Q8_0 else 0xFF  # largest code everywhere: no infinity meets its opposite inside the block
+        x = np.abs(synth.activations(9, M, K)) + 0.1
+        monkeypatch.setenv("GOMLX_HIPQ_GEMM_WREG", "4")
+        got = nn.quantized_dense(dev(torch, x), dev(torch, W), Quantization(ggml_type=t)).cpu().numpy()
+        want = oracle.c_qdense(t, x, W, None, oracle.ACT_NONE)
+        assert np.all(np.isposinf(want[:, 5])) and np.all(np.isposinf(got[:, 5]))
+        ok = np.arange(N) != 5
+        assert rel(got[:, ok], want[:, ok]) < TOL_F32
