@@ -947,7 +947,8 @@ namespace {
 // an image of few values does not pay for: from 2^25 values on, and where the estimate is 8 % ahead, the choice is the faster one in 130 of 133 problems
 // (the others 3 to 5 % behind).  E.g. (us, two passes | this): gated pair of 4096x14336 in Q4_K at 384, 512, 768 and 2048 rows 163 165 251 481 | 95 119 188 451;
 // 14336x4096 at 256, 384 and 512 rows 78 97 101 | 52 67 83; Q8_0: the pair 172 174 259 492 | 110 134 222 516 (not taken), 14336x4096 82 100 103 | 62 75 93; at
-// 4096x4096 and 512 rows, Q4_K 36 | 38 (not taken).
+// 4096x4096 and 512 rows, Q4_K 36 | 38 (not taken).  Few rows of less than 4096 values lie where neither estimate is good to 8 %: pair of 2048x12001 at 128 (Q4_K) and
+// 192 rows (Q8_0) 46 56 | 54 66 (not taken).
 // GOMLX_HIPQ_GEMM_WREG=0 keeps every call on the two passes, =tm or =tm,slices (tm 4, 6 or 8) forces this way wherever it applies (tuning runs
 // and tests; read at every call).
 constexpr int64_t kWregValues = (int64_t)1 << 25;
@@ -963,7 +964,7 @@ WregEnv wreg_env() {
 WregPlan plan_wreg(int type, bool bf16, int64_t M, int64_t K, int64_t tiles, int64_t cols, int64_t values, bool gated, bool may_split) {
     WregPlan best{false, 8, 1};
     const WregEnv env = wreg_env();
-    if (env.tm == 0 || !gemm_wreg_supported(type, M, K, cols) || (env.tm < 0 && values < kWregValues)) return best;
+    if (env.tm == 0 || !gemm_wreg_supported(type, M, K, cols) || (env.tm < 0 && (values < kWregValues || (K < 4096 && M <= 256)))) return best;
     constexpr int kTm[3] = {8, 6, 4};
     constexpr double kStep[4][3] = {{1.39, 1.11, 0.90}, {1.82, 1.46, 1.24}, {1.55, 1.25, 1.03}, {1.81, 1.44, 1.22}}, kFixed[3] = {14.2, 11.9, 10.8};
     const int row = type == kQ4_K ? 0 : type == kQ8_0 ? 1 : type == kQ4_0 ? 2 : 3;
