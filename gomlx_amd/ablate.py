@@ -79,14 +79,17 @@ _Q4K_NO_PARTIAL = """            asm volatile("" ::"v"(v));
 }
 
 // ---- several tiles of 32 batch rows per weight tile"""
-_Q4K_TILES_IMAGE = "    auto stage = [&](int sb, int h) __attribute__((always_inline)) {\n        uint8_t *dst = lds + h * L::kStageBytes;\n        for (int i = wave; i < NT * 8; i += G::kWaves) {\n"
-_Q4K_TILES_NO_IMAGE = "    auto stage = [&](int sb, int h) __attribute__((always_inline)) {\n        uint8_t *dst = lds + h * L::kStageBytes;\n        for (int i = wave; i < (sb == 0 ? NT * 8 : 0); i += G::kWaves) {\n"
-_Q4K_TILES_CONTRACT = "        q4k_tiles_half<NT, 0>(cur, lds, kg, col, magic, p1);\n"
+_Q4K_TILES_IMAGE = "            dma16(lds0 + (uint32_t)(h * L::kStageBytes + t * G::kHalfBytes + wave * 1024), irsrc[t], (uint32_t)lane * 16u, soff);\n"
+_Q4K_TILES_NO_IMAGE = "            if (sb == 0) dma16(lds0 + (uint32_t)(h * L::kStageBytes + t * G::kHalfBytes + wave * 1024), irsrc[t], (uint32_t)lane * 16u, soff);\n"
+_Q4K_TILES_CONTRACT = "        q4k_tiles_half<NT, 0>(cur, lds, kg, col, magic, w, p1);\n"
+_Q4K_TILES_EMPTY = _Q4K_KEEP + """        for (int t = 0; t < NT; t++)
+            for (int r = 0; r < 16; r++) p1[t][r] = 0.f;
+"""
 _Q4K_XPREP = """    if (int rc = x_is_bf16 ? (fine ? prep(mmq_xprep_kernel<true, 1>) : prep(mmq_xprep_kernel<true, 2>))
                            : (fine ? prep(mmq_xprep_kernel<false, 1>) : prep(mmq_xprep_kernel<false, 2>)))
         return rc;
 """
-_Q4K_REDUCE = "    if (count == 1) return launch_mmq_reduce(partial, partial2, xscale, nslices, M, K, N, items[0].bias, items[0].act, items[0].y, ex, s);\n"
+_Q4K_REDUCE = "    if (count == 1) return launch_mmq_reduce(partial, partial2, xscale, nslices, M, K, items[0].N, items[0].bias, items[0].act, items[0].y, ex, s);\n"
 
 _KS_STAGE = "                const Staged st = KS<T>::stage(p);\n"
 _KS_NO_STAGE = """                Staged st;
@@ -137,8 +140,8 @@ VARIANTS = {
     "q4k_tiles_no_image": ("mmq.hip", "the image copies of the kernel for several batch tiles after its first super-block (barriers kept)",
                            [(_Q4K_TILES_IMAGE, _Q4K_TILES_NO_IMAGE)]),
     "q4k_tiles_no_contract": ("mmq.hip", "unpacking and MFMAs of the kernel for several batch tiles (loads, image copies and barriers kept)",
-                              [(_Q4K_TILES_CONTRACT, _Q4K_KEEP),
-                               ("        q4k_tiles_half<NT, 1>(cur, lds + L::kStageBytes, kg, col, magic, p1);\n", "")]),
+                              [(_Q4K_TILES_CONTRACT, _Q4K_TILES_EMPTY),
+                               ("        q4k_tiles_half<NT, 1>(cur, lds + L::kStageBytes, kg, col, magic, w, p1);\n", "")]),
     "q4k_no_xprep": ("mmq.hip", "the activation pre-pass launch", [(_Q4K_XPREP, "    (void)prep;\n")]),
     "q4k_no_reduce": ("mmq.hip", "the reduction launch", [(_Q4K_REDUCE, "    if (count == 1) return GQ_OK;\n")]),
 }

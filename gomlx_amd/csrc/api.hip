@@ -4,6 +4,7 @@
 #include "common.hpp"
 #include "workspace.hpp"
 
+#include <algorithm>
 #include <atomic>
 #include <cstring>
 #include <cstdlib>
@@ -273,6 +274,38 @@ int64_t gated_split_k_to(int type, int64_t K, int64_t N) {
     }
 }
 
+// Whether an output's rows are whole float4 in memory, as the split-K kernels' reduction and the GEMMs' sums of K slices store them best.
+template <class... P> bool whole_rows(int64_t N, P... outputs) { return N % 4 == 0 && ((reinterpret_cast<uintptr_t>(outputs) | ...) & 15) == 0; }
+
+// The hand-over of a call whose rows are not (`whole` false).  Its two passes cannot slice K, which is what makes them wait on long rows, and on
+// short ones they were ahead of the lines above, which lie beyond the point where both are level; here the line is that point.  Measured
+// (time of the two passes over that of the split-K kernels; N 601 1501 3001 6001 12001):
+//   K 1024, 32 rows: Q4_K .94 .99 1.11 1.31 1.35, Q8_0 .88 .92 1.03 1.20 1.18, Q6_K .74 .77 .88 1.03 1.13; 64 rows: Q4_K .75 .78 .86 1.01 1.04
+//   K 2048, 64 rows: Q4_K 1.04 1.13 1.26 1.30 1.20 (96: .92 .98 1.06 1.05 1.03, gated 1.02 1.12 1.12 1.01 1.33), Q8_0 1.23 1.28 1.42 1.09 .90, Q4_0 1.27 1.34 1.47 1.30 1.12
+//     (96: 1.31 1.32 1.25 1.09 .80; gated 64: 1.32 1.43 1.36 1.01 1.10), IQ4_NL gated 64: 1.26 1.37 1.28 .96 1.07, Q6_K 32: 1.02 1.14 1.29 1.37 .97 (gated 1.06 1.24 1.28 .93 1.18; 33: .99 1.13 1.22 .94 .87)
+//   K 4096, 128 rows: Q4_K 1.27 1.29 1.25 1.22 1.32, Q8_0 1.82 1.40 1.12 1.06 .89 (96: 1.02 at 12001), Q4_0 1.87 1.59 1.25 1.07 .93, IQ4_NL 1.79 1.49 1.15 1.03 .90, gated .98 to 1.72;
+//     192: Q4_0 .72, IQ4_NL .68 at 12001; Q6_K 64: 1.60 1.71 1.16 1.05 1.07 (96: .80 at 6001)
+//   K 8192, 128 rows: Q8_0 2.07 1.61 1.48 1.39 1.60, Q4_0 2.36 1.81 1.53 1.45 1.28; 192: .91 to 1.03
+int64_t by_element_to(int type, int64_t K, int64_t N, bool gated) {
+    const int64_t one = weight_bytes_of(type, K, N);
+    const bool large = one >= kLargeWeightBytes;
+    // (matrices of fewer values stay with the two passes, whose results on unit vectors are the weights rounded once: 2048x601 1.04 to 1.5 at 64 rows)
+    if (K * N < ((int64_t)9 << 18)) return kGemvMaxRows;
+    if (K < 2048) return type == GQ_Q6_K || one < ((int64_t)3 << 20) ? kGemvMaxRows : 32;
+    if (K < 4096) {
+        if (type == GQ_Q4_K) return gated ? 96 : 64;
+        if (type == GQ_Q6_K) return gated ? kGemvMaxRows : 32;
+        return gated ? 48 : type == GQ_Q8_0 && large ? 32 : 64;
+    }
+    if (type == GQ_Q4_K) return INT64_MAX;
+    if (K < 8192) return type == GQ_Q6_K ? 64 : !gated && large ? 96 : 128;
+    return 128;
+}
+int64_t hand_over(int type, int64_t K, int64_t N, bool gated, bool whole) {
+    const int64_t to = gated ? gated_split_k_to(type, K, N) : split_k_to(type, K, N);
+    return whole || split_k_to_env() >= 0 ? to : std::min(to, by_element_to(type, K, N, gated));
+}
+
 // Whether y [M, N] lies over any part of x [M, K].  The split-K kernels and the two passes have read x before the launch that writes y; a kernel
 // whose workgroups read x while others write y must not have such a call.
 bool y_over_x(const void *x, bool x_is_bf16, const float *y, int64_t M, int64_t K, int64_t N) {
@@ -372,7 +405,7 @@ bool split_k_ahead(int type, int64_t M, int64_t K, int64_t one, int matrices) {
 bool takes_mmv(int type, int64_t M, int64_t K, int64_t N, const void *x, const void *gain, int matrices, bool extras, bool set = false) {
     if (M < 3 || !mmv_one_launch(K) || !mmv_supported(type, M, K, N, x, gain)) return false;
     const int64_t one = weight_bytes_of(type, K, N), bytes = one * matrices, MB = (int64_t)1 << 20;
-    if ((!set || type == GQ_Q4_K) && N % 4 == 0 && split_k_ahead(type, M, K, one, matrices)) return false;  // (what the split-K kernels take)
+    if ((!set || type == GQ_Q4_K) && split_k_ahead(type, M, K, one, matrices)) return false;  // (what the split-K kernels take)
     if (bytes < 9 * MB) return M * bytes >= 64 * MB;
     if (bytes < kLargeWeightBytes) return !(type == GQ_Q4_0 && M == 3) && M * bytes >= gemv_reach(type, K, K * N * matrices, matrices, extras, set) * MB;
     if (!extras && !set && M <= 4 && (type == GQ_Q8_0 || (type == GQ_Q4_0 && bytes < 64 * MB))) return false;  // one GEMV pass of four rows
@@ -390,6 +423,16 @@ int split_k(int type, const void *x, bool x_is_bf16, int64_t M, int64_t K, int c
     if (mmv) return launch_mmv(type, x, x_is_bf16, M, K, count, items, ex, s);
     if (count > 1) return launch_mmq_set(type, x, x_is_bf16, M, K, count, items, ex ? ex->norm : nullptr, s);
     return launch_mmq(type, x, x_is_bf16, M, K, items[0].W, items[0].N, items[0].bias, items[0].act, items[0].y, s, ex);
+}
+
+// Whether a call that the split-K kernels had no scratch memory for (a recording before the workspace exists, the static scratch array; nothing
+// has been launched then) goes on to the routes it would take without them: only where rows of N or the outputs' addresses are not
+// whole float4, calls which those routes served before the reduction stored them element by element.
+bool falls_back(int rc, bool whole) { return rc == GQ_ERR_INVALID && !whole; }
+bool whole_set(int count, const MmqSetItem *set) {
+    bool whole = true;
+    for (int i = 0; i < count; i++) whole = whole && whole_rows(set[i].N, set[i].bias, set[i].y);
+    return whole;
 }
 
 // large batches: W dequantised once into the stream's workspace, then a plain 16-bit GEMM
@@ -570,6 +613,7 @@ int gq_qdense_f32(int type, const float *dX, int64_t M, int64_t K, const void *d
     if (M == 0 || N == 0) return GQ_OK;
     if (int rc = use_device()) return rc;
     CallScope scope;
+    const bool whole = whole_rows(N, dBias, dY);
     // Small batches: GEMV passes cost about one third of the first pass per extra row; the split-K
     // MFMA kernels cost 19 .. 26 us (Q8_0 / Q4_0, K = 4096, N = 4096 .. 14336) for up to 32 rows and
     // 5 .. 18 us per further 32; the two passes 33 .. 62 us for anything up to 128 rows.  Measured
@@ -579,10 +623,13 @@ int gq_qdense_f32(int type, const float *dX, int64_t M, int64_t K, const void *d
         return launch_mmv(type, dX, false, M, K, 1, &one, nullptr, (hipStream_t)stream);
     const bool tp = gemm_two_pass_supported(type, false, M, K, N, dX);
     const bool ks = M <= kGemvMaxRows && gemv_ks_supported(type, K, N, dX);
-    const bool sk = M >= split_k_from(type, weight_bytes_of(type, K, N)) && mmq_supported(type, M, K, N, dX, dBias, dY) &&
-                    (M <= split_k_to(type, K, N) || !tp);
-    if (ks && !sk) return launch_gemv_ks(type, dX, false, M, K, (const uint8_t *)dW, N, dBias, act, dY, (hipStream_t)stream);
-    if (sk) return split_k(type, dX, false, M, K, 1, &one, nullptr, (hipStream_t)stream);
+    const bool sk = M >= split_k_from(type, weight_bytes_of(type, K, N)) && mmq_supported(type, M, K, N, dX) &&
+                    (M <= hand_over(type, K, N, false, whole) || !tp);
+    if (sk) {
+        const int rc = split_k(type, dX, false, M, K, 1, &one, nullptr, (hipStream_t)stream);
+        if (!falls_back(rc, whole)) return rc;
+    }
+    if (ks) return launch_gemv_ks(type, dX, false, M, K, (const uint8_t *)dW, N, dBias, act, dY, (hipStream_t)stream);
     // Shapes without a K-sliced plan (K not a multiple of 256: rare in models): a pass over W per row for up to 16
     // rows.  The 16-bit operands of the GEMMs below lean on averaging over many outputs and terms; on these few-row
     // problems seeded sweeps measured up to 0.9e-3 (1.25e-3 over a single block) through them, too close to the bound.
@@ -630,8 +677,10 @@ int gq_qdense_f32_batch(int count, const gq_dense_desc *descs, void *stream) {
         MmqSetItem set[4];
         if (set_takes_mmv(count, descs, nullptr, false, set))
             return launch_mmv(descs[0].type, descs[0].dX, false, descs[0].M, descs[0].K, count, set, nullptr, (hipStream_t)stream);
-        if (descs[0].M >= kSharedPassFromRows && takes_shared_pass(count, descs, nullptr, set))
-            return split_k(descs[0].type, descs[0].dX, false, descs[0].M, descs[0].K, count, set, nullptr, (hipStream_t)stream);
+        if (descs[0].M >= kSharedPassFromRows && takes_shared_pass(count, descs, nullptr, set)) {
+            const int rc = split_k(descs[0].type, descs[0].dX, false, descs[0].M, descs[0].K, count, set, nullptr, (hipStream_t)stream);
+            if (!falls_back(rc, whole_set(count, set))) return rc;
+        }
     }
     // problems that calls of their own would hand to the few-row kernel: up to four of one type, batch size and K in one launch, each with
     // its own input and share of the workgroups, and the bits of a call of its own (two Q4_K 4096x4096 at 3 and 5 rows 9.8 and 11.6 us; one launch each took 16.0 18.7,
@@ -704,6 +753,7 @@ int gq_qdense_bf16(int type, const uint16_t *dX, int64_t M, int64_t K, const voi
     if (M == 0 || N == 0) return GQ_OK;
     if (int rc = use_device()) return rc;
     CallScope scope;
+    const bool whole = whole_rows(N, dBias, dY);
     // Same crossovers as for fp32 activations: bf16 widens exactly to fp32 for the GEMV passes and to
     // the fp16 activation image of the split-K kernels (which have no bf16 rounding of W: tighter than
     // the bf16 MFMA paths).
@@ -712,10 +762,13 @@ int gq_qdense_bf16(int type, const uint16_t *dX, int64_t M, int64_t K, const voi
         return launch_mmv(type, dX, true, M, K, 1, &one, nullptr, (hipStream_t)stream);
     const bool tp = gemm_two_pass_supported(type, true, M, K, N, dX);
     const bool ks = M <= kGemvMaxRows && gemv_ks_supported(type, K, N, dX);
-    const bool sk = M >= split_k_from(type, weight_bytes_of(type, K, N)) && mmq_supported(type, M, K, N, dX, dBias, dY) &&
-                    (M <= split_k_to(type, K, N) || !tp);
-    if (ks && !sk) return launch_gemv_ks(type, dX, true, M, K, (const uint8_t *)dW, N, dBias, act, dY, (hipStream_t)stream);
-    if (sk) return split_k(type, dX, true, M, K, 1, &one, nullptr, (hipStream_t)stream);
+    const bool sk = M >= split_k_from(type, weight_bytes_of(type, K, N)) && mmq_supported(type, M, K, N, dX) &&
+                    (M <= hand_over(type, K, N, false, whole) || !tp);
+    if (sk) {
+        const int rc = split_k(type, dX, true, M, K, 1, &one, nullptr, (hipStream_t)stream);
+        if (!falls_back(rc, whole)) return rc;
+    }
+    if (ks) return launch_gemv_ks(type, dX, true, M, K, (const uint8_t *)dW, N, dBias, act, dY, (hipStream_t)stream);
     if (tp) return two_pass(type, true, dX, M, K, dW, N, dBias, act, dY, (hipStream_t)stream);
     return launch_gemm(type, true, dX, M, K, (const uint8_t *)dW, N, dBias, act, dY, (hipStream_t)stream);
 }
@@ -760,22 +813,22 @@ int64_t block_split_k_from(int type, int64_t weight_bytes, bool gated) {
     }
 }
 
-bool fold_into_gemv(int type, int64_t M, int64_t K, int64_t N, const float *x, const float *gain, const float *bias, const float *y, bool gated) {
+bool fold_into_gemv(int type, int64_t M, int64_t K, int64_t N, const float *x, const float *gain, bool gated) {
     if (!gemv_ks_ext_supported(type, M, K, N, x, gain)) return false;
-    return !(M >= block_split_k_from(type, weight_bytes_of(type, K, N), gated) && mmq_supported(type, M, K, N, x, bias, y));
+    return !(M >= block_split_k_from(type, weight_bytes_of(type, K, N), gated) && mmq_supported(type, M, K, N, x));
 }
 
 // Whether a projection with its neighbours runs on the split-K kernels (after fold_into_gemv() has declined).
-bool block_takes_split_k(int type, int64_t M, int64_t K, int64_t N, const float *x, const float *bias, const float *y, bool gated) {
+bool block_takes_split_k(int type, int64_t M, int64_t K, int64_t N, const float *x, bool gated, bool whole) {
     const bool tp = gated ? gemm_two_pass_block_supported(type, M, K, N, x, true) : gemm_two_pass_supported(type, false, M, K, N, x);
-    const int64_t to = gated ? gated_split_k_to(type, K, N) : split_k_to(type, K, N);
-    return M >= block_split_k_from(type, weight_bytes_of(type, K, N), gated) && mmq_supported(type, M, K, N, x, bias, y) && (M <= to || !tp);
+    const int64_t to = hand_over(type, K, N, gated, whole);
+    return M >= block_split_k_from(type, weight_bytes_of(type, K, N), gated) && mmq_supported(type, M, K, N, x) && (M <= to || !tp);
 }
 
 // Whether a plain dense call on these operands runs on the split-K kernels (the dispatch of gq_qdense_f32).
-bool dense_takes_split_k(int type, int64_t M, int64_t K, int64_t N, const float *x, const float *bias, const float *y) {
+bool dense_takes_split_k(int type, int64_t M, int64_t K, int64_t N, const float *x, bool whole) {
     const bool tp = gemm_two_pass_supported(type, false, M, K, N, x);
-    return M >= split_k_from(type, weight_bytes_of(type, K, N)) && mmq_supported(type, M, K, N, x, bias, y) && (M <= split_k_to(type, K, N) || !tp);
+    return M >= split_k_from(type, weight_bytes_of(type, K, N)) && mmq_supported(type, M, K, N, x) && (M <= hand_over(type, K, N, false, whole) || !tp);
 }
 
 // First batch size of the gated pair as one GEMM (wherever the split-K kernels have handed over: the composed form is never
@@ -787,13 +840,12 @@ int64_t gated_two_pass_from() {
 
 // Batches that a plain dense call would hand to the two-pass GEMM take its block form: the
 // normalisation rides on the activation pass, the residual and the gated product on the epilogue.
-bool block_takes_two_pass(int type, int64_t M, int64_t K, int64_t N, const float *x, const float *gain, const float *bias, const float *y,
-                          bool gated) {
+bool block_takes_two_pass(int type, int64_t M, int64_t K, int64_t N, const float *x, const float *gain, bool gated, bool whole) {
     if (M <= kGemvMaxRows || !gemm_two_pass_block_supported(type, M, K, N, x, gated)) return false;
     if (gated && M < gated_two_pass_from()) return false;
     if (gain && !aligned_to(gain, 16)) return false;
-    const int64_t to = gated ? gated_split_k_to(type, K, N) : split_k_to(type, K, N);
-    const bool sk = M >= split_k_from(type, weight_bytes_of(type, K, N)) && mmq_supported(type, M, K, N, x, bias, y) && M <= to;
+    const int64_t to = hand_over(type, K, N, gated, whole);
+    const bool sk = M >= split_k_from(type, weight_bytes_of(type, K, N)) && mmq_supported(type, M, K, N, x) && M <= to;
     return !sk;
 }
 // Whether a list of projections is one input contracted with two to four matrices that the shared split-K pass takes
@@ -822,7 +874,7 @@ bool takes_shared_pass(int count, const gq_dense_desc *descs, const float *gain,
     for (int i = 0; i < count; i++) ntot += descs[i].N;
     return mmq_set_supported(type, count, set, rows, K, descs[0].dX) &&
            rows >= block_split_k_from(type, weight_bytes_of(type, K, ntot), false) &&
-           (rows <= split_k_to(type, K, ntot) || !gemm_two_pass_supported(type, false, rows, K, ntot, descs[0].dX));
+           (rows <= hand_over(type, K, ntot, false, whole_set(count, set)) || !gemm_two_pass_supported(type, false, rows, K, ntot, descs[0].dX));
 }
 }  // namespace
 
@@ -836,24 +888,29 @@ int gq_qdense_block_f32(int type, const float *dX, int64_t M, int64_t K, const g
     if (M == 0 || N == 0) return GQ_OK;
     if (int rc = use_device()) return rc;
     CallScope scope;
+    const bool whole = whole_rows(N, dBias, dResidual, dY);
     RmsNorm rn{nullptr, 0.f, 0.f};
     if (norm) rn = RmsNorm{norm->dGain, norm->eps, norm->gain_offset};
     const MmqSetItem one{(const uint8_t *)dW, N, dBias, act, dY};
     const MmqExtra ex{nullptr, nullptr, dResidual, norm ? &rn : nullptr};
     if (takes_mmv(type, M, K, N, dX, rn.gain, 1, true) && !y_over_x(dX, false, dY, M, K, N))
         return launch_mmv(type, dX, false, M, K, 1, &one, &ex, (hipStream_t)stream);
-    if (fold_into_gemv(type, M, K, N, dX, rn.gain, dBias, dY, false))
+    if (fold_into_gemv(type, M, K, N, dX, rn.gain, false))
         return launch_gemv_ks_ext(type, dX, false, M, K, norm ? &rn : nullptr, (const uint8_t *)dW, dBias, nullptr, nullptr, dResidual, N, act, dY,
                                   (hipStream_t)stream);
-    if (block_takes_two_pass(type, M, K, N, dX, rn.gain, dBias, dY, false)) {
+    if (block_takes_two_pass(type, M, K, N, dX, rn.gain, false, whole)) {
         void *ws = nullptr;
         if (int rc = stream_workspace((hipStream_t)stream, gemm_two_pass_block_workspace(type, M, K, N, false), &ws)) return rc;
         return launch_gemm_two_pass_block(type, dX, M, K, norm ? &rn : nullptr, (const uint8_t *)dW, dBias, nullptr, nullptr, dResidual, N, act,
                                           dY, ws, (hipStream_t)stream);
     }
     // split-K range: the normalisation rides on the activation pre-pass and the reduction, the residual on the reduction
-    if (block_takes_split_k(type, M, K, N, dX, dBias, dY, false) && (!dResidual || aligned_to(dResidual, 16)) && (!rn.gain || aligned_to(rn.gain, 16)))
-        return split_k(type, dX, false, M, K, 1, &one, &ex, (hipStream_t)stream);
+    if (block_takes_split_k(type, M, K, N, dX, false, whole) && (!rn.gain || aligned_to(rn.gain, 16))) {
+        const int rc = split_k(type, dX, false, M, K, 1, &one, &ex, (hipStream_t)stream);
+        if (!falls_back(rc, whole) || !gemv_ks_ext_supported(type, M, K, N, dX, rn.gain)) return rc;
+        return launch_gemv_ks_ext(type, dX, false, M, K, norm ? &rn : nullptr, (const uint8_t *)dW, dBias, nullptr, nullptr, dResidual, N, act, dY,
+                                  (hipStream_t)stream);
+    }
     // composed: normalised activations into the stream's second workspace, the dense call, then the residual.  When y
     // overlaps the residual (a residual stream updated in place) the dense result goes to the workspace first: written
     // straight to y it would destroy the residual before the addition reads it.
@@ -873,7 +930,7 @@ int gq_qdense_block_f32(int type, const float *dX, int64_t M, int64_t K, const g
             x = xn;
         }
     }
-    if (dResidual && dense_takes_split_k(type, M, K, N, x, dBias, dY) && aligned_to(dResidual, 16)) {  // the residual rides on the reduction
+    if (dResidual && dense_takes_split_k(type, M, K, N, x, whole)) {  // the residual rides on the reduction
         const MmqExtra plain{nullptr, nullptr, dResidual, nullptr};
         return split_k(type, x, false, M, K, 1, &one, &plain, (hipStream_t)stream);
     }
@@ -924,7 +981,12 @@ int gq_qdense_norm_f32_batch(int count, const gq_dense_desc *descs, const gq_rms
     XsBatchItem items[8];
     if (merges_into_gemv(count, descs, norm, shared_pass, items))
         return launch_gemv_ks_batch_norm(descs[0].type, count, items, &rn, (hipStream_t)stream, (int)rows);
-    if (shared_pass) return split_k(descs[0].type, descs[0].dX, false, rows, descs[0].K, count, set, &ex, (hipStream_t)stream);
+    if (shared_pass) {
+        const int rc = split_k(descs[0].type, descs[0].dX, false, rows, descs[0].K, count, set, &ex, (hipStream_t)stream);
+        if (!falls_back(rc, whole_set(count, set))) return rc;
+        if (merges_into_gemv(count, descs, norm, false, items))
+            return launch_gemv_ks_batch_norm(descs[0].type, count, items, &rn, (hipStream_t)stream, (int)rows);
+    }
     // Past the split-K range the same projections share the two passes: one activation conversion, one image of all the
     // matrices, one GEMM (a decoder layer's q / k / v at 128 rows: two launches instead of six).
     if (same_input_set(count, descs, set) && rows > kGemvMaxRows && (!norm->dGain || aligned_to(norm->dGain, 16)) &&
@@ -949,24 +1011,29 @@ int gq_qdense_gated_f32(int type, const float *dX, int64_t M, int64_t K, const g
     if (M == 0 || N == 0) return GQ_OK;
     if (int rc = use_device()) return rc;
     CallScope scope;
+    const bool whole = whole_rows(N, dBiasGate, dBiasUp, dY);
     RmsNorm rn{nullptr, 0.f, 0.f};
     if (norm) rn = RmsNorm{norm->dGain, norm->eps, norm->gain_offset};
     const MmqSetItem one{(const uint8_t *)dWgate, N, dBiasGate, act, dY};
     const MmqExtra ex{(const uint8_t *)dWup, dBiasUp, nullptr, norm ? &rn : nullptr};
     if (takes_mmv(type, M, K, N, dX, rn.gain, 2, true) && !y_over_x(dX, false, dY, M, K, N))
         return launch_mmv(type, dX, false, M, K, 1, &one, &ex, (hipStream_t)stream);
-    if (fold_into_gemv(type, M, K, N, dX, rn.gain, dBiasGate, dY, true))
+    if (fold_into_gemv(type, M, K, N, dX, rn.gain, true))
         return launch_gemv_ks_ext(type, dX, false, M, K, norm ? &rn : nullptr, (const uint8_t *)dWgate, dBiasGate, (const uint8_t *)dWup, dBiasUp,
                                   nullptr, N, act, dY, (hipStream_t)stream);
-    if (block_takes_two_pass(type, M, K, N, dX, rn.gain, dBiasGate, dY, true)) {
+    if (block_takes_two_pass(type, M, K, N, dX, rn.gain, true, whole)) {
         void *ws = nullptr;
         if (int rc = stream_workspace((hipStream_t)stream, gemm_two_pass_block_workspace(type, M, K, N, true), &ws)) return rc;
         return launch_gemm_two_pass_block(type, dX, M, K, norm ? &rn : nullptr, (const uint8_t *)dWgate, dBiasGate, (const uint8_t *)dWup, dBiasUp,
                                           nullptr, N, act, dY, ws, (hipStream_t)stream);
     }
     // (split-K: both matrices against one activation image, which carries the gain; the reduction normalises and forms act(gate) * up)
-    if (block_takes_split_k(type, M, K, N, dX, dBiasGate, dY, true) && (!dBiasUp || aligned_to(dBiasUp, 16)) && (!rn.gain || aligned_to(rn.gain, 16)))
-        return split_k(type, dX, false, M, K, 1, &one, &ex, (hipStream_t)stream);
+    if (block_takes_split_k(type, M, K, N, dX, true, whole) && (!rn.gain || aligned_to(rn.gain, 16))) {
+        const int rc = split_k(type, dX, false, M, K, 1, &one, &ex, (hipStream_t)stream);
+        if (!falls_back(rc, whole) || !gemv_ks_ext_supported(type, M, K, N, dX, rn.gain)) return rc;
+        return launch_gemv_ks_ext(type, dX, false, M, K, norm ? &rn : nullptr, (const uint8_t *)dWgate, dBiasGate, (const uint8_t *)dWup, dBiasUp,
+                                  nullptr, N, act, dY, (hipStream_t)stream);
+    }
     // composed: [normalised activations,] act(gate) into the stream's second workspace, up into y, y *= act(gate)
     const size_t xn_bytes = norm ? ((size_t)M * (size_t)K * sizeof(float) + 255) / 256 * 256 : 0;
     void *ws = nullptr;
@@ -977,7 +1044,7 @@ int gq_qdense_gated_f32(int type, const float *dX, int64_t M, int64_t K, const g
         if (int rc = launch_rmsnorm(dX, M, K, rn.gain, rn.gain_offset, rn.eps, xn, (hipStream_t)stream)) return rc;
         x = xn;
     }
-    if (dense_takes_split_k(type, M, K, N, x, dBiasGate, dY) && (!dBiasUp || aligned_to(dBiasUp, 16))) {
+    if (dense_takes_split_k(type, M, K, N, x, whole)) {
         // both matrices against one activation image; the reduction forms act(gate) * up
         const MmqExtra plain{(const uint8_t *)dWup, dBiasUp, nullptr, nullptr};
         return split_k(type, x, false, M, K, 1, &one, &plain, (hipStream_t)stream);
@@ -1011,20 +1078,24 @@ int gq_qdense_block_bf16(int type, const uint16_t *dX, int64_t M, int64_t K, con
     if (M == 0 || N == 0) return GQ_OK;
     if (int rc = use_device()) return rc;
     CallScope scope;
+    const bool whole = whole_rows(N, dBias, dResidual, dY);
     const RmsNorm rn = norm ? RmsNorm{norm->dGain, norm->eps, norm->gain_offset} : RmsNorm{nullptr, 0.f, 0.f};
     const MmqSetItem one{(const uint8_t *)dW, N, dBias, act, dY};
     const MmqExtra ex{nullptr, nullptr, dResidual, norm ? &rn : nullptr};
     if (takes_mmv(type, M, K, N, dX, rn.gain, 1, true) && !y_over_x(dX, true, dY, M, K, N))
         return launch_mmv(type, dX, true, M, K, 1, &one, &ex, (hipStream_t)stream);
-    if (fold_into_gemv(type, M, K, N, reinterpret_cast<const float *>(dX), norm ? norm->dGain : nullptr, dBias, dY, false)) {
+    if (fold_into_gemv(type, M, K, N, reinterpret_cast<const float *>(dX), norm ? norm->dGain : nullptr, false)) {
         return launch_gemv_ks_ext(type, dX, true, M, K, norm ? &rn : nullptr, (const uint8_t *)dW, dBias, nullptr, nullptr, dResidual, N, act, dY,
                                   (hipStream_t)stream);
     }
     {   // the split-K kernels' pre-pass reads bf16 as well (where the fp32 call would take them too)
         const float *xa = reinterpret_cast<const float *>(dX), *gain = norm ? norm->dGain : nullptr;  // (only their alignment is looked at)
-        if (!block_takes_two_pass(type, M, K, N, xa, gain, dBias, dY, false) && block_takes_split_k(type, M, K, N, xa, dBias, dY, false) &&
-            (!dResidual || aligned_to(dResidual, 16)) && (!gain || aligned_to(gain, 16)))
-            return split_k(type, dX, true, M, K, 1, &one, &ex, (hipStream_t)stream);
+        if (!block_takes_two_pass(type, M, K, N, xa, gain, false, whole) && block_takes_split_k(type, M, K, N, xa, false, whole) && (!gain || aligned_to(gain, 16))) {
+            const int rc = split_k(type, dX, true, M, K, 1, &one, &ex, (hipStream_t)stream);
+            if (!falls_back(rc, whole) || !gemv_ks_ext_supported(type, M, K, N, dX, gain)) return rc;
+            return launch_gemv_ks_ext(type, dX, true, M, K, norm ? &rn : nullptr, (const uint8_t *)dW, dBias, nullptr, nullptr, dResidual, N, act, dY,
+                                      (hipStream_t)stream);
+        }
     }
     void *ws = nullptr;
     if (int rc = stream_workspace((hipStream_t)stream, widened_bytes(M, K), &ws, kWsWidenSlot)) return rc;
@@ -1042,20 +1113,24 @@ int gq_qdense_gated_bf16(int type, const uint16_t *dX, int64_t M, int64_t K, con
     if (M == 0 || N == 0) return GQ_OK;
     if (int rc = use_device()) return rc;
     CallScope scope;
+    const bool whole = whole_rows(N, dBiasGate, dBiasUp, dY);
     const RmsNorm rn = norm ? RmsNorm{norm->dGain, norm->eps, norm->gain_offset} : RmsNorm{nullptr, 0.f, 0.f};
     const MmqSetItem one{(const uint8_t *)dWgate, N, dBiasGate, act, dY};
     const MmqExtra ex{(const uint8_t *)dWup, dBiasUp, nullptr, norm ? &rn : nullptr};
     if (takes_mmv(type, M, K, N, dX, rn.gain, 2, true) && !y_over_x(dX, true, dY, M, K, N))
         return launch_mmv(type, dX, true, M, K, 1, &one, &ex, (hipStream_t)stream);
-    if (fold_into_gemv(type, M, K, N, reinterpret_cast<const float *>(dX), norm ? norm->dGain : nullptr, dBiasGate, dY, true)) {
+    if (fold_into_gemv(type, M, K, N, reinterpret_cast<const float *>(dX), norm ? norm->dGain : nullptr, true)) {
         return launch_gemv_ks_ext(type, dX, true, M, K, norm ? &rn : nullptr, (const uint8_t *)dWgate, dBiasGate, (const uint8_t *)dWup, dBiasUp, nullptr,
                                   N, act, dY, (hipStream_t)stream);
     }
     {
         const float *xa = reinterpret_cast<const float *>(dX), *gain = norm ? norm->dGain : nullptr;  // (only their alignment is looked at)
-        if (!block_takes_two_pass(type, M, K, N, xa, gain, dBiasGate, dY, true) && block_takes_split_k(type, M, K, N, xa, dBiasGate, dY, true) &&
-            (!dBiasUp || aligned_to(dBiasUp, 16)) && (!gain || aligned_to(gain, 16)))
-            return split_k(type, dX, true, M, K, 1, &one, &ex, (hipStream_t)stream);
+        if (!block_takes_two_pass(type, M, K, N, xa, gain, true, whole) && block_takes_split_k(type, M, K, N, xa, true, whole) && (!gain || aligned_to(gain, 16))) {
+            const int rc = split_k(type, dX, true, M, K, 1, &one, &ex, (hipStream_t)stream);
+            if (!falls_back(rc, whole) || !gemv_ks_ext_supported(type, M, K, N, dX, gain)) return rc;
+            return launch_gemv_ks_ext(type, dX, true, M, K, norm ? &rn : nullptr, (const uint8_t *)dWgate, dBiasGate, (const uint8_t *)dWup, dBiasUp, nullptr,
+                                      N, act, dY, (hipStream_t)stream);
+        }
     }
     void *ws = nullptr;
     if (int rc = stream_workspace((hipStream_t)stream, widened_bytes(M, K), &ws, kWsWidenSlot)) return rc;
@@ -1085,7 +1160,12 @@ int gq_qdense_norm_bf16_batch(int count, const gq_dense_desc *descs, const gq_rm
         XsBatchItem items[8];
         if (merges_into_gemv(count, descs, norm, shared_pass, items))
             return launch_gemv_ks_batch_norm(descs[0].type, count, items, &rn, (hipStream_t)stream, (int)descs[0].M, true);
-        if (shared_pass) return split_k(descs[0].type, descs[0].dX, true, descs[0].M, descs[0].K, count, set, &ex, (hipStream_t)stream);
+        if (shared_pass) {
+            const int rc = split_k(descs[0].type, descs[0].dX, true, descs[0].M, descs[0].K, count, set, &ex, (hipStream_t)stream);
+            if (!falls_back(rc, whole_set(count, set))) return rc;
+            if (merges_into_gemv(count, descs, norm, false, items))
+                return launch_gemv_ks_batch_norm(descs[0].type, count, items, &rn, (hipStream_t)stream, (int)descs[0].M, true);
+        }
     }
     // every distinct activation matrix (q / k / v share theirs) is widened once
     gq_dense_desc wide[64];

@@ -79,7 +79,7 @@ int launch_gemv_xs(int type, const float *x, int64_t M, int64_t K, const uint8_t
 bool gemv_ks_supported(int type, int64_t K, int64_t N, const void *x);
 int launch_gemv_ks(int type, const void *x, bool x_is_bf16, int64_t M, int64_t K, const uint8_t *W, int64_t N,
                    const float *bias, int act, float *y, hipStream_t s);
-bool mmq_supported(int type, int64_t M, int64_t K, int64_t N, const void *x, const void *bias, const void *y);
+bool mmq_supported(int type, int64_t M, int64_t K, int64_t N, const void *x);
 // RMS normalisation in front of a projection: x / sqrt(mean(x^2) + eps) * (gain + gain_offset); gain may be null.
 struct RmsNorm { const float *gain; float eps, gain_offset; };
 // Optional extras of a split-K call: a second matrix (the result becomes act(x.W + bias) * (x.W2 + bias2), both
@@ -96,7 +96,7 @@ bool mmq_set_supported(int type, int count, const MmqSetItem *items, int64_t M, 
 int launch_mmq_set(int type, const void *x, bool x_is_bf16, int64_t M, int64_t K, int count, const MmqSetItem *items, const RmsNorm *norm,
                    hipStream_t s);
 // 3 to 16 activation rows in one launch on the matrix cores (mmv.hip); more than 4096 values of K take a second launch, workspace
-// and what mmq_supported asks of N, bias, residual and y.
+// (sums of slices).
 bool mmv_supported(int type, int64_t M, int64_t K, int64_t N, const void *x, const void *gain);
 bool mmv_one_launch(int64_t K);
 // xs: every matrix with activations of its own (two to four of them, K in one launch, no extras).

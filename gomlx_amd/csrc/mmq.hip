@@ -66,6 +66,9 @@ template <int RT> struct Q4KTile {
 };
 constexpr int kQ4KRowTiles = 4;
 
+// The partial sums' rows are as long as a whole number of float4: N rounded up (the columns behind N are never read into an output).
+__host__ __device__ inline int64_t sum_cols(int64_t N) { return (N + 3) & ~(int64_t)3; }
+
 __device__ __forceinline__ uint32_t pack_h2(float a, float b) {
     h2 v;
     v.x = (_Float16)a;
@@ -925,22 +928,39 @@ __global__ __launch_bounds__(64 * RT * kParts) void mmq_q4k_coop_kernel(const vo
     }
 }
 
-// y[m][n] = act(sum_s partial[s][m][n] + bias[n]); N % 4 == 0 is guaranteed by the caller.  With a second
+// Four columns of an output row: as one float4 where `vec` says that every row and pointer is 16-byte aligned, else those of them
+// that are inside the row, one by one.
+__device__ __forceinline__ float4 load_cols(const float *p, int left, bool vec) {
+    if (vec) return *reinterpret_cast<const float4 *>(p);
+    return make_float4(p[0], left > 1 ? p[1] : 0.f, left > 2 ? p[2] : 0.f, left > 3 ? p[3] : 0.f);
+}
+__device__ __forceinline__ void store_cols(float *p, const float4 &v, int left, bool vec) {
+    if (vec) {
+        *reinterpret_cast<float4 *>(p) = v;
+        return;
+    }
+    p[0] = v.x;
+    if (left > 1) p[1] = v.y;
+    if (left > 2) p[2] = v.z;
+    if (left > 3) p[3] = v.w;
+}
+
+// y[m][n] = act(sum_s partial[s][m][n] + bias[n]); a thread owns four columns of the sums, whose rows are sum_cols(N) long.  With a second
 // set of partial sums (the other matrix of a gated pair) the result is multiplied by
 // sum_s partial2[s][m][n] + bias2[n]; a residual (which may be Y itself) is added last.
 // xscale[slice][M]: factor of each slice's partial sums of row m (the activations of a slice were scaled by its inverse).
 __global__ __launch_bounds__(256) void mmq_reduce_kernel(const float *__restrict__ partial, const float *__restrict__ partial2, int nslices,
-                                                         int64_t MN, int N, const float *__restrict__ bias, const float *__restrict__ bias2,
+                                                         int M, int N, int vec, const float *__restrict__ bias, const float *__restrict__ bias2,
                                                          int act, const float *residual, float *Y, const float *__restrict__ xscale,
                                                          const float *__restrict__ xss, float eps, float inv_k, uint32_t *flags, int nflags) {
     // (the main kernel that stages the activations itself raised these flags; the stream orders this kernel behind it)
     if (blockIdx.x == 0)
         for (int f = threadIdx.x; f < nflags; f += blockDim.x) flags[f] = 0u;
-    const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
-    if (i >= MN) return;
-    const bool small = MN <= (int64_t)INT32_MAX;  // (32-bit divisions are a fraction of the cost of 64-bit ones)
-    const int M = small ? (int)((uint32_t)MN / (uint32_t)N) : (int)(MN / N);
-    const int m = small ? (int)((uint32_t)i / (uint32_t)N) : (int)(i / N);
+    const int ld = (int)sum_cols(N);
+    const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4, ML = (int64_t)M * ld;
+    if (i >= ML) return;
+    // (32-bit divisions are a fraction of the cost of 64-bit ones)
+    const int m = ML <= (int64_t)INT32_MAX ? (int)((uint32_t)i / (uint32_t)ld) : (int)(i / ld), n = (int)(i - (int64_t)m * ld), left = N - n;
     // Slices are added in order, eight at a time: their loads (each a trip to another XCD's freshly written
     // lines) are all issued before the first sum needs one; a slice past the end re-reads the last and is not added.
     // xss: the activations carry an RMS normalisation whose 1 / sqrt(mean(x^2) + eps) is applied here, to the finished sums.
@@ -953,7 +973,7 @@ __global__ __launch_bounds__(256) void mmq_reduce_kernel(const float *__restrict
 #pragma unroll
             for (int j = 0; j < 8; j++) {
                 const int k = min(k0 + j, nslices - 1);
-                v[j] = *reinterpret_cast<const float4 *>(p + (int64_t)k * MN + i);
+                v[j] = *reinterpret_cast<const float4 *>(p + (int64_t)k * ML + i);
                 f[j] = xscale ? xscale[(int64_t)k * M + m] : 1.f;  // (no slice scales: the main kernel has applied its own)
                 q[j] = xss ? xss[(int64_t)k * M + m] : 0.f;
             }
@@ -970,7 +990,7 @@ __global__ __launch_bounds__(256) void mmq_reduce_kernel(const float *__restrict
             s.x /= r; s.y /= r; s.z /= r; s.w /= r;
         }
         if (b) {
-            const float4 v = *reinterpret_cast<const float4 *>(b + (int)(i % N));
+            const float4 v = load_cols(b + n, left, vec);
             s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
         }
         return s;
@@ -981,35 +1001,37 @@ __global__ __launch_bounds__(256) void mmq_reduce_kernel(const float *__restrict
         const float4 u = total(partial2, bias2);
         v.x *= u.x; v.y *= u.y; v.z *= u.z; v.w *= u.w;
     }
+    const int64_t at = (int64_t)m * N + n;
     if (residual) {
-        const float4 r = *reinterpret_cast<const float4 *>(residual + i);
+        const float4 r = load_cols(residual + at, left, vec);
         v.x += r.x; v.y += r.y; v.z += r.z; v.w += r.w;
     }
-    *reinterpret_cast<float4 *>(Y + i) = v;
+    store_cols(Y + at, v, left, vec);
 }
-
 // [xscale: nslices x M][xss: nslices x M] (the second only used with a normalisation)
 size_t mmq_scale_bytes(int nslices, int64_t M) { return ((size_t)2 * nslices * M * sizeof(float) + 255) & ~(size_t)255; }
 float *mmq_xss(const float *xscale, int nslices, int64_t M) { return const_cast<float *>(xscale) + (size_t)nslices * M; }
+template <class... P> bool whole_quads(int64_t N, P... p) { return N % 4 == 0 && (((reinterpret_cast<uintptr_t>(p)) | ...) & 15) == 0; }
 
 int launch_mmq_reduce(const float *partial, const float *partial2, const float *xscale, int nslices, int64_t M, int64_t K, int64_t N,
                       const float *bias, int act, float *y, const MmqExtra *ex, hipStream_t s, uint32_t *flags = nullptr, int nflags = 0) {
-    const int64_t MN = M * N;
+    const int64_t ML = M * sum_cols(N);
     const RmsNorm *norm = ex ? ex->norm : nullptr;
+    const float *bias2 = ex ? ex->bias2 : nullptr, *residual = ex ? ex->residual : nullptr;
     // (workgroups of 64 threads while 256 would leave CUs without one: the kernel is one round trip to memory long)
-    const int threads = MN / 4 / 256 >= 2 * device_cu_count() ? 256 : 64;
-    return launch(mmq_reduce_kernel, dim3((unsigned)((MN / 4 + threads - 1) / threads)), dim3(threads), 0, s, partial, partial2, nslices, MN, (int)N, bias,
-                  ex ? ex->bias2 : nullptr, act, ex ? ex->residual : nullptr, y, xscale, norm ? mmq_xss(xscale, nslices, M) : nullptr,
+    const int threads = ML / 4 / 256 >= 2 * device_cu_count() ? 256 : 64;
+    return launch(mmq_reduce_kernel, dim3((unsigned)((ML / 4 + threads - 1) / threads)), dim3(threads), 0, s, partial, partial2, nslices, (int)M, (int)N,
+                  whole_quads(N, bias, bias2, residual, y) ? 1 : 0, bias, bias2, act, residual, y, xscale, norm ? mmq_xss(xscale, nslices, M) : nullptr,
                   norm ? norm->eps : 0.f, 1.0f / (float)K, flags, nflags);
 }
 
 
 // The reduction for a set of matrices contracted in one launch: partial[slice][m][ntot] holds their columns side by
-// side; matrix p's columns n0[p] .. go to its own y[p] ([M, N[p]]) with its own bias and activation.  Every N[p] % 4 == 0.
+// side, each matrix's in sum_cols(N[p]); matrix p's columns n0[p] .. go to its own y[p] ([M, N[p]]) with its own bias and activation.
 struct MmqSetOut {
     const float *bias[kMaxSet];
     float *y[kMaxSet];
-    int N[kMaxSet], n0[kMaxSet], act[kMaxSet];
+    int N[kMaxSet], n0[kMaxSet], act[kMaxSet], vec[kMaxSet];
     int count, ntot;
 };
 __global__ __launch_bounds__(256) void mmq_reduce_set_kernel(const float *__restrict__ partial, int nslices, int M, MmqSetOut out,
@@ -1025,7 +1047,8 @@ __global__ __launch_bounds__(256) void mmq_reduce_set_kernel(const float *__rest
 #pragma unroll
     for (int j = 1; j < kMaxSet; j++)
         if (j < out.count && nt >= out.n0[j]) p = j;
-    const int n = nt - out.n0[p];
+    const int n = nt - out.n0[p], left = out.N[p] - n;
+    const bool vec = out.vec[p];
     float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
     float ss = 0.f;
     for (int k0 = 0; k0 < nslices; k0 += 8) {  // (all of a round's loads are issued before the first sum needs one)
@@ -1051,12 +1074,11 @@ __global__ __launch_bounds__(256) void mmq_reduce_set_kernel(const float *__rest
         s.x /= r; s.y /= r; s.z /= r; s.w /= r;
     }
     if (out.bias[p]) {
-        const float4 b = *reinterpret_cast<const float4 *>(out.bias[p] + n);
+        const float4 b = load_cols(out.bias[p] + n, left, vec);
         s.x += b.x; s.y += b.y; s.z += b.z; s.w += b.w;
     }
     const int act = out.act[p];
-    *reinterpret_cast<float4 *>(out.y[p] + (int64_t)m * out.N[p] + n) =
-        make_float4(apply_act(act, s.x), apply_act(act, s.y), apply_act(act, s.z), apply_act(act, s.w));
+    store_cols(out.y[p] + (int64_t)m * out.N[p] + n, make_float4(apply_act(act, s.x), apply_act(act, s.y), apply_act(act, s.z), apply_act(act, s.w)), left, vec);
 }
 
 // ---- small batches of the 32-value-block formats (Q8_0, Q4_0, IQ4_NL) --------------------------------------
@@ -1211,7 +1233,7 @@ __global__ __launch_bounds__(256) void mmq_b32_xprep_kernel(const void *__restri
     }
 }
 
-// partial[slice][m][n] = sum over the slice's k of x[m][k] * w[n][k];  grid (row ranges, slices, column tiles)
+// partial[slice][m][n] (rows of sum_cols(N)) = sum over the slice's k of x[m][k] * w[n][k];  grid (row ranges, slices, column tiles)
 // RT row tiles of 32 W rows per workgroup, two wavefronts each.  K % 256 == 0.
 // LDS: [activation image: S * 64 bytes][per wavefront: one stretch of 32 rows]
 template <int T, int RT>
@@ -1324,7 +1346,7 @@ __global__ __launch_bounds__(RT * 128) void mmq_b32_kernel(const uint8_t *__rest
 #pragma unroll
         for (int r = 0; r < 16; r++) {
             const int m = mt * kMT + 8 * (r >> 2) + 4 * kg + (r & 3);
-            if (m < M) partial[((int64_t)slice * M + m) * N + n] = acc[r] + xch[r * 64 + lane];
+            if (m < M) partial[((int64_t)slice * M + m) * sum_cols(N) + n] = acc[r] + xch[r * 64 + lane];
         }
     }
 }
@@ -1492,7 +1514,7 @@ __global__ __launch_bounds__(64 * Q4KTiles::kWaves) void mmq_b32_tiles_kernel(co
 #pragma unroll
             for (int r = 0; r < 16; r++) {
                 const int m = m0 + 32 * t + 8 * (r >> 2) + 4 * kg + (r & 3);
-                if (m < M) partial[((int64_t)slice * M + m) * N + n] = acc[t][r];
+                if (m < M) partial[((int64_t)slice * M + m) * sum_cols(N) + n] = acc[t][r];
             }
         }
     }
@@ -1657,7 +1679,7 @@ __global__ __launch_bounds__(64 * Q4KTiles::kWaves) void mmq_q8_tiles_kernel(con
 #pragma unroll
             for (int r = 0; r < 16; r++) {
                 const int m = m0 + 32 * t + 8 * (r >> 2) + 4 * kg + (r & 3);
-                if (m < M) partial[((int64_t)slice * M + m) * N + n] = acc[t][r];
+                if (m < M) partial[((int64_t)slice * M + m) * sum_cols(N) + n] = acc[t][r];
             }
         }
     }
@@ -1693,7 +1715,7 @@ int launch_mmq_b32(const void *x, bool x_is_bf16, int64_t M, int64_t K, const ui
     // workspace: [activation images: mtiles x nslices x S x 64 bytes][slice scales: nslices x M][partial sums: nslices x M x N fp32,
     // twice for a gated pair]
     const size_t img_bytes = (size_t)mtiles * nslices * S * 64;
-    const size_t part_bytes = (size_t)nslices * M * N * sizeof(float);
+    const size_t part_bytes = (size_t)nslices * M * sum_cols(N) * sizeof(float);
     void *ws = nullptr;
     if (int rc = stream_workspace(s, img_bytes + mmq_scale_bytes(nslices, M) + part_bytes * (W2 ? 2 : 1), &ws)) return rc;
     uint8_t *ximg = reinterpret_cast<uint8_t *>(ws);
@@ -1706,7 +1728,7 @@ int launch_mmq_b32(const void *x, bool x_is_bf16, int64_t M, int64_t K, const ui
                       norm ? mmq_xss(xscale, nslices, M) : nullptr);
     };
     if (int rc = x_is_bf16 ? prep(mmq_b32_xprep_kernel<true>) : prep(mmq_b32_xprep_kernel<false>)) return rc;
-    float *partial2 = W2 ? partial + (size_t)nslices * M * N : nullptr;
+    float *partial2 = W2 ? partial + (size_t)nslices * M * sum_cols(N) : nullptr;
     if constexpr (kHasTiles) {
         if (together) {
             static const bool tiles_lds_ok = [] {
@@ -1912,7 +1934,7 @@ __global__ __launch_bounds__(512) void mmq_q6k_kernel(const uint8_t *__restrict_
 #pragma unroll
         for (int r = 0; r < 16; r++) {
             const int m = mt * kMT + 8 * (r >> 2) + 4 * kg + (r & 3);
-            if (m < M) partial[((int64_t)slice * M + m) * N + n] = acc[r] + xch[r * 64 + lane];
+            if (m < M) partial[((int64_t)slice * M + m) * sum_cols(N) + n] = acc[r] + xch[r * 64 + lane];
         }
     }
 }
@@ -1932,7 +1954,7 @@ int launch_mmq_q6k_rt(const MmqExtra *ex, const void *x, bool x_is_bf16, int64_t
     const uint8_t *W2 = ex ? ex->W2 : nullptr;
     const RmsNorm *norm = ex ? ex->norm : nullptr;
     const size_t img_bytes = (size_t)mtiles * nslices * kQ6Slice * 64;
-    const size_t part_bytes = (size_t)nslices * M * N * sizeof(float);
+    const size_t part_bytes = (size_t)nslices * M * sum_cols(N) * sizeof(float);
     void *ws = nullptr;
     if (int rc = stream_workspace(s, img_bytes + mmq_scale_bytes(nslices, M) + part_bytes * (W2 ? 2 : 1), &ws)) return rc;
     uint8_t *ximg = reinterpret_cast<uint8_t *>(ws);
@@ -1946,7 +1968,7 @@ int launch_mmq_q6k_rt(const MmqExtra *ex, const void *x, bool x_is_bf16, int64_t
     };
     if (int rc = x_is_bf16 ? prep(mmq_b32_xprep_kernel<true>) : prep(mmq_b32_xprep_kernel<false>)) return rc;
     const dim3 grid((unsigned)((N + 32 * RT - 1) / (32 * RT)), (unsigned)nslices, (unsigned)mtiles * (W2 ? 2u : 1u));  // (a gated pair: one launch)
-    float *partial2 = W2 ? partial + (size_t)nslices * M * N : nullptr;
+    float *partial2 = W2 ? partial + (size_t)nslices * M * sum_cols(N) : nullptr;
     if (int rc = launch(mmq_q6k_kernel<RT>, grid, dim3(RT * 128), (size_t)kLds, s, (const uint8_t *)ximg, W, partial, (int)M, (int)K, (int)N,
                         row_bytes, mtiles, W2, partial2))
         return rc;
@@ -1963,12 +1985,12 @@ int launch_mmq_q6k(const MmqExtra *ex, const void *x, bool x_is_bf16, int64_t M,
 
 }  // namespace
 
-bool mmq_supported(int type, int64_t M, int64_t K, int64_t N, const void *x, const void *bias, const void *y) {
+bool mmq_supported(int type, int64_t M, int64_t K, int64_t N, const void *x) {
     // K <= 2^26: the kernels address the 32 rows of a tile by 32-bit byte offsets from its first row (31 rows of at most
     // 2^26 * 34 / 32 bytes stay below 2^32)
     // (Q4_K walks four tiles of 32 rows per launch and stays ahead of the two-pass GEMM for longer than the others)
-    const bool shape_ok = M >= 2 && M <= (type == kQ4_K ? 512 : 256) && N % 4 == 0 && N <= (int64_t)INT32_MAX / 2 && K <= ((int64_t)1 << 26) &&
-                          ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(bias) | reinterpret_cast<uintptr_t>(y)) & 15) == 0;
+    const bool shape_ok = M >= 2 && M <= (type == kQ4_K ? 512 : 256) && N <= (int64_t)INT32_MAX / 2 && K <= ((int64_t)1 << 26) &&
+                          (reinterpret_cast<uintptr_t>(x) & 15) == 0;
     if (type == kQ4_K) return shape_ok && K % 256 == 0;
     if (type == kQ8_0 || type == kQ4_0 || type == kIQ4_NL) return shape_ok && K % 256 == 0;  // whole stretches of 8 blocks
     if (type == kQ6_K) return shape_ok && K % 512 == 0;                   // whole, dword-aligned pairs of super-blocks
@@ -2029,12 +2051,13 @@ int run_q4k_set(const void *x, bool x_is_bf16, int64_t M, int64_t K, int count, 
     const int wg_rows = together ? Q4KTiles::kRows : Tile::kRows;
     Q4KSet set = {};
     MmqSetOut out = {};
-    int64_t rowwgs = 0, N = 0;  // workgroups along the rows of all matrices; their columns side by side
+    int64_t rowwgs = 0, N = 0;  // workgroups along the rows of all matrices; their sums' columns side by side
     for (int i = 0; i < count; i++) {
         set.W[i] = items[i].W; set.N[i] = (int)items[i].N; set.wg0[i] = (int)rowwgs; set.n0[i] = (int)N;
         out.bias[i] = items[i].bias; out.y[i] = items[i].y; out.N[i] = (int)items[i].N; out.n0[i] = (int)N; out.act[i] = items[i].act;
+        out.vec[i] = whole_quads(items[i].N, items[i].bias, items[i].y);
         rowwgs += (items[i].N + wg_rows - 1) / wg_rows;
-        N += items[i].N;
+        N += sum_cols(items[i].N);
     }
     set.count = out.count = count;
     set.ntot = out.ntot = (int)N;
@@ -2079,13 +2102,13 @@ int run_q4k_set(const void *x, bool x_is_bf16, int64_t M, int64_t K, int count, 
         if (!coop_lds_ok) return fail(GQ_ERR_HIP, "mmq: cannot reserve %d bytes of LDS", CTile::kLds);
         // workspace: [activation records: mtiles x nslices x 7 x kRecStride][partial sums: nslices x M x N fp32, twice for a gated pair]
         const size_t rec_bytes = (size_t)mtiles * nslices * CTile::kMaxSliceSB * kRecStride;
-        const size_t part_bytes = (size_t)nslices * M * N * sizeof(float);
+        const size_t part_bytes = (size_t)nslices * M * sum_cols(N) * sizeof(float);
         void *ws = nullptr;
         uint32_t *flags = nullptr;
         if (int rc = stream_workspace(s, rec_bytes + part_bytes * (W2 ? 2 : 1), &ws, 0, &flags)) return rc;
         uint8_t *ximg = reinterpret_cast<uint8_t *>(ws);
         float *partial = reinterpret_cast<float *>(ximg + rec_bytes);
-        partial2 = W2 ? partial + (size_t)nslices * M * N : nullptr;
+        partial2 = W2 ? partial + (size_t)nslices * M * sum_cols(N) : nullptr;
         const int spin = coop_spin_ticks();
         for (int64_t m0 = 0; m0 < M; m0 += kMT) {
             const int rc = x_is_bf16 ? launch(mmq_q4k_coop_kernel<kQ4KRowTiles, true>, grid, dim3(64 * CTile::kWaves), (size_t)CTile::kLds, s, x, ximg,
@@ -2095,7 +2118,7 @@ int run_q4k_set(const void *x, bool x_is_bf16, int64_t M, int64_t K, int count, 
             if (rc) return rc;
         }
         if (count == 1)
-            return launch_mmq_reduce(partial, partial2, nullptr, nslices, M, K, N, items[0].bias, items[0].act, items[0].y, ex, s, flags, nflags);
+            return launch_mmq_reduce(partial, partial2, nullptr, nslices, M, K, items[0].N, items[0].bias, items[0].act, items[0].y, ex, s, flags, nflags);
         const int64_t quads = M * N / 4;
         const int threads = quads / 256 >= 2 * device_cu_count() ? 256 : 64;
         return launch(mmq_reduce_set_kernel, dim3((unsigned)((quads + threads - 1) / threads)), dim3(threads), 0, s, (const float *)partial, nslices,
@@ -2104,7 +2127,7 @@ int run_q4k_set(const void *x, bool x_is_bf16, int64_t M, int64_t K, int count, 
     // workspace: [activation images: mtiles x nslices x kLdsBytes][slice scales: nslices x M][partial sums: nslices x M x N fp32,
     // twice for a gated pair]
     const size_t img_bytes = (size_t)mtiles * nslices * kLdsBytes;
-    const size_t part_bytes = (size_t)nslices * M * N * sizeof(float);
+    const size_t part_bytes = (size_t)nslices * M * sum_cols(N) * sizeof(float);
     void *ws = nullptr;
     if (int rc = stream_workspace(s, img_bytes + mmq_scale_bytes(nslices, M) + part_bytes * (W2 ? 2 : 1), &ws)) return rc;
     uint8_t *ximg = reinterpret_cast<uint8_t *>(ws);
@@ -2120,7 +2143,7 @@ int run_q4k_set(const void *x, bool x_is_bf16, int64_t M, int64_t K, int count, 
     if (int rc = x_is_bf16 ? (fine ? prep(mmq_xprep_kernel<true, 1>) : prep(mmq_xprep_kernel<true, 2>))
                            : (fine ? prep(mmq_xprep_kernel<false, 1>) : prep(mmq_xprep_kernel<false, 2>)))
         return rc;
-    partial2 = W2 ? partial + (size_t)nslices * M * N : nullptr;
+    partial2 = W2 ? partial + (size_t)nslices * M * sum_cols(N) : nullptr;
     // (the tiles are dealt evenly over the fewest launches: five tiles go as 3 + 2, not as 4 + 1 - every launch streams all of W)
     const int nlaunch = (mtiles + Q4KTiles::kMaxTiles - 1) / Q4KTiles::kMaxTiles;
     for (int l = 0, tile0 = 0; together && l < nlaunch; l++) {
@@ -2142,7 +2165,7 @@ int run_q4k_set(const void *x, bool x_is_bf16, int64_t M, int64_t K, int count, 
                             (int)M, (int)K, row_bytes, (int)m0, slice_sb, W2, partial2))
             return rc;
     }
-    if (count == 1) return launch_mmq_reduce(partial, partial2, xscale, nslices, M, K, N, items[0].bias, items[0].act, items[0].y, ex, s);
+    if (count == 1) return launch_mmq_reduce(partial, partial2, xscale, nslices, M, K, items[0].N, items[0].bias, items[0].act, items[0].y, ex, s);
     const int64_t quads = M * N / 4;
     const int threads = quads / 256 >= 2 * device_cu_count() ? 256 : 64;
     return launch(mmq_reduce_set_kernel, dim3((unsigned)((quads + threads - 1) / threads)), dim3(threads), 0, s, (const float *)partial, nslices, (int)M,
@@ -2160,16 +2183,20 @@ int launch_split_k_finish(const float *partial, const float *partial2, const flo
     MmqSetOut out = {};
     for (int i = 0; i < count; i++) {
         out.bias[i] = items[i].bias; out.y[i] = items[i].y; out.N[i] = (int)items[i].N; out.n0[i] = (int)N; out.act[i] = items[i].act;
-        N += items[i].N;
+        out.vec[i] = whole_quads(items[i].N, items[i].bias, items[i].y);
+        N += sum_cols(items[i].N);
     }
     out.count = count;
     out.ntot = (int)N;
-    const int64_t MN = M * N;
-    const int threads = MN / 4 / 256 >= 2 * device_cu_count() ? 256 : 64;
-    const dim3 grid((unsigned)((MN / 4 + threads - 1) / threads));
-    if (count == 1)
-        return launch(mmq_reduce_kernel, grid, dim3(threads), 0, s, partial, partial2, nslices, MN, (int)N, items[0].bias, ex ? ex->bias2 : nullptr, items[0].act,
-                      ex ? ex->residual : nullptr, items[0].y, (const float *)nullptr, xss, eps, inv_k, (uint32_t *)nullptr, 0);
+    const int64_t ML = M * N;
+    const int threads = ML / 4 / 256 >= 2 * device_cu_count() ? 256 : 64;
+    const dim3 grid((unsigned)((ML / 4 + threads - 1) / threads));
+    if (count == 1) {
+        const float *bias2 = ex ? ex->bias2 : nullptr, *residual = ex ? ex->residual : nullptr;
+        return launch(mmq_reduce_kernel, grid, dim3(threads), 0, s, partial, partial2, nslices, (int)M, (int)items[0].N,
+                      whole_quads(items[0].N, items[0].bias, bias2, residual, items[0].y) ? 1 : 0, items[0].bias, bias2, items[0].act, residual, items[0].y,
+                      (const float *)nullptr, xss, eps, inv_k, (uint32_t *)nullptr, 0);
+    }
     return launch(mmq_reduce_set_kernel, grid, dim3(threads), 0, s, partial, nslices, (int)M, out, (const float *)nullptr, xss, eps, inv_k,
                   (uint32_t *)nullptr, 0);
 }
@@ -2190,7 +2217,7 @@ bool mmq_set_supported(int type, int count, const MmqSetItem *items, int64_t M, 
     if (type != kQ4_K || count < 2 || count > kMaxSet) return false;
     int64_t total = 0;
     for (int i = 0; i < count; i++) {
-        if (!mmq_supported(type, M, K, items[i].N, x, items[i].bias, items[i].y)) return false;
+        if (!mmq_supported(type, M, K, items[i].N, x)) return false;
         total += items[i].N;
     }
     return total <= (int64_t)INT32_MAX / 2;

@@ -96,3 +96,36 @@ def test_gemm_with_weights_converted_in_registers_keeps_infinities(gpu, monkeypa
         assert np.all(np.isposinf(want[:, 5])) and np.all(np.isposinf(got[:, 5]))
         ok = np.arange(N) != 5
         assert rel(got[:, ok], want[:, ok]) < TOL_F32
+
+
+@pytest.mark.parametrize("t,M,K,N", [
+    (ggml.Q4_K, 6, 5120, 2305), (ggml.Q4_K, 12, 4096, 3075), (ggml.Q4_K, 32, 4096, 3074), (ggml.Q4_K, 77, 4096, 3073), (ggml.Q4_K, 128, 4096, 3077),
+    (ggml.Q8_0, 17, 4096, 1601), (ggml.Q8_0, 66, 4096, 1603), (ggml.Q4_0, 33, 4096, 2891), (ggml.IQ4_NL, 12, 5120, 2337), (ggml.Q6_K, 20, 4096, 2051),
+    (ggml.Q6_K, 5, 8192, 1025),
+])
+def test_split_k_rows_of_any_length(gpu, t, M, K, N):
+    """The split-K routes with N off every multiple of four (their sums' rows are padded, the outputs stored element by element): plain with
+    bias, behind a norm with a residual, a gated pair, q / k / v of one input, outputs that are not 16-byte aligned, bfloat16 rows."""
+    torch = gpu
+    W, W2, x = synth.weights(t, 3, N, K), synth.weights(t, 4, N, K), synth.activations(5 + M, M, K)
+    rng = np.random.default_rng(M)
+    bias, res = rng.standard_normal(N).astype(np.float32), rng.standard_normal((M, N)).astype(np.float32)
+    q, wd, w2d, xd = Quantization(ggml_type=t), dev(torch, W), dev(torch, W2), dev(torch, x)
+    gate, up = (oracle.c_qdense(t, x, w, None, oracle.ACT_NONE) for w in (W, W2))
+    peak = float(np.max(np.abs(gate)))
+    got = nn.quantized_dense(xd, wd, q, dev(torch, bias), Activation.RELU).cpu().numpy()
+    assert np.max(np.abs(got - np.maximum(gate + bias, 0))) < TOL_F32 * peak
+    got = nn.quantized_dense(xd, wd, q, dev(torch, np.concatenate([bias, bias]))[1:N + 1]).cpu().numpy()  # a bias off 16 bytes
+    assert np.max(np.abs(got - gate - np.concatenate([bias, bias])[1:N + 1])) < TOL_F32 * peak
+    norm = nn.RMSNorm(gain=dev(torch, np.ones(K, np.float32)), epsilon=1e-5)
+    scale = np.sqrt(np.mean(x.astype(np.float64) ** 2, axis=1, keepdims=True) + 1e-5)
+    got = nn.quantized_dense(xd, wd, q, norm=norm, residual=dev(torch, res)).cpu().numpy()
+    assert np.max(np.abs(got - res - gate / scale)) < TOL_F32 * np.max(np.abs(gate / scale)) + 1e-6 * np.max(np.abs(res))
+    got = nn.gated_feed_forward(xd, wd, w2d, q, Activation.RELU).cpu().numpy()
+    assert np.max(np.abs(got - np.maximum(gate, 0) * up)) < 2 * TOL_F32 * peak * np.max(np.abs(up))
+    outs = nn.quantized_dense_batch([(xd, w, q, None, None) for w in (wd, w2d, wd)], norm=norm)
+    for o, w in zip(outs, (gate, up, gate)):
+        assert rel(o.cpu().numpy(), w / scale) < TOL_F32
+    xb = xd.to(torch.bfloat16)
+    want = oracle.c_qdense(t, xb.float().cpu().numpy(), W, bias, oracle.ACT_NONE)
+    assert rel(nn.quantized_dense(xb, wd, q, dev(torch, bias)).cpu().numpy(), want) < TOL_F32
