@@ -129,3 +129,24 @@ def test_split_k_rows_of_any_length(gpu, t, M, K, N):
     xb = xd.to(torch.bfloat16)
     want = oracle.c_qdense(t, xb.float().cpu().numpy(), W, bias, oracle.ACT_NONE)
     assert rel(nn.quantized_dense(xb, wd, q, dev(torch, bias)).cpu().numpy(), want) < TOL_F32
+
+
+@pytest.mark.parametrize("count", [1, 1024, 1025, 16384, 16385])
+def test_gather_finds_a_bad_index_wherever_it_is(gpu, count):
+    """Lists around the check's workgroup and around the length up to which it runs in front of the rows, also behind work on the stream that takes
+    longer than the host spins for."""
+    torch = gpu
+    K, vocab = 32, 50
+    table = synth.weights(ggml.Q8_0, 3, vocab, K)
+    q, td = Quantization(ggml_type=ggml.Q8_0), dev(torch, table)
+    idx = (np.arange(count, dtype=np.int32) * 7 % vocab).reshape(-1, 1)
+    want = oracle.c_dequantize(ggml.Q8_0, table, K)[idx[:, 0]]
+    idx_d = dev(torch, idx)
+    for ahead in (0, 10_000_000):
+        torch.cuda._sleep(ahead)
+        assert np.array_equal(nn.quantized_gather(td, idx_d, q).cpu().numpy().view(np.uint32), want.view(np.uint32))
+    for bad, at in ((vocab, count - 1), (-1, 0), (vocab, count // 2)):
+        wrong = idx.copy()
+        wrong[at] = bad
+        with pytest.raises(IndexError):
+            nn.quantized_gather(td, dev(torch, wrong), q)
