@@ -1178,25 +1178,25 @@ template <int T> struct B32Geom {
 // columns of one slice (S / 256 octets per thread, consecutive threads on consecutive octets of a
 // column) and scales each column's slice by a power of two (pow2_scale); xscale[slice][M] receives the
 // inverse factors.  grid = column tiles x slices x 4.
-template <bool BF16X>
+// ITS: octets per thread at most, S / 256 of them used (S a multiple of 512, so that a wavefront's 64 octets belong to one column).
+template <bool BF16X, int ITS = 4>
 __global__ __launch_bounds__(256) void mmq_b32_xprep_kernel(const void *__restrict__ X, uint8_t *__restrict__ ximg, float *__restrict__ xscale,
                                                             int M, int K, int S, int nslices, const float *__restrict__ gain, float gain_offset,
                                                             float *__restrict__ xss) {
     __shared__ uint32_t red[8];
-    __shared__ float red_ss[8][2];  // a column's slice is one or two wavefronts' worth of octets
+    __shared__ float red_ss[8][4];  // a column's slice is one to four wavefronts' worth of octets
     const int tid = threadIdx.x;
     const int rg = (int)blockIdx.x & 3, ts = (int)blockIdx.x >> 2;
     const int slice = ts % nslices, mt = ts / nslices;
     const int opers = S / 8, its = S / 256;  // octets per column and slice; items per thread
     if (tid < 8) {
         red[tid] = 0u;
-        red_ss[tid][0] = 0.f;
-        red_ss[tid][1] = 0.f;
+        for (int i = 0; i < 4; i++) red_ss[tid][i] = 0.f;
     }
     __syncthreads();
-    float4 a[4], b[4];
+    float4 a[ITS], b[ITS];
 #pragma unroll
-    for (int it = 0; it < 4; it++) {
+    for (int it = 0; it < ITS; it++) {
         a[it] = make_float4(0.f, 0.f, 0.f, 0.f);
         b[it] = a[it];
         if (it < its) {
@@ -1206,7 +1206,7 @@ __global__ __launch_bounds__(256) void mmq_b32_xprep_kernel(const void *__restri
             if (ok) load_x8<BF16X>(X, (int64_t)row * K + k, a[it], b[it]);
             if (xss) {
                 const float ss = wave_sum(sumsq8(a[it], b[it]));
-                if ((tid & 63) == 0) red_ss[c][(oct >> 6) & 1] = ss;
+                if ((tid & 63) == 0) red_ss[c][oct >> 6] = ss;
                 if (gain && ok) apply_gain8(gain, gain_offset, k, a[it], b[it]);
             }
             const float am = wave_max(amax8(a[it], b[it]));  // a wavefront's 64 octets belong to one column
@@ -1215,7 +1215,7 @@ __global__ __launch_bounds__(256) void mmq_b32_xprep_kernel(const void *__restri
     }
     __syncthreads();
 #pragma unroll
-    for (int it = 0; it < 4; it++) {
+    for (int it = 0; it < ITS; it++) {
         if (it < its) {
             const int j = it * 256 + tid, c = j / opers, oct = j - c * opers;
             const int m = rg * 8 + c, row = mt * kMT + m;
@@ -1223,7 +1223,7 @@ __global__ __launch_bounds__(256) void mmq_b32_xprep_kernel(const void *__restri
             pow2_scale(__builtin_bit_cast(float, red[c]), sc, inv);
             if (oct == 0 && row < M) {
                 xscale[(size_t)slice * M + row] = inv;
-                if (xss) xss[(size_t)slice * M + row] = red_ss[c][0] + red_ss[c][1];
+                if (xss) xss[(size_t)slice * M + row] = (red_ss[c][0] + red_ss[c][1]) + (red_ss[c][2] + red_ss[c][3]);
             }
             const float4 p = a[it], q = b[it];
             const size_t g = (((size_t)mt * nslices + slice) * opers + oct) * 32 + m;
@@ -1701,12 +1701,20 @@ int launch_mmq_b32(const void *x, bool x_is_bf16, int64_t M, int64_t K, const ui
                           ((N + Q4KTiles::kRows - 1) / Q4KTiles::kRows) * ((K + 511) / 512) * (W2 ? 2 : 1) >= (int64_t)cus * 3 / 4;
     const int64_t rowwgs = together ? (N + Q4KTiles::kRows - 1) / Q4KTiles::kRows : (N + 32 * RT - 1) / (32 * RT);
     // slices of 1024 when that still leaves every CU a workgroup and a half (LDS holds a 1024-value image
-    // next to the parked stretches, not a 2048-value one); the kernel for several tiles has one workgroup per CU at a time
-    // and takes the long slices from three quarters of the CUs on
-    const int S = together ? (rowwgs * ((K + 1023) / 1024) * (W2 ? 2 : 1) >= (int64_t)cus * 3 / 4 ? 1024 : 512)
-                           : (rowwgs * ((K + 1023) / 1024) * mtiles >= (int64_t)cus * 3 / 2 ? 1024 : 512);
+    // next to the parked stretches, not a 2048-value one); the kernel for several tiles, which holds two halves of a stretch's image at a
+    // time, takes up to 2048 by the plan of run_q4k_set: rounds of workgroups, one per CU, times what one takes, and a slice's sums
+    // (the gated pair of 4096 x 14336 in Q4_0 at 128 rows: 4 slices in two rounds 79.7 us, 2 in one 74.9; 5120 x 13824 5 in two 68.8, 4 in one 55.2)
+    int S = rowwgs * ((K + 1023) / 1024) * mtiles >= (int64_t)cus * 3 / 2 ? 1024 : 512;
+    if (together) {
+        const int64_t z = W2 ? 2 : 1, sums = std::min<int64_t>(M, 128) * N * z * 8 / 4500, stretch_ns = 1100 + 700 * std::min(mtiles, 4);
+        int64_t best = INT64_MAX;
+        for (int len = 2048; len >= 512; len -= 512) {
+            const int64_t ns = (K + len - 1) / len, cost = (rowwgs * ns * z + cus - 1) / cus * (len / 256 * stretch_ns + 8000) + ns * sums;
+            if (cost < best) { best = cost; S = len; }
+        }
+    }
     const int nslices = (int)((K + S - 1) / S);
-    const size_t lds_bytes = (size_t)S * 64 + (size_t)2 * RT * B32Geom<T>::kWaveLds;  // image (later the handed-over tiles) + parked stretches
+    const size_t lds_bytes = (size_t)S * 64 + (size_t)2 * RT * B32Geom<T>::kWaveLds;  // image (later the handed-over tiles) + parked stretches (not of the kernel for several tiles)
     static const bool lds_ok = [] {
         return hipFuncSetAttribute(reinterpret_cast<const void *>(mmq_b32_kernel<T, RT>), hipFuncAttributeMaxDynamicSharedMemorySize,
                                    1024 * 64 + 2 * RT * B32Geom<T>::kWaveLds) == hipSuccess;
@@ -1727,7 +1735,9 @@ int launch_mmq_b32(const void *x, bool x_is_bf16, int64_t M, int64_t K, const ui
         return launch(kernel, xgrid, dim3(256), 0, s, x, ximg, xscale, (int)M, (int)K, S, nslices, norm ? norm->gain : nullptr, norm ? norm->gain_offset : 0.f,
                       norm ? mmq_xss(xscale, nslices, M) : nullptr);
     };
-    if (int rc = x_is_bf16 ? prep(mmq_b32_xprep_kernel<true>) : prep(mmq_b32_xprep_kernel<false>)) return rc;
+    if (int rc = S > 1024 ? (x_is_bf16 ? prep(mmq_b32_xprep_kernel<true, 8>) : prep(mmq_b32_xprep_kernel<false, 8>))
+                          : (x_is_bf16 ? prep(mmq_b32_xprep_kernel<true>) : prep(mmq_b32_xprep_kernel<false>)))
+        return rc;
     float *partial2 = W2 ? partial + (size_t)nslices * M * sum_cols(N) : nullptr;
     if constexpr (kHasTiles) {
         if (together) {

@@ -150,3 +150,21 @@ def test_gather_finds_a_bad_index_wherever_it_is(gpu, count):
         wrong[at] = bad
         with pytest.raises(IndexError):
             nn.quantized_gather(td, dev(torch, wrong), q)
+
+
+@pytest.mark.parametrize("t", [ggml.Q4_0, ggml.Q8_0, ggml.IQ4_NL])
+@pytest.mark.parametrize("K,N", [(4352, 16420), (2048, 33290)])
+def test_32_value_blocks_over_long_slices(gpu, t, K, N):
+    """Several tiles of batch rows over slices of more than 1024 values: three of 1536 or 2048 whose last is cut short, and one of 2048; with
+    a normalisation, whose sums of squares come from four wavefronts per slice then."""
+    torch, M = gpu, 40
+    W = synth.weights(t, 3, 131, K)
+    x = synth.activations(5, M, K)
+    want = oracle.c_qdense(t, x, W, None, oracle.ACT_NONE)
+    reps = -(-N // 131)
+    q, xd = Quantization(ggml_type=t), dev(torch, x)
+    wd = dev(torch, np.tile(W, (reps, 1))[:N])
+    assert rel(nn.quantized_dense(xd, wd, q).cpu().numpy(), np.tile(want, (1, reps))[:, :N]) < TOL_F32
+    norm = nn.RMSNorm(gain=dev(torch, np.ones(K, np.float32)), epsilon=1e-5)
+    want = want / np.sqrt(np.mean(x.astype(np.float64) ** 2, axis=1, keepdims=True) + 1e-5)
+    assert rel(nn.quantized_dense(xd, wd, q, norm=norm).cpu().numpy(), np.tile(want, (1, reps))[:, :N]) < TOL_F32
