@@ -301,6 +301,10 @@ int64_t by_element_to(int type, int64_t K, int64_t N, bool gated) {
     if (K < 8192) return type == GQ_Q6_K ? 64 : !gated && large ? 96 : 128;
     return 128;
 }
+// The first row count of such a call on the split-K kernels: up to 16 rows it keeps the GEMV and the few-row kernel, which hold activations in
+// more bits (16-bit fixed point per 32 values, two fp16) than the split-K kernels' one fp16: errors of 2e-5 and 1e-4 of the largest output.  (Those
+// take half the time there: Q4_K 14336 -> 4097 at 12 rows 25 against 52 us.) Beyond, the other routes are GEMMs on 16-bit operands, of weights as well.
+int64_t take_over(int64_t from, bool whole) { return whole ? from : std::max(from, kGemvMaxRows + 1); }
 int64_t hand_over(int type, int64_t K, int64_t N, bool gated, bool whole) {
     const int64_t to = gated ? gated_split_k_to(type, K, N) : split_k_to(type, K, N);
     return whole || split_k_to_env() >= 0 ? to : std::min(to, by_element_to(type, K, N, gated));
@@ -405,7 +409,7 @@ bool split_k_ahead(int type, int64_t M, int64_t K, int64_t one, int matrices) {
 bool takes_mmv(int type, int64_t M, int64_t K, int64_t N, const void *x, const void *gain, int matrices, bool extras, bool set = false) {
     if (M < 3 || !mmv_one_launch(K) || !mmv_supported(type, M, K, N, x, gain)) return false;
     const int64_t one = weight_bytes_of(type, K, N), bytes = one * matrices, MB = (int64_t)1 << 20;
-    if ((!set || type == GQ_Q4_K) && split_k_ahead(type, M, K, one, matrices)) return false;  // (what the split-K kernels take)
+    if ((!set || type == GQ_Q4_K) && N % 4 == 0 && split_k_ahead(type, M, K, one, matrices)) return false;  // (what the split-K kernels take)
     if (bytes < 9 * MB) return M * bytes >= 64 * MB;
     if (bytes < kLargeWeightBytes) return !(type == GQ_Q4_0 && M == 3) && M * bytes >= gemv_reach(type, K, K * N * matrices, matrices, extras, set) * MB;
     if (!extras && !set && M <= 4 && (type == GQ_Q8_0 || (type == GQ_Q4_0 && bytes < 64 * MB))) return false;  // one GEMV pass of four rows
@@ -623,7 +627,7 @@ int gq_qdense_f32(int type, const float *dX, int64_t M, int64_t K, const void *d
         return launch_mmv(type, dX, false, M, K, 1, &one, nullptr, (hipStream_t)stream);
     const bool tp = gemm_two_pass_supported(type, false, M, K, N, dX);
     const bool ks = M <= kGemvMaxRows && gemv_ks_supported(type, K, N, dX);
-    const bool sk = M >= split_k_from(type, weight_bytes_of(type, K, N)) && mmq_supported(type, M, K, N, dX) &&
+    const bool sk = M >= take_over(split_k_from(type, weight_bytes_of(type, K, N)), whole) && mmq_supported(type, M, K, N, dX) &&
                     (M <= hand_over(type, K, N, false, whole) || !tp);
     if (sk) {
         const int rc = split_k(type, dX, false, M, K, 1, &one, nullptr, (hipStream_t)stream);
@@ -762,7 +766,7 @@ int gq_qdense_bf16(int type, const uint16_t *dX, int64_t M, int64_t K, const voi
         return launch_mmv(type, dX, true, M, K, 1, &one, nullptr, (hipStream_t)stream);
     const bool tp = gemm_two_pass_supported(type, true, M, K, N, dX);
     const bool ks = M <= kGemvMaxRows && gemv_ks_supported(type, K, N, dX);
-    const bool sk = M >= split_k_from(type, weight_bytes_of(type, K, N)) && mmq_supported(type, M, K, N, dX) &&
+    const bool sk = M >= take_over(split_k_from(type, weight_bytes_of(type, K, N)), whole) && mmq_supported(type, M, K, N, dX) &&
                     (M <= hand_over(type, K, N, false, whole) || !tp);
     if (sk) {
         const int rc = split_k(type, dX, true, M, K, 1, &one, nullptr, (hipStream_t)stream);
@@ -813,22 +817,22 @@ int64_t block_split_k_from(int type, int64_t weight_bytes, bool gated) {
     }
 }
 
-bool fold_into_gemv(int type, int64_t M, int64_t K, int64_t N, const float *x, const float *gain, bool gated) {
+bool fold_into_gemv(int type, int64_t M, int64_t K, int64_t N, const float *x, const float *gain, bool gated, bool whole) {
     if (!gemv_ks_ext_supported(type, M, K, N, x, gain)) return false;
-    return !(M >= block_split_k_from(type, weight_bytes_of(type, K, N), gated) && mmq_supported(type, M, K, N, x));
+    return !(M >= take_over(block_split_k_from(type, weight_bytes_of(type, K, N), gated), whole) && mmq_supported(type, M, K, N, x));
 }
 
 // Whether a projection with its neighbours runs on the split-K kernels (after fold_into_gemv() has declined).
 bool block_takes_split_k(int type, int64_t M, int64_t K, int64_t N, const float *x, bool gated, bool whole) {
     const bool tp = gated ? gemm_two_pass_block_supported(type, M, K, N, x, true) : gemm_two_pass_supported(type, false, M, K, N, x);
     const int64_t to = hand_over(type, K, N, gated, whole);
-    return M >= block_split_k_from(type, weight_bytes_of(type, K, N), gated) && mmq_supported(type, M, K, N, x) && (M <= to || !tp);
+    return M >= take_over(block_split_k_from(type, weight_bytes_of(type, K, N), gated), whole) && mmq_supported(type, M, K, N, x) && (M <= to || !tp);
 }
 
 // Whether a plain dense call on these operands runs on the split-K kernels (the dispatch of gq_qdense_f32).
 bool dense_takes_split_k(int type, int64_t M, int64_t K, int64_t N, const float *x, bool whole) {
     const bool tp = gemm_two_pass_supported(type, false, M, K, N, x);
-    return M >= split_k_from(type, weight_bytes_of(type, K, N)) && mmq_supported(type, M, K, N, x) && (M <= hand_over(type, K, N, false, whole) || !tp);
+    return M >= take_over(split_k_from(type, weight_bytes_of(type, K, N)), whole) && mmq_supported(type, M, K, N, x) && (M <= hand_over(type, K, N, false, whole) || !tp);
 }
 
 // First batch size of the gated pair as one GEMM (wherever the split-K kernels have handed over: the composed form is never
@@ -872,9 +876,10 @@ bool takes_shared_pass(int count, const gq_dense_desc *descs, const float *gain,
     const int64_t rows = descs[0].M, K = descs[0].K;
     int64_t ntot = 0;
     for (int i = 0; i < count; i++) ntot += descs[i].N;
+    const bool whole = whole_set(count, set);
     return mmq_set_supported(type, count, set, rows, K, descs[0].dX) &&
-           rows >= block_split_k_from(type, weight_bytes_of(type, K, ntot), false) &&
-           (rows <= hand_over(type, K, ntot, false, whole_set(count, set)) || !gemm_two_pass_supported(type, false, rows, K, ntot, descs[0].dX));
+           rows >= take_over(block_split_k_from(type, weight_bytes_of(type, K, ntot), false), whole) &&
+           (rows <= hand_over(type, K, ntot, false, whole) || !gemm_two_pass_supported(type, false, rows, K, ntot, descs[0].dX));
 }
 }  // namespace
 
@@ -895,7 +900,7 @@ int gq_qdense_block_f32(int type, const float *dX, int64_t M, int64_t K, const g
     const MmqExtra ex{nullptr, nullptr, dResidual, norm ? &rn : nullptr};
     if (takes_mmv(type, M, K, N, dX, rn.gain, 1, true) && !y_over_x(dX, false, dY, M, K, N))
         return launch_mmv(type, dX, false, M, K, 1, &one, &ex, (hipStream_t)stream);
-    if (fold_into_gemv(type, M, K, N, dX, rn.gain, false))
+    if (fold_into_gemv(type, M, K, N, dX, rn.gain, false, whole))
         return launch_gemv_ks_ext(type, dX, false, M, K, norm ? &rn : nullptr, (const uint8_t *)dW, dBias, nullptr, nullptr, dResidual, N, act, dY,
                                   (hipStream_t)stream);
     if (block_takes_two_pass(type, M, K, N, dX, rn.gain, false, whole)) {
@@ -907,9 +912,7 @@ int gq_qdense_block_f32(int type, const float *dX, int64_t M, int64_t K, const g
     // split-K range: the normalisation rides on the activation pre-pass and the reduction, the residual on the reduction
     if (block_takes_split_k(type, M, K, N, dX, false, whole) && (!rn.gain || aligned_to(rn.gain, 16))) {
         const int rc = split_k(type, dX, false, M, K, 1, &one, &ex, (hipStream_t)stream);
-        if (!falls_back(rc, whole) || !gemv_ks_ext_supported(type, M, K, N, dX, rn.gain)) return rc;
-        return launch_gemv_ks_ext(type, dX, false, M, K, norm ? &rn : nullptr, (const uint8_t *)dW, dBias, nullptr, nullptr, dResidual, N, act, dY,
-                                  (hipStream_t)stream);
+        if (!falls_back(rc, whole)) return rc;
     }
     // composed: normalised activations into the stream's second workspace, the dense call, then the residual.  When y
     // overlaps the residual (a residual stream updated in place) the dense result goes to the workspace first: written
@@ -932,7 +935,8 @@ int gq_qdense_block_f32(int type, const float *dX, int64_t M, int64_t K, const g
     }
     if (dResidual && dense_takes_split_k(type, M, K, N, x, whole)) {  // the residual rides on the reduction
         const MmqExtra plain{nullptr, nullptr, dResidual, nullptr};
-        return split_k(type, x, false, M, K, 1, &one, &plain, (hipStream_t)stream);
+        const int rc = split_k(type, x, false, M, K, 1, &one, &plain, (hipStream_t)stream);
+        if (!falls_back(rc, whole)) return rc;
     }
     float *dense_out = in_place ? tmp : dY;
     if (int rc = gq_qdense_f32(type, x, M, K, dW, N, dBias, act, dense_out, stream)) return rc;
@@ -984,8 +988,6 @@ int gq_qdense_norm_f32_batch(int count, const gq_dense_desc *descs, const gq_rms
     if (shared_pass) {
         const int rc = split_k(descs[0].type, descs[0].dX, false, rows, descs[0].K, count, set, &ex, (hipStream_t)stream);
         if (!falls_back(rc, whole_set(count, set))) return rc;
-        if (merges_into_gemv(count, descs, norm, false, items))
-            return launch_gemv_ks_batch_norm(descs[0].type, count, items, &rn, (hipStream_t)stream, (int)rows);
     }
     // Past the split-K range the same projections share the two passes: one activation conversion, one image of all the
     // matrices, one GEMM (a decoder layer's q / k / v at 128 rows: two launches instead of six).
@@ -1018,7 +1020,7 @@ int gq_qdense_gated_f32(int type, const float *dX, int64_t M, int64_t K, const g
     const MmqExtra ex{(const uint8_t *)dWup, dBiasUp, nullptr, norm ? &rn : nullptr};
     if (takes_mmv(type, M, K, N, dX, rn.gain, 2, true) && !y_over_x(dX, false, dY, M, K, N))
         return launch_mmv(type, dX, false, M, K, 1, &one, &ex, (hipStream_t)stream);
-    if (fold_into_gemv(type, M, K, N, dX, rn.gain, true))
+    if (fold_into_gemv(type, M, K, N, dX, rn.gain, true, whole))
         return launch_gemv_ks_ext(type, dX, false, M, K, norm ? &rn : nullptr, (const uint8_t *)dWgate, dBiasGate, (const uint8_t *)dWup, dBiasUp,
                                   nullptr, N, act, dY, (hipStream_t)stream);
     if (block_takes_two_pass(type, M, K, N, dX, rn.gain, true, whole)) {
@@ -1030,9 +1032,7 @@ int gq_qdense_gated_f32(int type, const float *dX, int64_t M, int64_t K, const g
     // (split-K: both matrices against one activation image, which carries the gain; the reduction normalises and forms act(gate) * up)
     if (block_takes_split_k(type, M, K, N, dX, true, whole) && (!rn.gain || aligned_to(rn.gain, 16))) {
         const int rc = split_k(type, dX, false, M, K, 1, &one, &ex, (hipStream_t)stream);
-        if (!falls_back(rc, whole) || !gemv_ks_ext_supported(type, M, K, N, dX, rn.gain)) return rc;
-        return launch_gemv_ks_ext(type, dX, false, M, K, norm ? &rn : nullptr, (const uint8_t *)dWgate, dBiasGate, (const uint8_t *)dWup, dBiasUp,
-                                  nullptr, N, act, dY, (hipStream_t)stream);
+        if (!falls_back(rc, whole)) return rc;
     }
     // composed: [normalised activations,] act(gate) into the stream's second workspace, up into y, y *= act(gate)
     const size_t xn_bytes = norm ? ((size_t)M * (size_t)K * sizeof(float) + 255) / 256 * 256 : 0;
@@ -1047,7 +1047,8 @@ int gq_qdense_gated_f32(int type, const float *dX, int64_t M, int64_t K, const g
     if (dense_takes_split_k(type, M, K, N, x, whole)) {
         // both matrices against one activation image; the reduction forms act(gate) * up
         const MmqExtra plain{(const uint8_t *)dWup, dBiasUp, nullptr, nullptr};
-        return split_k(type, x, false, M, K, 1, &one, &plain, (hipStream_t)stream);
+        const int rc = split_k(type, x, false, M, K, 1, &one, &plain, (hipStream_t)stream);
+        if (!falls_back(rc, whole)) return rc;
     }
     float *gate = reinterpret_cast<float *>(static_cast<uint8_t *>(ws) + xn_bytes);
     if (int rc = gq_qdense_f32(type, x, M, K, dWgate, N, dBiasGate, act, gate, stream)) return rc;
@@ -1084,7 +1085,7 @@ int gq_qdense_block_bf16(int type, const uint16_t *dX, int64_t M, int64_t K, con
     const MmqExtra ex{nullptr, nullptr, dResidual, norm ? &rn : nullptr};
     if (takes_mmv(type, M, K, N, dX, rn.gain, 1, true) && !y_over_x(dX, true, dY, M, K, N))
         return launch_mmv(type, dX, true, M, K, 1, &one, &ex, (hipStream_t)stream);
-    if (fold_into_gemv(type, M, K, N, reinterpret_cast<const float *>(dX), norm ? norm->dGain : nullptr, false)) {
+    if (fold_into_gemv(type, M, K, N, reinterpret_cast<const float *>(dX), norm ? norm->dGain : nullptr, false, whole)) {
         return launch_gemv_ks_ext(type, dX, true, M, K, norm ? &rn : nullptr, (const uint8_t *)dW, dBias, nullptr, nullptr, dResidual, N, act, dY,
                                   (hipStream_t)stream);
     }
@@ -1092,9 +1093,7 @@ int gq_qdense_block_bf16(int type, const uint16_t *dX, int64_t M, int64_t K, con
         const float *xa = reinterpret_cast<const float *>(dX), *gain = norm ? norm->dGain : nullptr;  // (only their alignment is looked at)
         if (!block_takes_two_pass(type, M, K, N, xa, gain, false, whole) && block_takes_split_k(type, M, K, N, xa, false, whole) && (!gain || aligned_to(gain, 16))) {
             const int rc = split_k(type, dX, true, M, K, 1, &one, &ex, (hipStream_t)stream);
-            if (!falls_back(rc, whole) || !gemv_ks_ext_supported(type, M, K, N, dX, gain)) return rc;
-            return launch_gemv_ks_ext(type, dX, true, M, K, norm ? &rn : nullptr, (const uint8_t *)dW, dBias, nullptr, nullptr, dResidual, N, act, dY,
-                                      (hipStream_t)stream);
+            if (!falls_back(rc, whole)) return rc;
         }
     }
     void *ws = nullptr;
@@ -1119,7 +1118,7 @@ int gq_qdense_gated_bf16(int type, const uint16_t *dX, int64_t M, int64_t K, con
     const MmqExtra ex{(const uint8_t *)dWup, dBiasUp, nullptr, norm ? &rn : nullptr};
     if (takes_mmv(type, M, K, N, dX, rn.gain, 2, true) && !y_over_x(dX, true, dY, M, K, N))
         return launch_mmv(type, dX, true, M, K, 1, &one, &ex, (hipStream_t)stream);
-    if (fold_into_gemv(type, M, K, N, reinterpret_cast<const float *>(dX), norm ? norm->dGain : nullptr, true)) {
+    if (fold_into_gemv(type, M, K, N, reinterpret_cast<const float *>(dX), norm ? norm->dGain : nullptr, true, whole)) {
         return launch_gemv_ks_ext(type, dX, true, M, K, norm ? &rn : nullptr, (const uint8_t *)dWgate, dBiasGate, (const uint8_t *)dWup, dBiasUp, nullptr,
                                   N, act, dY, (hipStream_t)stream);
     }
@@ -1127,9 +1126,7 @@ int gq_qdense_gated_bf16(int type, const uint16_t *dX, int64_t M, int64_t K, con
         const float *xa = reinterpret_cast<const float *>(dX), *gain = norm ? norm->dGain : nullptr;  // (only their alignment is looked at)
         if (!block_takes_two_pass(type, M, K, N, xa, gain, true, whole) && block_takes_split_k(type, M, K, N, xa, true, whole) && (!gain || aligned_to(gain, 16))) {
             const int rc = split_k(type, dX, true, M, K, 1, &one, &ex, (hipStream_t)stream);
-            if (!falls_back(rc, whole) || !gemv_ks_ext_supported(type, M, K, N, dX, gain)) return rc;
-            return launch_gemv_ks_ext(type, dX, true, M, K, norm ? &rn : nullptr, (const uint8_t *)dWgate, dBiasGate, (const uint8_t *)dWup, dBiasUp, nullptr,
-                                      N, act, dY, (hipStream_t)stream);
+            if (!falls_back(rc, whole)) return rc;
         }
     }
     void *ws = nullptr;
@@ -1163,8 +1160,6 @@ int gq_qdense_norm_bf16_batch(int count, const gq_dense_desc *descs, const gq_rm
         if (shared_pass) {
             const int rc = split_k(descs[0].type, descs[0].dX, true, descs[0].M, descs[0].K, count, set, &ex, (hipStream_t)stream);
             if (!falls_back(rc, whole_set(count, set))) return rc;
-            if (merges_into_gemv(count, descs, norm, false, items))
-                return launch_gemv_ks_batch_norm(descs[0].type, count, items, &rn, (hipStream_t)stream, (int)descs[0].M, true);
         }
     }
     // every distinct activation matrix (q / k / v share theirs) is widened once

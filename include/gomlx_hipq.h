@@ -109,13 +109,15 @@ int gq_qdense_f32(int type, const float *dX, int64_t M, int64_t K, const void *d
                   const float *dBias, int act, float *dY, void *stream);
 /* gq_qdense_f32 for callers that cannot allocate device memory (code under HIP-graph capture, tight
  * serving loops, harnesses that forbid hipMalloc).  It has no counterpart in the reference.  Same
- * arguments, same kernels and, but for one case, bit-identical results; the scratch memory that batches
+ * arguments, same kernels and, but for two cases, bit-identical results; the scratch memory that batches
  * of 5 rows and more use (activation image, split-K partial sums) is a fixed 16 MiB device array inside
  * the library instead of a per-stream workspace (its first 4 KiB are the flag words every workspace starts
- * with: 16 MiB - 4 KiB serve the call), and the call makes no hipMalloc / hipFree at all.  The one case:
+ * with: 16 MiB - 4 KiB serve the call), and the call makes no hipMalloc / hipFree at all.  The first case:
  * a two-pass GEMM whose images fit that array, but not the sums of the K slices gq_qdense_f32 takes beside
  * them (some batches over a matrix of 2 to 8 Mi values), contracts K in one piece; the same products are
- * then added in another order, in fp32 as there, so that the results differ by a few fp32 roundings.  A
+ * then added in another order, in fp32 as there, so that the results differ by a few fp32 roundings.  The
+ * second: a call of 17 rows and more with N off every multiple of 4, or outputs off 16 bytes, whose split-K sums
+ * do not fit runs on the two passes instead, and differs by the rounding of their weights.  A
  * problem that needs more scratch than the array holds (the two-pass GEMM's 16-bit weight image of a large
  * matrix, or about M * N * K / 2048 > 3.5 Mi for the split-K kernels) fails with GQ_ERR_INVALID and a
  * message naming the size; nothing is launched then.  Every call on a GPU shares that GPU's array: calls
