@@ -7,7 +7,7 @@
 //
 //  * Activation traffic.  Every row tile of W needs all of x.  Fetching x per tile through
 //    the CU's vector-memory path would move several times more bytes than the weights themselves, so the
-//    work is split along K instead: a workgroup owns a K-slice of up to 7 super-blocks (1792 values; every n-th
+//    work is split along K instead: a workgroup owns a K-slice of up to 7 super-blocks (1792 values; 8 in the kernel for several tiles; every n-th
 //    super-block of a row for n slices, so that the slices' workgroups together read consecutive bytes),
 //    keeps the slice of x for 32 batch columns resident in LDS (fp16 in MFMA fragment order, written
 //    once by a pre-pass and copied global -> LDS without passing registers) and streams
