@@ -56,7 +56,6 @@ SIGNATURES = [
     ("gq_qdense_norm_bf16_batch", _int, [_int, _vp, _vp, _vp]),
     ("gq_qdense_gated_bf16", _int, [_int, _vp, _i64, _i64, _vp, _vp, _vp, _vp, _vp, _i64, _int, _vp, _vp]),
     ("gq_embedding_lookup", _int, [_int, _vp, _i64, _i64, _vp, _i64, _vp, _vp, _vp]),
-    ("gq_index_check", _int, [_vp, _i64, _i64, _vp, _vp]),
     ("gq_graph_begin", _int, [_vp]),
     ("gq_graph_end", _int, [_vp, ctypes.POINTER(_vp)]),
     ("gq_graph_launch", _int, [_vp, _vp]),
@@ -100,7 +99,7 @@ _fast_tried = False
 # Entry points the native host path calls, in the order in which csrc/binding.cpp takes them.
 _BOUND = ("gq_qdense_check", "gq_qdense_f32", "gq_qdense_bf16", "gq_qdense_block_f32", "gq_qdense_block_bf16", "gq_qdense_gated_f32",
           "gq_qdense_gated_bf16", "gq_qdense_f32_batch", "gq_qdense_norm_f32_batch", "gq_qdense_norm_bf16_batch", "gq_dequantize",
-          "gq_embedding_lookup", "gq_index_check", "gq_bytes_per_block", "gq_values_per_block")
+          "gq_embedding_lookup", "gq_bytes_per_block", "gq_values_per_block")
 
 
 def lib() -> ctypes.CDLL:

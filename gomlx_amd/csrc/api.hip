@@ -1208,14 +1208,6 @@ int gq_embedding_lookup(int type, const void *dTable, int64_t vocab, int64_t K, 
                                    (hipStream_t)stream);
 }
 
-int gq_index_check(const int32_t *dIndices, int64_t count, int64_t vocab, int32_t *status, void *stream) {
-    if (count < 0 || vocab < 0) return fail(GQ_ERR_INVALID, "gq_index_check: negative size");
-    if (!status || !aligned_to(status, 4) || (count > 0 && (!dIndices || !aligned_to(dIndices, 4))))
-        return fail(GQ_ERR_INVALID, "gq_index_check: null or misaligned pointer");
-    if (int rc = use_device()) return rc;
-    return launch_index_check(dIndices, count, vocab, status, (hipStream_t)stream);
-}
-
 int gq_graph_begin(void *stream) {
     if (!stream) return fail(GQ_ERR_INVALID, "gq_graph_begin: recording needs an explicit stream");
     if (profile_state().active) return fail(GQ_ERR_INVALID, "gq_graph_begin: kernel timing is active on this thread");

@@ -12,7 +12,6 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
 
-#include <chrono>
 #include <climits>
 #include <initializer_list>
 
@@ -33,11 +32,10 @@ struct Entry {
     decltype(&gq_qdense_norm_bf16_batch) norm_batch_bf16;
     decltype(&gq_dequantize) dequantize;
     decltype(&gq_embedding_lookup) lookup;
-    decltype(&gq_index_check) index_check;
     decltype(&gq_bytes_per_block) bytes_per_block;
     decltype(&gq_values_per_block) values_per_block;
 } g;
-constexpr int kEntries = 15;
+constexpr int kEntries = 14;
 bool g_bound = false;
 PyTypeObject *g_activation = nullptr;  // nn.Activation
 PyObject *s_scheme, *s_ggml_type, *s_gain, *s_epsilon, *s_scale_offset;
@@ -298,26 +296,7 @@ PyObject *gather(PyObject *, PyObject *const *a, Py_ssize_t n) {
         const void *tp = t->const_data_ptr();
         const int32_t *ip = idx->const_data_ptr<int32_t>();
         const hipStream_t s = static_cast<hipStream_t>(stream_of(*t));
-        // Up to kCheckedIndices indices are looked over by a launch of their own in front of the rows: the call waits for its answer, not for the
-        // rows (512 of them 15.8 -> 8.4 us a call among others).  Longer lists, and a stream that is being recorded, wait for the stream.
-        constexpr int64_t kCheckedIndices = 16384;
-        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-        const bool checked = idx->numel() <= kCheckedIndices && hipStreamIsCapturing(s, &capture) == hipSuccess && capture == hipStreamCaptureStatusNone;
         const int rc = without_gil([&] {
-            if (checked) {
-                int r = g.index_check(ip, idx->numel(), t->size(0), fp, s);
-                if (r != GQ_OK) return r;
-                r = g.lookup(type, tp, t->size(0), K, ip, idx->numel(), yp, nullptr, s);
-                const volatile int32_t *status = fp;
-                const auto give_up = std::chrono::steady_clock::now() + std::chrono::milliseconds(2);
-                while (*status == 0 && std::chrono::steady_clock::now() < give_up) {}
-                // (an answer that is late, behind long work on the stream, is waited for without spinning; one that never comes is an error.
-                // Either way nothing writes the flag after this.)
-                if (*status == 0 && hipStreamSynchronize(s) != hipSuccess) return (int)GQ_ERR_HIP;
-                if (r == GQ_OK && *status != 1) r = GQ_ERR_INVALID;
-                *fp = 0;
-                return r;
-            }
             const int r = g.lookup(type, tp, t->size(0), K, ip, idx->numel(), yp, fp, s);
             return r == GQ_OK && hipStreamSynchronize(s) != hipSuccess ? (int)GQ_ERR_HIP : r;
         });

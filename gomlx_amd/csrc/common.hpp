@@ -71,7 +71,6 @@ constexpr int64_t kLargeWeightBytes = (int64_t)24 << 20;
 int launch_dequantize(int type, const uint8_t *W, int64_t N, int64_t K, float *out, hipStream_t s);
 int launch_embedding_lookup(int type, const uint8_t *table, int64_t vocab, int64_t K, const int32_t *idx,
                             int64_t count, float *out, int32_t *err_flag, hipStream_t s);
-int launch_index_check(const int32_t *indices, int64_t count, int64_t vocab, int32_t *status, hipStream_t s);
 int launch_gemv(int type, const float *x, int64_t M, int64_t K, const uint8_t *W, int64_t N,
                 const float *bias, int act, float *y, hipStream_t s);
 bool gemv_xs_supported(int type, int64_t K, int64_t N, const void *x);

@@ -192,20 +192,6 @@ int dispatch_rows(int type, const uint8_t *W, float *out, int64_t N, int64_t K, 
 
 }  // namespace
 
-namespace {
-// Whether every index lies in [0, vocab), by one workgroup: the answer leaves for host memory (1: all do, 2: not) some 5 us after the launch,
-// while the rows are still being written.
-__global__ __launch_bounds__(1024) void index_check_kernel(const int32_t *__restrict__ indices, int64_t count, int64_t vocab, int32_t *status) {
-    int bad = 0;
-    for (int64_t i = threadIdx.x; i < count; i += 1024) bad |= indices[i] < 0 || indices[i] >= vocab;
-    bad = __syncthreads_or(bad);
-    if (threadIdx.x == 0) __hip_atomic_store(status, bad ? 2 : 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-}
-}  // namespace
-int launch_index_check(const int32_t *indices, int64_t count, int64_t vocab, int32_t *status, hipStream_t s) {
-    return launch(index_check_kernel, dim3(1), dim3(1024), 0, s, indices, count, vocab, status);
-}
-
 int launch_dequantize(int type, const uint8_t *W, int64_t N, int64_t K, float *out, hipStream_t s) {
     return dispatch_rows(type, W, out, N, K, nullptr, 0, nullptr, s);
 }

@@ -249,7 +249,7 @@ def quantized_dense(x: torch.Tensor, weights: torch.Tensor, quant: Quantization,
 
 def quantized_gather(table: torch.Tensor, indices: torch.Tensor, quant: Quantization) -> torch.Tensor:
     """nn.QuantizedGather: indices [batch..., 1] (int32) -> [batch..., K] float32 rows of the
-    dequantised table.  An out-of-range index raises IndexError."""
+    dequantised table.  An out-of-range index raises IndexError: the call waits for the stream, and returns with the rows written."""
     if _lib.fast is not None and (out := _lib.fast.gather(table, indices, quant)) is not None:
         return out
     if quant.scheme != QuantizationScheme.GGML:

@@ -229,11 +229,6 @@ int gq_qdense_gated_bf16(int type, const uint16_t *dX, int64_t M, int64_t K, con
 int gq_embedding_lookup(int type, const void *dTable, int64_t vocab, int64_t K,
                         const int32_t *dIndices, int64_t count, float *dOut,
                         int32_t *dErrFlag, void *stream);
-/* Whether `count` indices all lie in [0, vocab): *status, an int32 that the device can write
- * (pinned host memory, where a caller can wait for it without waiting for the stream), becomes
- * 1 if they do and 2 if not.  No counterpart in the reference. */
-int gq_index_check(const int32_t *dIndices, int64_t count, int64_t vocab, int32_t *status,
-                   void *stream);
 
 /* ---- Executable.Execute of a compiled graph (core/graph/graph.go:669): a sequence of
  * launches recorded once and replayed with one submission (HIP graph).  Between begin

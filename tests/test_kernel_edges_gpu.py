@@ -136,10 +136,9 @@ def test_split_k_rows_of_any_length(gpu, t, M, K, N):
     assert rel(nn.quantized_dense(xb, wd, q, dev(torch, bias)).cpu().numpy(), want) < TOL_F32
 
 
-@pytest.mark.parametrize("count", [1, 1024, 1025, 16384, 16385])
+@pytest.mark.parametrize("count", [1, 1024, 1025, 16385])
 def test_gather_finds_a_bad_index_wherever_it_is(gpu, count):
-    """Lists around the check's workgroup and around the length up to which it runs in front of the rows, also behind work on the stream that takes
-    longer than the host spins for."""
+    """First, middle and last index, alone on the stream and behind other work."""
     torch = gpu
     K, vocab = 32, 50
     table = synth.weights(ggml.Q8_0, 3, vocab, K)
@@ -155,6 +154,25 @@ def test_gather_finds_a_bad_index_wherever_it_is(gpu, count):
         wrong[at] = bad
         with pytest.raises(IndexError):
             nn.quantized_gather(td, dev(torch, wrong), q)
+
+
+@pytest.mark.parametrize("bad", [False, True])
+def test_gather_returns_with_its_rows_written(gpu, bad):
+    """256 MiB of rows, some 50 us of writing: the stream has nothing left to do when the call returns or raises, so that a reader on another
+    stream needs no event and memory of another stream may be released."""
+    torch = gpu
+    K, vocab, count = 4096, 64, 16384
+    td = dev(torch, synth.weights(ggml.Q8_0, 3, vocab, K))
+    idx = torch.arange(count, dtype=torch.int32, device="cuda").remainder_(vocab).view(-1, 1)
+    if bad:
+        idx[count - 1] = vocab
+    torch.cuda.synchronize()
+    if bad:
+        with pytest.raises(IndexError):
+            nn.quantized_gather(td, idx, Quantization(ggml_type=ggml.Q8_0))
+    else:
+        nn.quantized_gather(td, idx, Quantization(ggml_type=ggml.Q8_0))
+    assert torch.cuda.current_stream().query()
 
 
 @pytest.mark.parametrize("t", [ggml.Q4_0, ggml.Q8_0, ggml.IQ4_NL])
