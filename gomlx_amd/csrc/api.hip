@@ -274,7 +274,9 @@ int64_t gated_split_k_to(int type, int64_t K, int64_t N) {
     }
 }
 
-// Whether an output's rows are whole float4 in memory, as the split-K kernels' reduction and the GEMMs' sums of K slices store them best.
+// Whether an output's rows are whole float4 in memory, as the split-K kernels' reduction and the GEMMs' sums of K slices store them best: N, the
+// bias and y (of a gated pair: the gate's bias).  A residual or an up bias off 16 bytes is read element by element and moves no line: the exact
+// weights of the split-K kernels do not depend on it.
 template <class... P> bool whole_rows(int64_t N, P... outputs) { return N % 4 == 0 && ((reinterpret_cast<uintptr_t>(outputs) | ...) & 15) == 0; }
 
 // The hand-over of a call whose rows are not (`whole` false).  Its two passes cannot slice K, which is what makes them wait on long rows, and on
@@ -817,22 +819,24 @@ int64_t block_split_k_from(int type, int64_t weight_bytes, bool gated) {
     }
 }
 
-bool fold_into_gemv(int type, int64_t M, int64_t K, int64_t N, const float *x, const float *gain, bool gated, bool whole) {
+bool fold_into_gemv(int type, int64_t M, int64_t K, int64_t N, const float *x, const float *gain, bool gated, bool whole, bool up_whole = true) {
     if (!gemv_ks_ext_supported(type, M, K, N, x, gain)) return false;
-    return !(M >= take_over(block_split_k_from(type, weight_bytes_of(type, K, N), gated), whole) && mmq_supported(type, M, K, N, x));
+    return !(M >= take_over(block_split_k_from(type, weight_bytes_of(type, K, N), gated), whole && up_whole) && mmq_supported(type, M, K, N, x));
 }
 
 // Whether a projection with its neighbours runs on the split-K kernels (after fold_into_gemv() has declined).
-bool block_takes_split_k(int type, int64_t M, int64_t K, int64_t N, const float *x, bool gated, bool whole) {
+// up_whole: whether a gated pair's up bias is aligned as well.  Only the line up to 16 rows asks: off 16 bytes, that projection stayed on the GEMV and
+// the few-row kernel, whose activations have more bits (take_over).
+bool block_takes_split_k(int type, int64_t M, int64_t K, int64_t N, const float *x, bool gated, bool whole, bool up_whole = true) {
     const bool tp = gated ? gemm_two_pass_block_supported(type, M, K, N, x, true) : gemm_two_pass_supported(type, false, M, K, N, x);
     const int64_t to = hand_over(type, K, N, gated, whole);
-    return M >= take_over(block_split_k_from(type, weight_bytes_of(type, K, N), gated), whole) && mmq_supported(type, M, K, N, x) && (M <= to || !tp);
+    return M >= take_over(block_split_k_from(type, weight_bytes_of(type, K, N), gated), whole && up_whole) && mmq_supported(type, M, K, N, x) && (M <= to || !tp);
 }
 
 // Whether a plain dense call on these operands runs on the split-K kernels (the dispatch of gq_qdense_f32).
-bool dense_takes_split_k(int type, int64_t M, int64_t K, int64_t N, const float *x, bool whole) {
+bool dense_takes_split_k(int type, int64_t M, int64_t K, int64_t N, const float *x, bool whole, bool up_whole = true) {
     const bool tp = gemm_two_pass_supported(type, false, M, K, N, x);
-    return M >= take_over(split_k_from(type, weight_bytes_of(type, K, N)), whole) && mmq_supported(type, M, K, N, x) && (M <= hand_over(type, K, N, false, whole) || !tp);
+    return M >= take_over(split_k_from(type, weight_bytes_of(type, K, N)), whole && up_whole) && mmq_supported(type, M, K, N, x) && (M <= hand_over(type, K, N, false, whole) || !tp);
 }
 
 // First batch size of the gated pair as one GEMM (wherever the split-K kernels have handed over: the composed form is never
@@ -893,7 +897,7 @@ int gq_qdense_block_f32(int type, const float *dX, int64_t M, int64_t K, const g
     if (M == 0 || N == 0) return GQ_OK;
     if (int rc = use_device()) return rc;
     CallScope scope;
-    const bool whole = whole_rows(N, dBias, dResidual, dY);
+    const bool whole = whole_rows(N, dBias, dY);
     RmsNorm rn{nullptr, 0.f, 0.f};
     if (norm) rn = RmsNorm{norm->dGain, norm->eps, norm->gain_offset};
     const MmqSetItem one{(const uint8_t *)dW, N, dBias, act, dY};
@@ -1013,14 +1017,15 @@ int gq_qdense_gated_f32(int type, const float *dX, int64_t M, int64_t K, const g
     if (M == 0 || N == 0) return GQ_OK;
     if (int rc = use_device()) return rc;
     CallScope scope;
-    const bool whole = whole_rows(N, dBiasGate, dBiasUp, dY);
+    const bool whole = whole_rows(N, dBiasGate, dY);
+    const bool up = aligned_to(dBiasUp, 16);
     RmsNorm rn{nullptr, 0.f, 0.f};
     if (norm) rn = RmsNorm{norm->dGain, norm->eps, norm->gain_offset};
     const MmqSetItem one{(const uint8_t *)dWgate, N, dBiasGate, act, dY};
     const MmqExtra ex{(const uint8_t *)dWup, dBiasUp, nullptr, norm ? &rn : nullptr};
     if (takes_mmv(type, M, K, N, dX, rn.gain, 2, true) && !y_over_x(dX, false, dY, M, K, N))
         return launch_mmv(type, dX, false, M, K, 1, &one, &ex, (hipStream_t)stream);
-    if (fold_into_gemv(type, M, K, N, dX, rn.gain, true, whole))
+    if (fold_into_gemv(type, M, K, N, dX, rn.gain, true, whole, up))
         return launch_gemv_ks_ext(type, dX, false, M, K, norm ? &rn : nullptr, (const uint8_t *)dWgate, dBiasGate, (const uint8_t *)dWup, dBiasUp,
                                   nullptr, N, act, dY, (hipStream_t)stream);
     if (block_takes_two_pass(type, M, K, N, dX, rn.gain, true, whole)) {
@@ -1030,9 +1035,9 @@ int gq_qdense_gated_f32(int type, const float *dX, int64_t M, int64_t K, const g
                                           nullptr, N, act, dY, ws, (hipStream_t)stream);
     }
     // (split-K: both matrices against one activation image, which carries the gain; the reduction normalises and forms act(gate) * up)
-    if (block_takes_split_k(type, M, K, N, dX, true, whole) && (!rn.gain || aligned_to(rn.gain, 16))) {
+    if (block_takes_split_k(type, M, K, N, dX, true, whole, up) && (!rn.gain || aligned_to(rn.gain, 16))) {
         const int rc = split_k(type, dX, false, M, K, 1, &one, &ex, (hipStream_t)stream);
-        if (!falls_back(rc, whole)) return rc;
+        if (!falls_back(rc, whole && up)) return rc;
     }
     // composed: [normalised activations,] act(gate) into the stream's second workspace, up into y, y *= act(gate)
     const size_t xn_bytes = norm ? ((size_t)M * (size_t)K * sizeof(float) + 255) / 256 * 256 : 0;
@@ -1044,11 +1049,11 @@ int gq_qdense_gated_f32(int type, const float *dX, int64_t M, int64_t K, const g
         if (int rc = launch_rmsnorm(dX, M, K, rn.gain, rn.gain_offset, rn.eps, xn, (hipStream_t)stream)) return rc;
         x = xn;
     }
-    if (dense_takes_split_k(type, M, K, N, x, whole)) {
+    if (dense_takes_split_k(type, M, K, N, x, whole, up)) {
         // both matrices against one activation image; the reduction forms act(gate) * up
         const MmqExtra plain{(const uint8_t *)dWup, dBiasUp, nullptr, nullptr};
         const int rc = split_k(type, x, false, M, K, 1, &one, &plain, (hipStream_t)stream);
-        if (!falls_back(rc, whole)) return rc;
+        if (!falls_back(rc, whole && up)) return rc;
     }
     float *gate = reinterpret_cast<float *>(static_cast<uint8_t *>(ws) + xn_bytes);
     if (int rc = gq_qdense_f32(type, x, M, K, dWgate, N, dBiasGate, act, gate, stream)) return rc;
@@ -1079,7 +1084,7 @@ int gq_qdense_block_bf16(int type, const uint16_t *dX, int64_t M, int64_t K, con
     if (M == 0 || N == 0) return GQ_OK;
     if (int rc = use_device()) return rc;
     CallScope scope;
-    const bool whole = whole_rows(N, dBias, dResidual, dY);
+    const bool whole = whole_rows(N, dBias, dY);
     const RmsNorm rn = norm ? RmsNorm{norm->dGain, norm->eps, norm->gain_offset} : RmsNorm{nullptr, 0.f, 0.f};
     const MmqSetItem one{(const uint8_t *)dW, N, dBias, act, dY};
     const MmqExtra ex{nullptr, nullptr, dResidual, norm ? &rn : nullptr};
@@ -1112,21 +1117,22 @@ int gq_qdense_gated_bf16(int type, const uint16_t *dX, int64_t M, int64_t K, con
     if (M == 0 || N == 0) return GQ_OK;
     if (int rc = use_device()) return rc;
     CallScope scope;
-    const bool whole = whole_rows(N, dBiasGate, dBiasUp, dY);
+    const bool whole = whole_rows(N, dBiasGate, dY);
+    const bool up = aligned_to(dBiasUp, 16);
     const RmsNorm rn = norm ? RmsNorm{norm->dGain, norm->eps, norm->gain_offset} : RmsNorm{nullptr, 0.f, 0.f};
     const MmqSetItem one{(const uint8_t *)dWgate, N, dBiasGate, act, dY};
     const MmqExtra ex{(const uint8_t *)dWup, dBiasUp, nullptr, norm ? &rn : nullptr};
     if (takes_mmv(type, M, K, N, dX, rn.gain, 2, true) && !y_over_x(dX, true, dY, M, K, N))
         return launch_mmv(type, dX, true, M, K, 1, &one, &ex, (hipStream_t)stream);
-    if (fold_into_gemv(type, M, K, N, reinterpret_cast<const float *>(dX), norm ? norm->dGain : nullptr, true, whole)) {
+    if (fold_into_gemv(type, M, K, N, reinterpret_cast<const float *>(dX), norm ? norm->dGain : nullptr, true, whole, up)) {
         return launch_gemv_ks_ext(type, dX, true, M, K, norm ? &rn : nullptr, (const uint8_t *)dWgate, dBiasGate, (const uint8_t *)dWup, dBiasUp, nullptr,
                                   N, act, dY, (hipStream_t)stream);
     }
     {
         const float *xa = reinterpret_cast<const float *>(dX), *gain = norm ? norm->dGain : nullptr;  // (only their alignment is looked at)
-        if (!block_takes_two_pass(type, M, K, N, xa, gain, true, whole) && block_takes_split_k(type, M, K, N, xa, true, whole) && (!gain || aligned_to(gain, 16))) {
+        if (!block_takes_two_pass(type, M, K, N, xa, gain, true, whole) && block_takes_split_k(type, M, K, N, xa, true, whole, up) && (!gain || aligned_to(gain, 16))) {
             const int rc = split_k(type, dX, true, M, K, 1, &one, &ex, (hipStream_t)stream);
-            if (!falls_back(rc, whole)) return rc;
+            if (!falls_back(rc, whole && up)) return rc;
         }
     }
     void *ws = nullptr;

@@ -136,6 +136,43 @@ def test_split_k_rows_of_any_length(gpu, t, M, K, N):
     assert rel(nn.quantized_dense(xb, wd, q, dev(torch, bias)).cpu().numpy(), want) < TOL_F32
 
 
+def off16(torch, a):
+    """A copy of a float32 array on the GPU that starts 4 bytes behind a multiple of 16."""
+    buf = torch.empty(a.size + 1, dtype=torch.float32, device="cuda")
+    view = buf[1:].view(a.shape)
+    view.copy_(torch.from_numpy(a))
+    assert view.data_ptr() % 16 == 4
+    return view
+
+
+@pytest.mark.parametrize("t,M,K,N", [
+    (ggml.Q4_K, 17, 2048, 1024), (ggml.Q4_K, 96, 2048, 1024), (ggml.Q8_0, 40, 4096, 512), (ggml.Q4_0, 128, 2048, 1024), (ggml.IQ4_NL, 70, 2048, 8192),
+    (ggml.Q6_K, 33, 2048, 1024), (ggml.Q6_K, 96, 2048, 1024), (ggml.Q4_K, 300, 14336, 4096),
+    (ggml.Q8_0, 8, 8192, 1024), (ggml.Q4_K, 12, 14336, 4096),  # few rows: two launches of the few-row kernel, three of the split-K ones
+])
+@pytest.mark.parametrize("bf16", [False, True])
+def test_residual_and_up_bias_off_16_bytes_keep_the_route(gpu, t, M, K, N, bf16):
+    """A residual or an up bias off 16 bytes is read element by element: the same bits as an aligned one, on the split-K kernels, whose weights are exact,
+    up to the same row counts.  Up to 16 rows an up bias off 16 bytes keeps the pair on routes with more bits of the activations instead: within those of
+    the split-K kernels' fp16 (2^-11 of each value, 1e-4 rms of the largest output and a tenth of the bound of 1e-3 in either factor)."""
+    torch = gpu
+    reps = -(-N // 97)
+    wd, w2d = (dev(torch, np.tile(synth.weights(t, s, 97, K), (reps, 1))[:N]) for s in (3, 4))
+    x = dev(torch, synth.activations(5 + M, M, K))
+    x = x.to(torch.bfloat16) if bf16 else x
+    rng = np.random.default_rng(M)
+    res, bias = rng.standard_normal((M, N)).astype(np.float32), rng.standard_normal(N).astype(np.float32)
+    q, norm = Quantization(ggml_type=t), nn.RMSNorm(gain=dev(torch, 1 + 0.1 * rng.standard_normal(K).astype(np.float32)), epsilon=1e-5)
+    for n in (None, norm):
+        a, b = (nn.quantized_dense(x, wd, q, dev(torch, bias), norm=n, residual=r) for r in (dev(torch, res), off16(torch, res)))
+        assert torch.equal(a, b)
+        a, b = (nn.gated_feed_forward(x, wd, w2d, q, Activation.RELU, dev(torch, bias), u, norm=n) for u in (dev(torch, bias), off16(torch, bias)))
+        if M > 16:
+            assert torch.equal(a, b)
+        else:
+            assert float((a - b).abs().max()) < 2 * TOL_F32 * float(a.abs().max())
+
+
 @pytest.mark.parametrize("count", [1, 1024, 1025, 16385])
 def test_gather_finds_a_bad_index_wherever_it_is(gpu, count):
     """First, middle and last index, alone on the stream and behind other work."""
