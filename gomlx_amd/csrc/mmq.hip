@@ -635,13 +635,11 @@ __global__ __launch_bounds__(64 * Q4KTiles::kWaves) void mmq_q4k_tiles_kernel(co
         if (h == 1)
             dma16(lds0 + (uint32_t)(L::kRingBytes + (wave % NT) * 1024), srsrc, (uint32_t)(lane & 31) * 16u, (uint32_t)(kXFBytes + sb * 512));
     };
-    // (no fence: the loads that must have landed are waited for by count, and LDS reads have been consumed before a wavefront arrives)
+    // Loads that must have landed are waited for by count.  LDS reads too, all of them: what a wavefront has read the copies behind the barrier overwrite,
+    // and nothing else keeps a read's use - the sums' at the end of a super-block - in front of it (dma16 is not an LDS write to the compiler).
     auto meet = [&](bool all) __attribute__((always_inline)) {
-        // (the builtin, not written-out text: the compiler keeps its own count of loads into LDS and would otherwise wait for
-        // all of them in front of the first LDS read it cannot tell apart from their destinations)
-        if (all) __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
-        else __builtin_amdgcn_s_waitcnt(0x0F75);       // vmcnt(5)
-        asm volatile("" ::: "memory");
+        if (all) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        else asm volatile("s_waitcnt vmcnt(5) lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
     };
@@ -1419,9 +1417,12 @@ __global__ __launch_bounds__(64 * Q4KTiles::kWaves) void mmq_b32_tiles_kernel(co
                 (__attribute__((address_space(3))) void *)(dst + t * G::kHalfBytes + ck * 1024), 16, 0, 0);
         }
     };
-    auto meet = [&](bool all) __attribute__((always_inline)) {  // (see mmq_q4k_tiles_kernel)
-        if (all) __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
-        else __builtin_amdgcn_s_waitcnt(0x0F75);       // vmcnt(5)
+    auto meet = [&](bool all) __attribute__((always_inline)) {
+        // (as in mmq_q4k_tiles_kernel; the builtin, not written-out text: the compiler keeps its own count of its loads into LDS and would
+        // otherwise wait for all of them in front of the first LDS read it cannot tell apart from their destinations)
+        asm volatile("" ::: "memory");
+        if (all) __builtin_amdgcn_s_waitcnt(0x0070);   // vmcnt(0) lgkmcnt(0)
+        else __builtin_amdgcn_s_waitcnt(0x0075);       // vmcnt(5) lgkmcnt(0)
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
@@ -1586,9 +1587,12 @@ __global__ __launch_bounds__(64 * Q4KTiles::kWaves) void mmq_q8_tiles_kernel(con
                 (__attribute__((address_space(3))) void *)(dst + t * Q::kHalfBytes + ck * 1024), 16, 0, 0);
         }
     };
-    auto meet = [&](bool all) __attribute__((always_inline)) {  // (see mmq_q4k_tiles_kernel)
-        if (all) __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
-        else __builtin_amdgcn_s_waitcnt(0x0F79);       // vmcnt(9)
+    auto meet = [&](bool all) __attribute__((always_inline)) {
+        // (as in mmq_q4k_tiles_kernel; the builtin, not written-out text: the compiler keeps its own count of its loads into LDS and would
+        // otherwise wait for all of them in front of the first LDS read it cannot tell apart from their destinations)
+        asm volatile("" ::: "memory");
+        if (all) __builtin_amdgcn_s_waitcnt(0x0070);   // vmcnt(0) lgkmcnt(0)
+        else __builtin_amdgcn_s_waitcnt(0x0079);       // vmcnt(9) lgkmcnt(0)
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
