@@ -998,9 +998,9 @@ WregPlan plan_wreg_set(int type, int64_t M, int64_t K, int count, const MmqSetIt
     }
     return plan_wreg(type, false, M, K, tiles, cols, cols * K, false, may_split);
 }
-// [fp32 activations: fp16 rows, row scales (whole tiles of rows)][sums of the slices]
+// [fp32 activations: fp16 rows, row scales][sums of the slices]
 size_t wreg_front_bytes(bool bf16, int64_t M, int64_t K) {
-    return bf16 ? 0 : align256((size_t)M * K * 2) + align256((size_t)((M + 255) / 256 * 256) * sizeof(float));
+    return bf16 ? 0 : align256((size_t)M * K * 2) + align256((size_t)M * sizeof(float));
 }
 // (whatever the alignment of the outputs lets the plan be at the launch)
 size_t wreg_bytes(const WregPlan &split, bool bf16, int64_t M, int64_t K, int64_t cols) {
@@ -1030,7 +1030,8 @@ int run_wreg(int type, bool bf16, const void *x, int64_t M, int64_t K, const Rms
     return launch_slices_reduce(partial, p.slices, M, segs.n0[count], rowscale, nullptr, act, nullptr, nullptr, &segs, s);
 }
 }  // namespace
-// (The image's bytes also where gemm_wreg.hip needs none: an output that is not aligned for slices may take the other way at the launch.)
+// (The image's bytes also where gemm_wreg.hip needs none: outputs that are not aligned for slices may take the other way, and a recording of such a
+// call finds the workspace that an aligned one has left.)
 size_t gemm_two_pass_workspace(int type, bool x_is_bf16, int64_t M, int64_t K, int64_t N, bool split_k) {
     const int64_t Kp = padded_k(K);
     return std::max(two_pass_front_bytes(x_is_bf16, M, Kp, N) + (split_k ? gemm_partial_bytes(M, Kp, N) : 0),

@@ -119,7 +119,8 @@ int gq_qdense_f32(int type, const float *dX, int64_t M, int64_t K, const void *d
  * second: a call of 17 rows and more with N off every multiple of 4, or outputs off 16 bytes, whose split-K sums
  * do not fit runs on the two passes instead, and differs by the rounding of their weights.  A
  * problem that needs more scratch than the array holds (the two-pass GEMM's 16-bit weight image of a large
- * matrix, which the batches whose weights a GEMM converts in registers do without, or about M * N * K / 2048 > 3.5 Mi for the split-K kernels) fails with GQ_ERR_INVALID and a
+ * matrix, which is asked for also where a GEMM then converts the weights in registers, or about
+ * M * N * K / 2048 > 3.5 Mi for the split-K kernels) fails with GQ_ERR_INVALID and a
  * message naming the size; nothing is launched then.  Every call on a GPU shares that GPU's array: calls
  * that overlap in time on one GPU (different streams, or host threads that interleave) race; calls
  * on one stream from one thread are ordered and safe.  Not available while gq_profile_begin() is

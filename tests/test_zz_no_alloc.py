@@ -94,9 +94,10 @@ def test_static_scratch_entry_allocates_nothing(gpu, oracle):
         _lib.check(L.gq_stream_destroy(sp))
 
 
-def test_static_scratch_entry_rejects_what_does_not_fit(gpu):
+@pytest.mark.parametrize("t,M,K,N", [(ggml.Q8_0, 512, 4096, 4096),     # two-pass GEMM: a 32 MiB weight image
+                                     (ggml.Q4_K, 512, 14336, 4096)])  # one GEMM that converts the weights in registers: the image is asked for all the same
+def test_static_scratch_entry_rejects_what_does_not_fit(gpu, t, M, K, N):
     L = _lib.lib()
-    t, M, K, N = ggml.Q8_0, 512, 4096, 4096  # two-pass GEMM: a 32 MiB weight image
     W = gpu.zeros((N, ggml.row_bytes(t, K)), dtype=gpu.uint8, device="cuda")
     x = gpu.zeros((M, K), device="cuda")
     y = gpu.full((M, N), 7.0, device="cuda")
