@@ -2,10 +2,12 @@
 
 Bounds: max|got - want| / max|want| <= 1e-3 for fp32 activations (fp16 operands), 2e-2 for bfloat16 ones, as in test_parity_gpu.py.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
-from gomlx_amd import ggml, nn, synth
+from gomlx_amd import _lib, ggml, nn, synth
 from gomlx_amd.nn import Activation, Quantization
 from oracle import ggml_oracle as oracle
 
@@ -80,15 +82,54 @@ def test_gemm_with_weights_converted_in_registers(gpu, monkeypatch, t, tm, slice
     assert rel(nn.quantized_dense(xb, wd, q, dev(torch, bias)).cpu().numpy(), want) < TOL_BF16
 
 
+@pytest.mark.parametrize("t", GEMM_TYPES)
+@pytest.mark.parametrize("tm,slices,M", [(4, 2, 130), (6, 3, 200), (8, 2, 257)])
+def test_matrices_of_one_input_in_slices_with_weights_converted_in_registers(gpu, monkeypatch, t, tm, slices, M):
+    """Three matrices of different widths, the last workgroup of each partly filled, K in slices: each one's columns of the shared sums."""
+    torch, K, Ns = gpu, 5 * 256, (544, 288, 32)
+    monkeypatch.setenv("GOMLX_HIPQ_GEMM_WREG", f"{tm},{slices}")
+    x, Ws = synth.activations(5 + M, M, K), [synth.weights(t, 3 + i, n, K) for i, n in enumerate(Ns)]
+    gain = 1 + 0.1 * np.random.default_rng(M).standard_normal(K).astype(np.float32)
+    biases = [dev(torch, np.linspace(-1, 1, n, dtype=np.float32)) for n in Ns]
+    norm = nn.RMSNorm(gain=dev(torch, gain), epsilon=1e-5)
+    h = x * gain / np.sqrt(np.mean(x.astype(np.float64) ** 2, axis=1, keepdims=True) + 1e-5)
+    xd, q = dev(torch, x), Quantization(ggml_type=t)
+    outs = nn.quantized_dense_batch([(xd, dev(torch, w), q, b, None) for w, b in zip(Ws, biases)], norm=norm)
+    for out, w, b in zip(outs, Ws, biases):
+        want = oracle.c_qdense(t, h.astype(np.float32), w, None, oracle.ACT_NONE)
+        assert np.max(np.abs(out.cpu().numpy() - want - b.cpu().numpy())) < TOL_F32 * np.max(np.abs(want))
+
+
+@pytest.mark.parametrize("t", GEMM_TYPES)
+@pytest.mark.parametrize("bf16", [False, True])
+def test_gemm_with_weights_converted_in_registers_and_infinite_activations(gpu, monkeypatch, t, bf16):
+    """Rows with +inf, with -inf and with both, as in 64 bits on weights rounded to the operands' 16 bits, where a zero makes a NaN; the other rows stay finite."""
+    torch, M, K, N = gpu, 300, 512, 260
+    monkeypatch.setenv("GOMLX_HIPQ_GEMM_WREG", "8,1")
+    W = synth.weights(t, 77, N, K)
+    x = np.random.default_rng(M).standard_normal((M, K)).astype(np.float32)
+    x[1, K - 3], x[130, 5], x[299, 17], x[299, K - 300] = np.inf, -np.inf, np.inf, -np.inf
+    xd, w = dev(torch, x), torch.from_numpy(oracle.c_dequantize(t, W, K))
+    w = w.to(torch.bfloat16 if bf16 else torch.float16).double().numpy()
+    got = nn.quantized_dense(xd.to(torch.bfloat16) if bf16 else xd, dev(torch, W), Quantization(ggml_type=t)).cpu().numpy()
+    with np.errstate(invalid="ignore"):
+        want = x.astype(np.float64) @ w.T
+    for m in (1, 130, 299):
+        assert not np.isfinite(want[m]).any()
+        np.testing.assert_array_equal(got[m], want[m])
+    assert np.isfinite(np.delete(got, (1, 130, 299), axis=0)).all()
+
+
 def test_gemm_with_weights_converted_in_registers_keeps_infinities(gpu, monkeypatch):
     """A block of infinite scale in one weight row: that output column is infinite or NaN as the reference's, every other one untouched."""
     torch = gpu
     K, N, M = 512, 63, 40  # (an N that the split-K kernels do not take)
-    for t in (ggml.Q8_0, ggml.Q4_0, ggml.IQ4_NL):
+    for t in GEMM_TYPES:
         W = synth.weights(t, 3, N, K)
         W[5, 0:2] = np.frombuffer(np.float16(np.inf).tobytes(), np.uint8)
         bpb = ggml.bytes_per_block(t)
-        W[5, 2:bpb] = 0x7F if t == ggml.Q8_0 else 0xFF  # largest code everywhere: no infinity meets its opposite inside the block
+        # largest code (and sub-block scale) everywhere: no infinity meets a zero or its opposite inside the block
+        W[5, 4 if t == ggml.Q4_K else 2:bpb] = 0x7F if t == ggml.Q8_0 else 0xFF
         x = np.abs(synth.activations(9, M, K)) + 0.1
         monkeypatch.setenv("GOMLX_HIPQ_GEMM_WREG", "4")
         got = nn.quantized_dense(dev(torch, x), dev(torch, W), Quantization(ggml_type=t)).cpu().numpy()
@@ -171,6 +212,103 @@ def test_residual_and_up_bias_off_16_bytes_keep_the_route(gpu, t, M, K, N, bf16)
             assert torch.equal(a, b)
         else:
             assert float((a - b).abs().max()) < 2 * TOL_F32 * float(a.abs().max())
+
+
+@pytest.mark.parametrize("t,M,K,N,wreg", [
+    (ggml.Q4_K, 40, 4096, 1024, None), (ggml.Q8_0, 17, 4096, 1028, None), (ggml.Q4_0, 66, 4096, 1024, None), (ggml.Q6_K, 20, 4096, 1024, None),  # split-K
+    (ggml.Q8_0, 129, 512, 260, "4,1"), (ggml.Q4_K, 255, 512, 516, "8,1"), (ggml.IQ4_NL, 193, 768, 36, "6,1"),  # the GEMM that converts weights in registers
+])
+def test_outputs_off_16_bytes(gpu, monkeypatch, t, M, K, N, wreg):
+    """N a multiple of four and y off 16 bytes: stored element by element, the same bits as float4 - plain, a residual stream updated in place, a gated
+    pair - and no element outside y."""
+    torch = gpu
+    if wreg:
+        monkeypatch.setenv("GOMLX_HIPQ_GEMM_WREG", wreg)
+    L, stream = _lib.lib(), torch.cuda.current_stream().cuda_stream
+    W, W2, x = synth.weights(t, 3, N, K), synth.weights(t, 4, N, K), synth.activations(5 + M, M, K)
+    rng = np.random.default_rng(M)
+    bias, res = rng.standard_normal(N).astype(np.float32), rng.standard_normal((M, N)).astype(np.float32)
+    wd, w2d, xd, bd, rd = dev(torch, W), dev(torch, W2), dev(torch, x), dev(torch, bias), dev(torch, res)
+    def calls(y):
+        yp = y.data_ptr()
+        yield lambda: L.gq_qdense_f32(t, xd.data_ptr(), M, K, wd.data_ptr(), N, bd.data_ptr(), oracle.ACT_RELU, yp, stream)
+        yield lambda: L.gq_qdense_block_f32(t, xd.data_ptr(), M, K, None, wd.data_ptr(), N, bd.data_ptr(), oracle.ACT_NONE, yp, yp, stream)
+        yield lambda: L.gq_qdense_gated_f32(t, xd.data_ptr(), M, K, None, wd.data_ptr(), bd.data_ptr(), w2d.data_ptr(), None, N, oracle.ACT_RELU, yp, stream)
+    buf = torch.full((M * N + 8,), 7.0, device="cuda")
+    y, odd = torch.empty(M, N, device="cuda"), buf[5:5 + M * N].view(M, N)
+    gate, up = (oracle.c_qdense(t, x, w, b, oracle.ACT_NONE) for w, b in ((W, bias), (W2, None)))
+    wants = [np.maximum(gate, 0), gate + res, np.maximum(gate, 0) * up]
+    for a, b, want in zip(calls(y), calls(odd), wants):
+        for out, call in ((y, a), (odd, b)):
+            out.copy_(rd)
+            _lib.check(call())
+        assert torch.equal(y, odd)
+        assert np.max(np.abs(y.cpu().numpy() - want)) < 2 * TOL_F32 * np.max(np.abs(want))
+        assert bool((buf[:5] == 7).all()) and bool((buf[5 + M * N:] == 7).all())
+
+
+@pytest.mark.parametrize("recorded", [False, True])
+def test_split_k_without_room_falls_back(gpu, recorded):
+    """N off every multiple of four at 128 rows: the split-K kernels' scratch memory (23 MiB here) does not fit the static array, or what the stream holds when
+    a recording begins; the call goes on to the two passes (16 MiB), whose weights are rounded to 16 bits."""
+    torch, t, M, K, N = gpu, ggml.Q4_K, 128, 16384, 351
+    L = _lib.lib()
+    W, x = synth.weights(t, 3, N, K), synth.activations(4, 129, K)
+    wd, xd = dev(torch, W), dev(torch, x)
+    want = oracle.c_qdense(t, x[:M], W, None, oracle.ACT_NONE)
+    y = torch.zeros(M, N, device="cuda")
+    split = nn.quantized_dense(xd[:M], wd, Quantization(ggml_type=t)).cpu().numpy()
+    assert rel(split, want) < TOL_F32
+    if not recorded:
+        _lib.check(L.gq_qdense_f32_static(t, xd.data_ptr(), M, K, wd.data_ptr(), N, None, 0, y.data_ptr(), torch.cuda.current_stream().cuda_stream))
+        got = y.cpu().numpy()
+    else:
+        torch.cuda.synchronize()
+        sp = ctypes.c_void_p()
+        _lib.check(L.gq_stream_create(ctypes.byref(sp)))
+        dense = lambda rows, out: _lib.check(L.gq_qdense_f32(t, xd.data_ptr(), rows, K, wd.data_ptr(), N, None, 0, out.data_ptr(), sp))
+        one_more = torch.zeros(129, N, device="cuda")
+        torch.cuda.synchronize()
+        dense(129, one_more)  # two passes: the stream holds what they need
+        _lib.check(L.gq_sync(sp))
+        _lib.check(L.gq_graph_begin(sp))
+        dense(M, y)
+        g = ctypes.c_void_p()
+        _lib.check(L.gq_graph_end(sp, ctypes.byref(g)))
+        for _ in range(3):
+            y.fill_(float("nan"))
+            torch.cuda.synchronize()
+            dense(129, one_more)
+            _lib.check(L.gq_graph_launch(g, sp))
+            _lib.check(L.gq_sync(sp))
+            got = y.cpu().numpy()
+            assert np.array_equal(got, one_more[:M].cpu().numpy())
+        _lib.check(L.gq_graph_destroy(g))
+        _lib.check(L.gq_stream_destroy(sp))
+    assert rel(got, want) < TOL_F32 and not np.array_equal(got, split)
+
+
+@pytest.mark.parametrize("t", [ggml.Q8_0, ggml.Q4_0, ggml.IQ4_NL, ggml.Q6_K])
+@pytest.mark.parametrize("M,K,N", [(20, 4096, 2051), (40, 4096, 1602), (96, 8192, 1025)])
+@pytest.mark.parametrize("bf16", [False, True])
+def test_infinite_activations_of_batches_with_rows_of_any_length(gpu, t, M, K, N, bf16):
+    """N off every multiple of four on the split-K kernels: rows with +inf, with -inf and with both are the infinities and NaN of 64 bits, the other rows
+    finite, as on the routes these calls had before.  (Q4_K's sub-block minima are a second sum, in which an infinity meets its opposite.)"""
+    torch = gpu
+    W = np.tile(synth.weights(t, 77, 131, K), (-(-N // 131), 1))[:N]
+    x = np.random.default_rng(M + K).standard_normal((M, K)).astype(np.float32)
+    x[1, K - 3], x[3, 5], x[4, 17], x[4, K - 300] = np.inf, -np.inf, np.inf, -np.inf
+    xd = dev(torch, x)
+    if bf16:
+        xd = xd.to(torch.bfloat16)
+        x = xd.float().cpu().numpy()
+    got = nn.quantized_dense(xd, dev(torch, W), Quantization(ggml_type=t)).cpu().numpy()
+    with np.errstate(invalid="ignore"):
+        want = np.tile(x.astype(np.float64) @ oracle.c_dequantize(t, W[:131], K).astype(np.float64).T, (1, -(-N // 131)))[:, :N]
+    for m in (1, 3, 4):
+        assert not np.isfinite(want[m]).any()
+        np.testing.assert_array_equal(got[m], want[m])
+    assert np.isfinite(np.delete(got, (1, 3, 4), axis=0)).all()
 
 
 @pytest.mark.parametrize("count", [1, 1024, 1025, 16385])
