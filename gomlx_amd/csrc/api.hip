@@ -212,24 +212,25 @@ int64_t weight_bytes_of(int type, int64_t K, int64_t N) { return (int64_t)gq_row
 // 32 batch rows (Q6_K: per tile); the two passes pay the 16-bit image (written once and read once, in proportion to N K) and a GEMM that
 // splits K itself where its tiles leave CUs idle.
 // Measured (GOMLX_HIPQ_SPLIT_K_TO=100000 and =16; us per call on rotating weights, fp32 activations; rows 32 64 96 128 160 192 256;
-// split-K | two passes at the same rows):
-//   Q8_0   4096x4096  16 22 27 29 35 36 44 | 24 24 24 25 29 29 30
-//          4096x14336 31 36 43 49 69 76 88 | 51 54 53 54 64 65 65    14336x4096 31 37 44 50 70 77 90 | 53 55 56 58 68 74 76
-//   Q4_0   4096x4096  14 19 24 26 32 33 39 | 23 24 24 25 28 28 29
-//          4096x14336 25 32 39 44 61 67 79 | 47 48 49 50 59 60 60    14336x4096 26 33 39 44 62 69 82 | 51 51 53 55 66 71 73
-//   Q4_K   4096x4096  14 17 20 28 36 38 44 | 25 24 25 25 29 29 30
-//          4096x14336 21 27 32 37 52 57 68 | 48 49 50 51 61 61 61    14336x4096 21 28 33 38 54 59 71 | 50 52 54 56 66 72 74
-//   Q6_K   4096x4096  18 21 29 32 39 41 50 | 25 25 25 27 30 30 31
-//          4096x14336 34 55 76 89 109 130 163 | 53 54 55 56 66 66 66    14336x4096 35 55 77 90 111 132 167 | 54 56 57 59 70 75 77
-//   IQ4_NL 4096x4096  15 21 27 29 37 37 45 | 23 24 24 25 28 29 30
-//          4096x14336 28 34 41 46 65 72 84 | 47 48 49 50 60 61 61    14336x4096 29 35 41 47 67 73 86 | 51 52 54 56 66 71 74
-//          (Q4_K at 320 rows: 4096x14336 88 | 85, 14336x4096 92 | 92)
-// The hand-over lies up to 64 rows beyond the point where the two passes are level: the split-K kernels contract exact weights, the two passes
-// weights rounded to 16 bits (a relative error of 5.6e-4 for Q4_K where the split-K kernels have 2.6e-4), and these few per cent do not buy that.
-// GOMLX_HIPQ_SPLIT_K_TO=rows overrides the table (tuning runs only).
+// split-K | two passes - from 2^25 values on, but for Q6_K, in the one-GEMM form - at the same rows):
+//   Q8_0   4096x4096  16 22 26 29 35 36 45 | 23 24 27 25 27 28 30
+//          4096x14336 30 36 43 49 70 76 91 | 36 38 41 44 49 52 63    14336x4096 30 37 43 51 71 77 93 | 47 49 52 54 57 58 62
+//   Q4_0   4096x4096  14 19 25 27 33 34 42 | 26 25 26 27 27 28 30
+//          4096x14336 25 32 38 44 62 68 79 | 31 33 37 39 45 47 58    14336x4096 25 33 40 45 63 69 81 | 41 43 45 46 49 50 55
+//   Q4_K   4096x4096  14 17 21 28 37 39 45 | 25 27 27 28 29 29 31
+//          4096x14336 20 26 32 37 52 58 69 | 29 31 34 37 43 46 54    14336x4096 19 28 34 38 54 60 73 | 37 38 42 43 46 49 52
+//   Q6_K   4096x4096  18 21 30 32 41 42 52 | 25 26 27 28 29 29 32
+//          4096x14336 32 56 78 92 114 138 171 | 55 56 58 61 75 72 71    14336x4096 32 55 78 94 117 138 171 | 65 65 66 66 79 77 81
+//   IQ4_NL 4096x4096  16 21 28 29 38 39 47 | 25 26 27 27 27 28 31
+//          4096x14336 28 34 41 47 66 72 86 | 34 37 40 41 47 50 60    14336x4096 28 35 43 49 69 74 86 | 61 61 63 52 54 55 58
+//          (Q4_K at 320 rows: 4096x14336 91 | 64, 14336x4096 95 | 63)
+// The split-K kernels contract exact weights, the two passes weights rounded to 16 bits (a relative error of 5.6e-4 for Q4_K where the split-K kernels
+// have 2.6e-4).  So the hand-over lies beyond the point where both are level: by up to 64 rows over matrices that the image serves, and where it lay
+// in front of the one-GEMM form over those that this serves, at up to 1.5 times its time: bits that a batch has are not given up for time.
+// GOMLX_HIPQ_SPLIT_K_TO=rows overrides the table (tuning runs and tests; read at every call that the split-K kernels could take).
 int64_t split_k_to_env() {
-    static const int64_t v = [] { const char *e = std::getenv("GOMLX_HIPQ_SPLIT_K_TO"); return e ? (int64_t)std::atoll(e) : (int64_t)-1; }();
-    return v;
+    const char *e = std::getenv("GOMLX_HIPQ_SPLIT_K_TO");
+    return e ? (int64_t)std::atoll(e) : (int64_t)-1;
 }
 int64_t split_k_to(int type, int64_t K, int64_t N) {
     if (split_k_to_env() >= 0) return split_k_to_env();
@@ -246,18 +247,18 @@ int64_t split_k_to(int type, int64_t K, int64_t N) {
 
 // The same point for a gated pair act(x.Wgate) * (x.Wup): both matrices are contracted against one activation image by the
 // split-K kernels, or dequantised into one interleaved image for ONE GEMM by the two passes.  Measured (the same way, SiLU behind a
-// normalisation; rows 32 64 96 128 160 192 256; split-K | two passes):
-//   Q8_0   4096x4096  23 28 33 37 51 54 66 | 45 46 46 47 48 49 49
-//          4096x14336 53 63 76 88 126 139 165 | 115 118 123 129 144 145 152
-//   Q4_0   4096x4096  20 25 30 34 45 49 61 | 45 45 46 46 46 46 46
-//          4096x14336 43 54 67 78 110 122 144 | 106 111 113 120 135 131 137
-//   Q4_K   4096x4096  17 22 27 31 42 46 56 | 46 46 47 48 49 48 47
-//          4096x14336 31 45 55 64 93 103 125 | 108 112 115 122 137 133 139
-//   Q6_K   4096x4096  29 34 44 53 63 70 88 | 46 46 47 48 48 48 48
-//          4096x14336 58 92 132 166 204 235 308 | 117 120 126 131 144 146 153
-//   IQ4_NL 4096x4096  21 26 31 35 48 52 62 | 46 45 46 46 48 47 47
-//          4096x14336 48 59 72 82 120 133 155 | 108 111 114 120 130 132 131
-//          (Q4_K at 320 and 384 rows: 165 187 | 171 166; where the line lies and why: as above)
+// normalisation; rows 32 64 96 128 160 192 256; split-K | two passes or one GEMM):
+//   Q8_0   4096x4096  25 29 33 38 52 56 68 | 44 44 45 46 47 47 47
+//          4096x14336 56 63 76 86 124 132 155 | 89 89 92 93 92 93 95
+//   Q4_0   4096x4096  21 26 30 34 47 50 61 | 42 42 42 43 43 43 44
+//          4096x14336 44 54 67 77 105 114 132 | 72 72 75 76 79 79 80
+//   Q4_K   4096x4096  18 23 27 31 43 47 57 | 43 43 44 45 45 46 46
+//          4096x14336 30 39 49 58 83 92 110 | 62 63 66 69 76 78 79
+//   Q6_K   4096x4096  31 36 46 55 65 73 90 | 46 46 46 47 47 47 48
+//          4096x14336 64 96 137 170 211 243 316 | 118 118 123 127 138 138 145
+//   IQ4_NL 4096x4096  22 27 32 35 49 52 63 | 42 42 43 43 44 44 44
+//          4096x14336 49 60 72 82 114 123 141 | 82 83 85 85 90 88 90
+//          (Q4_K at 320 and 384 rows: 143 161 | 99 98; where the line lies and why: as above, here at up to 1.6 times the one GEMM's time)
 // (The pair composed of two dense calls and a multiplication is never ahead of the one GEMM: 127 - 159 against 118 - 143 us
 // for Q4_K 4096 -> 2 x 14336 at 64 - 256 rows.)
 int64_t gated_split_k_to(int type, int64_t K, int64_t N) {
@@ -288,19 +289,24 @@ template <class... P> bool whole_rows(int64_t N, P... outputs) { return N % 4 ==
 //   K 4096, 128 rows: Q4_K 1.27 1.29 1.25 1.22 1.32, Q8_0 1.82 1.40 1.12 1.06 .89 (96: 1.02 at 12001), Q4_0 1.87 1.59 1.25 1.07 .93, IQ4_NL 1.79 1.49 1.15 1.03 .90, gated .98 to 1.72;
 //     192: Q4_0 .72, IQ4_NL .68 at 12001; Q6_K 64: 1.60 1.71 1.16 1.05 1.07 (96: .80 at 6001)
 //   K 8192, 128 rows: Q8_0 2.07 1.61 1.48 1.39 1.60, Q4_0 2.36 1.81 1.53 1.45 1.28; 192: .91 to 1.03
+// and over small matrices (the range over five widths of 0.25 to 2.2 million values):
+//   K 1024, 17 rows: Q4_K 1.02 to 1.12, the others .76 to 1.11; 32: .71 to 1.01
+//   K 2048, 64 and 128 rows: Q4_K 1.03 to 1.07, .83 to .85 (gated 96: 1.00 to 1.07), Q6_K .98 to 1.02 at both (17: 1.03 to 1.09), Q8_0 Q4_0 IQ4_NL 1.18 to 1.29, 1.15 to 1.33
+//     (gated 96: 1.23 to 1.33, 128: 1.00 to 1.37)
+//   K 4096, 64 and 128 rows: Q4_K 1.59 to 1.67, 1.25 to 1.39, Q6_K 1.50 to 1.54, 1.53 to 1.62, the others 1.80 to 1.97, 1.76 to 2.07; gated 1.51 to 2.07, 1.20 to 2.08
+//   K 8192, 128 rows: 1.94 to 3.17
 int64_t by_element_to(int type, int64_t K, int64_t N, bool gated) {
     const int64_t one = weight_bytes_of(type, K, N);
-    const bool large = one >= kLargeWeightBytes;
-    // (matrices of fewer values stay with the two passes, whose results on unit vectors are the weights rounded once: 2048x601 1.04 to 1.5 at 64 rows)
-    if (K * N < ((int64_t)9 << 18)) return kGemvMaxRows;
+    const bool large = one >= kLargeWeightBytes, small = K * N < ((int64_t)9 << 18);  // (2.4 million values: between the small matrices above and 2048x1501)
     if (K < 2048) return type == GQ_Q6_K || one < ((int64_t)3 << 20) ? kGemvMaxRows : 32;
     if (K < 4096) {
         if (type == GQ_Q4_K) return gated ? 96 : 64;
         if (type == GQ_Q6_K) return gated ? kGemvMaxRows : 32;
+        if (small) return gated ? 96 : 128;
         return gated ? 48 : type == GQ_Q8_0 && large ? 32 : 64;
     }
     if (type == GQ_Q4_K) return INT64_MAX;
-    if (K < 8192) return type == GQ_Q6_K ? 64 : !gated && large ? 96 : 128;
+    if (K < 8192) return small ? 128 : type == GQ_Q6_K ? 64 : !gated && large ? 96 : 128;
     return 128;
 }
 // The first row count of such a call on the split-K kernels: up to 16 rows it keeps the GEMV and the few-row kernel, which hold activations in

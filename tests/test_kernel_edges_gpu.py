@@ -123,7 +123,8 @@ def test_gemm_with_weights_converted_in_registers_and_infinite_activations(gpu, 
 def test_gemm_with_weights_converted_in_registers_keeps_infinities(gpu, monkeypatch):
     """A block of infinite scale in one weight row: that output column is infinite or NaN as the reference's, every other one untouched."""
     torch = gpu
-    K, N, M = 512, 63, 40  # (an N that the split-K kernels do not take)
+    K, N, M = 512, 63, 40
+    monkeypatch.setenv("GOMLX_HIPQ_SPLIT_K_TO", "16")
     for t in GEMM_TYPES:
         W = synth.weights(t, 3, N, K)
         W[5, 0:2] = np.frombuffer(np.float16(np.inf).tobytes(), np.uint8)
@@ -175,6 +176,20 @@ def test_split_k_rows_of_any_length(gpu, t, M, K, N):
     xb = xd.to(torch.bfloat16)
     want = oracle.c_qdense(t, xb.float().cpu().numpy(), W, bias, oracle.ACT_NONE)
     assert rel(nn.quantized_dense(xb, wd, q, dev(torch, bias)).cpu().numpy(), want) < TOL_F32
+
+
+@pytest.mark.parametrize("t", GEMM_TYPES + [ggml.Q6_K])
+@pytest.mark.parametrize("K,N", [(2048, 131), (2048, 1150), (4608, 509)])
+def test_small_matrices_with_rows_of_any_length_keep_their_weights_exact(gpu, t, K, N):
+    """Less than 2.4 million values with N off every multiple of four: unit vectors return the weights themselves, which the split-K kernels
+    contract as they are (a 16-bit image would round them)."""
+    W = np.tile(synth.weights(t, 77 + t, 67, K), (-(-N // 67), 1))[:N]
+    cols = np.linspace(0, K - 1, 20).astype(int)
+    x = np.zeros((20, K), np.float32)
+    x[np.arange(20), cols] = 1.0
+    got = nn.quantized_dense(dev(gpu, x), dev(gpu, W), Quantization(ggml_type=t)).cpu().numpy()
+    want = np.tile(oracle.c_dequantize(t, W[:67], K), (-(-N // 67), 1))[:N, cols].T
+    assert np.array_equal(got, want)
 
 
 def off16(torch, a):

@@ -503,10 +503,10 @@ def test_infinite_activations_of_a_few_rows(gpu, oracle, t, M, K, N, bf16):
 @pytest.mark.parametrize("t", ALL_TYPES)
 @pytest.mark.parametrize("K,N", [(96, 131), (32, 2051), (2080, 67), (768, 1), (4352, 515)])
 @pytest.mark.parametrize("bf16", [False, True])
-def test_weight_image_of_the_two_pass_gemm_is_exact(gpu, oracle, t, K, N, bf16):
+def test_weight_image_of_the_two_pass_gemm_is_exact(gpu, oracle, monkeypatch, t, K, N, bf16):
     """Unit vectors through the two-pass GEMM return the columns of its 16-bit weight image: the exact values, rounded once.  Rows shorter
-    than a workgroup's 1024 octets and longer, last workgroups that are partly filled, K padded to the GEMM's step of 64 (N % 4 != 0 keeps
-    the split-K kernels away)."""
+    than a workgroup's 1024 octets and longer, last workgroups that are partly filled, K padded to the GEMM's step of 64."""
+    monkeypatch.setenv("GOMLX_HIPQ_SPLIT_K_TO", "16")
     K = -(-K // ggml.values_per_block(t)) * ggml.values_per_block(t)
     if bf16:
         K = -(-K // 64) * 64   # (other K go to the fused kernel)
