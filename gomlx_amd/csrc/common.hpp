@@ -96,7 +96,7 @@ bool mmq_set_supported(int type, int count, const MmqSetItem *items, int64_t M, 
 int launch_mmq_set(int type, const void *x, bool x_is_bf16, int64_t M, int64_t K, int count, const MmqSetItem *items, const RmsNorm *norm,
                    hipStream_t s);
 // 3 to 16 activation rows in one launch on the matrix cores (mmv.hip); more than 4096 values of K take a second launch, workspace
-// (sums of slices).
+// (sums of slices) and N % 4 == 0.
 bool mmv_supported(int type, int64_t M, int64_t K, int64_t N, const void *x, const void *gain);
 bool mmv_one_launch(int64_t K);
 // xs: every matrix with activations of its own (two to four of them, K in one launch, no extras).

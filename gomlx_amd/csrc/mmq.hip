@@ -40,7 +40,7 @@ typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef float f16v __attribute__((ext_vector_type(16)));
 
-constexpr int kSliceSB = 8;                 // super-blocks a slice's activation image has room for (a slice uses up to 7)
+constexpr int kSliceSB = 8;                 // super-blocks a slice's activation image has room for (mmq_q4k_kernel uses up to 7, mmq_q4k_tiles_kernel up to 8)
 constexpr int kSliceK = kSliceSB * 256;     // 2048 values
 constexpr int kParts = 2;                   // wavefronts sharing a row tile of 32 (interleaved super-blocks)
 constexpr int kMT = 32;                     // batch columns per pass
@@ -1356,7 +1356,7 @@ __global__ __launch_bounds__(RT * 128) void mmq_b32_kernel(const uint8_t *__rest
 // each, weight tiles parked in LDS by DMA two stretches ahead, the images of up to four tiles of 32 batch rows staged half
 // a stretch (four blocks) at a time through a ring of two stages with counted waits - and only the arithmetic differs:
 // per block two MFMAs per tile against fragments converted ONCE for all tiles, and the block's d applied to each tile's
-// sums in fp32.  Slices are S consecutive values (512 or 1024), the image is mmq_b32_xprep_kernel's.
+// sums in fp32.  Slices are S consecutive values (512, 1024, 1536 or 2048), the image is mmq_b32_xprep_kernel's.
 int tiles_together_mode();
 
 template <int NT> struct B32TilesOf {  // LDS: [ring: 2 stages x NT halves of 8 KiB][two parked stretches per wavefront]

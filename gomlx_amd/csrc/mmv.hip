@@ -810,7 +810,8 @@ bool mmv_supported(int type, int64_t M, int64_t K, int64_t N, const void *x, con
 }
 
 // The same activations against `count` matrices (one with W2, bias2: a gated pair; a residual goes with one matrix only).  K of
-// more than eight slices needs workspace.  xs: activations of their own for every matrix (two or more of up to eight slices, no extras).
+// more than eight slices needs workspace and, for the reduction, N % 4 == 0 (the dispatch sends other N here in one launch only).  xs: activations of
+// their own for every matrix (two or more of up to eight slices, no extras).
 int launch_mmv(int type, const void *x, bool x_is_bf16, int64_t M, int64_t K, int count, const MmqSetItem *items, const MmqExtra *ex, hipStream_t s,
                const void *const *xs) {
     if (count < 1 || count > kMaxProblems) return fail(GQ_ERR_NOT_IMPLEMENTED, "mmv: a set of %d matrices is not implemented", count);
@@ -824,7 +825,8 @@ int launch_mmv(int type, const void *x, bool x_is_bf16, int64_t M, int64_t K, in
         a.W[i] = items[i].W; a.bias[i] = items[i].bias; a.y[i] = items[i].y; a.N[i] = (int)items[i].N; a.act[i] = items[i].act;
         a.tile0[i] = (int)tiles; a.n0[i] = (int)ntot;
         tiles += (items[i].N + 15) / 16;
-        ntot += (items[i].N + 3) & ~(int64_t)3;  // (rows of sums of whole float4: launch_split_k_finish)
+        ntot += items[i].N;  // (two launches: the sums' rows are whole float4)
+        if (p.groups > 1 && items[i].N % 4 != 0) return fail(GQ_ERR_NOT_IMPLEMENTED, "mmv: N off 4 in two launches is not implemented");
     }
     if (tiles > INT32_MAX / 64 || ntot > INT32_MAX) return fail(GQ_ERR_NOT_IMPLEMENTED, "mmv: too many weight rows");
     a.count = count; a.ntiles = (int)tiles; a.M = (int)M; a.K = (int)K; a.nslices = p.nslices; a.ntot = (int)ntot;
