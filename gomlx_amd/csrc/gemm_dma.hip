@@ -948,7 +948,8 @@ namespace {
 // (the others 3 to 5 % behind).  E.g. (us, two passes | this): gated pair of 4096x14336 in Q4_K at 384, 512, 768 and 2048 rows 163 165 251 481 | 95 119 188 451;
 // 14336x4096 at 256, 384 and 512 rows 78 97 101 | 52 67 83; Q8_0: the pair 172 174 259 492 | 110 134 222 516 (not taken), 14336x4096 82 100 103 | 62 75 93; at
 // 4096x4096 and 512 rows, Q4_K 36 | 38 (not taken).  Few rows of less than 4096 values lie where neither estimate is good to 8 %: pair of 2048x12001 at 128 (Q4_K) and
-// 192 rows (Q8_0) 46 56 | 54 66 (not taken).
+// 192 rows (Q8_0) 46 56 | 54 66 (not taken).  A gated pair (two products' sums in the epilogue) and rows that are not whole float4 cost 4 us more per
+// round: of 445 further problems over the whole range, half of them with N off 4, 254 are taken, 6 of those 3 to 9 % behind the two passes.
 // GOMLX_HIPQ_GEMM_WREG=0 keeps every call on the two passes, =tm or =tm,slices (tm 4, 6 or 8) forces this way wherever it applies (tuning runs
 // and tests; read at every call).
 constexpr int64_t kWregValues = (int64_t)1 << 25;
@@ -977,7 +978,8 @@ WregPlan plan_wreg(int type, bool bf16, int64_t M, int64_t K, int64_t tiles, int
             if ((ns - 1) * per >= units || (env.slices > 0 && ns > 1 && ns != env.slices)) continue;
             const int64_t wgs = tiles * ((M + 32 * kTm[t] - 1) / (32 * kTm[t])) * ns, full = wgs / cus;
             const double frac = (double)(wgs % cus) / (double)cus;
-            double us = ((double)full + (frac > 0 ? 0.77 + 0.23 * frac : 0)) * ((double)(4 * per) * kStep[row][t] + kFixed[t]);
+            const double fixed = kFixed[t] + (gated ? 4.0 : 0.0) + (cols % 4 != 0 ? 4.0 : 0.0);
+            double us = ((double)full + (frac > 0 ? 0.77 + 0.23 * frac : 0)) * ((double)(4 * per) * kStep[row][t] + fixed);
             if (ns > 1) us += 3.4 + (double)(2 * ns + 1) * (double)M * (double)cols * 4.0 / 15.4e6;
             if (us < best_us || (ns > 1 && ns == env.slices)) { best_us = us; best.tm = kTm[t]; best.slices = ns; }
         }

@@ -425,21 +425,18 @@ __global__ __launch_bounds__(256, 1) void gemm_wreg_kernel(WregArgs a) {
     const float *const R = sliced ? nullptr : a.residual;
     const float *const B0 = sliced ? nullptr : a.bias[prob], *const B1 = GATED ? a.bias[1] : nullptr;
     const int act = sliced ? kActNone : a.act;
-    const bool vec = ((ld | N) & 3) == 0 && ((reinterpret_cast<uintptr_t>(Y) | reinterpret_cast<uintptr_t>(R) | reinterpret_cast<uintptr_t>(B0) |
-                                              reinterpret_cast<uintptr_t>(B1)) & 15) == 0;
     if (threadIdx.x < 32 * TM) {
         const int m = bm + (int)threadIdx.x;
         srow[threadIdx.x] = !sliced && a.rowscale && m < M ? a.rowscale[m] : 1.f;
     }
-    // the biases of a lane's columns: four of either tile (gated: of either matrix), or one
-    float4 bias[2] = {make_float4(0.f, 0.f, 0.f, 0.f), make_float4(0.f, 0.f, 0.f, 0.f)};
+    // the biases of a lane's four columns of either tile (gated: of either matrix)
+    float4 bias[2];
 #pragma unroll
     for (int j = 0; j < 2; j++) {
         const float *const B = GATED && j ? B1 : B0;
-        const int n = row0 + (GATED ? 0 : 32 * j) + (vec ? 4 * (lane & 7) : col);
-        if (!B || n >= N) continue;
-        if (vec) bias[j] = *reinterpret_cast<const float4 *>(B + n);
-        else bias[j].x = B[n];
+        const int n = row0 + (GATED ? 0 : 32 * j) + 4 * (lane & 7);
+        auto at = [&](int c) __attribute__((always_inline)) { return B && n + c < N ? B[n + c] : 0.f; };
+        bias[j] = make_float4(at(0), at(1), at(2), at(3));
     }
     __syncthreads();
     auto finish = [&](float v0, float v1, float s, float b, float b1, auto activate) __attribute__((always_inline)) {
@@ -447,12 +444,13 @@ __global__ __launch_bounds__(256, 1) void gemm_wreg_kernel(WregArgs a) {
         else return activate(fmaf(v0, s, b));
     };
     const int lr = 4 * ((lane >> 3) & 1) + (lane >> 4);  // a lane's row of eight
-    // pass p, tile j, four columns a lane
+    // pass p, tile j, four columns a lane.  Rows and pointers need not be whole float4: these instructions ask for whole dwords (an element at a time, behind
+    // a branch for its row and a switch for the activation, took 33 us of a 256 x 256 tile and 80 with a residual).
     auto store_vec = [&](int p, int j, auto activate) __attribute__((always_inline)) {
         const int n = row0 + 32 * j + 4 * (lane & 7);
         const float *const src = xch + j * (TH * 1024) + 4 * lane;
         const float4 b0 = j ? bias[1] : bias[0], b1 = bias[1];
-        if (n >= N) return;
+        if (n + 4 > N) return;
         // (buffer stores and loads: what lies past the last row is dropped resp. zero, so that no branch stands between one row's LDS reads and the next's)
         const uint64_t tail = (uint64_t)(M - bm) * (uint64_t)ld * 4;
         const uint32_t bytes = tail > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)tail;
@@ -493,6 +491,40 @@ __global__ __launch_bounds__(256, 1) void gemm_wreg_kernel(WregArgs a) {
             }
         }
     };
+    // the one to three columns in front of N that are no whole four: finished where they lie, one row after the other, then stored element by element
+    auto store_tail = [&](int p, int j) __attribute__((always_inline)) {
+        const int n = row0 + 32 * j + 4 * (lane & 7);
+        float *const src = xch + j * (TH * 1024) + 4 * lane;
+        const float4 b0 = j ? bias[1] : bias[0], b1 = bias[1];
+        if (n >= N || n + 4 <= N) return;
+#pragma unroll 1
+        for (int q = 0; q < 4 * TH; q++) {
+            const float s = srow[32 * TH * p + 8 * q + lr];
+#pragma unroll 1
+            for (int c = 0; c < 3; c++) {
+                const float bc = c == 0 ? b0.x : c == 1 ? b0.y : b0.z, b1c = c == 0 ? b1.x : c == 1 ? b1.y : b1.z;
+                src[256 * q + c] = finish(src[256 * q + c], GATED ? src[TH * 1024 + 256 * q + c] : 0.f, s, bc, b1c, [act](float v) { return apply_act(act, v); });
+            }
+        }
+        const int64_t at = (int64_t)(bm + 32 * TH * p + lr) * ld + n;
+        constexpr int D = TH == 3 ? 6 : 8;
+#pragma unroll 1
+        for (int q = 0; q < 4 * TH; q += D) {
+            float r[D][3];
+#pragma unroll
+            for (int i = 0; i < D; i++)
+#pragma unroll
+                for (int c = 0; c < 3; c++) {
+                    r[i][c] = src[256 * (q + i) + c];
+                    if (R && n + c < N && bm + 32 * TH * p + lr + 8 * (q + i) < M) r[i][c] += R[at + (int64_t)(8 * (q + i)) * ld + c];
+                }
+#pragma unroll
+            for (int i = 0; i < D; i++)
+#pragma unroll
+                for (int c = 0; c < 3; c++)
+                    if (n + c < N && bm + 32 * TH * p + lr + 8 * (q + i) < M) Y[at + (int64_t)(8 * (q + i)) * ld + c] = r[i][c];
+        }
+    };
 #pragma unroll
     for (int p = 0; p < 2; p++) {
         const int mp = bm + 32 * TH * p;
@@ -508,23 +540,10 @@ __global__ __launch_bounds__(256, 1) void gemm_wreg_kernel(WregArgs a) {
         asm volatile("" ::: "memory");
 #pragma unroll 1
         for (int j = 0; j < (GATED ? 1 : 2); j++) {
-            if (vec) {
-                if (act == kActNone) store_vec(p, j, [](float v) { return v; });
-                else if (act == kActSilu) store_vec(p, j, [](float v) { return v / (1.0f + __expf(-v)); });
-                else store_vec(p, j, [act](float v) { return apply_act(act, v); });
-            } else {
-                const int n = row0 + 32 * j + col;
-                const float *const src = xch + j * (TH * 1024) + lane;
-                const float b0 = j ? bias[1].x : bias[0].x;
-#pragma unroll 1
-                for (int q = 0; q < 16 * TH; q++) {
-                    const int m = mp + 8 * (q >> 2) + 4 * h + (q & 3);
-                    float v = finish(src[64 * q], GATED ? src[TH * 1024 + 64 * q] : 0.f, srow[m - bm], b0, bias[1].x, [act](float v) { return apply_act(act, v); });
-                    if (n >= N || m >= M) continue;
-                    if (R) v += R[(int64_t)m * ld + n];
-                    Y[(int64_t)m * ld + n] = v;
-                }
-            }
+            if (act == kActNone) store_vec(p, j, [](float v) { return v; });
+            else if (act == kActSilu) store_vec(p, j, [](float v) { return v / (1.0f + __expf(-v)); });
+            else store_vec(p, j, [act](float v) { return apply_act(act, v); });
+            if (N & 3) store_tail(p, j);
         }
     }
 #undef GQ_PUBLISH

@@ -51,6 +51,8 @@ GEMM_TYPES = [ggml.Q4_K, ggml.Q8_0, ggml.Q4_0, ggml.IQ4_NL]
     (6, 1, 193, 1280, 36),     # one row over, N inside the first wavefront's tiles
     (8, 2, 255, 1280, 516),    # one row short, uneven slices
     (8, 1, 288, 512, 320),     # a whole tile and a whole 32-row part of the second
+    (4, 1, 130, 512, 259),     # three columns that are no whole four, in the second workgroup's first wavefront
+    (6, 1, 191, 512, 94),      # two, in the second wavefront
 ])
 def test_gemm_with_weights_converted_in_registers(gpu, monkeypatch, t, tm, slices, M, K, N):
     """Every epilogue of gemm_wreg.hip (plain, bias and activation, residual behind a norm, gated pair, q / k / v of one input) at the edges of
@@ -232,10 +234,11 @@ def test_residual_and_up_bias_off_16_bytes_keep_the_route(gpu, t, M, K, N, bf16)
 @pytest.mark.parametrize("t,M,K,N,wreg", [
     (ggml.Q4_K, 40, 4096, 1024, None), (ggml.Q8_0, 17, 4096, 1028, None), (ggml.Q4_0, 66, 4096, 1024, None), (ggml.Q6_K, 20, 4096, 1024, None),  # split-K
     (ggml.Q8_0, 129, 512, 260, "4,1"), (ggml.Q4_K, 255, 512, 516, "8,1"), (ggml.IQ4_NL, 193, 768, 36, "6,1"),  # the GEMM that converts weights in registers
+    (ggml.Q4_0, 257, 512, 289, "8,1"), (ggml.Q8_0, 190, 512, 34, "6,1"), (ggml.Q4_K, 129, 512, 3, "4,1"),
 ])
 def test_outputs_off_16_bytes(gpu, monkeypatch, t, M, K, N, wreg):
-    """N a multiple of four and y off 16 bytes: stored element by element, the same bits as float4 - plain, a residual stream updated in place, a gated
-    pair - and no element outside y."""
+    """y off 16 bytes, N a multiple of four and not: the same bits as at an aligned address - plain, a residual stream updated in place, a gated pair - and
+    no element outside y."""
     torch = gpu
     if wreg:
         monkeypatch.setenv("GOMLX_HIPQ_GEMM_WREG", wreg)
