@@ -122,6 +122,12 @@ __device__ __forceinline__ float wave_sum(float v) {
     return v;
 }
 
+// An octet of a column's slice that holds exactly one infinity (see stage_x; a NaN stays).
+__device__ __forceinline__ float4 lone_infinity(const float4 &v) {
+    auto of = [](float x) __attribute__((always_inline)) { return fabsf(x) == INFINITY ? copysignf(1.f, x) : x * 0.f; };
+    return make_float4(of(v.x), of(v.y), of(v.z), of(v.w));
+}
+
 // ---- stage the K-slice of x into LDS in MFMA fragment order ---------------------------------
 //
 // One item = 8 consecutive activations of one batch column ("octet").  Inside a super-block the
@@ -134,6 +140,9 @@ __device__ __forceinline__ float wave_sum(float v) {
 // columns a half-wave later reads from one slot) over all LDS banks.
 // The eight sub-block sums of (sbl, m) are stored in the order (0, 2, 1, 3, 4, 6, 5, 7) too.
 // `active`: the thread's octet belongs to the slice (slices may hold fewer than 8 super-blocks).
+// An infinity would meet a code of zero, and the minima's sum its opposite: NaN whatever the weight.  Where a column's slice holds one, it goes
+// to the image as 1 or -1, the slice's finite values as zeros, and the inverse scale is infinite: the product is the weight's
+// sign times infinity, NaN for a weight of zero, as in the reference's arithmetic.  Several in one slice make NaN.
 // red: [2][2][ROUNDS][4] floats of shared memory; inv_scale[m] receives the slice's inverse scale of column m0 + m.
 // With xss (normalisation folded in): x is multiplied by gain + gain_offset (gain may be null) and xss[m0 + m] receives
 // the slice's sum of squares of the raw x.
@@ -174,15 +183,41 @@ __device__ __forceinline__ void stage_x(const void *__restrict__ X, int M, int K
         if ((tid & 63) == 0) red[(half * ROUNDS + r) * 4 + wih] = am;
     }
     __syncthreads();
+    float sc[ROUNDS], inv[ROUNDS], top = 0.f;
 #pragma unroll
     for (int r = 0; r < ROUNDS; r++) {
-        const int m = (tid >> 8) + 2 * (round0 + r);
-        const bool ok = k_ok && (m0 + m < M);
         const float *rr = red + (half * ROUNDS + r) * 4;
-        float sc, inv;
-        pow2_scale(fmaxf(fmaxf(rr[0], rr[1]), fmaxf(rr[2], rr[3])), sc, inv);
+        const float t = fmaxf(fmaxf(rr[0], rr[1]), fmaxf(rr[2], rr[3]));
+        pow2_scale(t, sc[r], inv[r]);
+        top = fmaxf(top, t);
+    }
+    if (__builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, top)) == 0x7F800000) {  // (a wavefront's threads look at the same columns)
+#pragma unroll
+        for (int r = 0; r < ROUNDS; r++) {
+            int infinities = 0;  // counted over the whole slice by each of its wavefronts: nothing is added to the ordinary case
+            for (int o = tid & 63; o < 256; o += 64) {
+                const int ko = ((o >> 5) * sb_stride + sb_first) * 256 + 8 * (o & 31);
+                float4 v = make_float4(0.f, 0.f, 0.f, 0.f), w = v;
+                if (ko < K) {
+                    load_x8<BF16X>(X, (int64_t)min(m0 + half + 2 * (round0 + r), M - 1) * K + ko, v, w);
+                    if (xss && gain) apply_gain8(gain, gain_offset, ko, v, w);
+                }
+                const float e[8] = {v.x, v.y, v.z, v.w, w.x, w.y, w.z, w.w};
+                for (int i = 0; i < 8; i++) infinities += (int)__popcll(__ballot(fabsf(e[i]) == INFINITY));
+            }
+            if (infinities == 1) {
+                lo[r] = lone_infinity(lo[r]);
+                hi[r] = lone_infinity(hi[r]);
+                inv[r] = INFINITY;
+            }
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < ROUNDS; r++) {
+        const int m = half + 2 * (round0 + r);
+        const bool ok = k_ok && (m0 + m < M);
         if (oct == 0 && m0 + m < M) {
-            inv_scale[m0 + m] = inv;
+            inv_scale[m0 + m] = inv[r];
             if (xss) {
                 const float *rs = red_ss + (half * ROUNDS + r) * 4;
                 xss[m0 + m] = (rs[0] + rs[1]) + (rs[2] + rs[3]);
@@ -191,7 +226,7 @@ __device__ __forceinline__ void stage_x(const void *__restrict__ X, int M, int K
         if (!active) continue;
         const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
         float4 a = ok ? lo[r] : z, b = ok ? hi[r] : z;
-        a.x *= sc; a.y *= sc; a.z *= sc; a.w *= sc; b.x *= sc; b.y *= sc; b.z *= sc; b.w *= sc;
+        a.x *= sc[r]; a.y *= sc[r]; a.z *= sc[r]; a.w *= sc[r]; b.x *= sc[r]; b.y *= sc[r]; b.z *= sc[r]; b.w *= sc[r];
         uint4 o;  // bytes (0,2,1,3,4,6,5,7)
         o.x = pack_h2(a.x, a.z);
         o.y = pack_h2(a.y, a.w);
